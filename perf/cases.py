@@ -241,7 +241,9 @@ def _network(widths, seed):
     w = _ints(widths)
     layers = []
     for a, b in zip(w, w[1:]):
-        layers += [nn.Linear(a, b, device=DEVICE), nn.ReLU()]
+        # (a smooth activation: with ReLU a rounding error now and then decides whether a unit is
+        # on, and two correct implementations differ by that unit's whole gradient)
+        layers += [nn.Linear(a, b, device=DEVICE), nn.Tanh()]
     return nn.Sequential(*layers[:-1])
 
 
@@ -256,8 +258,12 @@ def _prepare_network(case, seed):
         opt = torchsso.optim.SecondOrderOptimizer(model, 'Cov', {'Linear': 'Kron'}, kron, lr=1e-3,
                                                   momentum=0.9, weight_decay=case['weight_decay'])
     elif case['kind'] == 'noisy':
+        # (a KL weight under which the samples stay close to the mean: with samples that swamp
+        # the network, rounding errors grow a hundredfold per step, and two correct
+        # implementations part after three steps)
         opt = torchsso.optim.VIOptimizer(model, 50000, 'Cov', {'Linear': 'Kron'}, kron, lr=1e-3,
-                                         momentum=0.9, num_mc_samples=case['samples'], seed=1)
+                                         momentum=0.9, num_mc_samples=case['samples'],
+                                         kl_weighting=1e-3, seed=1)
     else:
         opt = torchsso.optim.VOGN(model, dataset_size=50000, num_mc_samples=case['samples'],
                                   warmup_kl_weighting_steps=None,
