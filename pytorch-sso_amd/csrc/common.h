@@ -16,7 +16,7 @@ bool enable_large_lds(const void* kernel, int bytes);
 
 #define KFAC_LAUNCH_TILE2(kernel, grid, stream, ...)                                         \
   do {                                                                                       \
-    constexpr int lds_bytes_ = kfac::Cfg<2, 2>::SMEM_FLOATS * (int)sizeof(float);            \
+    constexpr int lds_bytes_ = kfac::SplitCfg<2, 2>::SMEM_BYTES;                           \
     if (kfac::enable_large_lds((const void*)(kernel), lds_bytes_))                           \
       hipLaunchKernelGGL((kernel), (grid), dim3(kfac::NTHREADS), lds_bytes_, (stream),       \
                          __VA_ARGS__);                                                       \

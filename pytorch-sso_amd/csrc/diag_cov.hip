@@ -34,7 +34,7 @@ struct EpiWeightBias {
   }
 };
 
-__global__ __launch_bounds__(NTHREADS, 3) void diag_linear_kernel(const float* g, const float* a,
+__global__ __launch_bounds__(NTHREADS, 2) void diag_linear_kernel(const float* g, const float* a,
                                                                   int n, int fout, int fin,
                                                                   int add_bias, float alpha,
                                                                   float* W, float* bvec) {
@@ -43,7 +43,7 @@ __global__ __launch_bounds__(NTHREADS, 3) void diag_linear_kernel(const float* g
   SqDenseKM P{{g, nullptr, fout, fout, 0}};
   SqDenseKM Q{{a, nullptr, fin, N, add_bias ? 1 : 0}};
   EpiWeightBias epi{W, bvec, fout, N, fin, alpha};
-  gemm_tile(P, Q, blockIdx.y * BM, blockIdx.x * BN, 0, n, false, epi, smem);
+  split_tile(P, Q, blockIdx.y * BM, blockIdx.x * BN, 0, n, false, epi, smem);
 }
 
 // sum of squares of the accumulators over the calls of the tile engine

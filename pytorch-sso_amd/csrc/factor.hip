@@ -124,7 +124,7 @@ static SyrkPlan plan_syrk(int d, long K) {
 }
 
 template <class OP, int W>
-__global__ __launch_bounds__(64 * W * W, W == 2 ? 3 : 1) void syrk_kernel(OP op, int d, int K, int T, int ntiles,
+__global__ __launch_bounds__(64 * W * W, W == 2 ? 2 : 1) void syrk_kernel(OP op, int d, int K, int T, int ntiles,
                                                           int splits, int chunks_per_split,
                                                           float* C, const float* Cin,
                                                           float alpha, float beta, float* ws) {
@@ -141,13 +141,9 @@ __global__ __launch_bounds__(64 * W * W, W == 2 ? 3 : 1) void syrk_kernel(OP op,
   const int kbeg = split * chunks_per_split * KC;
   int kend = kbeg + chunks_per_split * KC;
   if (kend > K) kend = K;
-  if (splits == 1) {
-    EpiStore epi{C, d, d, d, alpha, beta, bi != bj, Cin};
-    gemm_tile_cfg<W, W, true>(op, op, bi * TS, bj * TS, kbeg, kend, bi == bj, epi, smem);
-  } else {
-    EpiPartial epi{ws + ((size_t)split * ntiles + tile) * (TS * TS), bi * TS, bj * TS, d, d, TS};
-    gemm_tile_cfg<W, W, true>(op, op, bi * TS, bj * TS, kbeg, kend, bi == bj, epi, smem);
-  }
+  const EpiStore whole{C, d, d, d, alpha, beta, bi != bj, Cin};
+  const EpiPartial part{ws + ((size_t)split * ntiles + tile) * (TS * TS), bi * TS, bj * TS, d, d, TS};
+  syrk_tile<W>(op, bi, bj, kbeg, kend, splits == 1, whole, part, smem);
 }
 
 template <int TS>
@@ -172,7 +168,7 @@ static void launch_syrk_cfg(const OP& op, const SyrkPlan& p, int d, int64_t K, f
                             float beta, const float* Cin, float* C, void* workspace,
                             hipStream_t stream) {
   constexpr int TS = 64 * W;
-  constexpr int lds_bytes = Cfg<W, W>::SMEM_FLOATS * (int)sizeof(float);
+  constexpr int lds_bytes = syrk_lds_bytes<W>();
   if (!enable_large_lds((const void*)syrk_kernel<OP, W>, lds_bytes)) return;
   hipLaunchKernelGGL((syrk_kernel<OP, W>), dim3(p.ntiles, p.splits), dim3(64 * W * W), lds_bytes,
                      stream, op, d, (int)K, p.T, p.ntiles, p.splits, p.cps, C, Cin, alpha, beta,

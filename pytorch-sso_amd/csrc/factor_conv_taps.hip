@@ -36,6 +36,7 @@ namespace kfac {
 // x[n][c][u0 + ry + dy][v0 + rx + dx] for k = (n, ry, rx) inside a hh x ww rectangle
 struct ShiftX {
   static constexpr int layout = MK;
+  static constexpr int kruns = K_RUNS;
   static constexpr bool has_second = false;
   const float* p;
   int C, H, W, u0, v0, hh, ww;     // u0, v0 already include the displacement
@@ -55,6 +56,18 @@ struct ShiftX {
   }
   __device__ __forceinline__ unsigned off(const MS& m, const KS& k) const { return m.off + k.off; }
   __device__ __forceinline__ bool is_one(const MS&) const { return false; }
+  // the positions of a row of the rectangle are consecutive
+  __device__ __forceinline__ bool runs() const { return ww >= 4; }
+  __device__ __forceinline__ bool quads() const { return (ww & 3) == 0; }
+  __device__ __forceinline__ KRun run(int k) const {
+    const int n = by_area.div(k);
+    const int rem = k - n * hh * ww;
+    const int ry = by_ww.div(rem);
+    const int rx = rem - ry * ww;
+    const int row = n * C * H * W + (u0 + ry) * W + v0;
+    const int next = ry + 1 < hh ? row + W : (n + 1) * C * H * W + u0 * W + v0;
+    return KRun{(unsigned)(row + rx) * 4u, (unsigned)next * 4u, ww - rx};
+  }
 };
 
 struct JobDesc {
@@ -107,7 +120,10 @@ __device__ __forceinline__ void corr_product(const float* x, int nimg, int C, in
   ShiftX P{x, C, H, Wd, jd.u0, jd.v0, jd.hh, jd.ww, by_area, by_ww};
   ShiftX Q{x, C, H, Wd, jd.u0 + jd.dy, jd.v0 + jd.dx, jd.hh, jd.ww, by_area, by_ww};
   EpiStore epi{ws + (size_t)(jd.part0 + split) * C * C, C, C, C, 1.f, 0.f, false};
-  gemm_tile_cfg<W, W>(P, Q, bi * TS, bj * TS, kbeg, kend, false, epi, smem);
+  if constexpr (W == 2)
+    split_tile(P, Q, bi * TS, bj * TS, kbeg, kend, false, epi, smem);
+  else
+    gemm_tile_cfg<W, W>(P, Q, bi * TS, bj * TS, kbeg, kend, false, epi, smem);
 }
 
 // work item `item` of one layer's plan -> (job, split, tile), job by job
@@ -125,7 +141,7 @@ __device__ __forceinline__ void corr_item(const float* x, int nimg, int C, int H
 }
 
 template <int W>
-__global__ __launch_bounds__(64 * W * W, W == 2 ? 3 : 1) void corr_kernel(
+__global__ __launch_bounds__(64 * W * W, W == 2 ? 2 : 1) void corr_kernel(
     const float* x, int nimg, int C, int H, int Wd, const TapPlanDev plan, int tiles_side,
     float* ws) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
@@ -171,7 +187,7 @@ __device__ __forceinline__ int find_layer(const int* __restrict__ cum, int n, in
 
 // the correlation items of all layers of one tile size in one launch
 template <int W>
-__global__ __launch_bounds__(64 * W * W, W == 2 ? 3 : 1) void corr_grouped_kernel(
+__global__ __launch_bounds__(64 * W * W, W == 2 ? 2 : 1) void corr_grouped_kernel(
     const TapLayer* __restrict__ layers, const TapPlanDev* __restrict__ plans,
     const TapOrder* __restrict__ order, const unsigned* __restrict__ entries,
     const int* __restrict__ index, const int* __restrict__ cum, int nlayers) {
@@ -294,7 +310,10 @@ __device__ __forceinline__ void interleave_item(const TapPlanDev& plan, const fl
   const size_t CC = (size_t)C * C;
   const int tid = threadIdx.x;
   for (int t2 = 0; t2 < T; ++t2) {
-    if (t <= t2) {
+    // the block of a tap with itself is symmetric up to the rounding of its products: its
+    // upper triangle stands for both
+    const bool mixed = t == t2 && c0 < q0 + IL_COLS && q0 < c0 + IL_ROWS;
+    if (t < t2 || mixed || (t == t2 && c0 < q0)) {
       // B[(t,t2)][c][c2]: lanes along c2
       const float* blk = B + plan.pair_of[t * T + t2] * CC;
       const int j = tid % IL_COLS;
@@ -302,7 +321,8 @@ __device__ __forceinline__ void interleave_item(const TapPlanDev& plan, const fl
       for (int k = 0; k < IL_ROWS * IL_COLS / 256; ++k) {
         const int i = tid / IL_COLS + (256 / IL_COLS) * k;
         const int c = c0 + i, c2 = q0 + j;
-        out[i][j * T + t2] = (c < C && c2 < C) ? blk[(size_t)c * C + c2] : 0.f;
+        const bool flip = mixed && c > c2;
+        out[i][j * T + t2] = (c < C && c2 < C) ? blk[flip ? (size_t)c2 * C + c : (size_t)c * C + c2] : 0.f;
       }
     } else {
       // transposed block B[(t2,t)][c2][c]: lanes along c
@@ -557,7 +577,7 @@ int conv_a_taps(const float* x, int n, int c, int H, int W, int kh, int kw, int 
     hipLaunchKernelGGL(corr_kernel<1>, dim3(hp.items), dim3(64), lds, stream, x, n, c, H, W,
                        hp.dev, hp.tiles_side, ws);
   } else {
-    constexpr int lds = Cfg<2, 2>::SMEM_FLOATS * (int)sizeof(float);
+    constexpr int lds = SplitCfg<2, 2>::SMEM_BYTES;
     if (!enable_large_lds((const void*)corr_kernel<2>, lds)) return KFAC_ERR_LAUNCH;
     hipLaunchKernelGGL(corr_kernel<2>, dim3(hp.items), dim3(256), lds, stream, x, n, c, H, W,
                        hp.dev, hp.tiles_side, ws);
@@ -781,7 +801,7 @@ int conv_a_taps_grouped(int count, const TapsJob* jobs, void* workspace, size_t 
   const TapOrder* dord = (const TapOrder*)(table + gp.orders_off);
   const unsigned* dent = (const unsigned*)(table + gp.entries_off);
   if (!gp.members[1].empty()) {
-    constexpr int lds = Cfg<2, 2>::SMEM_FLOATS * (int)sizeof(float);
+    constexpr int lds = SplitCfg<2, 2>::SMEM_BYTES;
     if (!enable_large_lds((const void*)corr_grouped_kernel<2>, lds)) return KFAC_ERR_LAUNCH;
     hipLaunchKernelGGL(corr_grouped_kernel<2>, dim3(gp.cum_corr[1].back()), dim3(256), lds, stream,
                        dl, dp, dord, dent, (const int*)(table + gp.index_off[1]),

@@ -66,7 +66,7 @@ __device__ __forceinline__ int find_job(const int* __restrict__ cum, int njobs, 
 }
 
 template <class OP, int W>
-__global__ __launch_bounds__(64 * W * W, W == 2 ? 3 : 1) void syrk_grouped_kernel(
+__global__ __launch_bounds__(64 * W * W, W == 2 ? 2 : 1) void syrk_grouped_kernel(
     const SyJob<OP>* __restrict__ jobs, const int* __restrict__ cum, int njobs) {
   constexpr int TS = 64 * W;
   constexpr int KC = Cfg<W, W>::KC;
@@ -86,13 +86,9 @@ __global__ __launch_bounds__(64 * W * W, W == 2 ? 3 : 1) void syrk_grouped_kerne
   int kend = kbeg + jb.cps * KC;
   if (kend > K) kend = K;
   const OP op = jb.op;
-  if (splits == 1) {
-    EpiStore epi{jb.C, d, d, d, jb.alpha, jb.beta, bi != bj, jb.Cin};
-    gemm_tile_cfg<W, W, true>(op, op, bi * TS, bj * TS, kbeg, kend, bi == bj, epi, smem);
-  } else {
-    EpiPartial epi{jb.ws + ((size_t)split * ntiles + tile) * (TS * TS), bi * TS, bj * TS, d, d, TS};
-    gemm_tile_cfg<W, W, true>(op, op, bi * TS, bj * TS, kbeg, kend, bi == bj, epi, smem);
-  }
+  const EpiStore whole{jb.C, d, d, d, jb.alpha, jb.beta, bi != bj, jb.Cin};
+  const EpiPartial part{jb.ws + ((size_t)split * ntiles + tile) * (TS * TS), bi * TS, bj * TS, d, d, TS};
+  syrk_tile<W>(op, bi, bj, kbeg, kend, splits == 1, whole, part, smem);
 }
 
 // many splits: item = (tile, row of the tile, 64-wide segment)
@@ -645,7 +641,7 @@ static Launch fill_planes(TableWriter& tw, const GroupedPlan& gp, const kfac_fac
 template <class OP, int W>
 static bool launch_syrk_group(const Launch& l, char* table, hipStream_t stream) {
   if (l.njobs == 0) return true;
-  constexpr int lds_bytes = Cfg<W, W>::SMEM_FLOATS * (int)sizeof(float);
+  constexpr int lds_bytes = syrk_lds_bytes<W>();
   if (!enable_large_lds((const void*)syrk_grouped_kernel<OP, W>, lds_bytes)) return false;
   hipLaunchKernelGGL((syrk_grouped_kernel<OP, W>), dim3(l.items), dim3(64 * W * W), lds_bytes,
                      stream, (const SyJob<OP>*)(table + l.jobs_off),

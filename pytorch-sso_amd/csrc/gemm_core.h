@@ -46,7 +46,7 @@ struct Cfg {
   static constexpr int TM = 64 * WM;
   static constexpr int TN = 64 * WN;
   static constexpr int NT = 64 * WM * WN;
-  static constexpr int KC = 16;
+  static constexpr int KC = 16;                  // (that of SplitCfg too)
   static constexpr int LDS_MK = KC + 4;          // padded row of an MK chunk (conflict-free b128)
   static constexpr int P_FLOATS = LDS_MK * TM;   // >= KC*TM and TM*LDS_MK
   static constexpr int Q_FLOATS = LDS_MK * TN;
@@ -425,52 +425,10 @@ __device__ __forceinline__ void gemm_tile_loop(const OPP& P, const OPQ& Q, int m
 
 }
 
-template <int WM, int WN, bool SAME, bool SKIP, class OPP, class OPQ, class EPI>
-__device__ __forceinline__ void gemm_tile_impl(const OPP& P, const OPQ& Q, int m0, int n0,
-                                               int kbeg, int kend, EPI& epi, float* smem) {
-  typedef Cfg<WM, WN> C;
-  constexpr bool same = SAME;
-  const int t = threadIdx.x & (C::NT - 1);
-  const int lane = t & 63;
-  const int wave = t >> 6;
-  const int r = lane & 31;
-  const int h = lane >> 5;
-  int wm = (wave / WN) * 64;
-  int wn = (wave % WN) * 64;
-  static_assert(SAME || !SKIP, "only a diagonal tile of a symmetric product has blocks to skip");
-  static_assert(!SKIP || (WM == WN && WM <= 2), "skipping is written for 64- and 128-wide tiles");
-  int mode = WAVE_FULL;
-  if (SKIP) {
-    if (wm == wn) {
-      mode = WAVE_DIAG;
-    } else if (wm < wn) {
-      mode = WAVE_ROW0;
-    } else {             // the quadrant below the diagonal: the lower half of the one above
-      mode = WAVE_ROW1;
-      wm = 0;
-      wn = 64;
-    }
-  }
-
-  v16f acc[2][2];
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.f;
-
-  // (uniform per workgroup: the tile lies inside the columns that vector loads may fetch)
-  constexpr bool can_vec = offers_vec4<OPP>::value || (!SAME && offers_vec4<OPQ>::value);
-  bool vec = false;
-  if constexpr (can_vec) vec = vec_tile_ok(P, m0, C::TM) && (same || vec_tile_ok(Q, n0, C::TN));
-  if constexpr (can_vec) {
-    if (vec)
-      gemm_tile_loop<WM, WN, SAME, SKIP, true>(P, Q, m0, n0, kbeg, kend, smem, wm, wn, mode, acc);
-  }
-  if (!vec)
-    gemm_tile_loop<WM, WN, SAME, SKIP, false>(P, Q, m0, n0, kbeg, kend, smem, wm, wn, mode, acc);
-
+// The accumulators of the calling wave's quadrant through the epilogue.
+template <bool SKIP, class EPI>
+__device__ __forceinline__ void store_tile(const v16f (&acc)[2][2], int m0, int n0, int wm, int wn,
+                                           int mode, EPI& epi) {
   // A diagonal tile of a symmetric product: the blocks above the tile's diagonal are
   // stored at their mirror position too, the blocks below it were not computed.
   auto computed = [&](int a, int b) {
@@ -524,6 +482,55 @@ __device__ __forceinline__ void gemm_tile_impl(const OPP& P, const OPQ& Q, int m
           if (mirrored(a, b)) epi.store(col, row, acc[a][b][i]);
         }
       }
+}
+
+template <int WM, int WN, bool SAME, bool SKIP, class OPP, class OPQ, class EPI>
+__device__ __forceinline__ void gemm_tile_impl(const OPP& P, const OPQ& Q, int m0, int n0,
+                                               int kbeg, int kend, EPI& epi, float* smem) {
+  typedef Cfg<WM, WN> C;
+  constexpr bool same = SAME;
+  const int t = threadIdx.x & (C::NT - 1);
+  const int lane = t & 63;
+  const int wave = t >> 6;
+  const int r = lane & 31;
+  const int h = lane >> 5;
+  int wm = (wave / WN) * 64;
+  int wn = (wave % WN) * 64;
+  static_assert(SAME || !SKIP, "only a diagonal tile of a symmetric product has blocks to skip");
+  static_assert(!SKIP || (WM == WN && WM <= 2), "skipping is written for 64- and 128-wide tiles");
+  int mode = WAVE_FULL;
+  if (SKIP) {
+    if (wm == wn) {
+      mode = WAVE_DIAG;
+    } else if (wm < wn) {
+      mode = WAVE_ROW0;
+    } else {             // the quadrant below the diagonal: the lower half of the one above
+      mode = WAVE_ROW1;
+      wm = 0;
+      wn = 64;
+    }
+  }
+
+  v16f acc[2][2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.f;
+
+  // (uniform per workgroup: the tile lies inside the columns that vector loads may fetch)
+  constexpr bool can_vec = offers_vec4<OPP>::value || (!SAME && offers_vec4<OPQ>::value);
+  bool vec = false;
+  if constexpr (can_vec) vec = vec_tile_ok(P, m0, C::TM) && (same || vec_tile_ok(Q, n0, C::TN));
+  if constexpr (can_vec) {
+    if (vec)
+      gemm_tile_loop<WM, WN, SAME, SKIP, true>(P, Q, m0, n0, kbeg, kend, smem, wm, wn, mode, acc);
+  }
+  if (!vec)
+    gemm_tile_loop<WM, WN, SAME, SKIP, false>(P, Q, m0, n0, kbeg, kend, smem, wm, wn, mode, acc);
+
+  store_tile<SKIP>(acc, m0, n0, wm, wn, mode, epi);
 }
 
 // SKIP_LOWER: a diagonal tile (`same`) leaves out its blocks below the diagonal.

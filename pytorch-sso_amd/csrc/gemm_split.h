@@ -1,0 +1,570 @@
+// Tile engine on the bf16 matrix cores with float32 results (gfx950, CDNA4, wave64).
+//
+// One workgroup of 256 threads (4 waves, 2x2) computes a 128x128 tile of
+//     C[m][n] = sum_k  P(k, m) * Q(k, n)          k in [kbeg, kend)
+// The fp32 matrix instructions of this chip run at 157 TFLOP/s, the bf16 ones at 2500.  A
+// float32 is the exact sum of three bf16 numbers (8 + 8 + 8 significant bits, each the
+// rounded rest of the ones before), x = h + m + l, so a product of two floats is nine
+// products of bf16 numbers, each exact in float32:
+//     x y = h h' + (h m' + m h') + (h l' + m m' + l h') + [m l' + l m' + l l'].
+// The bracket is at most 2^-23 and on average 2^-26 of x y, below the rounding of one float32
+// accumulation, and is left out; the other six run as v_mfma_f32_32x32x16_bf16.  The leading
+// products and the five corrections have accumulators of their own: the leading ones are
+// rounded once per 16 reduction steps, the corrections are 2^-8 of them, and the two are
+// added at the end.  Measured against float64 on one 32x32 tile (relative 2-norm, this
+// engine / v_mfma_f32_32x32x2_f32 on the same data):
+//     N(0,1):           K = 128  6.3e-8 / 2.2e-7    K = 4096  4.0e-7 / 1.1e-6    K = 65536  1.7e-6 / 4.6e-6
+//     max(0, N(0,1)):   K = 128  4.4e-8 / 8.6e-8    K = 4096  3.2e-7 / 5.0e-7    K = 65536  1.4e-6 / 2.0e-6
+// (with all six products in one accumulator the errors are those of the fp32 instruction,
+// and sums of positive terms drift by -1.3e-6 at K = 65536: the accumulation inside the
+// instruction rounds down.)
+//
+// A 64x64 sub-tile per wave takes 24 matrix instructions (768 cycles) per 16 reduction
+// steps where the fp32 instruction takes 2048 cycles.  The operands are split on their way
+// into LDS, once per workgroup; that is 5.5 vector instructions per element, which run
+// beside the matrix instructions of the other wave on the SIMD.
+#pragma once
+#include "gemm_core.h"
+
+namespace kfac {
+
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+typedef unsigned v2u __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) char lds_c;
+typedef __attribute__((address_space(3))) v4u lds_u4;
+typedef __attribute__((address_space(3))) v2u lds_u2;
+
+// LDS of one operand chunk (16 reduction steps): three planes (h, m, l), each with the 16-byte
+// groups of 8 consecutive k of all rows, the two groups of a row in two halves:
+//     plane * PLANE + (k / 8) * HALF + row * 16 + (k % 8) * 2
+// A fragment of the matrix instruction (lane: row = lane % 32, k = 8 * (lane / 32) + 0..7) is
+// one ds_read_b128.  The halves are 128 bytes further apart than their size, so that a
+// wave that writes 8-byte pieces of both at once meets every bank once.
+template <int ROWS>
+struct SplitChunk {
+    static constexpr int HALF = ROWS * 16 + 64;
+  static constexpr int PLANE = 2 * HALF;
+  static constexpr int BYTES = 3 * PLANE;
+};
+
+template <int WM, int WN>
+struct SplitCfg {
+  static constexpr int TM = 64 * WM;
+  static constexpr int TN = 64 * WN;
+  static constexpr int NT = 64 * WM * WN;
+  static constexpr int KC = 16;
+  static constexpr int STAGE = SplitChunk<TM>::BYTES + SplitChunk<TN>::BYTES;
+  static constexpr int SMEM_BYTES = 2 * STAGE;
+};
+
+__device__ __forceinline__ unsigned pack_bf16(float a, float b) {
+  v2bf r;
+  r[0] = (__bf16)a;
+  r[1] = (__bf16)b;
+  return __builtin_bit_cast(unsigned, r);
+}
+__device__ __forceinline__ float bf16_lo(unsigned p) { return __builtin_bit_cast(float, p << 16); }
+__device__ __forceinline__ float bf16_hi(unsigned p) {
+  return __builtin_bit_cast(float, p & 0xffff0000u);
+}
+// two floats -> their h, m and l parts, packed
+__device__ __forceinline__ void split_pair(float a, float b, unsigned& h, unsigned& m, unsigned& l) {
+  h = pack_bf16(a, b);
+  asm("" : "+v"(h));       // (or the low half would be converted a second time)
+  const float ra = a - bf16_lo(h), rb = b - bf16_hi(h);
+  m = pack_bf16(ra, rb);
+  asm("" : "+v"(m));
+  l = pack_bf16(ra - bf16_lo(m), rb - bf16_hi(m));
+}
+
+// the element at `off` (per lane, range-checked) + `at` (the same for all lanes)
+__device__ __forceinline__ float buffer_load_at(__amdgpu_buffer_rsrc_t r, unsigned off, unsigned at) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, (int)at, 0));
+}
+
+// ---------------------------------------------------------------------------
+// global -> registers -> LDS, one chunk of an operand.  Two chunks are in flight (SET): a
+// chunk is fetched two steps ahead of its use, split and stored one step ahead, in PIECES of
+// two elements that the tile loop deals out between its matrix instructions.
+// ---------------------------------------------------------------------------
+// How four consecutive k of an MK operand lie in memory (`kruns`):
+//   K_FLAT   always next to each other (a matrix row)
+//   K_RUNS   in runs of at least 4 if `runs()`: `KRun run(k)` gives the offset of k, how many
+//            elements its run still holds (itself included) and the offset of the next run;
+//            `quads()`: all runs are multiples of 4 long
+//   K_ANY    anywhere (one offset per element)
+enum { K_FLAT = 0, K_RUNS = 1, K_ANY = 2 };
+struct KRun {
+  unsigned off, next;
+  int len;
+};
+
+template <class OP, int ROWS, int NT, int LAYOUT = OP::layout>
+struct SplitStager;
+
+// Consecutive m contiguous: a thread takes 8 consecutive k of one column.
+template <class OP, int ROWS, int NT>
+struct SplitStager<OP, ROWS, NT, KM> {
+  static constexpr int NI = ROWS * 2 / NT;
+  static constexpr int PIECES = 4 * NI;
+  static_assert(ROWS * 2 % NT == 0 && ROWS % 64 == 0, "a wave's lanes share their k");
+  typename OP::MS ms[NI];
+  float regs[2][NI][8];
+  unsigned ones[2];          // bit 8i + j: element j of column i is the constant 1
+  v4u ph, pm, pl;            // the column being split
+
+  static __device__ __forceinline__ int tid() { return threadIdx.x & (NT - 1); }
+  static __device__ __forceinline__ int kgroup(int i) {
+    return __builtin_amdgcn_readfirstlane((tid() + NT * i) / ROWS);
+  }
+  // the tile lies inside the columns that are plain memory
+  static __device__ __forceinline__ bool fast(const OP& op, int m0) {
+    return op.vec_cols() == op.M || m0 + ROWS <= op.vec_cols();
+  }
+  __device__ __forceinline__ void init(const OP& op, int m0) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) ms[i] = op.mstate(m0 + ((tid() + NT * i) & (ROWS - 1)));
+  }
+  // a chunk inside the k range of a `fast` tile, load by load
+  static constexpr int LOADS = 8 * NI;
+  template <int SET, int LOAD>
+  __device__ __forceinline__ void fetch_load(const OP& op, int k0) {
+    constexpr int i = LOAD / 8, j = LOAD % 8;
+    regs[SET][i][j] = buffer_load_at(op.rsrc(), ms[i].off, (k0 + 8 * kgroup(i) + j) * op.kstride());
+  }
+  // any chunk
+  template <int SET>
+  __device__ __forceinline__ void fetch(const OP& op, int k0, int kend) {
+    unsigned one = 0;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int k = k0 + 8 * kgroup(i);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        // (k is the same for all lanes: its offset is a scalar)
+        const bool in = k + j < kend;
+        const unsigned at = in ? (k + j) : 0;
+        regs[SET][i][j] = buffer_load_at(op.rsrc(), in ? ms[i].off : INV_M, at * op.kstride());
+        if (op.second())
+          regs[SET][i][j] += buffer_load_at(op.rsrc2(), in ? ms[i].off2 : INV_M, at * 4u);
+        one |= (unsigned)(op.is_one(ms[i]) && in) << (8 * i + j);
+      }
+    }
+    ones[SET] = one;
+  }
+  template <int SET, int PIECE, bool FAST>
+  __device__ __forceinline__ void commit(lds_c* chunk) {
+    typedef SplitChunk<ROWS> L;
+    constexpr int i = PIECE / 4, j = PIECE % 4;
+    float v[2] = {regs[SET][i][2 * j], regs[SET][i][2 * j + 1]};
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      if (!FAST) v[e] = ((ones[SET] >> (8 * i + 2 * j + e)) & 1u) ? 1.f : v[e];
+      if (squares_elements<OP>::value) v[e] *= v[e];
+    }
+    unsigned h, m, l;
+    split_pair(v[0], v[1], h, m, l);
+    ph[j] = h;
+    pm[j] = m;
+    pl[j] = l;
+    if (j == 3) {
+      lds_c* const at = chunk + kgroup(i) * L::HALF + ((tid() + NT * i) & (ROWS - 1)) * 16;
+      *(lds_u4*)at = ph;
+      *(lds_u4*)(at + L::PLANE) = pm;
+      *(lds_u4*)(at + 2 * L::PLANE) = pl;
+    }
+  }
+};
+
+// Consecutive k contiguous: a thread takes 4 consecutive k of NI rows.
+template <class OP, int ROWS, int NT>
+struct SplitStager<OP, ROWS, NT, MK> {
+  static constexpr int NI = ROWS * 4 / NT;
+  static constexpr int PIECES = 2 * NI;
+  static constexpr int STEP = NT / 4;
+  typename OP::MS ms[NI];
+  v4f regs[2][NI];
+  unsigned ones;             // bit i: row i is the row of ones (K_ANY operands)
+  unsigned kin[2];           // bit j: element j lies inside the k range (where `ones` matters)
+  v2u ph, pm, pl;            // the row being split
+
+  static __device__ __forceinline__ int tid() { return threadIdx.x & (NT - 1); }
+  static __device__ __forceinline__ bool fast(const OP& op, int) {
+    if constexpr (OP::kruns == K_RUNS) return op.quads();
+    return OP::kruns == K_FLAT;
+  }
+  __device__ __forceinline__ void init(const OP& op, int m0) {
+    ones = 0;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      ms[i] = op.mstate(m0 + (tid() >> 2) + STEP * i);
+      if (OP::kruns == K_ANY) ones |= (unsigned)op.is_one(ms[i]) << i;
+    }
+  }
+  static constexpr int LOADS = NI;
+  unsigned koff;             // of the chunk being fetched by fetch_load
+  template <int SET, int LOAD>
+  __device__ __forceinline__ void fetch_load(const OP& op, int k0) {
+    const int k = k0 + 4 * (tid() & 3);
+    if (LOAD == 0) {
+      if constexpr (OP::kruns == K_RUNS) koff = op.run(k).off; else koff = op.kstate(k, true).off;
+    }
+    regs[SET][LOAD] = buffer_load4(op.rsrc(), ms[LOAD].off + koff);
+  }
+  template <int SET>
+  __device__ __forceinline__ void fetch(const OP& op, int k0, int kend) {
+    const __amdgpu_buffer_rsrc_t rs = op.rsrc();
+    const int k = k0 + 4 * (tid() & 3);
+    if constexpr (OP::kruns == K_RUNS) {
+      if (op.runs()) {
+        const KRun run = op.run(k);
+        const bool whole = run.len >= 4 && k + 4 <= kend;
+        if (__builtin_amdgcn_ballot_w64(!whole) == 0) {
+#pragma unroll
+          for (int i = 0; i < NI; ++i) regs[SET][i] = buffer_load4(rs, ms[i].off + run.off);
+        } else if (whole) {
+#pragma unroll
+          for (int i = 0; i < NI; ++i) regs[SET][i] = buffer_load4(rs, ms[i].off + run.off);
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const unsigned off = j < run.len ? run.off + 4 * j : run.next + 4 * (j - run.len);
+            const unsigned ko = k + j < kend ? off : INV_K;
+#pragma unroll
+            for (int i = 0; i < NI; ++i) regs[SET][i][j] = buffer_load(rs, ms[i].off + ko);
+          }
+        }
+        return;
+      }
+    }
+    unsigned in = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const typename OP::KS ks = op.kstate(k + j, k + j < kend);
+      in |= (unsigned)(k + j < kend) << j;
+#pragma unroll
+      for (int i = 0; i < NI; ++i) regs[SET][i][j] = buffer_load(rs, op.off(ms[i], ks));
+    }
+    kin[SET] = in;
+  }
+  template <int SET, int PIECE, bool FAST>
+  __device__ __forceinline__ void commit(lds_c* chunk) {
+    typedef SplitChunk<ROWS> L;
+    constexpr int i = PIECE / 2, j = PIECE % 2;
+    float v[2] = {regs[SET][i][2 * j], regs[SET][i][2 * j + 1]};
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      if (OP::kruns == K_ANY) v[e] = ((ones >> i) & (kin[SET] >> (2 * j + e)) & 1u) ? 1.f : v[e];
+      if (squares_elements<OP>::value) v[e] *= v[e];
+    }
+    unsigned h, m, l;
+    split_pair(v[0], v[1], h, m, l);
+    ph[j] = h;
+    pm[j] = m;
+    pl[j] = l;
+    if (j == 1) {
+      lds_c* const at = chunk + ((tid() >> 1) & 1) * L::HALF + ((tid() >> 2) + STEP * i) * 16 +
+                        (tid() & 1) * 8;
+      *(lds_u2*)at = ph;
+      *(lds_u2*)(at + L::PLANE) = pm;
+      *(lds_u2*)(at + 2 * L::PLANE) = pl;
+    }
+  }
+};
+
+template <int ROWS>
+__device__ __forceinline__ v8bf load_frag(const lds_c* chunk, int row0, int lane, int plane) {
+  typedef SplitChunk<ROWS> L;
+  const lds_c* const at = chunk + plane * L::PLANE + (lane >> 5) * L::HALF + (row0 + (lane & 31)) * 16;
+  return __builtin_bit_cast(v8bf, *(const lds_u4*)at);
+}
+
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (N > 0) {
+    static_for<N - 1>(f);
+    f(std::integral_constant<int, N - 1>{});
+  }
+}
+
+// The 32x32 blocks of a tile that one wave computes.
+// FULL: the four blocks of its 64x64 quadrant, block (a, b) = rows a of P against rows b of Q.
+// TRI: a diagonal tile of a symmetric product (P = Q) is symmetric itself; its blocks on and
+// above the diagonal (10 of 16 in a 128-wide tile, 3 of 4 in a 64-wide one) are dealt to the
+// waves three at a time, as products of three fragment rows r0, r1, r2 of the one operand:
+//     block 0 = (r0, r1)    block 1 = (r0, r2)    block 2 = (r1, r1)
+//   waves 0 / 1 of a 128-wide tile: r = (0, 1, 0) / (2, 3, 2), the three blocks of a diagonal
+//   quadrant;  waves 2 / 3: r = (0, 2, 3) / (1, 2, 3), a row of the quadrant above the
+//   diagonal (their block 2 repeats one of wave 1's and is not stored).
+// Every wave runs the same code, and the tile is done in three quarters of the time.
+struct SplitTri {
+  int r[3];
+  bool last;           // block 2 is this wave's to store
+};
+template <int W>
+__device__ __forceinline__ SplitTri split_tri(int wave) {
+  if (W == 1 || wave == 0) return SplitTri{{0, 1, 0}, true};
+  if (wave == 1) return SplitTri{{2, 3, 2}, true};
+  return SplitTri{{wave - 2, 2, 3}, false};
+}
+
+// fragments of one chunk: [h, m, l][row]; a FULL wave keeps P's two rows and Q's two
+template <bool TRI>
+struct SplitFrags {
+  v8bf p[3][TRI ? 3 : 2];
+  v8bf q[3][TRI ? 1 : 2];
+};
+
+// Accumulates C = P Q over [kbeg, kend) into the wave's blocks (leading products in acc, the
+// corrections in cor).  prow / qrow: the tile rows of its fragments (TRI: prow only).
+template <int WM, int WN, bool TRI, bool FAST, class OPP, class OPQ>
+__device__ __forceinline__ void split_tile_loop(const OPP& P, const OPQ& Q, int m0, int n0, int kbeg,
+                                                int kend, lds_c* sm, const int (&prow)[3],
+                                                const int (&qrow)[2], v16f (&acc)[TRI ? 3 : 4],
+                                                v16f (&cor)[TRI ? 3 : 4]) {
+  typedef SplitCfg<WM, WN> C;
+  constexpr int KC = C::KC;
+  constexpr int QOFF = SplitChunk<C::TM>::BYTES;
+  constexpr int NB = TRI ? 3 : 4;
+  const int lane = threadIdx.x & 63;
+  typedef SplitStager<OPP, C::TM, C::NT> SP;
+  typedef SplitStager<OPQ, C::TN, C::NT> SQ;
+  SP sp;
+  SQ sq;
+  sp.init(P, m0);
+  if (!TRI) sq.init(Q, n0);
+  const int nchunks = (kend - kbeg + KC - 1) / KC;
+  const int nfull = (kend - kbeg) / KC;
+  if (nchunks <= 0) return;
+  auto fetch = [&](auto set_, int c) {
+    constexpr int SET = decltype(set_)::value;
+    sp.template fetch<SET>(P, kbeg + c * KC, kend);
+    if (!TRI) sq.template fetch<SET>(Q, kbeg + c * KC, kend);
+  };
+  constexpr int LOADS = SP::LOADS + (TRI ? 0 : SQ::LOADS);
+  auto fetch_load = [&](auto set_, auto load_, int c) {
+    constexpr int SET = decltype(set_)::value, X = decltype(load_)::value;
+    if constexpr (X < SP::LOADS)
+      sp.template fetch_load<SET, X>(P, kbeg + c * KC);
+    else
+      sq.template fetch_load<SET, X - SP::LOADS>(Q, kbeg + c * KC);
+  };
+  constexpr int PIECES = SP::PIECES + (TRI ? 0 : SQ::PIECES);
+  auto commit = [&](auto set_, auto piece_, lds_c* stage) {
+    constexpr int SET = decltype(set_)::value, X = decltype(piece_)::value;
+    if constexpr (X < SP::PIECES)
+      sp.template commit<SET, X, FAST>(stage);
+    else
+      sq.template commit<SET, X - SP::PIECES, FAST>(stage + QOFF);
+  };
+  SplitFrags<TRI> fr[2];
+  auto load_frags = [&](auto set_, auto plane_) {
+    constexpr int SET = decltype(set_)::value, PL = decltype(plane_)::value;
+    const lds_c* const tp = sm + SET * C::STAGE;
+#pragma unroll
+    for (int i = 0; i < (TRI ? 3 : 2); ++i) fr[SET].p[PL][i] = load_frag<C::TM>(tp, prow[i], lane, PL);
+    if (!TRI) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) fr[SET].q[PL][i] = load_frag<C::TN>(tp + QOFF, qrow[i], lane, PL);
+    }
+  };
+  constexpr std::integral_constant<int, 0> S0{};
+  constexpr std::integral_constant<int, 1> S1{};
+  // (chunks past the end are fetched like the others: their elements lie outside the k
+  // range and cost no memory access, and the number of loads in flight is the same on every
+  // path, so that a commit waits for its own chunk only)
+  fetch(S0, 0);
+  fetch(S1, 1);
+  static_for<PIECES>([&](auto x) { commit(S0, x, sm); });
+  __syncthreads();
+  load_frags(S0, std::integral_constant<int, 0>{});
+
+  // One chunk.  Its leading planes are in registers already; the loads of chunk c + 2 and the
+  // pieces of chunk c + 1 are dealt out between the matrix instructions of the first four
+  // products; then the workgroup meets (chunk c has been read and chunk c + 1 written by
+  // every wave), and the leading planes of chunk c + 1 come in under the last two products.
+  auto step = [&](auto set_, auto full_, int c) {
+    constexpr int SET = decltype(set_)::value;
+    constexpr bool FULL = decltype(full_)::value;
+    lds_c* const next = sm + (SET ^ 1) * C::STAGE;
+    load_frags(set_, std::integral_constant<int, 1>{});
+    load_frags(set_, std::integral_constant<int, 2>{});
+    if (!FULL) fetch(set_, c + 2);
+    __builtin_amdgcn_sched_barrier(0);
+    static_for<6>([&](auto prod_) {
+      constexpr int PR = decltype(prod_)::value;
+      constexpr int PA = PR == 2 || PR == 3 ? 1 : PR == 5 ? 2 : 0;
+      constexpr int PB = PR == 1 || PR == 3 ? 1 : PR == 4 ? 2 : 0;
+      if constexpr (PR == 4) {
+        __syncthreads();
+        load_frags(std::integral_constant<int, SET ^ 1>{}, std::integral_constant<int, 0>{});
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      static_for<NB>([&](auto blk_) {
+        constexpr int B = decltype(blk_)::value;
+        constexpr int IDX = PR * NB + B;
+        v16f& t = PR == 0 ? acc[B] : cor[B];
+        v8bf a, b;
+        if constexpr (TRI) {
+          a = fr[SET].p[PA][B == 2 ? 1 : 0];
+          b = fr[SET].p[PB][B == 1 ? 2 : 1];
+        } else {
+          a = fr[SET].p[PA][B >> 1];
+          b = fr[SET].q[PB][B & 1];
+        }
+        t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, t, 0, 0, 0);
+        if constexpr (PR < 4) {
+          constexpr int LAST = 4 * NB;
+          constexpr int l0 = IDX * LOADS / LAST, l1 = (IDX + 1) * LOADS / LAST;
+          if constexpr (FULL)
+            static_for<l1 - l0>([&](auto x) {
+              fetch_load(set_, std::integral_constant<int, l0 + decltype(x)::value>{}, c + 2);
+            });
+          constexpr int p0 = IDX * PIECES / LAST, p1 = (IDX + 1) * PIECES / LAST;
+          static_for<p1 - p0>([&](auto x) {
+            commit(std::integral_constant<int, SET ^ 1>{},
+                   std::integral_constant<int, p0 + decltype(x)::value>{}, next);
+          });
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    });
+  };
+  constexpr std::false_type ANY{};
+  int c = 0;
+  if (FAST) {
+    constexpr std::true_type FULL{};
+    for (; c + 3 < nfull; c += 2) {       // (chunks c + 2 and c + 3 lie inside the range)
+      step(S0, FULL, c);
+      step(S1, FULL, c + 1);
+    }
+  }
+  for (; c < nchunks; c += 2) {           // (a chunk past the end adds zeros)
+    step(S0, ANY, c);
+    step(S1, ANY, c + 1);
+  }
+  __syncthreads();       // (the next tile of this workgroup may overwrite the stages)
+}
+
+// the sum of a wave's blocks over [kbeg, kend), in acc
+template <int WM, int WN, bool TRI, class OPP, class OPQ>
+__device__ __forceinline__ void split_blocks(const OPP& P, const OPQ& Q, int m0, int n0, int kbeg,
+                                             int kend, float* smem, const int (&prow)[3],
+                                             const int (&qrow)[2], v16f (&acc)[TRI ? 3 : 4]) {
+  typedef SplitCfg<WM, WN> C;
+  v16f cor[TRI ? 3 : 4];
+#pragma unroll
+  for (int b = 0; b < (TRI ? 3 : 4); ++b)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[b][i] = cor[b][i] = 0.f;
+  lds_c* const sm = (lds_c*)smem;
+  // (uniform per workgroup)
+  if (SplitStager<OPP, C::TM, C::NT>::fast(P, m0) &&
+      (TRI || SplitStager<OPQ, C::TN, C::NT>::fast(Q, n0)))
+    split_tile_loop<WM, WN, TRI, true>(P, Q, m0, n0, kbeg, kend, sm, prow, qrow, acc, cor);
+  else
+    split_tile_loop<WM, WN, TRI, false>(P, Q, m0, n0, kbeg, kend, sm, prow, qrow, acc, cor);
+#pragma unroll
+  for (int b = 0; b < (TRI ? 3 : 4); ++b) acc[b] += cor[b];
+}
+
+// The 32x32 blocks of a wave, rows from `row0`, columns from `col0`, through the epilogue.
+// `what`: nothing (the block is another wave's), the block, the block and its mirror image, or,
+// for a block on the diagonal, its upper triangle with or without the mirror image.  (The two
+// orders in which the corrections h m' and m h' are added round differently, so that only
+// one triangle of such a block is used: the result is symmetric to the bit.)
+enum { BLK_NONE = 0, BLK_PLAIN = 1, BLK_BOTH = 2, BLK_UPPER = 3, BLK_UPPER_BOTH = 4 };
+template <int NB, class EPI>
+__device__ __forceinline__ void store_blocks(const v16f (&acc)[NB], const int (&row0)[NB],
+                                             const int (&col0)[NB], const int (&what)[NB],
+                                             const EPI& epi) {
+  const int lane = threadIdx.x & 63;
+  const int r = lane & 31, h = lane >> 5;
+  auto row_of = [&](int b, int i) { return row0[b] + 8 * (i >> 2) + 4 * h + (i & 3); };
+  auto put = [&](int b, auto&& element) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int row = row_of(b, i), col = col0[b] + r;
+      if (what[b] < BLK_UPPER || row <= col) element(i, row, col);
+      if (what[b] == BLK_BOTH || (what[b] == BLK_UPPER_BOTH && row < col)) element(i, col, row);
+    }
+  };
+  if constexpr (reading_epilogue<EPI>::value) {
+    // C = alpha*acc + beta*C_old: the old values of two blocks are loaded ahead of the stores.
+    // Interleaved load/store pairs would each wait for their own load (a store to C may alias
+    // the next load of C, so the compiler keeps them in order).
+    if (epi.reads()) {
+#pragma unroll
+      for (int b0 = 0; b0 < NB; b0 += 2) {
+        float old[2][16];
+#pragma unroll
+        for (int b = b0; b < b0 + 2 && b < NB; ++b)
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            old[b - b0][i] = what[b] != BLK_NONE ? epi.fetch(row_of(b, i), col0[b] + r) : 0.f;
+        // (the old values are symmetric like the new ones)
+#pragma unroll
+        for (int b = b0; b < b0 + 2 && b < NB; ++b)
+          if (what[b] != BLK_NONE)
+            put(b, [&](int i, int row, int col) { epi.store_with(row, col, acc[b][i], old[b - b0][i]); });
+      }
+      return;
+    }
+  }
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+    if (what[b] != BLK_NONE)
+      put(b, [&](int i, int row, int col) { epi.store(row, col, acc[b][i]); });
+}
+
+// a tile of a product of two operands
+template <int WM, int WN, class OPP, class OPQ, class STORE>
+__device__ __forceinline__ void split_tile_full(const OPP& P, const OPQ& Q, int m0, int n0, int kbeg,
+                                                int kend, float* smem, const STORE& store) {
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x & (64 * WM * WN - 1)) >> 6);
+  const int wm = (wave / WN) * 64, wn = (wave % WN) * 64;
+  const int prow[3] = {wm, wm + 32, 0}, qrow[2] = {wn, wn + 32};
+  v16f acc[4];
+  split_blocks<WM, WN, false>(P, Q, m0, n0, kbeg, kend, smem, prow, qrow, acc);
+  const int row0[4] = {m0 + wm, m0 + wm, m0 + wm + 32, m0 + wm + 32};
+  const int col0[4] = {n0 + wn, n0 + wn + 32, n0 + wn, n0 + wn + 32};
+  const int what[4] = {BLK_PLAIN, BLK_PLAIN, BLK_PLAIN, BLK_PLAIN};
+  store([&](const auto& epi) { store_blocks<4>(acc, row0, col0, what, epi); });
+}
+
+// a diagonal tile of a symmetric product: with `both`, the blocks above its diagonal are stored
+// at their mirror positions too
+template <int W, class OP, class STORE>
+__device__ __forceinline__ void split_tile_tri(const OP& P, int m0, int kbeg, int kend, float* smem,
+                                               bool both, const STORE& store) {
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x & (64 * W * W - 1)) >> 6);
+  const SplitTri t = split_tri<W>(wave);
+  const int prow[3] = {32 * t.r[0], 32 * t.r[1], 32 * t.r[2]}, qrow[2] = {0, 0};
+  v16f acc[3];
+  split_blocks<W, W, true>(P, P, m0, m0, kbeg, kend, smem, prow, qrow, acc);
+  const int row0[3] = {m0 + prow[0], m0 + prow[0], m0 + prow[1]};
+  const int col0[3] = {m0 + prow[1], m0 + prow[2], m0 + prow[1]};
+  const int above = both ? BLK_BOTH : BLK_PLAIN, on = both ? BLK_UPPER_BOTH : BLK_UPPER;
+  const int what[3] = {above, t.r[0] == t.r[2] ? on : above, t.last ? on : BLK_NONE};
+  store([&](const auto& epi) { store_blocks<3>(acc, row0, col0, what, epi); });
+}
+
+// The tile (m0, n0) of the product, 128x128 on 256 threads; `same`: P and Q describe the same
+// columns (a diagonal tile of a symmetric product, of which, without `both`, the 32x32 blocks
+// below the diagonal are not written).
+template <class OPP, class OPQ, class EPI>
+__device__ __forceinline__ void split_tile(const OPP& P, const OPQ& Q, int m0, int n0, int kbeg,
+                                           int kend, bool same, const EPI& epi, float* smem,
+                                           bool both = true) {
+  auto store = [&](auto&& put) { put(epi); };
+  if constexpr (std::is_same<OPP, OPQ>::value) {
+    if (same) {
+      split_tile_tri<2>(P, m0, kbeg, kend, smem, both, store);
+      return;
+    }
+  }
+  split_tile_full<2, 2>(P, Q, m0, n0, kbeg, kend, smem, store);
+}
+
+}  // namespace kfac

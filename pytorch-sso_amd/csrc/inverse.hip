@@ -453,7 +453,7 @@ __global__ __launch_bounds__(DIAG_THREADS) void potrf_diag_kernel(const MatDesc*
 }
 
 // row panel of the blocked Cholesky: U[p, j] = Ypp^T * A[p, j], j > p
-__global__ __launch_bounds__(NTHREADS) void potrf_panel_kernel(const MatDesc* table, int p,
+__global__ __launch_bounds__(NTHREADS, 2) void potrf_panel_kernel(const MatDesc* table, int p,
                                                                const WorkList wl) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
   int mat, local;
@@ -466,7 +466,7 @@ __global__ __launch_bounds__(NTHREADS) void potrf_panel_kernel(const MatDesc* ta
   DenseKM P{m.Y + (size_t)r0 * n + r0, nullptr, n, DB, 0};
   DenseKM Q{m.U + (size_t)r0 * n, nullptr, n, n, 0};
   EpiStore epi{m.U + (size_t)r0 * n, n, DB, n, 1.f, 0.f, false};
-  gemm_tile(P, Q, 0, bj * BN, 0, DB, false, epi, smem);
+  split_tile(P, Q, 0, bj * BN, 0, DB, false, epi, smem);
 }
 
 // Tile (bi <= bj) number `local` of the trailing update of block rows [row_lo, row_hi).
@@ -513,7 +513,7 @@ constexpr int GROUP_BLOCKS = 4;
 // 9217 / 4097 / 4097 matrices 10.12 / 10.03 / 9.95 / 9.92 ms and 10.58 ms with 64)
 constexpr int TAIL_BLOCKS = 24;
 
-__global__ __launch_bounds__(NTHREADS, 3) void potrf_trail_kernel(const MatDesc* table, int kb0,
+__global__ __launch_bounds__(NTHREADS, 2) void potrf_trail_kernel(const MatDesc* table, int kb0,
                                                                int nk, int row_lo, int row_hi,
                                                                const WorkList wl) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
@@ -525,7 +525,8 @@ __global__ __launch_bounds__(NTHREADS, 3) void potrf_trail_kernel(const MatDesc*
   const int n = m.n;
   DenseKM P{m.U + (size_t)kb0 * DB * n, nullptr, n, n, 0};
   EpiStore epi{m.U, n, n, n, -1.f, 1.f, false};
-  gemm_tile(P, P, bi * BM, bj * BN, 0, nk * DB, bi == bj, epi, smem);
+  // (nobody reads U below its diagonal)
+  split_tile(P, P, bi * BM, bj * BN, 0, nk * DB, bi == bj, epi, smem, false);
 }
 
 // Diagonal blocks p and, beside them, the part of panel p-1's update that nothing needs
@@ -780,7 +781,7 @@ __device__ __forceinline__ MergeTile merge_tile(const MatDesc& m, int depth, int
 
 // first product:  W^T[j][i] = sum_{k <= j} Y22[k][j] * U12[i][k], stored at
 // Y[X2 rows][X1 cols] (the unused lower triangle of Y)
-__global__ __launch_bounds__(NTHREADS) void trtri_w_kernel(const MatDesc* table, int depth,
+__global__ __launch_bounds__(NTHREADS, 2) void trtri_w_kernel(const MatDesc* table, int depth,
                                                            const WorkList wl) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
   int mat, local;
@@ -792,11 +793,11 @@ __global__ __launch_bounds__(NTHREADS) void trtri_w_kernel(const MatDesc* table,
   DenseKM P{m.Y + (size_t)t.X2 * n + t.X2, nullptr, n, t.b2, 0};
   DenseMK Q{m.U + (size_t)t.X1 * n + t.X2, n, t.b1};
   EpiStore epi{m.Y + (size_t)t.X2 * n + t.X1, n, t.b2, t.b1, 1.f, 0.f, false};
-  gemm_tile(P, Q, t.jt * BM, t.it * BN, 0, min(t.b2, (t.jt + 1) * DB), false, epi, smem);
+  split_tile(P, Q, t.jt * BM, t.it * BN, 0, min(t.b2, (t.jt + 1) * DB), false, epi, smem);
 }
 
 // second product:  Y12[i][j] = - sum_{k >= i} Y11[i][k] * W^T[j][k]
-__global__ __launch_bounds__(NTHREADS) void trtri_y_kernel(const MatDesc* table, int depth,
+__global__ __launch_bounds__(NTHREADS, 2) void trtri_y_kernel(const MatDesc* table, int depth,
                                                            const WorkList wl) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
   int mat, local;
@@ -808,7 +809,7 @@ __global__ __launch_bounds__(NTHREADS) void trtri_y_kernel(const MatDesc* table,
   DenseMK P{m.Y + (size_t)t.X1 * n + t.X1, n, t.b1};
   DenseMK Q{m.Y + (size_t)t.X2 * n + t.X1, n, t.b2};
   EpiStore epi{m.Y + (size_t)t.X1 * n + t.X2, n, t.b1, t.b2, -1.f, 0.f, false};
-  gemm_tile(P, Q, t.it * BM, t.jt * BN, t.it * DB, t.b1, false, epi, smem);
+  split_tile(P, Q, t.it * BM, t.jt * BN, t.it * DB, t.b1, false, epi, smem);
 }
 
 // Which upper tile (bi <= bj) of Y Y^T a workgroup takes.  The tiles of a column bj all
@@ -890,7 +891,7 @@ struct EpiSymFlip {
 };
 
 // dst = Y Y^T over the upper tiles (k >= the later block), mirrored
-__global__ __launch_bounds__(NTHREADS) void lauum_kernel(const MatDesc* table, const WorkList wl) {
+__global__ __launch_bounds__(NTHREADS, 2) void lauum_kernel(const MatDesc* table, const WorkList wl) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
   int mat, local;
   work_find(wl, mat, local);
@@ -901,7 +902,7 @@ __global__ __launch_bounds__(NTHREADS) void lauum_kernel(const MatDesc* table, c
   const int n = m.n;
   DenseMK P{m.Y, n, n};
   EpiSymFlip epi{m.U, n, m.rev ? n - 1 : 0, m.rev ? -1 : 1, bi != bj};
-  gemm_tile(P, P, bi * BM, bj * BN, bj * DB, n, bi == bj, epi, smem);
+  split_tile(P, P, bi * BM, bj * BN, bj * DB, n, bi == bj, epi, smem);
 }
 
 // W = J Y^T J (J = reversal) for the matrices factored back to front: with S = J X J = R^T R

@@ -1,6 +1,6 @@
 // Operand and epilogue functors for the tile engine in gemm_core.h.
 #pragma once
-#include "gemm_core.h"
+#include "gemm_split.h"
 
 namespace kfac {
 
@@ -44,6 +44,8 @@ struct DenseKM {
   static constexpr bool vec4 = true;
   // (the columns in memory; the optional last one is not)
   __device__ __forceinline__ int vec_cols() const { return extra ? M - 1 : M; }
+  // (bytes from one k to the next)
+  __device__ __forceinline__ unsigned kstride() const { return (unsigned)ld * 4u; }
   const float* p;
   const float* vec;
   int ld, M, extra;
@@ -77,6 +79,7 @@ struct DenseKM {
 // Dense row-major matrix read as P(k, m) = p[m*ld + k]  (k contiguous), M rows.
 struct DenseMK {
   static constexpr int layout = MK;
+  static constexpr int kruns = K_FLAT;
   static constexpr bool has_second = false;
   const float* p;
   int ld, M;
@@ -98,6 +101,7 @@ struct DenseMK {
 // Output gradient of a Conv2d, g[n][c][hw], read as P(k=(n,pos), m=c).
 struct ConvG {
   static constexpr int layout = MK;
+  static constexpr int kruns = K_RUNS;
   static constexpr bool has_second = false;
   const float* p;
   int C, HW;
@@ -117,6 +121,13 @@ struct ConvG {
     const int n = by_hw.div(k);
     return KS{k_offset_or_invalid((unsigned)(n * C * HW + (k - n * HW)) * 4u, valid)};
   }
+  // the positions of an image are consecutive
+  __device__ __forceinline__ bool runs() const { return HW >= 4; }
+  __device__ __forceinline__ bool quads() const { return (HW & 3) == 0; }
+  __device__ __forceinline__ KRun run(int k) const {
+    const int n = by_hw.div(k), pos = k - n * HW, image = n * C * HW;
+    return KRun{(unsigned)(image + pos) * 4u, (unsigned)(image + C * HW) * 4u, HW - pos};
+  }
   __device__ __forceinline__ unsigned off(const MS& m, const KS& k) const { return m.off + k.off; }
   __device__ __forceinline__ bool is_one(const MS&) const { return false; }
 };
@@ -126,6 +137,7 @@ struct ConvG {
 // (0 in the padding), plus an optional trailing row of ones (m == M-1).
 struct ConvA {
   static constexpr int layout = MK;
+  static constexpr int kruns = K_ANY;
   static constexpr bool has_second = false;
   const float* p;
   int C, H, W, KH, KW, SH, SW, PH, PW, DH, DW, OH, OW, M, ones;
@@ -197,6 +209,7 @@ struct ConvA {
 // every image: a constant substituted after the load costs the inner loop about 7 %.
 struct ConvP {
   static constexpr int layout = MK;
+  static constexpr int kruns = K_RUNS;
   static constexpr bool has_second = false;
   const float* p;
   int C, KH, KW, SH, DH, Hs, OHW, OW, M, ones;
@@ -227,6 +240,12 @@ struct ConvP {
   __device__ __forceinline__ KS kstate(int k, bool valid) const {
     const int n = by_l.div(k);
     return KS{k_offset_or_invalid((unsigned)(n * image + (k - n * OHW)) * 4u, valid)};
+  }
+  __device__ __forceinline__ bool runs() const { return OHW >= 4; }
+  __device__ __forceinline__ bool quads() const { return (OHW & 3) == 0; }
+  __device__ __forceinline__ KRun run(int k) const {
+    const int n = by_l.div(k), pos = k - n * OHW;
+    return KRun{(unsigned)(n * image + pos) * 4u, (unsigned)((n + 1) * image) * 4u, OHW - pos};
   }
   __device__ __forceinline__ unsigned off(const MS& m, const KS& k) const { return m.off + k.off; }
   __device__ __forceinline__ bool is_one(const MS&) const { return false; }

@@ -172,14 +172,14 @@ __device__ __forceinline__ void tile_or_piece(const LayerDesc& m, const TileItem
                                               const EPI& epi, float* smem) {
   if (it.pieces == 1) {
     EPI e = epi;
-    gemm_tile(P, Q, m0, n0, k0, k1, false, e, smem);
+    split_tile(P, Q, m0, n0, k0, k1, false, e, smem);
     return;
   }
   const int kbeg = k0 + it.piece * (pb * BM);
   const int kend = min(k1, kbeg + pb * BM);
   float* parts = m.parts + ((size_t)tile_id * max_pieces + it.piece) * (BM * BN);
   EpiPartial part{parts, m0, n0, M, N, BN};
-  gemm_tile(P, Q, m0, n0, kbeg, kend, false, part, smem);
+  split_tile(P, Q, m0, n0, kbeg, kend, false, part, smem);
 }
 
 // where the products of a layer between the first and the last put their result
@@ -204,7 +204,7 @@ __device__ __forceinline__ EpiSplit fourth_epilogue(const LayerDesc& m) {
 }
 
 template <bool SAMPLE>
-__global__ __launch_bounds__(NTHREADS, 3) void precond_first_kernel(const LayerDesc* table,
+__global__ __launch_bounds__(NTHREADS, 2) void precond_first_kernel(const LayerDesc* table,
                                                                  const WorkList wl, int pb) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
   int layer, local;
@@ -232,7 +232,7 @@ __global__ __launch_bounds__(NTHREADS, 3) void precond_first_kernel(const LayerD
 }
 
 template <bool SAMPLE>
-__global__ __launch_bounds__(NTHREADS, 3) void precond_second_kernel(const LayerDesc* table,
+__global__ __launch_bounds__(NTHREADS, 2) void precond_second_kernel(const LayerDesc* table,
                                                                  const WorkList wl, int pb) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
   int layer, local;
@@ -257,7 +257,7 @@ __global__ __launch_bounds__(NTHREADS, 3) void precond_second_kernel(const Layer
 }
 
 // third product, layers whose R is the factor Ya:  X' = X Ya^T, reduction a >= j
-__global__ __launch_bounds__(NTHREADS, 3) void precond_third_kernel(const LayerDesc* table,
+__global__ __launch_bounds__(NTHREADS, 2) void precond_third_kernel(const LayerDesc* table,
                                                                 const WorkList wl, int pb) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
   int layer, local;
@@ -273,7 +273,7 @@ __global__ __launch_bounds__(NTHREADS, 3) void precond_third_kernel(const LayerD
 }
 
 // fourth product, layers whose L is the factor Yg:  U = Yg X', reduction k >= i
-__global__ __launch_bounds__(NTHREADS, 3) void precond_fourth_kernel(const LayerDesc* table,
+__global__ __launch_bounds__(NTHREADS, 2) void precond_fourth_kernel(const LayerDesc* table,
                                                                  const WorkList wl, int pb) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
   int layer, local;

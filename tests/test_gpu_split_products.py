@@ -1,0 +1,96 @@
+"""Products on the bf16 matrix cores with float32 results (csrc/gemm_split.h): every element
+within the rounding of a float32 sum of its exact products, at the edges of tiles, chunks and
+runs, and over the range of magnitudes of the data type."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope='module')
+def dev():
+    return torch.device('cuda:0')
+
+
+@pytest.fixture(scope='module')
+def ops():
+    from torchsso import _ops
+    return _ops
+
+
+def _assert_float32_sum(got, a, b, what):
+    """got = a^T b for float64 copies a [K, m], b [K, n] of float32 operands.  An element is a
+    sum of exact products, of which the terms of relative size 2^-23 and below are left
+    out, added to float32 accumulators in at most K / 16 + 1 steps each for the leading and
+    the correction terms (16 products per step, each step within 2^-23 of the running sum of
+    absolute values), over at most K / 128 + 1 partial sums."""
+    K = a.shape[0]
+    want = a.t() @ b
+    mass = a.abs().t() @ b.abs()
+    bound = mass * (2. ** -23) * (2 * (K // 16 + 1) + K // 128 + 4) + 1e-37
+    over = ((got.double() - want).abs() / bound).max().item()
+    assert over <= 1., '%s: error %.2f times the bound' % (what, over)
+
+
+@pytest.mark.parametrize('bias', [False, True])
+@pytest.mark.parametrize('rows', [1, 15, 16, 17, 33, 47, 130])
+@pytest.mark.parametrize('f', [193, 255, 256, 257, 384])
+def test_dense_symmetric(ops, dev, f, rows, bias):
+    gen = torch.Generator(device=dev).manual_seed(f * 1000 + rows)
+    x = torch.randn(rows, f, device=dev, generator=gen)
+    out = ops.factor_linear(x, bias, 1.)
+    a = x.double()
+    if bias:
+        a = torch.cat([a, torch.ones(rows, 1, device=dev, dtype=torch.float64)], 1)
+    _assert_float32_sum(out, a, a, 'factor of %d x %d' % (rows, f))
+    assert torch.equal(out, out.t())
+
+
+@pytest.mark.parametrize('hw', [(1, 1), (1, 3), (2, 2), (3, 3), (7, 7), (5, 13), (8, 8)])
+@pytest.mark.parametrize('n', [1, 5])
+def test_positions_in_runs(ops, dev, n, hw):
+    c = 200
+    gen = torch.Generator(device=dev).manual_seed(n * 100 + hw[0] * hw[1])
+    g = torch.randn(n, c, *hw, device=dev, generator=gen)
+    out = ops.factor_conv_g(g, 1.)
+    a = g.double().permute(0, 2, 3, 1).reshape(-1, c)
+    _assert_float32_sum(out, a, a, 'output gradients %dx%dx%d' % ((n,) + hw))
+    assert torch.equal(out, out.t())
+
+
+@pytest.mark.parametrize('exponent', [-15, 0, 15])
+def test_magnitudes(ops, dev, exponent):
+    # columns of very different sizes: each keeps its own 24 bits
+    gen = torch.Generator(device=dev).manual_seed(3)
+    x = torch.randn(200, 300, device=dev, generator=gen)
+    x *= 10. ** torch.linspace(exponent - 3, exponent + 3, 300, device=dev)
+    out = ops.factor_linear(x, False, 1.)
+    _assert_float32_sum(out, x.double(), x.double(), 'magnitudes around 1e%d' % exponent)
+
+
+def test_positive_terms(ops, dev):
+    # no drift where all terms have one sign
+    gen = torch.Generator(device=dev).manual_seed(4)
+    x = torch.rand(4096, 256, device=dev, generator=gen)
+    out = ops.factor_linear(x, False, 1.)
+    want = x.double().t() @ x.double()
+    assert ((out.double() - want) / want).mean().abs().item() < 2. ** -22
+
+
+@pytest.mark.parametrize('shape', [(1, 2), (129, 258), (300, 77), (128, 513)])
+def test_preconditioned_gradient(ops, dev, shape):
+    dG, dA = shape
+    gen = torch.Generator(device=dev).manual_seed(dG + dA)
+    Gi = torch.randn(dG, dG, device=dev, generator=gen)
+    Ai = torch.randn(dA, dA, device=dev, generator=gen)
+    Gi, Ai = Gi + Gi.t(), Ai + Ai.t()
+    w = torch.randn(dG, dA - 1, device=dev, generator=gen)
+    b = torch.randn(dG, device=dev, generator=gen)
+    full = torch.cat([w, b[:, None]], 1).double()
+    want = Gi.double() @ full @ Ai.double()
+    ops.precondition_batched([Gi], [Ai], [w], [b])
+    got = torch.cat([w, b[:, None]], 1).double()
+    # two products, each a float32 sum; the bound in the 2-norm
+    mass = Gi.double().abs() @ full.abs() @ Ai.double().abs()
+    steps = 2 * (dG // 16 + dA // 16 + 2) + 8
+    assert (got - want).abs().div(mass * 2. ** -23 * steps).max().item() <= 1.
