@@ -17,6 +17,8 @@
 //   3. Y = U^-1 by recursive doubling over the 128-blocks:
 //      Y12 = -Y11 * U12 * Y22, two MFMA products per level, log2(n/128) levels;
 //   4. dst = Y Y^T on the MFMA tile engine (upper tiles, mirrored).
+//   Batches whose tiles fit beside a diagonal block have steps 3 and 4 done by the launches of
+//   step 2 (the sweep, potrf_step_kernel).
 //
 // Every launch covers all matrices that still have work at that step (matrices
 // are processed in descending size order so the active ones form a prefix),
@@ -542,6 +544,51 @@ constexpr int STEP_TILES_PER_WG = DIAG_THREADS / NTHREADS;
 static_assert(STEP_TILES_PER_WG * SMEM_FLOATS * (int)sizeof(float) <= DIAG_SMEM_BYTES,
               "the tiles of a workgroup share the diagonal block's LDS");
 
+//
+// SWEEP: the whole inversion rides in these launches (see use_sweep).  With Z = U^-T, whose
+// rows obey  Z[i] = Y_ii^T (I[i] - sum_{k < i} U[k,i]^T Z[k]),  and X = Z^T Z the inverse, the
+// launch of diagonal block p applies block row k = p - 1 of U and Z to everything:
+//   A[i,j] -= U[k,i]^T U[k,j]   p <= i <= j        (T - p)(T - p + 1) / 2 tiles
+//   Z[i,j] -= U[k,i]^T Z[k,j]   p <= i, j <= k     (T - p) p
+//   X[i,j] += Z[k,i]^T Z[k,j]   i <= j <= k        p (p + 1) / 2
+// about T^2 / 2 tiles at every p, and the launch of p = T finishes X.  A finished row of Z lies
+// in column k of Y (Y = Z^T), a pending one below Y's diagonal; X grows in the columns of U
+// that no later step reads.
+__host__ __device__ inline int sweep_items(int T, int p, bool x) {
+  if (p > T) return 0;
+  const int Tr = T - p;
+  return Tr * (Tr + 1) / 2 + Tr * p + (x ? p * (p + 1) / 2 : 0);
+}
+
+__device__ __forceinline__ void sweep_tile(const MatDesc& m, int p, int local, float* smem) {
+  const int n = m.n, Tr = m.T - p, k0 = (p - 1) * DB;
+  const int nA = Tr * (Tr + 1) / 2;
+  const DenseKM uk{m.U + (size_t)k0 * n, nullptr, n, n, 0};
+  const DenseMK zk{m.Y + k0, n, n};
+  int bi, bj;
+  if (local < nA) {
+    upper_tile(xcd_remap(local, nA), Tr, bi, bj);
+    if (bj == 0) return;                     // tile (p, p): the diagonal block's own workgroup
+    bi += p;
+    bj += p;
+    EpiStore epi{m.U, n, n, n, -1.f, 1.f, false};
+    gemm_tile(uk, uk, bi * BM, bj * BN, 0, DB, bi == bj, epi, smem);
+  } else if (local < nA + Tr * p) {
+    const int at = xcd_remap(local - nA, Tr * p);
+    bi = at / p;
+    bj = at - bi * p;
+    bi += p;
+    // (column p - 1 of these rows meets its first update: what lies there is not a value yet)
+    EpiStore epi{m.Y, n, n, n, -1.f, bj == p - 1 ? 0.f : 1.f, false};
+    gemm_tile(uk, zk, bi * BM, bj * BN, 0, DB, false, epi, smem);
+  } else {
+    upper_tile(xcd_remap(local - nA - Tr * p, p * (p + 1) / 2), p, bi, bj);
+    EpiStore epi{m.U, n, n, n, 1.f, bj == p - 1 ? 0.f : 1.f, p == m.T && bi != bj};
+    gemm_tile(zk, zk, bi * BM, bj * BN, 0, min(DB, n - k0), bi == bj, epi, smem);
+  }
+}
+
+template <bool SWEEP>
 __global__ __launch_bounds__(DIAG_THREADS) void potrf_step_kernel(const MatDesc* table, int p,
                                                                    int* info, int ndiag,
                                                                    int row_lo, int row_hi, int tpw,
@@ -553,7 +600,7 @@ __global__ __launch_bounds__(DIAG_THREADS) void potrf_step_kernel(const MatDesc*
   }
   // A tile is the work of four waves.  A launch with more tiles than compute units packs
   // `tpw` (up to three) of them into a workgroup, each group of four waves with its own
-  // 40 KB of the launch's LDS; every tile of this launch reduces over the same 128 rows, so
+  // 40 KB of the launch's LDS; every tile of this launch reduces over at most 128 rows, and
   // the groups meet at the same barriers (a group that has returned no longer counts).
   const int group = (int)threadIdx.x / NTHREADS;
   if (group >= tpw) return;
@@ -561,6 +608,10 @@ __global__ __launch_bounds__(DIAG_THREADS) void potrf_step_kernel(const MatDesc*
   if (item >= wl.cum[wl.n]) return;
   int mat, local, bi, bj;
   work_find_item(wl, item, mat, local);
+  if constexpr (SWEEP) {
+    sweep_tile(table[mat], p, local, dsm + group * SMEM_FLOATS);
+    return;
+  }
   if (!trail_tile(table[mat].T, row_lo, row_hi, local, bi, bj)) return;
   if (bj == p) return;                       // tile (p, p): the diagonal block's own workgroup
   const MatDesc m = table[mat];
@@ -579,6 +630,34 @@ constexpr int FINE_THREADS = 1024;
 constexpr int FINE_SMEM_BYTES = 2 * DB * DB * (int)sizeof(float);
 constexpr int FINE_MAX_TILES = 256;      // one workgroup per CU
 
+// Tile `local` of row panel p.  U[p,j] = Y_pp^T A[p,j] in place for j > p, and in a sweep, after
+// those T - p - 1 tiles, the finished row p of Z for j < p: Z[p,j] = Y_pp^T (pending row), read
+// below the diagonal of Y and stored transposed above it.
+struct PanelTile {
+  const float* q;      // right-hand operand (row k at q + k n), `cols` columns wide
+  float* c;            // where the result goes: U[p,j], or Y[j,p]
+  int rows, cols;      // of the tile (rows: also the depth of the reduction)
+  bool z;
+};
+__device__ __forceinline__ bool panel_tile(const MatDesc& m, int p, int local, PanelTile& t) {
+  const int n = m.n, right = m.T - p - 1;
+  t.z = local >= right;
+  if (!t.z) {
+    const int bj = p + 1 + local;
+    t.q = t.c = m.U + (size_t)p * DB * n + bj * DB;
+    t.rows = DB;
+    t.cols = min(DB, n - bj * DB);
+    return true;
+  }
+  const int bj = local - right;
+  if (bj >= p) return false;
+  t.q = m.Y + (size_t)p * DB * n + bj * DB;
+  t.c = m.Y + (size_t)bj * DB * n + p * DB;
+  t.rows = min(DB, n - p * DB);
+  t.cols = DB;
+  return true;
+}
+
 __global__ __launch_bounds__(FINE_THREADS) void potrf_fine_kernel(const MatDesc* table, int p,
                                                                   const WorkList wl) {
   extern __shared__ __attribute__((aligned(16))) float fsm[];
@@ -588,26 +667,24 @@ __global__ __launch_bounds__(FINE_THREADS) void potrf_fine_kernel(const MatDesc*
   work_find(wl, mat, local);
   const MatDesc m = table[mat];
   const int n = m.n;
-  const int bj = p + 1 + local;
-  if (bj >= m.T) return;
-  // P(k, i) = Y_pp;  Q(k, j) = A[p, bj], j < qw;  C[i][j] = U[p, bj] over Q
+  PanelTile pt;
+  if (!panel_tile(m, p, local, pt)) return;
+  // P(k, i) = Y_pp;  Q(k, j);  C[i][j], or C[j][i]
   const float* P = m.Y + (size_t)p * DB * n + p * DB;
-  const float* Q = m.U + (size_t)p * DB * n + bj * DB;
-  float* C = m.U + (size_t)p * DB * n + bj * DB;
-  const int qw = min(DB, n - bj * DB);
   const int t = threadIdx.x;
   const int wave = t >> 6, lane = t & 63;
   const int r = lane & 31, h = lane >> 5;
   const int wr = wave >> 2, wc = wave & 3;
 
   const int mm = t & (DB - 1), kq = t >> 7;
-  const __amdgpu_buffer_rsrc_t rp = make_rsrc(P), rq = make_rsrc(Q);
+  const __amdgpu_buffer_rsrc_t rp = make_rsrc(P), rq = make_rsrc(pt.q);
   float vp[16], vq[16];
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
     const unsigned off = (unsigned)((kq + 8 * i) * n + mm) * 4u;
-    vp[i] = buffer_load(rp, off);
-    vq[i] = buffer_load(rq, mm < qw ? off : INV_M);
+    const bool in = kq + 8 * i < pt.rows;
+    vp[i] = buffer_load(rp, in && mm < pt.rows ? off : INV_M);
+    vq[i] = buffer_load(rq, in && mm < pt.cols ? off : INV_M);
   }
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
@@ -615,11 +692,15 @@ __global__ __launch_bounds__(FINE_THREADS) void potrf_fine_kernel(const MatDesc*
     tq[(kq + 8 * i) * DB + mm] = vq[i];
   }
   __syncthreads();
-  const v16f acc = lds_mma32(tp + 32 * wr, DB, 1, tq + 32 * wc, DB, 1, DB);
+  // (the transposed result comes from the exchanged operands: rows j, and lanes along i)
+  const lds_f* const left = pt.z ? tq : tp;
+  const lds_f* const right = pt.z ? tp : tq;
+  const int nrow = pt.z ? pt.cols : pt.rows, ncol = pt.z ? pt.rows : pt.cols;
+  const v16f acc = lds_mma32(left + 32 * wr, DB, 1, right + 32 * wc, DB, 1, DB);
 #pragma unroll
   for (int e = 0; e < 16; ++e) {
     const int row = 32 * wr + 8 * (e >> 2) + 4 * h + (e & 3), col = 32 * wc + r;
-    if (col < qw) C[(size_t)row * n + col] = acc[e];
+    if (row < nrow && col < ncol) pt.c[(size_t)row * n + col] = acc[e];
   }
 }
 
@@ -643,38 +724,38 @@ __global__ __launch_bounds__(SUB_THREADS) void potrf_sub_kernel(const MatDesc* t
   const int local = item >> 2, sj = item & 3;
   const MatDesc m = table[mat];
   const int n = m.n;
-  const int bj = p + 1 + local;
-  if (bj >= m.T) return;
+  PanelTile pt;
+  if (!panel_tile(m, p, local, pt)) return;
   const float* P = m.Y + (size_t)p * DB * n + p * DB;
-  const float* Q = m.U + (size_t)p * DB * n + bj * DB;
-  float* C = m.U + (size_t)p * DB * n + bj * DB;
-  const int qw = min(DB, n - bj * DB);
   const int t = threadIdx.x;
   const int wave = t >> 6, lane = t & 63;
   const int r = lane & 31, h = lane >> 5;
   const int br = wave & 3, khalf = wave >> 2;
-  const int row0 = 32 * br, col0 = WQ * sj;         // of this wave's block in the tile
+  const int row0 = 32 * br, col0 = WQ * sj;         // of this wave's block in the tile (U[p,j])
 
-  const __amdgpu_buffer_rsrc_t rp = make_rsrc(P), rq = make_rsrc(Q);
+  const __amdgpu_buffer_rsrc_t rp = make_rsrc(P), rq = make_rsrc(pt.q);
   float vp[WP / 4], vq[WQ / 4];
 #pragma unroll
   for (int i = 0; i < WP / 4; ++i) {
     const int idx = t + SUB_THREADS * i;
-    vp[i] = buffer_load(rp, (unsigned)((idx / WP) * n + idx % WP) * 4u);
+    const int k = idx / WP, col = idx % WP;
+    vp[i] = buffer_load(rp, k < pt.rows && col < pt.rows ? (unsigned)(k * n + col) * 4u : INV_M);
   }
 #pragma unroll
   for (int i = 0; i < WQ / 4; ++i) {
     const int idx = t + SUB_THREADS * i;
     const int k = idx / WQ, col = WQ * sj + idx % WQ;
-    vq[i] = buffer_load(rq, col < qw ? (unsigned)(k * n + col) * 4u : INV_M);
+    vq[i] = buffer_load(rq, k < pt.rows && col < pt.cols ? (unsigned)(k * n + col) * 4u : INV_M);
   }
 #pragma unroll
   for (int i = 0; i < WP / 4; ++i) tp[t + SUB_THREADS * i] = vp[i];
 #pragma unroll
   for (int i = 0; i < WQ / 4; ++i) tq[t + SUB_THREADS * i] = vq[i];
   __syncthreads();
-  const v16f acc = lds_mma32(tp + 64 * khalf * WP + 32 * br, WP, 1, tq + 64 * khalf * WQ, WQ, 1,
-                             64);
+  const lds_f* const bp = tp + 64 * khalf * WP + 32 * br;
+  const lds_f* const bq = tq + 64 * khalf * WQ;
+  // (the transposed result comes from the exchanged operands: rows j, and lanes along i)
+  const v16f acc = lds_mma32(pt.z ? bq : bp, pt.z ? WQ : WP, 1, pt.z ? bp : bq, pt.z ? WP : WQ, 1, 64);
   __syncthreads();
   // the second halves of the reduction travel through LDS (the operands are spent)
   lds_f* const red = tp + br * 1024;
@@ -686,9 +767,11 @@ __global__ __launch_bounds__(SUB_THREADS) void potrf_sub_kernel(const MatDesc* t
   if (khalf == 0) {
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      const int row = row0 + 8 * (e >> 2) + 4 * h + (e & 3), col = col0 + r;
+      const int at = 8 * (e >> 2) + 4 * h + (e & 3);
+      const int row = (pt.z ? col0 : row0) + at, col = (pt.z ? row0 : col0) + r;
       const float v = acc[e] + red[e * 64 + lane];
-      if (col < qw) C[(size_t)row * n + col] = v;
+      if (row < (pt.z ? pt.cols : pt.rows) && col < (pt.z ? pt.rows : pt.cols))
+        pt.c[(size_t)row * n + col] = v;
     }
   }
 }
@@ -984,6 +1067,27 @@ static size_t inverse_workspace_bytes(const std::vector<int>& dims) {
 
 enum { MODE_INVERSE = 0, MODE_CHOLESKY = 1 };
 
+// The sweep (SWEEP of potrf_step_kernel) or, after the factorisation, the recursive triangular
+// inverse and Y Y^T.  The sweep has two launches per 128 columns and nothing after them, but its
+// products are 128 deep and read and write their results every time; the recursive one adds
+// 2 log2(T) + 1 launches, each as long as its longest tile, of deep products.  So the line
+// lies where the tiles of a step, about T^2 / 2 per matrix, no longer fit beside a diagonal block:
+// three per compute unit.  Recursive / sweep, one matrix of n rows, us (same step tiles):
+//     300: 191 / 164   1000: 472 / 346   2305: 1049 / 753   3500 (406 tiles): 1575 / 1367
+//     4600 (666): 2230 / 2177;   five matrices of 728 tiles in all: 2418 / 2264
+//     the layers of a ResNet-50 (several thousand): 10.8 / 12.3 ms
+// (a matrix of one block has no panels: Y Y^T by its own kernel, 70 us instead of 75.)
+constexpr long SWEEP_MAX_TILES = 3 * 255;
+static bool use_sweep(const std::vector<int>& Ts) {
+  long tiles = 0;
+  int longest = 0;
+  for (int T : Ts) {
+    tiles += (long)T * (T + 1) / 2;
+    longest = std::max(longest, T);
+  }
+  return longest > 1 && tiles <= SWEEP_MAX_TILES;
+}
+
 static int run_batched(std::vector<HostMat>& mats, int mode, int* info, void* workspace,
                        size_t workspace_bytes, hipStream_t stream) {
   const int nmat = (int)mats.size();
@@ -995,7 +1099,8 @@ static int run_batched(std::vector<HostMat>& mats, int mode, int* info, void* wo
 
   // kernels that need more than the default 64 KiB of LDS (registered once per process)
   if (!enable_large_lds((const void*)potrf_diag_kernel, DIAG_SMEM_BYTES) ||
-      !enable_large_lds((const void*)potrf_step_kernel, DIAG_SMEM_BYTES) ||
+      !enable_large_lds((const void*)potrf_step_kernel<false>, DIAG_SMEM_BYTES) ||
+      !enable_large_lds((const void*)potrf_step_kernel<true>, DIAG_SMEM_BYTES) ||
       !enable_large_lds((const void*)potrf_fine_kernel, FINE_SMEM_BYTES) ||
       !enable_large_lds((const void*)potrf_sub_kernel, SUB_SMEM_BYTES))
     return KFAC_ERR_LAUNCH;
@@ -1049,18 +1154,23 @@ static int run_batched(std::vector<HostMat>& mats, int mode, int* info, void* wo
   };
 
   // Runs `launch(worklist)` over the first `count` matrices of the sorted table,
-  // WL_MAX at a time, with items(T) work items for a matrix of T blocks; matrices
+  // WL_MAX at a time, with items(s) work items for the matrix at position s; matrices
   // without items are skipped at the ends and cost nothing in between.
-  auto for_worklists = [&](int count, auto&& items, auto&& launch) {
+  auto for_matrices = [&](int count, auto&& items, auto&& launch) {
     for (int s0 = 0; s0 < count; s0 += WL_MAX) {
       WorkList wl;
       wl.first = s0;
       wl.n = std::min(WL_MAX, count - s0);
       wl.cum[0] = 0;
-      for (int i = 0; i < wl.n; ++i) wl.cum[i + 1] = wl.cum[i] + std::max(0, (int)items(Ts[s0 + i]));
+      for (int i = 0; i < wl.n; ++i) wl.cum[i + 1] = wl.cum[i] + std::max(0, (int)items(s0 + i));
       for (int i = wl.n + 1; i <= WL_MAX; ++i) wl.cum[i] = wl.cum[wl.n];
       if (wl.cum[wl.n] > 0) launch(wl, wl.cum[wl.n]);
     }
+  };
+
+  // ... with items(T) work items for a matrix of T blocks
+  auto for_worklists = [&](int count, auto&& items, auto&& launch) {
+    for_matrices(count, [&](int s) { return items(Ts[s]); }, launch);
   };
 
   bool any_pi = false;
@@ -1070,7 +1180,43 @@ static int run_batched(std::vector<HostMat>& mats, int mode, int* info, void* wo
     hipLaunchKernelGGL(inv_copy_damp_kernel, dim3(grid), dim3(256), 0, stream, table, info, wl);
   });
 
-  for (int P0 = 0, Pend = 0; P0 < Tmax; P0 = Pend) {
+  const bool sweep = mode == MODE_INVERSE && use_sweep(Ts);
+  // (a matrix factored back to front is written back through a reversal: its Y Y^T comes after)
+  auto sweep_x = [&](int s) {
+    const HostMat& h = mats[order[s]];
+    return h.fac == nullptr && h.std == nullptr;
+  };
+  for (int p = 0; sweep && p <= Tmax; ++p) {
+    const int na = active(p + 1);
+    if (p == 0) {
+      hipLaunchKernelGGL(potrf_diag_kernel, dim3(na), dim3(DIAG_THREADS), DIAG_SMEM_BYTES, stream,
+                         table, p, info);
+    } else {
+      bool first = true;
+      for_matrices(active(p), [&](int s) { return sweep_items(Ts[s], p, sweep_x(s)); },
+                   [&](const WorkList& wl, int grid) {
+        const int nd = first ? na : 0;
+        first = false;
+        const int tpw = std::min(STEP_TILES_PER_WG, std::max(1, cdiv(grid, 256)));
+        hipLaunchKernelGGL(potrf_step_kernel<true>, dim3(nd + cdiv(grid, tpw)), dim3(DIAG_THREADS),
+                           DIAG_SMEM_BYTES, stream, table, p, info, nd, p, Tmax, tpw, wl);
+      });
+    }
+    int panels = 0;
+    auto panel_items = [&](int T) { return T > p ? T - 1 : 0; };
+    for (int s = 0; s < na; ++s) panels += panel_items(Ts[s]);
+    if (panels <= SUB_MAX_TILES)
+      for_worklists(na, [&](int T) { return 4 * panel_items(T); }, [&](const WorkList& wl, int grid) {
+        hipLaunchKernelGGL(potrf_sub_kernel, dim3(grid), dim3(SUB_THREADS), SUB_SMEM_BYTES, stream,
+                           table, p, wl);
+      });
+    else
+      for_worklists(na, panel_items, [&](const WorkList& wl, int grid) {
+        hipLaunchKernelGGL(potrf_fine_kernel, dim3(grid), dim3(FINE_THREADS), FINE_SMEM_BYTES,
+                           stream, table, p, wl);
+      });
+  }
+  for (int P0 = 0, Pend = 0; !sweep && P0 < Tmax; P0 = Pend) {
     Pend = Tmax - P0 <= TAIL_BLOCKS ? Tmax : std::min(P0 + GROUP_BLOCKS, Tmax);
     auto total_items = [&](int count, auto&& items) {
       long sum = 0;
@@ -1097,7 +1243,7 @@ static int run_batched(std::vector<HostMat>& mats, int mode, int* info, void* wo
           first = false;
           // (one workgroup runs per compute unit: beyond 256 tiles, up to three to a workgroup)
           const int tpw = std::min(STEP_TILES_PER_WG, std::max(1, cdiv(grid, 256)));
-          hipLaunchKernelGGL(potrf_step_kernel, dim3(nd + cdiv(grid, tpw)), dim3(DIAG_THREADS),
+          hipLaunchKernelGGL(potrf_step_kernel<false>, dim3(nd + cdiv(grid, tpw)), dim3(DIAG_THREADS),
                              DIAG_SMEM_BYTES, stream, table, p, info, nd, p, Pend, tpw, wl);
         });
       }
@@ -1134,7 +1280,7 @@ static int run_batched(std::vector<HostMat>& mats, int mode, int* info, void* wo
     });
     return launch_status();
   }
-  if (Tmax > 1) {
+  if (Tmax > 1 && !sweep) {
     int D = 0;
     while ((1 << D) < Tmax) ++D;
     const int na = active(2);
@@ -1155,8 +1301,9 @@ static int run_batched(std::vector<HostMat>& mats, int mode, int* info, void* wo
     any_std |= h.std != nullptr;
     any_fac |= h.fac != nullptr;
   }
-  if (any_inv)
-    for_worklists(nmat, [](int T) { return T * (T + 1) / 2; }, [&](const WorkList& wl, int grid) {
+  if (any_inv)      // (in a sweep, those of its matrices that it did not finish)
+    for_matrices(nmat, [&](int s) { return sweep && sweep_x(s) ? 0 : Ts[s] * (Ts[s] + 1) / 2; },
+                 [&](const WorkList& wl, int grid) {
       KFAC_LAUNCH_TILE2(lauum_kernel, dim3(grid), stream, table, wl);
     });
   if (any_fac)   // the triangular inversion kept intermediate products below the diagonal
