@@ -531,19 +531,189 @@ __global__ __launch_bounds__(NTHREADS, 2) void potrf_trail_kernel(const MatDesc*
   split_tile(P, P, bi * BM, bj * BN, 0, nk * DB, bi == bj, epi, smem, false);
 }
 
+// One 128x128 tile of a rank-128 update beside a diagonal block, by the first 8 waves of the
+// workgroup (64x32 per wave):  C[m][n] = beta C + sign * sum_k P(k, m) Q(k, n), k < depth <= 128.
+// Such a tile is alone on its compute unit (the launch carries the diagonal block's LDS), so
+// it is a chain of latencies: memory -> split -> LDS -> matrix instructions -> memory.  The
+// operands come in two halves of 64 k, split into bf16 parts as in gemm_split.h; the whole
+// first half is in flight at once, the second under the products of the first, and C's old
+// values under those of the second.  A workgroup takes one tile after the other.
+// Bound by memory where every unit has one: 128 KB of C and up to 128 KB of operands per tile,
+// 11 us each with 510 tiles in a launch (the fp32 tile engine, three tiles to a workgroup:
+// 19 us).  Inverse of a 2900^2 / 3500^2 / 4600^2 matrix 1121 -> 920 / 1367 -> 1124 /
+// 2177 -> 1922 us, and 2.5 times closer to float64 (6.7e-5 -> 2.7e-5 at 2900).
+// PMK / QMK: the operand has consecutive k next to each other (P(k, m) = p[m n + k]) instead of
+// consecutive m (p[k n + m]).
+// `upper`: only elements on and above the diagonal of C are stored, with `mirror` at their
+// mirror positions too (a tile on the diagonal is symmetric except for rounding).
+constexpr int STEP_THREADS = 512;
+typedef SplitChunk<128> StepGroup;                  // (HALF: 8 k of 128 rows)
+constexpr int STEP_PLANE = 8 * StepGroup::HALF;     // 64 k
+constexpr int STEP_OPERAND = 3 * STEP_PLANE;
+static_assert(2 * STEP_OPERAND <= DIAG_SMEM_BYTES, "a tile lives in the diagonal block's LDS");
+
+template <bool MKL>
+struct StepOperand {
+  const float* p;
+  int n, m0, depth;
+  float v[16];
+  // k in [64 half, 64 half + 64): 16 elements per thread
+  __device__ __forceinline__ void load(int half) {
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(p);
+    const int t = threadIdx.x;
+    if constexpr (MKL) {
+      const int k = 64 * half + 4 * (t & 15);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int m = m0 + (t >> 4) + 32 * i;
+        const unsigned off = (unsigned)(m * n + k) * 4u;
+        if (depth == DB) {
+          const v4f x = buffer_load4(rs, m < n ? off : INV_M);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[4 * i + j] = x[j];
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            v[4 * i + j] = buffer_load(rs, m < n && k + j < depth ? off + 4 * j : INV_M);
+        }
+      }
+    } else {
+      // (never the last block row: all 128 k are there)
+      const int m = m0 + (t & 127);
+      const int k = 64 * half + 8 * __builtin_amdgcn_readfirstlane(t >> 7);
+      const unsigned off = m < n ? (unsigned)m * 4u : INV_M;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          v[8 * i + j] = buffer_load_at(rs, off, (unsigned)((k + 32 * i + j) * n) * 4u);
+    }
+  }
+  __device__ __forceinline__ void commit(lds_c* at) const {
+    const int t = threadIdx.x;
+    if constexpr (MKL) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        v2u h, m, l;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          unsigned a, b, c;
+          split_pair(v[4 * i + 2 * j], v[4 * i + 2 * j + 1], a, b, c);
+          h[j] = a;
+          m[j] = b;
+          l[j] = c;
+        }
+        lds_c* const o = at + ((t & 15) >> 1) * StepGroup::HALF + ((t >> 4) + 32 * i) * 16 + (t & 1) * 8;
+        *(lds_u2*)o = h;
+        *(lds_u2*)(o + STEP_PLANE) = m;
+        *(lds_u2*)(o + 2 * STEP_PLANE) = l;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        v4u h, m, l;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          unsigned a, b, c;
+          split_pair(v[8 * i + 2 * j], v[8 * i + 2 * j + 1], a, b, c);
+          h[j] = a;
+          m[j] = b;
+          l[j] = c;
+        }
+        lds_c* const o = at + ((t >> 7) + 4 * i) * StepGroup::HALF + (t & 127) * 16;
+        *(lds_u4*)o = h;
+        *(lds_u4*)(o + STEP_PLANE) = m;
+        *(lds_u4*)(o + 2 * STEP_PLANE) = l;
+      }
+    }
+  }
+};
+
+template <bool PMK, bool QMK>
+__device__ __forceinline__ void step_tile(const float* p, const float* q, float* C, int n, int m0,
+                                          int n0, int depth, float sign, bool fresh, bool upper,
+                                          bool mirror, lds_c* sm) {
+  StepOperand<PMK> P{p, n, m0, depth};
+  StepOperand<QMK> Q{q, n, n0, depth};
+  lds_c* const sq = sm + STEP_OPERAND;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+  const int wm = (wave & 1) * 64, wn = (wave >> 1) * 32;
+  v16f acc[2], cor[2];
+#pragma unroll
+  for (int b = 0; b < 2; ++b)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[b][e] = cor[b][e] = 0.f;
+  auto products = [&]() {
+#pragma unroll 1
+    for (int ks = 0; ks < 4; ++ks) {
+      v8bf a[3][2], b[3];
+#pragma unroll
+      for (int pl = 0; pl < 3; ++pl) {
+        const lds_c* const at = sm + pl * STEP_PLANE + (2 * ks + h) * StepGroup::HALF + r * 16;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) a[pl][i] = __builtin_bit_cast(v8bf, *(const lds_u4*)(at + (wm + 32 * i) * 16));
+        b[pl] = __builtin_bit_cast(v8bf, *(const lds_u4*)(at + STEP_OPERAND + wn * 16));
+      }
+      static_for<6>([&](auto prod_) {
+        constexpr int PR = decltype(prod_)::value;
+        constexpr int PA = PR == 2 || PR == 3 ? 1 : PR == 5 ? 2 : 0;
+        constexpr int PB = PR == 1 || PR == 3 ? 1 : PR == 4 ? 2 : 0;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          v16f& x = PR == 0 ? acc[i] : cor[i];
+          x = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[PA][i], b[PB], x, 0, 0, 0);
+        }
+      });
+    }
+  };
+  P.load(0);
+  Q.load(0);
+  P.commit(sm);
+  Q.commit(sq);
+  P.load(1);
+  Q.load(1);
+  __syncthreads();
+  products();
+  __syncthreads();
+  P.commit(sm);
+  Q.commit(sq);
+  const __amdgpu_buffer_rsrc_t rc = make_rsrc(C);
+  const int col = n0 + wn + r;
+  float old[2][16];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int row = m0 + wm + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
+      const bool in = !fresh && row < n && col < n && (!upper || row <= col);
+      old[i][e] = buffer_load(rc, in ? (unsigned)(row * n + col) * 4u : INV_M);
+    }
+  __syncthreads();
+  products();
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    acc[i] += cor[i];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int row = m0 + wm + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
+      if (row < n && col < n && (!upper || row <= col)) {
+        const float v = fmaf(sign, acc[i][e], old[i][e]);
+        C[(size_t)row * n + col] = v;
+        if (mirror && row < col) C[(size_t)col * n + row] = v;
+      }
+    }
+  }
+  __syncthreads();       // (the next tile overwrites the operands)
+}
+
 // Diagonal blocks p and, beside them, the part of panel p-1's update that nothing needs
 // before the next row panel:   A[i,j] -= U[p-1,i]^T U[p-1,j]   for block rows
 // row_lo <= i < row_hi (row_lo = p + 1: row p got its update in a launch of its own).
-// The first `ndiag` workgroups take one diagonal block each (potrf_diag_kernel's work),
-// the others `tpw` tiles each.  The launch carries the diagonal block's LDS, so one
-// workgroup runs per CU: the tile workgroups use the CUs that the few diagonal blocks
-// leave idle, for about as long as a diagonal block takes; a launch with more tiles than
-// CUs puts up to three tiles into a workgroup, as many waves per CU as in a launch of
-// their own.
-constexpr int STEP_TILES_PER_WG = DIAG_THREADS / NTHREADS;
-static_assert(STEP_TILES_PER_WG * SMEM_FLOATS * (int)sizeof(float) <= DIAG_SMEM_BYTES,
-              "the tiles of a workgroup share the diagonal block's LDS");
-
+// The first `ndiag` workgroups take one diagonal block each (potrf_diag_kernel's work).  The
+// launch carries the diagonal block's LDS, so one workgroup runs per CU: the others use the
+// CUs that the few diagonal blocks leave idle, for about as long as a diagonal block takes,
+// and where there are more tiles than such CUs they walk the list of tiles.
 //
 // SWEEP: the whole inversion rides in these launches (see use_sweep).  With Z = U^-T, whose
 // rows obey  Z[i] = Y_ii^T (I[i] - sum_{k < i} U[k,i]^T Z[k]),  and X = Z^T Z the inverse, the
@@ -560,66 +730,64 @@ __host__ __device__ inline int sweep_items(int T, int p, bool x) {
   return Tr * (Tr + 1) / 2 + Tr * p + (x ? p * (p + 1) / 2 : 0);
 }
 
-__device__ __forceinline__ void sweep_tile(const MatDesc& m, int p, int local, float* smem) {
+__device__ __forceinline__ void sweep_tile(const MatDesc& m, int p, int local, lds_c* sm) {
   const int n = m.n, Tr = m.T - p, k0 = (p - 1) * DB;
   const int nA = Tr * (Tr + 1) / 2;
-  const DenseKM uk{m.U + (size_t)k0 * n, nullptr, n, n, 0};
-  const DenseMK zk{m.Y + k0, n, n};
+  const float* const uk = m.U + (size_t)k0 * n;
+  const float* const zk = m.Y + k0;
   int bi, bj;
   if (local < nA) {
     upper_tile(xcd_remap(local, nA), Tr, bi, bj);
     if (bj == 0) return;                     // tile (p, p): the diagonal block's own workgroup
     bi += p;
     bj += p;
-    EpiStore epi{m.U, n, n, n, -1.f, 1.f, false};
-    gemm_tile(uk, uk, bi * BM, bj * BN, 0, DB, bi == bj, epi, smem);
+    step_tile<false, false>(uk, uk, m.U, n, bi * BM, bj * BN, DB, -1.f, false, true, false, sm);
   } else if (local < nA + Tr * p) {
     const int at = xcd_remap(local - nA, Tr * p);
     bi = at / p;
     bj = at - bi * p;
     bi += p;
     // (column p - 1 of these rows meets its first update: what lies there is not a value yet)
-    EpiStore epi{m.Y, n, n, n, -1.f, bj == p - 1 ? 0.f : 1.f, false};
-    gemm_tile(uk, zk, bi * BM, bj * BN, 0, DB, false, epi, smem);
+    step_tile<false, true>(uk, zk, m.Y, n, bi * BM, bj * BN, DB, -1.f, bj == p - 1, false, false, sm);
   } else {
     upper_tile(xcd_remap(local - nA - Tr * p, p * (p + 1) / 2), p, bi, bj);
-    EpiStore epi{m.U, n, n, n, 1.f, bj == p - 1 ? 0.f : 1.f, p == m.T && bi != bj};
-    gemm_tile(zk, zk, bi * BM, bj * BN, 0, min(DB, n - k0), bi == bj, epi, smem);
+    step_tile<true, true>(zk, zk, m.U, n, bi * BM, bj * BN, min(DB, n - k0), 1.f, bj == p - 1, true,
+                          p == m.T, sm);
   }
 }
 
 template <bool SWEEP>
 __global__ __launch_bounds__(DIAG_THREADS) void potrf_step_kernel(const MatDesc* table, int p,
                                                                    int* info, int ndiag,
-                                                                   int row_lo, int row_hi, int tpw,
+                                                                   int row_lo, int row_hi,
                                                                    const WorkList wl) {
   extern __shared__ __attribute__((aligned(16))) float dsm[];
   if ((int)blockIdx.x < ndiag) {
     diag_block(table[blockIdx.x], p, info, dsm, true);
     return;
   }
-  // A tile is the work of four waves.  A launch with more tiles than compute units packs
-  // `tpw` (up to three) of them into a workgroup, each group of four waves with its own
-  // 40 KB of the launch's LDS; every tile of this launch reduces over at most 128 rows, and
-  // the groups meet at the same barriers (a group that has returned no longer counts).
-  const int group = (int)threadIdx.x / NTHREADS;
-  if (group >= tpw) return;
-  const int item = ((int)blockIdx.x - ndiag) * tpw + group;
-  if (item >= wl.cum[wl.n]) return;
-  int mat, local, bi, bj;
-  work_find_item(wl, item, mat, local);
-  if constexpr (SWEEP) {
-    sweep_tile(table[mat], p, local, dsm + group * SMEM_FLOATS);
-    return;
+  if (threadIdx.x >= STEP_THREADS) return;     // (a wave that has returned no longer counts)
+  const int total = wl.cum[wl.n];
+  for (int item = (int)blockIdx.x - ndiag; item < total; item += (int)gridDim.x - ndiag) {
+    int mat, local, bi, bj;
+    work_find_item(wl, item, mat, local);
+    const MatDesc m = table[mat];
+    if constexpr (SWEEP) {
+      sweep_tile(m, p, local, (lds_c*)dsm);
+    } else {
+      if (!trail_tile(m.T, row_lo, row_hi, local, bi, bj)) continue;
+      if (bj == p) continue;                   // tile (p, p): the diagonal block's own workgroup
+      const float* const uk = m.U + (size_t)(p - 1) * DB * m.n;
+      step_tile<false, false>(uk, uk, m.U, m.n, bi * BM, bj * BN, DB, -1.f, false, true, false,
+                              (lds_c*)dsm);
+    }
   }
-  if (!trail_tile(table[mat].T, row_lo, row_hi, local, bi, bj)) return;
-  if (bj == p) return;                       // tile (p, p): the diagonal block's own workgroup
-  const MatDesc m = table[mat];
-  const int n = m.n;
-  DenseKM P{m.U + (size_t)(p - 1) * DB * n, nullptr, n, n, 0};
-  EpiStore epi{m.U, n, n, n, -1.f, 1.f, false};
-  gemm_tile(P, P, bi * BM, bj * BN, 0, DB, bi == bj, epi, dsm + group * SMEM_FLOATS);
 }
+
+// Workgroups of a step launch behind its `nd` diagonal blocks: one per tile, at most one per
+// compute unit.
+constexpr int STEP_CUS = 256;
+static int step_workgroups(int nd, int tiles) { return std::min(tiles, std::max(STEP_CUS - nd, 64)); }
 
 // The row panel for launches of few tiles: the same 128x128x128 product, but by 16 waves
 // with one 32x32 block each instead of 4 waves with four.  A tile is a chain of
@@ -1197,9 +1365,9 @@ static int run_batched(std::vector<HostMat>& mats, int mode, int* info, void* wo
                    [&](const WorkList& wl, int grid) {
         const int nd = first ? na : 0;
         first = false;
-        const int tpw = std::min(STEP_TILES_PER_WG, std::max(1, cdiv(grid, 256)));
-        hipLaunchKernelGGL(potrf_step_kernel<true>, dim3(nd + cdiv(grid, tpw)), dim3(DIAG_THREADS),
-                           DIAG_SMEM_BYTES, stream, table, p, info, nd, p, Tmax, tpw, wl);
+        hipLaunchKernelGGL(potrf_step_kernel<true>, dim3(nd + step_workgroups(nd, grid)),
+                           dim3(DIAG_THREADS), DIAG_SMEM_BYTES, stream, table, p, info, nd, p, Tmax,
+                           wl);
       });
     }
     int panels = 0;
@@ -1241,10 +1409,9 @@ static int run_batched(std::vector<HostMat>& mats, int mode, int* info, void* wo
         for_worklists(na, rest_items, [&](const WorkList& wl, int grid) {
           const int nd = first ? na : 0;
           first = false;
-          // (one workgroup runs per compute unit: beyond 256 tiles, up to three to a workgroup)
-          const int tpw = std::min(STEP_TILES_PER_WG, std::max(1, cdiv(grid, 256)));
-          hipLaunchKernelGGL(potrf_step_kernel<false>, dim3(nd + cdiv(grid, tpw)), dim3(DIAG_THREADS),
-                             DIAG_SMEM_BYTES, stream, table, p, info, nd, p, Pend, tpw, wl);
+          hipLaunchKernelGGL(potrf_step_kernel<false>, dim3(nd + step_workgroups(nd, grid)),
+                             dim3(DIAG_THREADS), DIAG_SMEM_BYTES, stream, table, p, info, nd, p,
+                             Pend, wl);
         });
       }
       const int nb = active(p + 2);
