@@ -136,15 +136,19 @@ def f32_array(values):
 
 def ptr_array(tensors, what='tensor', allow_none=False):
     """Host array of device addresses (0 for None when allowed)."""
-    out = (ctypes.c_void_p * len(tensors))()
+    f32 = torch.float32
+    out = []
     for i, t in enumerate(tensors):
         if t is None:
             if not allow_none:
                 raise KfacHipError('%s %d is None' % (what, i))
-            out[i] = None
+            out.append(None)
+        # (dev_ptr's conditions; its message is put together only where one fails)
+        elif isinstance(t, torch.Tensor) and t.is_cuda and t.dtype is f32 and t.is_contiguous():
+            out.append(t.data_ptr())
         else:
-            out[i] = dev_ptr(t, '%s %d' % (what, i))
-    return out
+            out.append(dev_ptr(t, '%s %d' % (what, i)))
+    return (ctypes.c_void_p * len(out))(*out)
 
 
 def signatures():
@@ -196,7 +200,10 @@ def stream_ptr(device=None, stream=None):
     """Raw handle of `stream` (a torch.cuda.Stream), or of torch's current stream."""
     if stream is not None:
         return stream.cuda_stream
-    return torch.cuda.current_stream(device).cuda_stream
+    index = getattr(device, 'index', None)
+    if index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(index)     # (no Stream object around the handle)
 
 
 _all_workspaces = []     # the `bufs` dict of every thread's _Workspace

@@ -94,6 +94,22 @@ def mode():
     return _mode
 
 
+_stream_objects = {}       # what identifies a stream to torch -> a Stream object for it
+
+
+def _current_stream(idx):
+    """torch.cuda.current_stream(idx) for a device index, with the object that wraps the
+    stream made once and not for every hook."""
+    ident = torch._C._cuda_getCurrentStream(idx)
+    st = _stream_objects.get(ident)
+    if st is None:
+        if len(_stream_objects) >= 64:
+            _stream_objects.clear()
+        st = torch.cuda.current_stream(idx)
+        _stream_objects[(st.stream_id, st.device_index, st.device_type)] = st
+    return st
+
+
 def set_flush_work(work):
     """Grouped mode: the queue of a device also runs as soon as the products collected
     amount to `work` multiply-adds (d^2 * K summed over them), so that the engine starts on
@@ -117,7 +133,7 @@ def defer(device, key, job, keep, work=0., backward=False):
     product belongs to a backward hook; the first of those runs what the forward hooks have
     queued, so that the input factors are computed beside the backward pass."""
     idx = device.index if device.index is not None else torch.cuda.current_device()
-    stream = torch.cuda.current_stream(device)
+    stream = _current_stream(idx)
     with _lock:
         q = _deferred.get(idx)
         if q is None:
@@ -143,7 +159,7 @@ def defer_bn(device, key, job):
     in ONE launch on the caller's stream when the queue runs.  A backward hook: the first
     one of a pass runs what the forward hooks have queued."""
     idx = device.index if device.index is not None else torch.cuda.current_device()
-    stream = torch.cuda.current_stream(device)
+    stream = _current_stream(idx)
     with _lock:
         q = _deferred.get(idx)
         if q is None:

@@ -11,7 +11,7 @@ import torch
 import torch.nn as nn
 
 from torchsso import _lanes, _ops
-from torchsso.curv.curvature import Curvature, DiagCurvature
+from torchsso.curv.curvature import Curvature, DiagCurvature, _attach
 
 
 class CovBatchNorm1d(Curvature):
@@ -48,8 +48,8 @@ class _DiagCovBatchNorm(DiagCurvature):
             x_hat = (out - bn.bias.detach().view(shape)) / bn.weight.detach().view(shape)
         else:
             x_hat = None
-        setattr(module, 'data_input', x_hat)
-        setattr(module, 'data_output', output)
+        _attach(module, 'data_input', x_hat)
+        _attach(module, 'data_output', output)
         if output.requires_grad:
             output.register_hook(self._on_grad_output)
 

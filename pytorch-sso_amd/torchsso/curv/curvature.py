@@ -29,6 +29,20 @@ from torchsso import _lanes, _ops
 PI_TYPE_TRACENORM = 'tracenorm'
 
 
+def _attach(module, name, value):
+    """setattr(module, name, value) for what the hooks leave on a module.  A plain tensor under
+    a name that is no parameter, buffer, child or member of the class is an ordinary attribute,
+    stored without Module.__setattr__'s search through those (1 us a time, 400 times in a
+    ResNet-50 pass)."""
+    if ((value is None or type(value) is torch.Tensor)
+            and type(module).__setattr__ is nn.Module.__setattr__
+            and name not in module._parameters and name not in module._buffers
+            and name not in module._modules and not hasattr(type(module), name)):
+        module.__dict__[name] = value
+    else:
+        setattr(module, name, value)
+
+
 class Curvature(object):
     """Base class (reference: curvature.py:10-212)."""
 
@@ -123,8 +137,8 @@ class Curvature(object):
         """Forward hook (reference: curvature.py:118-139)."""
         assert self._module == module
         data_input = input[0].detach()
-        setattr(module, 'data_input', data_input)
-        setattr(module, 'data_output', output)
+        _attach(module, 'data_input', data_input)
+        _attach(module, 'data_output', output)
         self.update_in_forward(data_input)
         if isinstance(output, torch.Tensor) and output.requires_grad:
             output.register_hook(self._on_grad_output)
@@ -143,8 +157,8 @@ class Curvature(object):
         if grad_input is not None:
             index = 1 if self.bias else 0
             grad_input = None if grad_input[index] is None else grad_input[index].detach()
-        setattr(module, 'grad_input', grad_input)
-        setattr(module, 'grad_output', grad_output)
+        _attach(module, 'grad_input', grad_input)
+        _attach(module, 'grad_output', grad_output)
         self.update_in_backward(grad_output)
 
     def adjust_data_scale(self, scale):

@@ -131,11 +131,17 @@ class VIOptimizer(SecondOrderOptimizer):
 
     def zero_grad(self, set_to_none=False):
         """Clears the gradients of the parameters and of the posterior means."""
+        dense = []
         for group in self.param_groups:
             for t in list(group['mean']) + list(group['params']):
                 if t.grad is not None:
                     t.grad.detach_()
-                    t.grad.zero_()
+                    if t.grad.layout == torch.strided:
+                        dense.append(t.grad)
+                    else:
+                        t.grad.zero_()
+        if dense:
+            torch._foreach_zero_(dense)          # (one launch instead of one per tensor)
 
     @property
     def seed(self):
@@ -165,11 +171,16 @@ class VIOptimizer(SecondOrderOptimizer):
 
     @staticmethod
     def _means_into(groups, with_grads):
+        to, source = [], []
         for group in groups:
             for p, m in zip(group['params'], group['mean']):
-                p.data.copy_(m.data)
+                to.append(p.data)
+                source.append(m.data)
                 if with_grads and p.grad is not None and m.grad is not None:
-                    p.grad.copy_(m.grad)
+                    to.append(p.grad)
+                    source.append(m.grad)
+        if to:
+            torch._foreach_copy_(to, source)     # (one launch instead of one per tensor)
 
     def copy_mean_to_params(self):
         self._means_into(self.param_groups, with_grads=True)
