@@ -56,15 +56,20 @@ int conv_a_taps_grouped(int count, const TapsJob* jobs, void* workspace, size_t 
 
 // Blocks per piece of the cut reductions of a launch of 128x128 tiles (0: none is cut).
 // `work` = sum over the tiles of their reduction length in blocks, `longest` = the longest
-// of them: with the work spread evenly over the chip's resident workgroups (3 per CU) the
-// launch would last work / 768 block times, and it cannot end before its longest tile does
-// (which shares its compute unit with two other workgroups until the launch thins out).
+// of them: with the work spread evenly over the chip's resident workgroups (2 per CU) the
+// launch would last work / 512 block times, and it cannot end before its longest tile does
+// (which shares its compute unit with another workgroup until the launch thins out).
 // Where the longest tile is the longer of the two, reductions are cut into pieces that are
 // work items of the same launch and store raw partial tiles; a short launch afterwards adds
 // the pieces of every cut tile up in order (splitk_sum).
-constexpr int MIN_PIECE_BLOCKS = 4;
+// MIN_PIECE_BLOCKS: a shorter piece writes and reads its partial for too little work.
+// Preconditioning of a 784-1000-1000-10 network / a conv net (1600, 3201) / slim and full
+// ResNet-50 with pieces of at least 1, 2, 3, 4 blocks: 207 176 172 187 / 252 219 185 194 /
+// 565 562 540 538 / 988 992 992 995 us (4 blocks and work / 768: 192 / 195 / 546 / 1113).
+constexpr int MIN_PIECE_BLOCKS = 3;
+constexpr int RESIDENT_TILES = 512;
 inline int piece_blocks(long work, int longest) {
-  const long even = work / 768 + 1;
+  const long even = work / RESIDENT_TILES + 1;
   if (longest <= MIN_PIECE_BLOCKS || 3 * (long)longest <= 4 * even) return 0;
   const long pb = even / 2 > MIN_PIECE_BLOCKS ? even / 2 : MIN_PIECE_BLOCKS;
   return pb >= longest ? 0 : (int)pb;

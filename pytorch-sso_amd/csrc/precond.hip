@@ -359,7 +359,7 @@ static size_t piece_floats(int dG, int dA, const int (&pbs)[4]) {
   return most > 1 ? (size_t)ta * tg * most * (BM * BN) : 0;
 }
 
-// scratch: one descriptor table per product, then per layer dG*dA floats (twice that when
+// scratch: the descriptor tables, then per layer dG*dA floats (twice that when
 // `factored`: a layer with a factored side keeps two results in flight) and its piece area
 static size_t precond_workspace(int layers, const int* dG, const int* dA, bool factored) {
   size_t bytes = PRODUCTS * align256((size_t)layers * sizeof(LayerDesc));
@@ -391,9 +391,10 @@ static int run_layers(int layers, const int* dG, const int* dA, const float* con
   }
   // Longest tiles first, so that the tail of a launch is made of short tiles: each
   // product walks the layers in the order of ITS reduction length (dG for the first and
-  // fourth, dA for the second and third), through a descriptor table of its own.
-  const size_t table_bytes = align256((size_t)layers * sizeof(LayerDesc));
-  char* tbase = (char*)workspace + PRODUCTS * table_bytes;
+  // fourth, dA for the second and third), through a descriptor table in that order.
+  // (two orders, so two tables, one behind the other; uploaded together, which for a few
+  // layers is one launch)
+  char* tbase = (char*)workspace + PRODUCTS * align256((size_t)layers * sizeof(LayerDesc));
   // pieces as large as the scratch was sized for, at least (the query assumed that every
   // side is a triangular factor), and none where it left no room
   const std::vector<int> no_flags(layers, 0);     // explicit inverses on both sides
@@ -437,38 +438,41 @@ static int run_layers(int layers, const int* dG, const int* dA, const float* con
     shape(product, l, part, tri, tslow, tfast);
     return part && piece_count(tfast, pbs[product]) > 1 ? tslow * tfast : 0;
   };
-  std::vector<int> order(layers);
+  std::vector<int> by_g(layers), by_a(layers);
+  for (int l = 0; l < layers; ++l) by_g[l] = by_a[l] = l;
+  std::stable_sort(by_g.begin(), by_g.end(), [&](int a, int b) { return dG[a] > dG[b]; });
+  std::stable_sort(by_a.begin(), by_a.end(), [&](int a, int b) { return dA[a] > dA[b]; });
+  for (int s0 = 0; s0 < 2 * layers; s0 += LAYER_CHUNK) {
+    LayerChunk chunk;
+    const int cnt = std::min(LAYER_CHUNK, 2 * layers - s0);
+    for (int k = 0; k < cnt; ++k) {
+      const int at = s0 + k;
+      const int l = at < layers ? by_g[at] : by_a[at - layers];
+      LayerDesc& d = chunk.d[k];
+      d.L = L[l];
+      d.R = R[l];
+      d.V = V[l];
+      d.vb = vb ? vb[l] : nullptr;
+      d.meanW = meanW ? meanW[l] : nullptr;
+      d.meanb = meanb ? meanb[l] : nullptr;
+      d.outW = outW[l];
+      d.outb = outb ? outb[l] : nullptr;
+      d.Tt = (float*)(tbase + toff[l]);
+      d.dG = dG[l];
+      d.dA = dA[l];
+      d.dAw = dA[l] - (has_bias[l] ? 1 : 0);
+      d.scale = scale;
+      d.flags = flags ? flags[l] : 0;
+      d.parts = (float*)(tbase + poff[l]);
+    }
+    hipLaunchKernelGGL(layer_setup_kernel, dim3(1), dim3(LAYER_CHUNK), 0, stream, chunk,
+                       (LayerDesc*)workspace, s0, cnt);
+  }
   for (int product = 0; product < PRODUCTS; ++product) {
     if (!any[product]) continue;
-    LayerDesc* const table = (LayerDesc*)((char*)workspace + product * table_bytes);
-    const int* key = (product == 0 || product == 3) ? dG : dA;
-    for (int l = 0; l < layers; ++l) order[l] = l;
-    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return key[a] > key[b]; });
-    for (int s0 = 0; s0 < layers; s0 += LAYER_CHUNK) {
-      LayerChunk chunk;
-      const int cnt = std::min(LAYER_CHUNK, layers - s0);
-      for (int k = 0; k < cnt; ++k) {
-        const int l = order[s0 + k];
-        LayerDesc& d = chunk.d[k];
-        d.L = L[l];
-        d.R = R[l];
-        d.V = V[l];
-        d.vb = vb ? vb[l] : nullptr;
-        d.meanW = meanW ? meanW[l] : nullptr;
-        d.meanb = meanb ? meanb[l] : nullptr;
-        d.outW = outW[l];
-        d.outb = outb ? outb[l] : nullptr;
-        d.Tt = (float*)(tbase + toff[l]);
-        d.dG = dG[l];
-        d.dA = dA[l];
-        d.dAw = dA[l] - (has_bias[l] ? 1 : 0);
-        d.scale = scale;
-        d.flags = flags ? flags[l] : 0;
-        d.parts = (float*)(tbase + poff[l]);
-      }
-      hipLaunchKernelGGL(layer_setup_kernel, dim3(1), dim3(LAYER_CHUNK), 0, stream, chunk,
-                         table, s0, cnt);
-    }
+    const bool g_order = product == 0 || product == 3;
+    const std::vector<int>& order = g_order ? by_g : by_a;
+    LayerDesc* const table = (LayerDesc*)workspace + (g_order ? 0 : layers);
     // every launch of a product is enqueued before any of the next one (stream order is
     // the dependency)
     const int pb = pbs[product];
