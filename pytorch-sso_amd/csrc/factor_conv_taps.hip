@@ -59,6 +59,7 @@ struct ShiftX {
   // the positions of a row of the rectangle are consecutive
   __device__ __forceinline__ bool runs() const { return ww >= 4; }
   __device__ __forceinline__ bool quads() const { return (ww & 3) == 0; }
+  __device__ __forceinline__ bool padded() const { return false; }
   __device__ __forceinline__ KRun run(int k) const {
     const int n = by_area.div(k);
     const int rem = k - n * hh * ww;

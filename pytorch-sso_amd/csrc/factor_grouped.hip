@@ -233,10 +233,11 @@ struct Classified {
   int OH, OW;
   int Hs;                // P_CONVP: rows of a plane of the copy
   size_t copy_bytes;     // P_CONVP: 0 when the input itself serves
+  int positions;         // P_CONVG, P_CONVP: index positions of an image (see padded_run)
 };
 
-static Classified classify(const kfac_factor_job& j) {
-  Classified c{P_BAD, 0, 0, 0, 0, 0, 0};
+static Classified classify_shape(const kfac_factor_job& j) {
+  Classified c{P_BAD, 0, 0, 0, 0, 0, 0, 0};
   if (j.rows <= 0 || j.c <= 0) return c;
   const int bias = j.add_bias ? 1 : 0;
   if (j.kind == KFAC_FACTOR_LINEAR) {
@@ -291,6 +292,16 @@ static Classified classify(const kfac_factor_job& j) {
       c.copy_bytes = as_is ? 0 : (size_t)copy;
     }
   }
+  return c;
+}
+
+// ... and the reduction index of products in runs, on 128-wide tiles with padded runs
+static Classified classify(const kfac_factor_job& j) {
+  Classified c = classify_shape(j);
+  if (c.path != P_CONVG && c.path != P_CONVP) return c;
+  const int run = c.path == P_CONVG ? j.H * j.W : c.OH * c.OW;
+  c.positions = c.d > GROUP_W1_MAX_DIM ? padded_run(run) : run;
+  c.K = (long)j.rows * c.positions;
   return c;
 }
 
@@ -511,8 +522,8 @@ DenseKM make_op<DenseKM>(const kfac_factor_job& j, const Classified& c) {
   return DenseKM{j.x, nullptr, j.c, c.d, j.add_bias ? 1 : 0};
 }
 template <>
-ConvG make_op<ConvG>(const kfac_factor_job& j, const Classified&) {
-  return ConvG(j.x, j.c, j.H * j.W);
+ConvG make_op<ConvG>(const kfac_factor_job& j, const Classified& c) {
+  return ConvG(j.x, j.c, j.H * j.W, c.positions);
 }
 template <>
 ConvA make_op<ConvA>(const kfac_factor_job& j, const Classified& c) {
@@ -522,7 +533,8 @@ ConvA make_op<ConvA>(const kfac_factor_job& j, const Classified& c) {
 
 template <>
 ConvP make_op<ConvP>(const kfac_factor_job& j, const Classified& c) {
-  return ConvP(j.x, j.c, j.kh, j.kw, j.sh, j.dh, c.Hs, c.OH, c.OW, c.d, j.add_bias ? 1 : 0);
+  return ConvP(j.x, j.c, j.kh, j.kw, j.sh, j.dh, c.Hs, c.OH, c.OW, c.d, j.add_bias ? 1 : 0,
+               c.positions);
 }
 
 struct Launch {

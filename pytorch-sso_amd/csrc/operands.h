@@ -104,11 +104,14 @@ struct ConvG {
   static constexpr int kruns = K_RUNS;
   static constexpr bool has_second = false;
   const float* p;
+  static constexpr bool pads_runs = true;
   int C, HW;
-  FastDiv by_hw;
+  int HWp;             // index positions of an image (HW, or padded_run(HW))
+  FastDiv by_hw;       // division by HWp
   ConvG() = default;
-  __host__ __device__ ConvG(const float* p_, int C_, int HW_)
-      : p(p_), C(C_), HW(HW_), by_hw((unsigned)HW_) {}
+  __host__ __device__ ConvG(const float* p_, int C_, int HW_) : ConvG(p_, C_, HW_, HW_) {}
+  __host__ __device__ ConvG(const float* p_, int C_, int HW_, int HWp_)
+      : p(p_), C(C_), HW(HW_), HWp(HWp_), by_hw((unsigned)HWp_) {}
   struct MS { unsigned off; };
   struct KS { unsigned off; };
   __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc() const {
@@ -118,15 +121,17 @@ struct ConvG {
     return MS{m < C ? (unsigned)(m * HW) * 4u : INV_M};
   }
   __device__ __forceinline__ KS kstate(int k, bool valid) const {
-    const int n = by_hw.div(k);
-    return KS{k_offset_or_invalid((unsigned)(n * C * HW + (k - n * HW)) * 4u, valid)};
+    const int n = by_hw.div(k), pos = k - n * HWp;
+    return KS{k_offset_or_invalid((unsigned)(n * C * HW + pos) * 4u, valid && pos < HW)};
   }
   // the positions of an image are consecutive
   __device__ __forceinline__ bool runs() const { return HW >= 4; }
   __device__ __forceinline__ bool quads() const { return (HW & 3) == 0; }
+  __device__ __forceinline__ bool padded() const { return HWp != HW; }
   __device__ __forceinline__ KRun run(int k) const {
-    const int n = by_hw.div(k), pos = k - n * HW, image = n * C * HW;
-    return KRun{(unsigned)(image + pos) * 4u, (unsigned)(image + C * HW) * 4u, HW - pos};
+    const int n = by_hw.div(k), pos = k - n * HWp, image = n * C * HW;
+    return KRun{(unsigned)(image + pos) * 4u, padded() ? INV_K : (unsigned)(image + C * HW) * 4u,
+                HW - pos};
   }
   __device__ __forceinline__ unsigned off(const MS& m, const KS& k) const { return m.off + k.off; }
   __device__ __forceinline__ bool is_one(const MS&) const { return false; }
@@ -212,15 +217,17 @@ struct ConvP {
   static constexpr int kruns = K_RUNS;
   static constexpr bool has_second = false;
   const float* p;
+  static constexpr bool pads_runs = true;
   int C, KH, KW, SH, DH, Hs, OHW, OW, M, ones;
   int image;           // floats per image: C*SH*KW planes (+ OH*OW ones)
-  FastDiv by_l;        // division by OH*OW
+  int Lp;              // index positions of an image (OH*OW, or padded_run of it)
+  FastDiv by_l;        // division by Lp
   ConvP() = default;
   __host__ __device__ ConvP(const float* p_, int C_, int KH_, int KW_, int SH_, int DH_, int Hs_,
-                            int OH_, int OW_, int M_, int ones_)
+                            int OH_, int OW_, int M_, int ones_, int Lp_)
       : p(p_), C(C_), KH(KH_), KW(KW_), SH(SH_), DH(DH_), Hs(Hs_), OHW(OH_ * OW_), OW(OW_), M(M_),
         ones(ones_), image(C_ * SH_ * KW_ * Hs_ * OW_ + (ones_ ? OH_ * OW_ : 0)),
-        by_l((unsigned)(OH_ * OW_)) {}
+        Lp(Lp_), by_l((unsigned)Lp_) {}
   struct MS { unsigned off; };
   struct KS { unsigned off; };
   __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc() const { return make_rsrc(p); }
@@ -238,14 +245,16 @@ struct ConvP {
     return s;
   }
   __device__ __forceinline__ KS kstate(int k, bool valid) const {
-    const int n = by_l.div(k);
-    return KS{k_offset_or_invalid((unsigned)(n * image + (k - n * OHW)) * 4u, valid)};
+    const int n = by_l.div(k), pos = k - n * Lp;
+    return KS{k_offset_or_invalid((unsigned)(n * image + pos) * 4u, valid && pos < OHW)};
   }
   __device__ __forceinline__ bool runs() const { return OHW >= 4; }
   __device__ __forceinline__ bool quads() const { return (OHW & 3) == 0; }
+  __device__ __forceinline__ bool padded() const { return Lp != OHW; }
   __device__ __forceinline__ KRun run(int k) const {
-    const int n = by_l.div(k), pos = k - n * OHW;
-    return KRun{(unsigned)(n * image + pos) * 4u, (unsigned)((n + 1) * image) * 4u, OHW - pos};
+    const int n = by_l.div(k), pos = k - n * Lp;
+    return KRun{(unsigned)(n * image + pos) * 4u, padded() ? INV_K : (unsigned)((n + 1) * image) * 4u,
+                OHW - pos};
   }
   __device__ __forceinline__ unsigned off(const MS& m, const KS& k) const { return m.off + k.off; }
   __device__ __forceinline__ bool is_one(const MS&) const { return false; }

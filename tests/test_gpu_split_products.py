@@ -46,6 +46,37 @@ def test_dense_symmetric(ops, dev, f, rows, bias):
     assert torch.equal(out, out.t())
 
 
+# one run of a multiple of 4, padded runs (6 = 8 - 2, 7, 9 = 12 - 3, ...), runs left as they are (1 .. 5)
+@pytest.mark.parametrize('hw', [(1, 1), (1, 3), (2, 2), (1, 5), (2, 3), (1, 7), (3, 3), (2, 5), (3, 5),
+                                (7, 7), (5, 13), (8, 8)])
+@pytest.mark.parametrize('n', [1, 2, 5, 40])
+def test_positions_in_runs_of_a_grouped_call(ops, dev, n, hw):
+    """Output gradients of two sizes, a pointwise and a strided convolution's input in one call;
+    nothing but the positions themselves may reach the sums, whatever lies beside a run."""
+    gen = torch.Generator(device=dev).manual_seed(n * 100 + hw[0] * hw[1])
+    randn = lambda *shape: torch.randn(*shape, device=dev, generator=gen)
+    positions = lambda t: t.double().permute(0, 2, 3, 1).reshape(-1, t.shape[1])
+    g, h, x = randn(n, 200, *hw), randn(n, 65, *hw), randn(n, 257, *hw)
+    s = randn(n, 23, 2 * hw[0] + 1, 2 * hw[1] + 1)          # 3x3, stride 2: hw output positions
+    g[0, 199], g[0, 198] = 1e18, 1.
+    cols = torch.nn.functional.unfold(s.double(), 3, stride=2)         # [n, 23 * 9, positions]
+    jobs, outs, rows = [], [], []
+    for kind, t, rows64, geometry in (
+            ('conv_g', g, positions(g), {}), ('conv_g', h, positions(h), {}),
+            ('conv_a', x, positions(x), dict(kernel_size=1, stride=1, padding=0, dilation=1)),
+            ('conv_a', s, cols.permute(0, 2, 1).reshape(-1, cols.shape[1]),
+             dict(kernel_size=3, stride=2, padding=0, dilation=1))):
+        out = torch.full((rows64.shape[1],) * 2, float('nan'), device=dev)
+        jobs.append(ops.factor_job(kind, t, 1., out, **geometry))
+        outs.append(out)
+        rows.append(rows64)
+    ops.factor_grouped(jobs, dev)
+    torch.cuda.synchronize()
+    for k, (out, a) in enumerate(zip(outs, rows)):
+        _assert_float32_sum(out, a, a, 'product %d, %d images of %dx%d' % ((k, n) + hw))
+        assert torch.equal(out, out.t())
+
+
 @pytest.mark.parametrize('hw', [(1, 1), (1, 3), (2, 2), (3, 3), (7, 7), (5, 13), (8, 8)])
 @pytest.mark.parametrize('n', [1, 5])
 def test_positions_in_runs(ops, dev, n, hw):
