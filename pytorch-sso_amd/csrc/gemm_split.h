@@ -78,6 +78,14 @@ __device__ __forceinline__ void split_pair(float a, float b, unsigned& h, unsign
   l = pack_bf16(ra - bf16_lo(m), rb - bf16_hi(m));
 }
 
+// Leading sums + corrections.  An infinite element has no rest (inf - inf), and beyond 3.4e38
+// the corrections overflow with either sign: where they are not finite the leading sum is the
+// result, infinite with its sign as a float32 sum's, and NaN only where that is.
+__device__ __forceinline__ void add_corrections(v16f& acc, const v16f& cor) {
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] += __builtin_isfinite(cor[i]) ? cor[i] : 0.f;
+}
+
 // the element at `off` (per lane, range-checked) + `at` (the same for all lanes)
 __device__ __forceinline__ float buffer_load_at(__amdgpu_buffer_rsrc_t r, unsigned off, unsigned at) {
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, (int)at, 0));
@@ -517,7 +525,7 @@ __device__ __forceinline__ void split_blocks(const OPP& P, const OPQ& Q, int m0,
     split_tile_loop<WM, WN, TRI, ANY_K>(P, Q, m0, n0, kbeg, kend, sm, prow, qrow, acc, cor);
   }
 #pragma unroll
-  for (int b = 0; b < (TRI ? 3 : 4); ++b) acc[b] += cor[b];
+  for (int b = 0; b < (TRI ? 3 : 4); ++b) add_corrections(acc[b], cor[b]);
 }
 
 // The 32x32 blocks of a wave, rows from `row0`, columns from `col0`, through the epilogue.

@@ -698,7 +698,7 @@ __device__ __forceinline__ void step_tile(const float* p, const float* q, float*
   products();
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    acc[i] += cor[i];
+    add_corrections(acc[i], cor[i]);
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
       const int row = m0 + wm + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);

@@ -99,6 +99,27 @@ def test_magnitudes(ops, dev, exponent):
     _assert_float32_sum(out, x.double(), x.double(), 'magnitudes around 1e%d' % exponent)
 
 
+@pytest.mark.parametrize('hw', [(4, 8), (7, 7)])
+def test_infinities_and_overflow(ops, dev, hw):
+    """What a float32 sum gives where it is not finite: inf with its sign, NaN only for
+    NaN and for inf - inf; everything else as if those elements were not there."""
+    gen = torch.Generator(device=dev).manual_seed(6)
+    g = torch.rand(3, 300, *hw, device=dev, generator=gen) + 0.1
+    g[1, 10, 1, 2] = float('inf')
+    g[0, 140, -1, -3] = -float('inf')    # (brought twice by a padded run's last load)
+    g[2, 270, -1, -1] = float('nan')
+    g[:, 20] *= 1.1e25                        # its square overflows, nothing else does
+    x = g.permute(0, 2, 3, 1).reshape(-1, 300).contiguous()
+    want = x.cpu().t() @ x.cpu()
+    for out in (ops.factor_conv_g(g, 1.), ops.factor_linear(x, False, 1.)):
+        out = out.cpu()
+        assert torch.equal(out.isnan(), want.isnan())
+        assert torch.equal(out.isposinf(), want.isposinf())
+        assert torch.equal(out.isneginf(), want.isneginf())
+        ok = want.isfinite()
+        assert ((out - want)[ok] / want[ok]).abs().max().item() < 1e-5
+
+
 def test_positive_terms(ops, dev):
     # no drift where all terms have one sign
     gen = torch.Generator(device=dev).manual_seed(4)
