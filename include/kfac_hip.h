@@ -156,8 +156,8 @@ double kfac_factor_grouped_executed_flops(int count, const kfac_factor_job* jobs
  * n x n buffer per matrix.  `dims` is a HOST array of `count` sizes. */
 size_t kfac_inverse_workspace_bytes(int count, const int* dims);
 
-/* Plan query: the fp32 MFMA flops the batched inversion executes for matrices of these
- * sizes (HOST arrays): blocked Cholesky (diagonal blocks, row panels, trailing updates
+/* Plan query: the flops of float32 products that the batched inversion executes on the matrix
+ * cores for matrices of these sizes (HOST arrays): blocked Cholesky (diagonal blocks, row panels, trailing updates
  * with whole diagonal tiles), the triangular inverse, and Y Y^T for the matrices whose
  * explicit inverse is formed (factored[i] == 0, or factored == NULL). */
 double kfac_inverse_executed_flops(int count, const int* dims, const int* factored);

@@ -1586,8 +1586,19 @@ double kfac_inverse_executed_flops(int count, const int* dims, const int* factor
   // strips (12 + 8 blocks, 32 deep), the pending panel (10 blocks, 128 deep)
   const double diag = 4096. * (4 * 120 + 20 * 16 + 10 * 64);
   double total = 0.;
+  std::vector<int> Ts(count);
+  for (int i = 0; i < count; ++i) Ts[i] = cdiv(dims[i], DB);
+  if (use_sweep(Ts)) {
+    for (int i = 0; i < count; ++i) {
+      const int T = Ts[i];
+      total += T * diag + B * T * (T - 1);      // diagonal blocks; row panels of U and Z
+      for (int p = 1; p <= T; ++p)              // (tile (p, p) is the diagonal block's)
+        total += B * (sweep_items(T, p, !(factored && factored[i])) - (p < T ? 1 : 0));
+    }
+    return total;
+  }
   for (int i = 0; i < count; ++i) {
-    const double T = cdiv(dims[i], DB);
+    const double T = Ts[i];
     // Cholesky: row panels, trailing updates (whole diagonal tiles)
     total += T * diag + B * (T * (T - 1) / 2 + (T - 1) * T * (T + 1) / 6);
     // triangular inverse: per merge of r x c blocks, W tiles reduce over 1..c blocks,
