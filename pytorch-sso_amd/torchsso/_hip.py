@@ -200,7 +200,7 @@ def stream_ptr(device=None, stream=None):
     """Raw handle of `stream` (a torch.cuda.Stream), or of torch's current stream."""
     if stream is not None:
         return stream.cuda_stream
-    index = getattr(device, 'index', None)
+    index = device.index if isinstance(device, torch.device) else None
     if index is None:
         return torch.cuda.current_stream(device).cuda_stream
     return torch._C._cuda_getCurrentRawStream(index)     # (no Stream object around the handle)
