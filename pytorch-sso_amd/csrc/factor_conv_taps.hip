@@ -38,9 +38,11 @@ struct ShiftX {
   static constexpr int layout = MK;
   static constexpr int kruns = K_RUNS;
   static constexpr bool has_second = false;
+  static constexpr bool pads_runs = true;
   const float* p;
   int C, H, W, u0, v0, hh, ww;     // u0, v0 already include the displacement
-  FastDiv by_area, by_ww;
+  int wwp;                         // index positions of a row (row_positions)
+  FastDiv by_area, by_ww;          // divisions by hh * wwp and by wwp
   struct MS { unsigned off; };
   struct KS { unsigned off; };
   __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc() const { return make_rsrc(p); }
@@ -49,33 +51,41 @@ struct ShiftX {
   }
   __device__ __forceinline__ KS kstate(int k, bool valid) const {
     const int n = by_area.div(k);
-    const int rem = k - n * hh * ww;
+    const int rem = k - n * hh * wwp;
     const int ry = by_ww.div(rem);
-    const int rx = rem - ry * ww;
-    return KS{k_offset_or_invalid((unsigned)(n * C * H * W + (u0 + ry) * W + v0 + rx) * 4u, valid)};
+    const int rx = rem - ry * wwp;
+    return KS{k_offset_or_invalid((unsigned)(n * C * H * W + (u0 + ry) * W + v0 + rx) * 4u,
+                                  valid && rx < ww)};
   }
   __device__ __forceinline__ unsigned off(const MS& m, const KS& k) const { return m.off + k.off; }
   __device__ __forceinline__ bool is_one(const MS&) const { return false; }
   // the positions of a row of the rectangle are consecutive
   __device__ __forceinline__ bool runs() const { return ww >= 4; }
   __device__ __forceinline__ bool quads() const { return (ww & 3) == 0; }
-  __device__ __forceinline__ bool padded() const { return false; }
+  __device__ __forceinline__ bool padded() const { return wwp != ww; }
+  // what the offset of a k inside the range is beyond that of `o`, another displacement
+  __device__ __forceinline__ unsigned k_shift(const ShiftX& o) const {
+    return (unsigned)((u0 - o.u0) * W + v0 - o.v0) * 4u;
+  }
   __device__ __forceinline__ KRun run(int k) const {
     const int n = by_area.div(k);
-    const int rem = k - n * hh * ww;
+    const int rem = k - n * hh * wwp;
     const int ry = by_ww.div(rem);
-    const int rx = rem - ry * ww;
+    const int rx = rem - ry * wwp;
     const int row = n * C * H * W + (u0 + ry) * W + v0;
     const int next = ry + 1 < hh ? row + W : (n + 1) * C * H * W + u0 * W + v0;
-    return KRun{(unsigned)(row + rx) * 4u, (unsigned)next * 4u, ww - rx};
+    return KRun{(unsigned)(row + rx) * 4u, padded() ? INV_K : (unsigned)next * 4u, ww - rx};
   }
 };
 
+// Index positions of a row of a rectangle: padded (padded_run) for 128-wide tiles.
+__host__ __device__ inline int row_positions(int ww, int w) { return w == 2 ? padded_run(ww) : ww; }
+
 struct JobDesc {
-  short u0, v0, hh, ww;    // rectangle of the first factor; the reduction runs over n * hh * ww
+  short u0, v0, hh, ww;    // rectangle of the first factor; the reduction runs over its rows (row_positions)
   short dy, dx;            // displacement of the second factor
   short splits;            // k-splits
-  unsigned char sh_area, sh_ww;   // shifts of the two FastDiv (by hh * ww and by ww)
+  unsigned char sh_area, sh_ww;   // shifts of the two FastDiv of a ShiftX
   unsigned m_area, m_ww;          // their multipliers
   int cps;                 // chunks per split
   int part0;               // index (in C*C units) of its first partial in the workspace
@@ -109,7 +119,8 @@ __device__ __forceinline__ void corr_product(const float* x, int nimg, int C, in
   constexpr int KC = Cfg<W, W>::KC;
   const JobDesc jd = plan.jobs[j];
   const int bi = tile / tiles_side, bj = tile - bi * tiles_side;
-  const int K = nimg * jd.hh * jd.ww;
+  const int wwp = row_positions(jd.ww, W);
+  const int K = nimg * jd.hh * wwp;
   const int kbeg = split * jd.cps * KC;
   int kend = kbeg + jd.cps * KC;
   if (kend > K) kend = K;
@@ -118,8 +129,8 @@ __device__ __forceinline__ void corr_product(const float* x, int nimg, int C, in
   by_area.sh = jd.sh_area;
   by_ww.m = jd.m_ww;
   by_ww.sh = jd.sh_ww;
-  ShiftX P{x, C, H, Wd, jd.u0, jd.v0, jd.hh, jd.ww, by_area, by_ww};
-  ShiftX Q{x, C, H, Wd, jd.u0 + jd.dy, jd.v0 + jd.dx, jd.hh, jd.ww, by_area, by_ww};
+  ShiftX P{x, C, H, Wd, jd.u0, jd.v0, jd.hh, jd.ww, wwp, by_area, by_ww};
+  ShiftX Q{x, C, H, Wd, jd.u0 + jd.dy, jd.v0 + jd.dx, jd.hh, jd.ww, wwp, by_area, by_ww};
   EpiStore epi{ws + (size_t)(jd.part0 + split) * C * C, C, C, C, 1.f, 0.f, false};
   if constexpr (W == 2)
     split_tile(P, Q, bi * TS, bj * TS, kbeg, kend, false, epi, smem);
@@ -447,6 +458,7 @@ static TapPlanHost plan_taps(int n, int c, int H, int Wd, int kh, int kw, int ph
                              int dw, int group_cps = 0) {
   TapPlanHost hp;
   hp.ok = false;
+  hp.w = c <= 64 ? 1 : 2;
   const int T = kh * kw;
   if (T < 2 || T > MAX_TAPS) return hp;
   const int OH = H + 2 * ph - dh * (kh - 1), OW = Wd + 2 * pw - dw * (kw - 1);
@@ -477,7 +489,8 @@ static TapPlanHost plan_taps(int n, int c, int H, int Wd, int kh, int kw, int ph
             jd.v0 = (short)ax.pieces[px].lo;
             jd.ww = (short)(ax.pieces[px].hi - ax.pieces[px].lo);
             jd.dx = (short)ax.pieces[px].delta;
-            const FastDiv fa((unsigned)(jd.hh * jd.ww)), fw((unsigned)jd.ww);
+            const int wwp = row_positions(jd.ww, hp.w);
+            const FastDiv fa((unsigned)(jd.hh * wwp)), fw((unsigned)wwp);
             jd.m_area = fa.m;
             jd.sh_area = (unsigned char)fa.sh;
             jd.m_ww = fw.m;
@@ -490,13 +503,12 @@ static TapPlanHost plan_taps(int n, int c, int H, int Wd, int kh, int kw, int ph
       pd.pair_first[pd.npairs] = (short)npj;
     }
   // tiles and k-splits: work items in proportion to each job's length
-  hp.w = c <= 64 ? 1 : 2;
   const int ts = 64 * hp.w;
   hp.tiles_side = cdiv(c, ts);
   const int ntiles = hp.tiles_side * hp.tiles_side;
   const int kc = hp.w == 1 ? Cfg<1, 1>::KC : Cfg<2, 2>::KC;
   double total = 0;
-  auto job_k = [&](const JobDesc& jd) { return (long)n * jd.hh * jd.ww; };
+  auto job_k = [&](const JobDesc& jd) { return (long)n * jd.hh * row_positions(jd.ww, hp.w); };
   for (int j = 0; j < pd.njobs; ++j) total += (double)job_k(pd.jobs[j]);
   // All workgroups of a launch that fits the chip are resident at once (3 four-wave
   // workgroups per CU: 768) and share the matrix cores of their CU, so the launch lasts as
@@ -549,7 +561,7 @@ static double plan_executed_flops(const TapPlanHost& hp, int n) {
   double total = 0.;
   for (int j = 0; j < hp.dev.njobs; ++j) {
     const JobDesc& jd = hp.dev.jobs[j];
-    const long K = (long)n * jd.hh * jd.ww;
+    const long K = (long)n * jd.hh * row_positions(jd.ww, hp.w);
     total += ntiles * (double)((K + kc - 1) / kc) * kc * 2.0 * ts * ts;
   }
   return total;

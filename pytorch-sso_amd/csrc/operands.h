@@ -128,6 +128,7 @@ struct ConvG {
   __device__ __forceinline__ bool runs() const { return HW >= 4; }
   __device__ __forceinline__ bool quads() const { return (HW & 3) == 0; }
   __device__ __forceinline__ bool padded() const { return HWp != HW; }
+  __device__ __forceinline__ unsigned k_shift(const ConvG&) const { return 0; }
   __device__ __forceinline__ KRun run(int k) const {
     const int n = by_hw.div(k), pos = k - n * HWp, image = n * C * HW;
     return KRun{(unsigned)(image + pos) * 4u, padded() ? INV_K : (unsigned)(image + C * HW) * 4u,
@@ -251,6 +252,7 @@ struct ConvP {
   __device__ __forceinline__ bool runs() const { return OHW >= 4; }
   __device__ __forceinline__ bool quads() const { return (OHW & 3) == 0; }
   __device__ __forceinline__ bool padded() const { return Lp != OHW; }
+  __device__ __forceinline__ unsigned k_shift(const ConvP&) const { return 0; }
   __device__ __forceinline__ KRun run(int k) const {
     const int n = by_l.div(k), pos = k - n * Lp;
     return KRun{(unsigned)(n * image + pos) * 4u, padded() ? INV_K : (unsigned)((n + 1) * image) * 4u,

@@ -46,7 +46,7 @@ def test_dense_symmetric(ops, dev, f, rows, bias):
     assert torch.equal(out, out.t())
 
 
-# one run of a multiple of 4, padded runs (6 = 8 - 2, 7, 9 = 12 - 3, ...), runs left as they are (1 .. 5)
+# one run of a multiple of 4, padded runs (5 = 8 - 3, 6, 7, 9, ...), runs left as they are (1 .. 3)
 @pytest.mark.parametrize('hw', [(1, 1), (1, 3), (2, 2), (1, 5), (2, 3), (1, 7), (3, 3), (2, 5), (3, 5),
                                 (7, 7), (5, 13), (8, 8)])
 @pytest.mark.parametrize('n', [1, 2, 5, 40])
@@ -87,6 +87,24 @@ def test_positions_in_runs(ops, dev, n, hw):
     a = g.double().permute(0, 2, 3, 1).reshape(-1, c)
     _assert_float32_sum(out, a, a, 'output gradients %dx%dx%d' % ((n,) + hw))
     assert torch.equal(out, out.t())
+
+
+# rows of the correlations' rectangles: W - 2 inside, 1 at the edges (runs of 1 .. 12)
+@pytest.mark.parametrize('w', [3, 5, 6, 7, 8, 9, 11, 13, 14])
+@pytest.mark.parametrize('c', [66, 200])
+def test_correlations_in_runs(ops, dev, c, w):
+    gen = torch.Generator(device=dev).manual_seed(100 * c + w)
+    x = torch.randn(3, c, 6, w, device=dev, generator=gen)
+    x[1, c - 1, 2, w - 1], x[1, c - 1, 3, 0] = 1e18, -1e18
+    a = torch.nn.functional.unfold(x.double(), 3, padding=1).permute(0, 2, 1).reshape(-1, 9 * c)
+    single = ops.factor_conv_a(x, (3, 3), (1, 1), (1, 1), (1, 1), False, 1.)
+    out = torch.full((9 * c,) * 2, float('nan'), device=dev)
+    ops.factor_grouped([ops.factor_job('conv_a', x, 1., out, kernel_size=3, stride=1, padding=1,
+                                       dilation=1)], dev)
+    torch.cuda.synchronize()
+    for got in (single, out):
+        # (a block is the sum of up to 9 rectangles' products)
+        _assert_float32_sum(got, a, a, 'correlations of %d channels of 6x%d' % (c, w))
 
 
 @pytest.mark.parametrize('exponent', [-15, 0, 15])
