@@ -41,7 +41,7 @@ PEAK_FP32_MFMA_TFLOPS = 157.3
 # rocprofv3 --pmc readings of the factor-build kernels of a resnet50 step, kept with the
 # profile summary they come from (counter runs cannot be made from inside this script):
 #   traffic_bytes_per_launch   HBM bytes per launch (FETCH_SIZE, WRITE_SIZE, calibrated)
-#   executed_flop_per_step_pmc 512 x SQ_INSTS_VALU_MFMA_MOPS_F32
+#   executed_flop_per_step_pmc 512 x (SQ_INSTS_VALU_MFMA_MOPS_F32 + SQ_INSTS_VALU_MFMA_MOPS_BF16 / 6)
 # The second one is the check on the plan arithmetic below: if the flops this script
 # derives from the library's tile / split plan differ from it by more than 3 %, the plan
 # has changed since the counters were read, and the line says so instead of quoting them.
