@@ -76,11 +76,11 @@ inline int piece_blocks(long work, int longest) {
 }
 
 // Tiles' worth of MFMA work in the T(T+1)/2 upper tiles of a symmetric product with T tiles
-// per side: a diagonal tile leaves out its 32x32 blocks below the diagonal, 6 of 16 for a
-// 128-wide tile of four waves, 1 of 4 for a 64-wide tile of one.
+// per side: of a diagonal tile's 32x32 blocks a 128-wide tile of four waves computes 12 of 16 (three
+// each, split_tile_tri) and a 64-wide tile of one wave 3 of 4.
 inline double syrk_tile_units(int T, int w) {
-  const double diag = w == 2 ? 10. / 16. : 3. / 4.;
-  return (double)T * (T - 1) / 2 + T * diag;
+  (void)w;
+  return (double)T * (T - 1) / 2 + T * (3. / 4.);
 }
 
 inline int launch_status() {
