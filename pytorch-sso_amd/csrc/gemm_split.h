@@ -32,6 +32,7 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 typedef unsigned v2u __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) char lds_c;
+typedef __attribute__((address_space(3))) unsigned lds_u;
 typedef __attribute__((address_space(3))) v4u lds_u4;
 typedef __attribute__((address_space(3))) v2u lds_u2;
 
@@ -55,7 +56,8 @@ struct SplitCfg {
   static constexpr int NT = 64 * WM * WN;
   static constexpr int KC = 16;
   static constexpr int STAGE = SplitChunk<TM>::BYTES + SplitChunk<TN>::BYTES;
-  static constexpr int SMEM_BYTES = 2 * STAGE;
+  static constexpr int VOTES = 2 * STAGE;                // a word per wave (split_blocks)
+  static constexpr int SMEM_BYTES = VOTES + 4 * WM * WN;
 };
 
 __device__ __forceinline__ unsigned pack_bf16(float a, float b) {
@@ -78,9 +80,9 @@ __device__ __forceinline__ void split_pair(float a, float b, unsigned& h, unsign
   l = pack_bf16(ra - bf16_lo(m), rb - bf16_hi(m));
 }
 
-// Leading sums + corrections.  An infinite element has no rest (inf - inf), and beyond 3.4e38
-// the corrections overflow with either sign: where they are not finite the leading sum is the
-// result, infinite with its sign as a float32 sum's, and NaN only where that is.
+// Leading sums + corrections.  An infinite element has no rest (inf - inf): where the corrections
+// are not finite the leading sum is the result, infinite with its sign as a float32 sum's, and
+// NaN only where that is.  (Finite elements that round to an infinite leading part: split_blocks.)
 __device__ __forceinline__ void add_corrections(v16f& acc, const v16f& cor) {
 #pragma unroll
   for (int i = 0; i < 16; ++i) acc[i] += __builtin_isfinite(cor[i]) ? cor[i] : 0.f;
@@ -189,8 +191,8 @@ struct SplitStager<OP, ROWS, NT, KM> {
     }
     ones[SET] = one;
   }
-  template <int SET, int PIECE, int MODE>
-  __device__ __forceinline__ void commit(lds_c* chunk) {
+  template <int SET, int PIECE, int MODE, bool SCALED = false>
+  __device__ __forceinline__ void commit(lds_c* chunk, float scale = 1.f) {
     typedef SplitChunk<ROWS> L;
     constexpr int i = PIECE / 4, j = PIECE % 4;
     float v[2] = {regs[SET][i][2 * j], regs[SET][i][2 * j + 1]};
@@ -198,6 +200,7 @@ struct SplitStager<OP, ROWS, NT, KM> {
     for (int e = 0; e < 2; ++e) {
       if (MODE == ANY_K) v[e] = ((ones[SET] >> (8 * i + 2 * j + e)) & 1u) ? 1.f : v[e];
       if (squares_elements<OP>::value) v[e] *= v[e];
+      if (SCALED) v[e] *= scale;
     }
     unsigned h, m, l;
     split_pair(v[0], v[1], h, m, l);
@@ -301,8 +304,8 @@ struct SplitStager<OP, ROWS, NT, MK> {
     }
     kin[SET] = in;
   }
-  template <int SET, int PIECE, int MODE>
-  __device__ __forceinline__ void commit(lds_c* chunk) {
+  template <int SET, int PIECE, int MODE, bool SCALED = false>
+  __device__ __forceinline__ void commit(lds_c* chunk, float scale = 1.f) {
     typedef SplitChunk<ROWS> L;
     constexpr int i = PIECE / 2, j = PIECE % 2;
     float v[2] = {regs[SET][i][2 * j], regs[SET][i][2 * j + 1]};
@@ -311,6 +314,7 @@ struct SplitStager<OP, ROWS, NT, MK> {
       if (MODE == PADDED_K && 2 * j + e < 3) v[e] = cut[SET] > 2 * j + e ? 0.f : v[e];
       if (OP::kruns == K_ANY) v[e] = ((ones >> i) & (kin[SET] >> (2 * j + e)) & 1u) ? 1.f : v[e];
       if (squares_elements<OP>::value) v[e] *= v[e];
+      if (SCALED) v[e] *= scale;
     }
     unsigned h, m, l;
     split_pair(v[0], v[1], h, m, l);
@@ -369,6 +373,22 @@ struct SplitFrags {
   v8bf p[3][TRI ? 3 : 2];
   v8bf q[3][TRI ? 1 : 2];
 };
+
+// product PR of the six (in the order h h', h m', m h', m m', h l', l h') for block B
+template <bool TRI, int PR, int B>
+__device__ __forceinline__ void split_product(const SplitFrags<TRI>& fr, v16f& sum) {
+  constexpr int PA = PR == 2 || PR == 3 ? 1 : PR == 5 ? 2 : 0;
+  constexpr int PB = PR == 1 || PR == 3 ? 1 : PR == 4 ? 2 : 0;
+  v8bf a, b;
+  if constexpr (TRI) {
+    a = fr.p[PA][B == 2 ? 1 : 0];
+    b = fr.p[PB][B == 1 ? 2 : 1];
+  } else {
+    a = fr.p[PA][B >> 1];
+    b = fr.q[PB][B & 1];
+  }
+  sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, sum, 0, 0, 0);
+}
 
 // Accumulates C = P Q over [kbeg, kend) into the wave's blocks (leading products in acc, the
 // corrections in cor).  prow / qrow: the tile rows of its fragments (TRI: prow only).
@@ -453,8 +473,6 @@ __device__ __forceinline__ void split_tile_loop(const OPP& P, const OPQ& Q, int 
     __builtin_amdgcn_sched_barrier(0);
     static_for<6>([&](auto prod_) {
       constexpr int PR = decltype(prod_)::value;
-      constexpr int PA = PR == 2 || PR == 3 ? 1 : PR == 5 ? 2 : 0;
-      constexpr int PB = PR == 1 || PR == 3 ? 1 : PR == 4 ? 2 : 0;
       if constexpr (PR == 4) {
         __syncthreads();
         load_frags(std::integral_constant<int, SET ^ 1>{}, std::integral_constant<int, 0>{});
@@ -463,16 +481,7 @@ __device__ __forceinline__ void split_tile_loop(const OPP& P, const OPQ& Q, int 
       static_for<NB>([&](auto blk_) {
         constexpr int B = decltype(blk_)::value;
         constexpr int IDX = PR * NB + B;
-        v16f& t = PR == 0 ? acc[B] : cor[B];
-        v8bf a, b;
-        if constexpr (TRI) {
-          a = fr[SET].p[PA][B == 2 ? 1 : 0];
-          b = fr[SET].p[PB][B == 1 ? 2 : 1];
-        } else {
-          a = fr[SET].p[PA][B >> 1];
-          b = fr[SET].q[PB][B & 1];
-        }
-        t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, t, 0, 0, 0);
+        split_product<TRI, PR, B>(fr[SET], PR == 0 ? acc[B] : cor[B]);
         if constexpr (PR < 4) {
           constexpr int LAST = 4 * NB;
           constexpr int l0 = IDX * LOADS / LAST, l1 = (IDX + 1) * LOADS / LAST;
@@ -503,24 +512,89 @@ __device__ __forceinline__ void split_tile_loop(const OPP& P, const OPQ& Q, int 
     step(S0, ANY, c);
     step(S1, ANY, c + 1);
   }
-  __syncthreads();       // (the next tile of this workgroup may overwrite the stages)
 }
 
-// the sum of a wave's blocks over [kbeg, kend), in acc
+// The same in a rolled loop, one chunk after the other, the loads of the next one in flight under
+// the products of this one, with every element multiplied by `scale`.
+template <int WM, int WN, bool TRI, class OPP, class OPQ>
+__device__ __forceinline__ void split_tile_rolled(const OPP& P, const OPQ& Q, int m0, int n0, int kbeg,
+                                                  int kend, lds_c* sm, const int (&prow)[3],
+                                                  const int (&qrow)[2], float scale,
+                                                  v16f (&acc)[TRI ? 3 : 4], v16f (&cor)[TRI ? 3 : 4]) {
+  typedef SplitCfg<WM, WN> C;
+  constexpr int KC = C::KC;
+  constexpr int QOFF = SplitChunk<C::TM>::BYTES;
+  const int lane = threadIdx.x & 63;
+  typedef SplitStager<OPP, C::TM, C::NT> SP;
+  typedef SplitStager<OPQ, C::TN, C::NT> SQ;
+  SP sp;
+  SQ sq;
+  sp.init(P, m0);
+  if (!TRI) sq.init(Q, n0);
+  sp.template fetch<0>(P, kbeg, kend);
+  if (!TRI) sq.template fetch<0>(Q, kbeg, kend);
+  int stage = 0;
+#pragma unroll 1
+  for (int k0 = kbeg; k0 < kend; k0 += KC) {
+    lds_c* const at = sm + stage;
+    stage ^= C::STAGE;
+    static_for<SP::PIECES>(
+        [&](auto x) { sp.template commit<0, decltype(x)::value, ANY_K, true>(at, scale); });
+    if (!TRI)
+      static_for<SQ::PIECES>(
+          [&](auto x) { sq.template commit<0, decltype(x)::value, ANY_K, true>(at + QOFF, scale); });
+    if (k0 + KC < kend) {
+      sp.template fetch<0>(P, k0 + KC, kend);
+      if (!TRI) sq.template fetch<0>(Q, k0 + KC, kend);
+    }
+    __syncthreads();       // (every wave is done with the chunk before this one: its stage is free)
+    SplitFrags<TRI> fr;
+#pragma unroll
+    for (int pl = 0; pl < 3; ++pl) {
+#pragma unroll
+      for (int i = 0; i < (TRI ? 3 : 2); ++i) fr.p[pl][i] = load_frag<C::TM>(at, prow[i], lane, pl);
+      if (!TRI) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) fr.q[pl][i] = load_frag<C::TN>(at + QOFF, qrow[i], lane, pl);
+      }
+    }
+    static_for<6>([&](auto prod_) {
+      constexpr int PR = decltype(prod_)::value;
+      static_for<(TRI ? 3 : 4)>([&](auto blk_) {
+        constexpr int B = decltype(blk_)::value;
+        split_product<TRI, PR, B>(fr, PR == 0 ? acc[B] : cor[B]);
+      });
+    });
+  }
+}
+
+// The sum of a wave's blocks over [kbeg, kend), in acc.
+// A finite element beyond the largest bf16 number (3.3895e38) rounds to an infinite leading part,
+// and every sum that it enters comes out as inf or NaN.  So a tile with such a sum is computed
+// once more from halves of the elements, and the sums taken four times: what is finite then, is
+// what a float32 sum gives, and what is not, is not there either.  (Half of an element is exact,
+// but for a last bit of 2^-149.)  The waves vote across the barrier that ends a tile anyway.
 template <int WM, int WN, bool TRI, class OPP, class OPQ>
 __device__ __forceinline__ void split_blocks(const OPP& P, const OPQ& Q, int m0, int n0, int kbeg,
                                              int kend, float* smem, const int (&prow)[3],
                                              const int (&qrow)[2], v16f (&acc)[TRI ? 3 : 4]) {
   typedef SplitCfg<WM, WN> C;
-  v16f cor[TRI ? 3 : 4];
-#pragma unroll
-  for (int b = 0; b < (TRI ? 3 : 4); ++b)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) acc[b][i] = cor[b][i] = 0.f;
+  constexpr int NB = TRI ? 3 : 4;
+  v16f cor[NB];
   lds_c* const sm = (lds_c*)smem;
+  lds_u* const votes = (lds_u*)(sm + C::VOTES);
+  const int wave = (int)(threadIdx.x & (C::NT - 1)) >> 6;
   // (uniform per workgroup; operands in padded runs are two of a kind)
   const int mode = SplitStager<OPP, C::TM, C::NT>::fast(P, m0);
   const int qmode = TRI ? mode : SplitStager<OPQ, C::TN, C::NT>::fast(Q, n0);
+  auto clear = [&]() {
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[b][i] = cor[b][i] = 0.f;
+  };
+  clear();
+  if (kend <= kbeg) return;
   if (mode == FAST_K && qmode == FAST_K) {
     split_tile_loop<WM, WN, TRI, FAST_K>(P, Q, m0, n0, kbeg, kend, sm, prow, qrow, acc, cor);
   } else if (has_padded_runs<OPP>::value && mode == PADDED_K) {
@@ -529,8 +603,31 @@ __device__ __forceinline__ void split_blocks(const OPP& P, const OPQ& Q, int m0,
   } else {
     split_tile_loop<WM, WN, TRI, ANY_K>(P, Q, m0, n0, kbeg, kend, sm, prow, qrow, acc, cor);
   }
+  // (0 times a correction that is not finite is NaN; the third part of an element with an
+  // infinite leading part is NaN, and so are all the corrections that it enters)
+  float probe = 0.f;
 #pragma unroll
-  for (int b = 0; b < (TRI ? 3 : 4); ++b) add_corrections(acc[b], cor[b]);
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      probe = fmaf(cor[b][i], 0.f, probe);
+      acc[b][i] += cor[b][i];
+    }
+  votes[wave] = __builtin_amdgcn_ballot_w64(probe != 0.f) != 0;
+  __syncthreads();           // (and the next tile of this workgroup may overwrite the stages)
+  unsigned any = 0;
+#pragma unroll
+  for (int w = 0; w < C::NT / 64; ++w) any |= votes[w];
+  if (__builtin_expect(__builtin_amdgcn_readfirstlane((int)any) != 0, 0)) {
+    clear();
+    split_tile_rolled<WM, WN, TRI>(P, Q, m0, n0, kbeg, kend, sm, prow, qrow, 0.5f, acc, cor);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      add_corrections(acc[b], cor[b]);
+      acc[b] *= 4.f;
+    }
+    __syncthreads();
+  }
 }
 
 // The 32x32 blocks of a wave, rows from `row0`, columns from `col0`, through the epilogue.

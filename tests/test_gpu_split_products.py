@@ -18,7 +18,7 @@ def ops():
     return _ops
 
 
-def _assert_float32_sum(got, a, b, what):
+def _assert_float32_sum(got, a, b, what, where=None):
     """got = a^T b for float64 copies a [K, m], b [K, n] of float32 operands.  An element is a
     sum of exact products, of which the terms of relative size 2^-23 and below are left
     out, added to float32 accumulators in at most K / 16 + 1 steps each for the leading and
@@ -28,7 +28,8 @@ def _assert_float32_sum(got, a, b, what):
     want = a.t() @ b
     mass = a.abs().t() @ b.abs()
     bound = mass * (2. ** -23) * (2 * (K // 16 + 1) + K // 128 + 4) + 1e-37
-    over = ((got.double() - want).abs() / bound).max().item()
+    over = (got.double() - want).abs() / bound
+    over = (over if where is None else over[where]).max().item()
     assert over <= 1., '%s: error %.2f times the bound' % (what, over)
 
 
@@ -136,6 +137,37 @@ def test_infinities_and_overflow(ops, dev, hw):
         assert torch.equal(out.isneginf(), want.isneginf())
         ok = want.isfinite()
         assert ((out - want)[ok] / want[ok]).abs().max().item() < 1e-5
+
+
+@pytest.mark.parametrize('hw', [(4, 8), (7, 7)])
+def test_finite_elements_beyond_the_largest_bf16(ops, dev, hw):
+    """3.4e38 is a float32 like any other, though its nearest bf16 number is infinite: its products
+    with small elements are finite, and only its square overflows."""
+    gen = torch.Generator(device=dev).manual_seed(7)
+    g = 1e-30 * (torch.rand(3, 300, *hw, device=dev, generator=gen) + 0.1)
+    g[1, 10, 1, 2] = 3.4e38
+    g[0, 140, -1, -3] = -3.4e38
+    g[2, 270, -1, -1] = 3.3962e38            # (the smallest ones that round up: 3.39618e38)
+    x = g.permute(0, 2, 3, 1).reshape(-1, 300).contiguous()
+    pointwise = ops.factor_conv_a(g, 1, 1, 0, 1, False, 1.)
+    for out in (ops.factor_conv_g(g, 1.), ops.factor_linear(x, False, 1.), pointwise):
+        a = x.double()
+        large = (a.abs() > 1e38).any(0)
+        finite = (a.t() @ a).abs() < 3.4e38
+        assert torch.equal(out.isfinite(), finite) and int((~finite).sum()) == 3
+        _assert_float32_sum(torch.where(finite, out, 0.), a * ~large, a, 'small elements by all',
+                            where=finite & ~large[:, None])
+        _assert_float32_sum(torch.where(finite, out, 0.), a * large, a, 'large elements by all',
+                            where=finite & large[:, None])
+    # (in sums of two operands too)
+    Gi = torch.randn(300, 300, device=dev, generator=gen)
+    Gi = Gi + Gi.t()
+    w = 1e-30 * torch.randn(300, 200, device=dev, generator=gen)
+    Gi[:, 5], Gi[5, :] = 1e-9, 1e-9
+    w[5, 7] = 3.4e38
+    want = Gi.double() @ w.double()
+    ops.precondition_batched([Gi], [torch.eye(200, device=dev)], [w], [None])
+    assert ((w.double() - want).abs() / (want.abs() + 1e-30)).max().item() < 1e-4
 
 
 def test_positive_terms(ops, dev):
