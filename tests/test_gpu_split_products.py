@@ -47,6 +47,23 @@ def test_dense_symmetric(ops, dev, f, rows, bias):
     assert torch.equal(out, out.t())
 
 
+# the last reduction in one rolled loop (48 steps) and the first that is not, of products of one
+# operand, of two, and of operands whose consecutive k are next to each other
+@pytest.mark.parametrize('rows', [31, 32, 48, 49, 64])
+def test_short_reductions(ops, dev, rows):
+    gen = torch.Generator(device=dev).manual_seed(rows)
+    x = torch.randn(rows, 300, device=dev, generator=gen)
+    g = torch.randn(rows, 200, device=dev, generator=gen)
+    a = torch.cat([x.double(), torch.ones(rows, 1, device=dev, dtype=torch.float64)], 1)
+    _assert_float32_sum(ops.factor_linear(x, True, 1.), a, a, 'factor, %d rows' % rows)
+    w, b = ops.diag_cov_linear(g, x, True, 1.)
+    # (the squares are float32 too: another rounding of either factor)
+    _assert_float32_sum(torch.cat([w, b[:, None]], 1), g.double() ** 2, a ** 2, 'squares, %d' % rows)
+    c = torch.randn(1, 300, 1, rows, device=dev, generator=gen)
+    a = c.double().reshape(300, rows).t()
+    _assert_float32_sum(ops.factor_conv_g(c, 1.), a, a, 'positions, %d' % rows)
+
+
 # one run of a multiple of 4, padded runs (5 = 8 - 3, 6, 7, 9, ...), runs left as they are (1 .. 3)
 @pytest.mark.parametrize('hw', [(1, 1), (1, 3), (2, 2), (1, 5), (2, 3), (1, 7), (3, 3), (2, 5), (3, 5),
                                 (7, 7), (5, 13), (8, 8)])
