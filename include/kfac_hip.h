@@ -87,8 +87,9 @@ int kfac_factor_conv_a(const float* x, int n, int c, int H, int W,
 
 /* Plan queries (no device needed): the fp32 MFMA flops the factor builders execute for a
  * d x d factor reduced over K terms (kfac_factor_linear, kfac_factor_conv_g and the
- * pointwise case of kfac_factor_conv_a) and for a Conv2d input factor of the given
- * geometry: whole tiles of the upper triangle, whole reduction chunks, the shared spatial
+ * pointwise case of kfac_factor_conv_a; images of h*w positions with h*w no multiple of 4
+ * execute up to 3 more of them each in 128-wide tiles, which the first query does not
+ * know) and for a Conv2d input factor of the given geometry: whole tiles of the upper triangle, whole reduction chunks, the shared spatial
  * correlations of a stride-1 k x k layer.  For utilisation figures next to the
  * algorithmic 2*d*d*K. */
 double kfac_factor_executed_flops(int d, int64_t K);

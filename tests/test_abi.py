@@ -106,6 +106,14 @@ def test_grouped_factor_plan_needs_no_device():
               + lib.kfac_factor_conv_a_executed_flops(32, 64, 56, 56, 3, 3, 1, 1, 1, 1, 1, 1, 0)
               + lib.kfac_factor_conv_a_executed_flops(32, 128, 28, 28, 3, 3, 2, 2, 1, 1, 1, 1, 0))
     assert abs(lib.kfac_factor_grouped_executed_flops(len(jobs), arr) - single) <= 1e-9 * single
+    # images of odd length: single products pad their runs as grouped ones do, within the scratch
+    # of a product of as many terms
+    for c, n, h, w in ((600, 8, 3, 3), (300, 32, 1, 7), (2048, 32, 7, 7), (512, 1, 1, 5)):
+        odd = (_hip.FactorJob * 1)(_job(_hip.FACTOR_CONV_A, c, n, h, w))
+        assert lib.kfac_factor_conv_a_executed_flops(n, c, h, w, 1, 1, 1, 1, 0, 0, 1, 1, 0) \
+            == lib.kfac_factor_grouped_executed_flops(1, odd)
+        assert lib.kfac_factor_conv_a_workspace_bytes(n, c, h, w, 1, 1, 1, 1, 0, 0, 1, 1, 0) \
+            == lib.kfac_factor_workspace_bytes(c, n * h * w)
     assert lib.kfac_factor_grouped(0, None, None, 0, None) == 0
     assert lib.kfac_factor_grouped(1, None, None, 0, None) == 1
     assert lib.kfac_factor_grouped(len(jobs), arr, None, 0, None) == 2            # no scratch

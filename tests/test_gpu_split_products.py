@@ -18,15 +18,15 @@ def ops():
     return _ops
 
 
-def _assert_float32_sum(got, a, b, what, where=None):
-    """got = a^T b for float64 copies a [K, m], b [K, n] of float32 operands.  An element is a
+def _assert_float32_sum(got, a, b, what, where=None, plus=0.):
+    """got = a^T b (+ plus) for float64 copies a [K, m], b [K, n] of float32 operands.  An element is a
     sum of exact products, of which the terms of relative size 2^-23 and below are left
     out, added to float32 accumulators in at most K / 16 + 1 steps each for the leading and
     the correction terms (16 products per step, each step within 2^-23 of the running sum of
     absolute values), over at most K / 128 + 1 partial sums."""
     K = a.shape[0]
-    want = a.t() @ b
-    mass = a.abs().t() @ b.abs()
+    want = a.t() @ b + plus
+    mass = a.abs().t() @ b.abs() + abs(plus)
     bound = mass * (2. ** -23) * (2 * (K // 16 + 1) + K // 128 + 4) + 1e-37
     over = (got.double() - want).abs() / bound
     over = (over if where is None else over[where]).max().item()
@@ -105,6 +105,23 @@ def test_positions_in_runs(ops, dev, n, hw):
     a = g.double().permute(0, 2, 3, 1).reshape(-1, c)
     _assert_float32_sum(out, a, a, 'output gradients %dx%dx%d' % ((n,) + hw))
     assert torch.equal(out, out.t())
+
+
+# single products on 128-wide tiles (more than 256 rows), with the old contents of the output, and
+# with the reduction cut into pieces
+@pytest.mark.parametrize('hw', [(1, 1), (1, 3), (1, 5), (2, 3), (1, 7), (3, 3), (7, 7), (5, 13), (8, 8)])
+@pytest.mark.parametrize('n', [1, 5, 60])
+def test_positions_in_runs_of_a_single_call(ops, dev, n, hw):
+    c = 300
+    gen = torch.Generator(device=dev).manual_seed(n * 100 + hw[0] * hw[1])
+    g = torch.randn(n, c, *hw, device=dev, generator=gen)
+    old = torch.rand(c, c, device=dev, generator=gen)
+    old = old + old.t()
+    a = g.double().permute(0, 2, 3, 1).reshape(-1, c)
+    for out in (ops.factor_conv_g(g, 1., out=old.clone(), beta=1.),
+                ops.factor_conv_a(g, 1, 1, 0, 1, False, 1., out=old.clone(), beta=1.)):
+        _assert_float32_sum(out, a, a, 'positions %dx%dx%d' % ((n,) + hw), plus=old.double())
+        assert torch.equal(out, out.t())
 
 
 # rows of the correlations' rectangles: W - 2 inside, 1 at the edges (runs of 1 .. 12)
