@@ -81,6 +81,16 @@ struct ShiftX {
 // Index positions of a row of a rectangle: padded (padded_run) for 128-wide tiles.
 __host__ __device__ inline int row_positions(int ww, int w) { return w == 2 ? padded_run(ww) : ww; }
 
+// Time of a chunk of a job against one in runs of at least 4.  Rows of up to three positions (the
+// strips beside the left and right edge) are loaded element by element, every lane of a load in a
+// line of its own: on 128-wide tiles such a chunk lasts several times as long, and a plan that
+// counts it as one ends with the few items of those strips.  Factor of 32 images of 128x56x56 /
+// 256x14x14 / 64 of 128x14x14, one product: 667 / 190 / 110 us counted as 1, 349 / 125 / 76 as 5,
+// 331 / 117 / 71 as 6, 302 / 112 / 71 as 8 (but 32 of 512x9x9, where every job is short: 207 / 210 /
+// 209 / 224).  The 64-wide tiles load everything element by element.
+constexpr int SHORT_RUN_COST = 6;
+static int chunk_cost(int ww, int w) { return w == 2 && ww < 4 ? SHORT_RUN_COST : 1; }
+
 struct JobDesc {
   short u0, v0, hh, ww;    // rectangle of the first factor; the reduction runs over its rows (row_positions)
   short dy, dx;            // displacement of the second factor
@@ -507,22 +517,26 @@ static TapPlanHost plan_taps(int n, int c, int H, int Wd, int kh, int kw, int ph
   hp.tiles_side = cdiv(c, ts);
   const int ntiles = hp.tiles_side * hp.tiles_side;
   const int kc = hp.w == 1 ? Cfg<1, 1>::KC : Cfg<2, 2>::KC;
-  double total = 0;
   auto job_k = [&](const JobDesc& jd) { return (long)n * jd.hh * row_positions(jd.ww, hp.w); };
-  for (int j = 0; j < pd.njobs; ++j) total += (double)job_k(pd.jobs[j]);
-  // All workgroups of a launch that fits the chip are resident at once (3 four-wave
-  // workgroups per CU: 768) and share the matrix cores of their CU, so the launch lasts as
-  // long as the fullest CU: a little under one full round (the split counts round up) beats
-  // 1.3 rounds by a quarter.  The one-wave workgroups (8 per CU) do best at 1.5 rounds.
-  const double target_items = hp.w == 1 ? 3072.0 : 700.0;
+  // (in chunks in runs)
+  auto job_work = [&](const JobDesc& jd) { return (job_k(jd) + kc - 1) / kc * chunk_cost(jd.ww, hp.w); };
+  double total = 0;
+  for (int j = 0; j < pd.njobs; ++j) total += (double)job_work(pd.jobs[j]);
+  // All workgroups of a launch that fits the chip are resident at once (RESIDENT_TILES) and share
+  // the matrix cores of their CU, so the launch lasts as long as the fullest CU: about one full
+  // round of items of one duration.  (A target of 440 / 480 / 512 items, as above: 341 / 348 /
+  // 331, 121 / 125 / 117 and 74 / 76 / 71 us; 700, of the time when three workgroups fitted a
+  // CU: 310 / 140 / 88.)  The one-wave workgroups (8 per CU) do best at 1.5 rounds.
+  const double target_items = hp.w == 1 ? 3072.0 : (double)RESIDENT_TILES;
   int item = 0, part = 0;
   for (int j = 0; j < pd.njobs; ++j) {
     JobDesc& jd = pd.jobs[j];
     const long nchunks = (job_k(jd) + kc - 1) / kc;
-    long splits = group_cps > 0
-                      ? (nchunks + group_cps / 2) / group_cps
-                      : (long)(target_items * ((double)job_k(jd) / total) / ntiles + 0.5);
-    const long max_splits = std::max<long>(1, nchunks / (128 / kc));
+    const long work = job_work(jd);
+    long splits = group_cps > 0 ? (work + group_cps / 2) / group_cps
+                                : (long)(target_items * ((double)work / total) / ntiles + 0.5);
+    // (an item lasts as long as 128 steps in runs, at least, and is a chunk, at least)
+    const long max_splits = std::max<long>(1, std::min(nchunks, work / (128 / kc)));
     splits = std::max<long>(1, std::min(std::min(splits, max_splits), 4096L));
     long cps = (nchunks + splits - 1) / splits;
     splits = (nchunks + cps - 1) / cps;
@@ -661,7 +675,7 @@ static TapsGroupPlan* make_taps_group_plan(int count, const TapsJob* jobs) {
   gp->partial_floats = 0;
   gp->executed_flops = 0.;
   // chunks per item: the default where a tile size has plenty of work, shorter items where
-  // its launch would not fill the chip twice (3 layers of 64 channels, say)
+  // its launch would not fill the chip (3 layers of 64 channels, say)
   double units[2] = {0., 0.};
   for (int i = 0; i < count; ++i) {
     const TapsJob& j = jobs[i];
@@ -673,9 +687,12 @@ static TapsGroupPlan* make_taps_group_plan(int count, const TapsJob* jobs) {
   }
   int group_cps[2];
   for (int w = 0; w < 2; ++w) {
-    const double slots = w == 0 ? 2048. : 768.;
+    // (resident workgroups: RESIDENT_TILES of four waves, 2048 of one; 1.5 rounds of the longer
+    // ones: 32 images of 512x7x7 / 384x13x13 / 64 of 128x14x14 in 1.5 / 2 rounds 178 / 139 / 87 us,
+    // 188 / 150 / 89)
+    const double items = w == 0 ? 2. * 2048. : 1.5 * RESIDENT_TILES;
     const int dflt = w == 0 ? TAPS_GROUP_CPS1 : TAPS_GROUP_CPS2;
-    long t = (long)(units[w] / (2. * slots));
+    long t = (long)(units[w] / items);
     group_cps[w] = (int)std::max(8L, std::min((long)dflt, t));
   }
   for (int i = 0; i < count; ++i) {

@@ -91,6 +91,18 @@ def _job(kind, c, rows, H=1, W=1, k=1, stride=1, pad=0, x=256, C=512):
     return j
 
 
+@pytest.mark.parametrize('n,c,side', [(32, 128, 28), (32, 256, 14), (64, 128, 14)])
+def test_correlation_plan_fits_one_round(n, c, side):
+    """A correlation launch of 128-wide tiles holds about as many items as two resident
+    workgroups per compute unit (512), the last of each job rounded up: their number follows from
+    the scratch, one c x c partial per split and 45 block sums."""
+    lib = _hip.load()
+    size = lib.kfac_factor_conv_a_workspace_bytes(n, c, side, side, 3, 3, 1, 1, 1, 1, 1, 1, 0)
+    splits = size // (4 * c * c) - 45
+    tiles = (-(-c // 128)) ** 2
+    assert 256 < splits * tiles <= 512 + 64 // 2
+
+
 def test_grouped_factor_plan_needs_no_device():
     """The plan of a grouped call (scratch, executed flops) is host arithmetic; bad lists are
     refused before anything is launched."""
