@@ -4,6 +4,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "../../include/kfac_hip.h"
 
 namespace kfac {
@@ -73,6 +75,20 @@ inline int piece_blocks(long work, int longest) {
   if (longest <= MIN_PIECE_BLOCKS || 3 * (long)longest <= 4 * even) return 0;
   const long pb = even / 2 > MIN_PIECE_BLOCKS ? even / 2 : MIN_PIECE_BLOCKS;
   return pb >= longest ? 0 : (int)pb;
+}
+
+// Chunks per item of a launch of factor products that hold `units` (tile, chunk) pairs, on tiles
+// of w x w waves: `dflt` where the launch holds plenty of items at that length, shorter items
+// where it would not fill the chip: twice with workgroups of one wave (8 per CU are resident), 1.5
+// times with those of four (output gradients of 32 images of 2048x7x7 / 1024x13x13 / 256x56x56 in
+// 1.5 / 2 / 3 rounds: 79 / 87 / 98, 69 / 73 / 82, 73 / 78 / 91 us), or once where that would take
+// items of less than 8 chunks (a strided pointwise layer, 256 rows, 588 items of 8 chunks 64 us,
+// one round of 10 chunks 54).
+inline long group_item_chunks(int w, double units, long dflt) {
+  const double resident = w == 1 ? 2048. : RESIDENT_TILES;
+  long t = (long)(units / ((w == 1 ? 2. : 1.5) * resident));
+  if (t < 8) t = w == 1 ? 8 : std::max(8L, (long)(units / resident) + 1);
+  return std::min(t, dflt);
 }
 
 // Tiles' worth of MFMA work in the T(T+1)/2 upper tiles of a symmetric product with T tiles

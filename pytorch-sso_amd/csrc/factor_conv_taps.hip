@@ -687,13 +687,7 @@ static TapsGroupPlan* make_taps_group_plan(int count, const TapsJob* jobs) {
   }
   int group_cps[2];
   for (int w = 0; w < 2; ++w) {
-    // (resident workgroups: RESIDENT_TILES of four waves, 2048 of one; 1.5 rounds of the longer
-    // ones: 32 images of 512x7x7 / 384x13x13 / 64 of 128x14x14 in 1.5 / 2 rounds 178 / 139 / 87 us,
-    // 188 / 150 / 89)
-    const double items = w == 0 ? 2. * 2048. : 1.5 * RESIDENT_TILES;
-    const int dflt = w == 0 ? TAPS_GROUP_CPS1 : TAPS_GROUP_CPS2;
-    long t = (long)(units[w] / items);
-    group_cps[w] = (int)std::max(8L, std::min((long)dflt, t));
+    group_cps[w] = (int)group_item_chunks(w + 1, units[w], w == 0 ? TAPS_GROUP_CPS1 : TAPS_GROUP_CPS2);
   }
   for (int i = 0; i < count; ++i) {
     const TapsJob& j = jobs[i];

@@ -211,18 +211,8 @@ static GroupPlan plan_group(int d, long K, long target) {
   return p;
 }
 
-// Chunks per item for one launch: the default when the launch holds plenty of items at that
-// length, shorter items when it would not fill the chip: twice with workgroups of one wave (8 per
-// CU are resident), 1.5 times with those of four (RESIDENT_TILES; output gradients of 32 images of
-// 2048x7x7 / 1024x13x13 / 256x56x56 in 1.5 / 2 / 3 rounds: 79 / 87 / 98, 69 / 73 / 82, 73 / 78 /
-// 91 us).
 static long launch_target(int w, double total_units) {
-  const long dflt = w == 1 ? GROUP_TARGET_CPS_W1 : GROUP_TARGET_CPS_W2;
-  const double items = w == 1 ? 2. * 2048. : 1.5 * RESIDENT_TILES;
-  long t = (long)(total_units / items);
-  if (t > dflt) t = dflt;
-  if (t < 8) t = 8;
-  return t;
+  return group_item_chunks(w, total_units, w == 1 ? GROUP_TARGET_CPS_W1 : GROUP_TARGET_CPS_W2);
 }
 
 enum Path { P_DENSE, P_CONVG, P_CONVA, P_CONVP, P_TAPS, P_SINGLE, P_BAD };

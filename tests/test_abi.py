@@ -126,6 +126,10 @@ def test_grouped_factor_plan_needs_no_device():
             == lib.kfac_factor_grouped_executed_flops(1, odd)
         assert lib.kfac_factor_conv_a_workspace_bytes(n, c, h, w, 1, 1, 1, 1, 0, 0, 1, 1, 0) \
             == lib.kfac_factor_workspace_bytes(c, n * h * w)
+    # a launch too small for 1.5 rounds of items of 8 chunks is one round (512), not a little more
+    # (the scratch is one 128 x 128 partial per item, and a little for the tables)
+    pointwise = (_hip.FactorJob * 1)(_job(_hip.FACTOR_CONV_A, 256, 32, 56, 56, stride=2))
+    assert 256 < lib.kfac_factor_grouped_workspace_bytes(1, pointwise) / 4. / 128 ** 2 < 513
     assert lib.kfac_factor_grouped(0, None, None, 0, None) == 0
     assert lib.kfac_factor_grouped(1, None, None, 0, None) == 1
     assert lib.kfac_factor_grouped(len(jobs), arr, None, 0, None) == 2            # no scratch
