@@ -575,10 +575,12 @@ __device__ __forceinline__ void split_tile_rolled(const OPP& P, const OPQ& Q, in
 
 // The sum of a wave's blocks over [kbeg, kend), in acc.
 // A finite element beyond the largest bf16 number (3.3895e38) rounds to an infinite leading part,
-// and every sum that it enters comes out as inf or NaN.  So a tile with such a sum is computed
-// once more from halves of the elements, and the sums taken four times: what is finite then, is
-// what a float32 sum gives, and what is not, is not there either.  (Half of an element is exact,
-// but for a last bit of 2^-149.)  The waves vote across the barrier that ends a tile anyway.
+// and every sum that it enters comes out as inf or NaN; and leading parts that are rounded up have
+// an infinite sum where the elements' own is still finite (above 0.992 of the largest float32:
+// the square of 2^64 - 2^54).  So a tile with a sum that is not finite is computed once more
+// from halves of the elements, and the sums taken four times: what is finite then, is what a
+// float32 sum gives, and what is not, is not there either.  (Half of an element is exact, but for
+// a last bit of 2^-149.)  The waves vote across the barrier that ends a tile anyway.
 template <int WM, int WN, bool TRI, class OPP, class OPQ>
 __device__ __forceinline__ void split_blocks(const OPP& P, const OPQ& Q, int m0, int n0, int kbeg,
                                              int kend, float* smem, const int (&prow)[3],
@@ -610,15 +612,15 @@ __device__ __forceinline__ void split_blocks(const OPP& P, const OPQ& Q, int m0,
   } else {
     split_tile_loop<WM, WN, TRI, ANY_K>(P, Q, m0, n0, kbeg, kend, sm, prow, qrow, acc, cor);
   }
-  // (0 times a correction that is not finite is NaN; the third part of an element with an
-  // infinite leading part is NaN, and so are all the corrections that it enters)
+  // (0 times a sum that is not finite is NaN; the third part of an element with an infinite leading
+  // part is NaN, and so are all the corrections that it enters)
   float probe = 0.f;
 #pragma unroll
   for (int b = 0; b < NB; ++b)
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      probe = fmaf(cor[b][i], 0.f, probe);
       acc[b][i] += cor[b][i];
+      probe = fmaf(acc[b][i], 0.f, probe);
     }
   votes[wave] = __builtin_amdgcn_ballot_w64(probe != 0.f) != 0;
   __syncthreads();           // (and the next tile of this workgroup may overwrite the stages)

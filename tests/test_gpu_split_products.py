@@ -204,6 +204,24 @@ def test_finite_elements_beyond_the_largest_bf16(ops, dev, hw):
     assert ((w.double() - want).abs() / (want.abs() + 1e-30)).max().item() < 1e-4
 
 
+@pytest.mark.parametrize('rows', [3, 100])
+def test_sums_just_below_the_largest_float32(ops, dev, rows):
+    """2^64 - 2^54 is 2^64 in bf16: its square is finite, that of its leading part is not.  In a
+    reduction in one rolled loop and in the pipelined one, with the sign, and in a sum of two."""
+    big = 2. ** 64 - 2. ** 54
+    x = torch.zeros(rows, 300, device=dev)
+    x[1, 5], x[1, 290] = big, -big                                  # products of both signs
+    x[0, 100], x[2, 100] = big * 0.75, big * 0.65                   # 0.985 of it
+    x[0, 200], x[1, 200] = big, big                                 # overflows in float32 too
+    want = x.double().t() @ x.double()
+    over = want > 3.4028235e38
+    assert int(over.sum()) == 1 and (want[5, 5] > 3.39e38) and (want[5, 290] < -3.39e38)
+    for out in (ops.factor_linear(x, False, 1.), ops.factor_conv_g(x.t().reshape(1, 300, 1, rows), 1.)):
+        assert torch.equal(out.isposinf(), over) and not out.isneginf().any() and not out.isnan().any()
+        # (each product here is a float32 number up to its last bits)
+        assert ((out.double() - want)[~over].abs() <= 2. ** -22 * want[~over].abs()).all()
+
+
 def test_positive_terms(ops, dev):
     # no drift where all terms have one sign
     gen = torch.Generator(device=dev).manual_seed(4)
