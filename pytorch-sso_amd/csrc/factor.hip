@@ -96,13 +96,17 @@ static SyrkPlan plan_syrk(int d, long K) {
   splits = (nchunks + cps - 1) / cps;
   if (splits < 1) splits = 1;
   if (p.w == 2) {
-    // All workgroups of up to 3 per CU are resident at once and share the CU's matrix
-    // cores, so the launch takes (workgroups on the fullest CU) x (chunks per split):
-    // a few more splits can take a whole round off.  Every extra split costs one more
-    // partial tile written and read (the last term, in chunk times).
+    // Two workgroups per CU are resident and share its matrix cores; one that is left alone, the last
+    // of an odd number, takes 1.5 times its share.  So the launch takes (workgroups on the fullest
+    // CU, and a half if they are odd) x (chunks per split): more splits than fit at once take
+    // time off some products and add to others.  Every extra split costs one more partial tile
+    // written and read (the last term, in chunk times).  8192 rows of 1600 / 2176 in 5 / 3 splits
+    // (2 workgroups on the fullest CU) 137 / 224 us, in 8 / 5 (3) 153 / 243; of 2304 / 2432 in 2 splits
+    // (2) 286 / 297, in 4 (3) 264 / 272.
     const int ncu = 256;
     auto cost = [&](long s, long c) {
-      return (double)cdiv((int)(s * p.ntiles), ncu) * (c + 3) + (s > 1 ? 0.035 * s * p.ntiles : 0.);
+      const int on_one = cdiv((int)(s * p.ntiles), ncu);
+      return (on_one + on_one % 2 * 0.5) * (c + 3) + (s > 1 ? 0.035 * s * p.ntiles : 0.);
     };
     double best = cost(splits, cps);
     long best_s = splits, best_cps = cps;

@@ -103,6 +103,15 @@ def test_correlation_plan_fits_one_round(n, c, side):
     assert 256 < splits * tiles <= 512 + 64 // 2
 
 
+@pytest.mark.parametrize('d,rows,splits', [(1600, 8192, 5), (2176, 8192, 3), (2304, 8192, 4),
+                                           (2304, 2000, 2)])
+def test_splits_of_a_single_product(d, rows, splits):
+    """Two workgroups per compute unit are resident: three on the fullest one pay off where they are a
+    good deal shorter than two (2304 rows of a factor), not in exchange for little."""
+    tiles = -(-d // 128) * (-(-d // 128) + 1) // 2
+    assert _hip.load().kfac_factor_workspace_bytes(d, rows) == 4 * 128 * 128 * tiles * splits
+
+
 def test_grouped_factor_plan_needs_no_device():
     """The plan of a grouped call (scratch, executed flops) is host arithmetic; bad lists are
     refused before anything is launched."""
