@@ -527,28 +527,37 @@ static TapPlanHost plan_taps(int n, int c, int H, int Wd, int kh, int kw, int ph
   // round of items of one duration.  (A target of 440 / 480 / 512 items, as above: 341 / 348 /
   // 331, 121 / 125 / 117 and 74 / 76 / 71 us; 700, of the time when three workgroups fitted a
   // CU: 310 / 140 / 88.)  The one-wave workgroups (8 per CU) do best at 1.5 rounds.
-  const double target_items = hp.w == 1 ? 3072.0 : (double)RESIDENT_TILES;
-  int item = 0, part = 0;
-  for (int j = 0; j < pd.njobs; ++j) {
-    JobDesc& jd = pd.jobs[j];
-    const long nchunks = (job_k(jd) + kc - 1) / kc;
-    const long work = job_work(jd);
-    long splits = group_cps > 0 ? (work + group_cps / 2) / group_cps
-                                : (long)(target_items * ((double)work / total) / ntiles + 0.5);
-    // (an item lasts as long as 128 steps in runs, at least, and is a chunk, at least)
-    const long max_splits = std::max<long>(1, std::min(nchunks, work / (128 / kc)));
-    splits = std::max<long>(1, std::min(std::min(splits, max_splits), 4096L));
-    long cps = (nchunks + splits - 1) / splits;
-    splits = (nchunks + cps - 1) / cps;
-    jd.splits = (short)splits;
-    jd.cps = (int)cps;
-    pd.item0[j] = item;
-    jd.part0 = part;
-    item += (int)splits * ntiles;
-    part += (int)splits;
-  }
+  // Where the splits of the jobs, rounded to whole ones, make a good deal more than one round all the
+  // same (9 tiles and more to a job), shorter items end more evenly: 39 images of 400x16x16, 672
+  // items 518 us, 880 462; 2 of 324x52x52, 612 and 846, 208 and 188; but 32 of 512x7x7 180 and 189,
+  // 32 of 521x14x14 1144 and 1174.
+  constexpr double ROUND_LIMIT = 1.15 * RESIDENT_TILES, LONG_ROUND = 1.375 * RESIDENT_TILES;
+  auto deal = [&](double target_items) {
+    int item = 0, part = 0;
+    for (int j = 0; j < pd.njobs; ++j) {
+      JobDesc& jd = pd.jobs[j];
+      const long nchunks = (job_k(jd) + kc - 1) / kc;
+      const long work = job_work(jd);
+      long splits = group_cps > 0 ? (work + group_cps / 2) / group_cps
+                                  : (long)(target_items * ((double)work / total) / ntiles + 0.5);
+      // (an item lasts as long as 128 steps in runs, at least, and is a chunk, at least)
+      const long max_splits = std::max<long>(1, std::min(nchunks, work / (128 / kc)));
+      splits = std::max<long>(1, std::min(std::min(splits, max_splits), 4096L));
+      long cps = (nchunks + splits - 1) / splits;
+      splits = (nchunks + cps - 1) / cps;
+      jd.splits = (short)splits;
+      jd.cps = (int)cps;
+      pd.item0[j] = item;
+      jd.part0 = part;
+      item += (int)splits * ntiles;
+      part += (int)splits;
+    }
+    hp.items = item;
+    return part;
+  };
+  int part = deal(hp.w == 1 ? 3072.0 : (double)RESIDENT_TILES);
+  if (hp.w == 2 && group_cps == 0 && hp.items > ROUND_LIMIT) part = deal(LONG_ROUND);
   for (int j = pd.njobs; j < MAX_JOBS; ++j) pd.item0[j] = INT_MAX;
-  hp.items = item;
   hp.partial_floats = (size_t)(part + pd.npairs) * c * c;     // partials, then the block sums
   hp.sum_offset = (size_t)part * c * c;
   hp.ok = true;

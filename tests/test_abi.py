@@ -103,6 +103,13 @@ def test_correlation_plan_fits_one_round(n, c, side):
     assert 256 < splits * tiles <= 512 + 64 // 2
 
 
+@pytest.mark.parametrize('n,c,side', [(39, 400, 16), (2, 324, 52)])
+def test_correlation_plan_of_many_tiles(n, c, side):
+    """Where whole splits make a good deal more than one round of items in any case, they are shorter."""
+    size = _hip.load().kfac_factor_conv_a_workspace_bytes(n, c, side, side, 3, 3, 1, 1, 1, 1, 1, 1, 0)
+    assert (size // (4 * c * c) - 45) * (-(-c // 128)) ** 2 > 1.375 * 512
+
+
 @pytest.mark.parametrize('d,rows,splits', [(1600, 8192, 5), (2176, 8192, 3), (2304, 8192, 4),
                                            (2304, 2000, 2)])
 def test_splits_of_a_single_product(d, rows, splits):
