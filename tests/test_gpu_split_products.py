@@ -23,11 +23,16 @@ def _assert_float32_sum(got, a, b, what, where=None, plus=0.):
     sum of exact products, of which the terms of relative size 2^-23 and below are left
     out, added to float32 accumulators in at most K / 16 + 1 steps each for the leading and
     the correction terms (16 products per step, each step within 2^-23 of the running sum of
-    absolute values), over at most K / 128 + 1 partial sums."""
+    absolute values), over at most K / 128 + 1 partial sums.  At the small end of the range an
+    element below 2^-109 is rounded to a multiple of 2^-133, the smallest bf16 number, and
+    a sum to one of 2^-149 at every step of either accumulator."""
     K = a.shape[0]
     want = a.t() @ b + plus
     mass = a.abs().t() @ b.abs() + abs(plus)
-    bound = mass * (2. ** -23) * (2 * (K // 16 + 1) + K // 128 + 4) + 1e-37
+    tiny = lambda x: ((x.abs() < 2. ** -109) & (x != 0)).double()
+    rounded = 2. ** -134 * (tiny(a).t() @ b.abs() + a.abs().t() @ tiny(b))
+    bound = mass * (2. ** -23) * (2 * (K // 16 + 1) + K // 128 + 4) + rounded \
+        + 2. ** -149 * (2 * (K // 16 + 1) + K // 128 + 4)
     over = (got.double() - want).abs() / bound
     over = (over if where is None else over[where]).max().item()
     assert over <= 1., '%s: error %.2f times the bound' % (what, over)
@@ -150,6 +155,16 @@ def test_magnitudes(ops, dev, exponent):
     x *= 10. ** torch.linspace(exponent - 3, exponent + 3, 300, device=dev)
     out = ops.factor_linear(x, False, 1.)
     _assert_float32_sum(out, x.double(), x.double(), 'magnitudes around 1e%d' % exponent)
+
+
+@pytest.mark.parametrize('rows', [20, 200])
+def test_smallest_elements(ops, dev, rows):
+    # columns from 1e-38 to 1e18: subnormal parts, subnormal products and elements of less than 24 bits
+    gen = torch.Generator(device=dev).manual_seed(5)
+    x = torch.randn(rows, 300, device=dev, generator=gen)
+    x *= 10. ** torch.linspace(-38, 18, 300, device=dev, dtype=torch.float64).float()
+    out = ops.factor_linear(x, False, 1.)
+    _assert_float32_sum(out, x.double(), x.double(), 'columns from 1e-38 on')
 
 
 @pytest.mark.parametrize('hw', [(4, 8), (7, 7)])
