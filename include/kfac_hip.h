@@ -19,6 +19,9 @@
  *  - sizes: any single matrix (factor, inverse, gradient viewed as 2-D) is at most
  *    1 GiB (16384 x 16384 fp32); layer inputs of any size are accepted (the factor
  *    builders consume them in slices of at most 1 GiB along the batch dimension);
+ *  - precision: products are float32 sums of exact products, infinities and NaN included.
+ *    An element below 1.5e-33 (2^-109) enters the products of 128-wide tiles rounded to a
+ *    multiple of 2^-133: its products with large elements keep 2^-134 / |x| instead of 2^-24;
  *  - entry points are re-entrant: they may be called from any host thread
  *    (the backward hooks of the host code run on autograd's worker thread).
  */
@@ -85,13 +88,13 @@ int kfac_factor_conv_a(const float* x, int n, int c, int H, int W,
                        int add_bias, float alpha, float beta, const float* C_prev, float* C,
                        void* workspace, size_t workspace_bytes, void* stream);
 
-/* Plan queries (no device needed): the fp32 MFMA flops the factor builders execute for a
- * d x d factor reduced over K terms (kfac_factor_linear, kfac_factor_conv_g and the
- * pointwise case of kfac_factor_conv_a; images of h*w positions with h*w no multiple of 4
+/* Plan queries (no device needed): the flops of float32 products that the factor builders
+ * execute for a d x d factor reduced over K terms (kfac_factor_linear, kfac_factor_conv_g and
+ * the pointwise case of kfac_factor_conv_a; images of h*w positions with h*w no multiple of 4
  * execute up to 3 more of them each in 128-wide tiles, which the first query does not
- * know) and for a Conv2d input factor of the given geometry: whole tiles of the upper triangle, whole reduction chunks, the shared spatial
- * correlations of a stride-1 k x k layer.  For utilisation figures next to the
- * algorithmic 2*d*d*K. */
+ * know) and for a Conv2d input factor of the given geometry: whole tiles of the upper
+ * triangle, whole reduction chunks, the shared spatial correlations of a stride-1 k x k
+ * layer.  For utilisation figures next to the algorithmic 2*d*d*K. */
 double kfac_factor_executed_flops(int d, int64_t K);
 double kfac_factor_conv_a_executed_flops(int n, int c, int H, int W, int kh, int kw,
                                          int sh, int sw, int ph, int pw, int dh, int dw,
@@ -148,7 +151,7 @@ size_t kfac_factor_grouped_workspace_bytes(int count, const kfac_factor_job* job
 int kfac_factor_grouped(int count, const kfac_factor_job* jobs, void* workspace,
                         size_t workspace_bytes, void* stream);
 
-/* Plan query: the fp32 MFMA flops kfac_factor_grouped executes for this list. */
+/* Plan query: the flops of float32 products that kfac_factor_grouped executes for this list. */
 double kfac_factor_grouped_executed_flops(int count, const kfac_factor_job* jobs);
 
 /* ---- Damped factor inversion ------------------------------------------- */
@@ -262,7 +265,7 @@ int kfac_cholesky_upper_batched(int count, const int* dims, const float* const* 
 /* Scratch for the two routines below (dG, dA: HOST arrays). */
 size_t kfac_precondition_workspace_bytes(int layers, const int* dG, const int* dA);
 
-/* Plan query: the fp32 MFMA flops the preconditioning of these layers executes (HOST
+/* Plan query: the flops of float32 products that the preconditioning of these layers executes (HOST
  * arrays; a NULL flag array: no side is given by its triangular factor): whole 128 x 128
  * tiles; a triangular operand is applied twice, each time over the non-zero part of the
  * reduction (the diagonal tiles' zero half included). */

@@ -92,10 +92,9 @@ inline long group_item_chunks(int w, double units, long dflt) {
 }
 
 // Tiles' worth of MFMA work in the T(T+1)/2 upper tiles of a symmetric product with T tiles
-// per side: of a diagonal tile's 32x32 blocks a 128-wide tile of four waves computes 12 of 16 (three
-// each, split_tile_tri) and a 64-wide tile of one wave 3 of 4.
-inline double syrk_tile_units(int T, int w) {
-  (void)w;
+// per side: of the 32x32 blocks of a diagonal tile a 128-wide one of four waves computes 12 of 16
+// (three each, split_tile_tri), a 64-wide one of one wave 3 of 4.
+inline double syrk_tile_units(int T) {
   return (double)T * (T - 1) / 2 + T * (3. / 4.);
 }
 

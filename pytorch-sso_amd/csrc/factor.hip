@@ -251,7 +251,7 @@ static double syrk_executed_flops(int d, int64_t terms, int64_t K) {
   const SyrkPlan p = plan_syrk(d, (long)terms);
   const int kc = p.w == 1 ? Cfg<1, 1>::KC : Cfg<2, 2>::KC;
   const double chunks = (double)((K + kc - 1) / kc);
-  return syrk_tile_units(p.T, p.w) * chunks * kc * 2.0 * p.ts * p.ts;
+  return syrk_tile_units(p.T) * chunks * kc * 2.0 * p.ts * p.ts;
 }
 
 double kfac_factor_executed_flops(int d, int64_t K) {

@@ -412,7 +412,7 @@ static GroupedPlan make_plan(int count, const kfac_factor_job* jobs) {
         else if (p.splits > 1)
           gp.reduce_tile[w].push_back(i);
         gp.executed_flops +=
-            syrk_tile_units(p.T, p.w) * (double)((c.K + 15) / 16) * 16 * 2.0 * p.ts * p.ts;
+            syrk_tile_units(p.T) * (double)((c.K + 15) / 16) * 16 * 2.0 * p.ts * p.ts;
       }
     }
   for (int path = 0; path < SYRK_PATHS; ++path)

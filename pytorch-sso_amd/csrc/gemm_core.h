@@ -1,14 +1,14 @@
 // fp32 MFMA GEMM tile engine for gfx950 (CDNA4, wave64).
 //
-// One workgroup of 256 threads (4 waves, 2x2) computes a 128x128 tile of
+// One workgroup of 64 threads (one wave), or of 256 (4 waves, 2x2), computes a 64x64 or 128x128
+// tile of
 //     C[m][n] = sum_k  P(k, m) * Q(k, n)          k in [kbeg, kend)
 // with v_mfma_f32_32x32x2_f32.  Each wave owns a 64x64 sub-tile (2x2 MFMA
 // blocks, 64 accumulator registers).  Operands are described by functors that
-// map (k, m) to a global-memory element, so the same engine serves
-//   * factor builds (X^T X for Linear, implicit im2col for Conv2d),
-//   * the trailing updates / triangular products of the blocked inverse,
-//   * the two chained preconditioning GEMMs,
-// without ever materialising a transposed, concatenated or unfolded copy.
+// map (k, m) to a global-memory element, so the same engine serves the 64-wide tiles of all factor
+// builds (X^T X for Linear, implicit im2col and correlations for Conv2d) and the 128-wide ones of
+// the per-sample gradients of a convolution, without ever materialising a transposed,
+// concatenated or unfolded copy.  All other products run on the bf16 matrix cores (gemm_split.h).
 //
 // Operand functor contract (details in operands.h):
 //   static constexpr int layout;      KM: consecutive m are contiguous in memory
@@ -36,8 +36,8 @@ constexpr int NTHREADS = 256;    // threads of the default configuration
 
 // A configuration is WM x WN waves, each owning a 64x64 sub-tile:
 //   tile = (64*WM) x (64*WN), threads = 64*WM*WN.
-// 2x2 is the default; 1x1 (one wave, 64x64) serves small factors, where a
-// 128-wide tile would be mostly padding.
+// 1x1 (one wave, 64x64) serves small factors, where a 128-wide tile would be mostly
+// padding.
 // KC = 16 is the reduction depth per LDS stage (32 MFMAs per wave and stage);
 // two stages of the 2x2 configuration take 40 KiB, so that three workgroups
 // fit the 160 KiB of a CU.
@@ -303,46 +303,20 @@ __device__ __forceinline__ void acc_coords(int m0, int n0, int a, int b, int i, 
 }
 
 // The MFMAs of k-steps [S0, S1) of a 16-deep slice.  A diagonal tile of a symmetric product
-// is symmetric itself: with SKIP its 32x32 blocks below the diagonal are not computed, and
-// the blocks above it are stored twice.  The 10 blocks of a 128-wide tile are dealt 3, 2, 2, 3
-// over its four waves: the waves on the diagonal quadrants take the three blocks of theirs,
-// and the quadrant above the diagonal is shared by the wave that owns it (upper two blocks)
-// and the wave of the quadrant below the diagonal (lower two), so the tile is done in three
-// quarters of the time.  The single wave of a 64-wide tile takes its three blocks.  The
-// matrix cores this leaves alone serve the other workgroups of the compute unit; a launch
-// with few workgroups per unit has little to gain and pays for the mirrored stores.
-enum { WAVE_FULL = 0, WAVE_DIAG = 1, WAVE_ROW0 = 2, WAVE_ROW1 = 3 };
+// is symmetric itself: with SKIP (64-wide tiles of one wave) its 32x32 block below the diagonal is not
+// computed, and the one above it is stored twice: three quarters of the time.  The matrix cores
+// this leaves alone serve the other workgroups of the compute unit; a launch with few workgroups
+// per unit has little to gain and pays for the mirrored stores.
 template <int S0, int S1, bool SKIP>
 __device__ __forceinline__ void mma_slice(const float (&fa)[2][8], const float (&fb)[2][8],
-                                          v16f (&acc)[2][2], int mode) {
-  if (!SKIP || mode == WAVE_FULL) {
+                                          v16f (&acc)[2][2]) {
 #pragma unroll
-    for (int s = S0; s < S1; ++s)
+  for (int s = S0; s < S1; ++s)
 #pragma unroll
-      for (int a = 0; a < 2; ++a)
+    for (int a = 0; a < 2; ++a)
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
-          acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[a][s], fb[b][s], acc[a][b], 0, 0, 0);
-  } else if (mode == WAVE_DIAG) {
-#pragma unroll
-    for (int s = S0; s < S1; ++s) {
-      acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[0][s], fb[0][s], acc[0][0], 0, 0, 0);
-      acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[0][s], fb[1][s], acc[0][1], 0, 0, 0);
-      acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[1][s], fb[1][s], acc[1][1], 0, 0, 0);
-    }
-  } else if (mode == WAVE_ROW0) {
-#pragma unroll
-    for (int s = S0; s < S1; ++s) {
-      acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[0][s], fb[0][s], acc[0][0], 0, 0, 0);
-      acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[0][s], fb[1][s], acc[0][1], 0, 0, 0);
-    }
-  } else {
-#pragma unroll
-    for (int s = S0; s < S1; ++s) {
-      acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[1][s], fb[0][s], acc[1][0], 0, 0, 0);
-      acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[1][s], fb[1][s], acc[1][1], 0, 0, 0);
-    }
-  }
+      for (int b = SKIP ? a : 0; b < 2; ++b)
+        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[a][s], fb[b][s], acc[a][b], 0, 0, 0);
 }
 
 // acc_coords for a wave whose quadrant starts at (wm, wn) of the tile
@@ -359,7 +333,7 @@ __device__ __forceinline__ void quad_coords(int m0, int n0, int wm, int wn, int 
 // vector access are staged with 16-byte loads (the caller has checked that the tile allows it).
 template <int WM, int WN, bool SAME, bool SKIP, bool VEC, class OPP, class OPQ>
 __device__ __forceinline__ void gemm_tile_loop(const OPP& P, const OPQ& Q, int m0, int n0, int kbeg,
-                                               int kend, float* smem, int wm, int wn, int mode,
+                                               int kend, float* smem, int wm, int wn,
                                                v16f (&acc)[2][2]) {
   typedef Cfg<WM, WN> C;
   constexpr bool same = SAME;
@@ -410,14 +384,14 @@ __device__ __forceinline__ void gemm_tile_loop(const OPP& P, const OPQ& Q, int m
           load_frags<OPQ::layout, C::TN, C::LDS_MK>(tqc, wn, r, h, 16 * sl, fb);
       }
       if (sl == KC / 16 - 1) {
-        mma_slice<0, 4, SKIP>(fa, fb, acc, mode);
+        mma_slice<0, 4, SKIP>(fa, fb, acc);
         if (more) {
           sp.commit(tpn);
           if (!same) sq.commit(tpn + C::P_FLOATS);
         }
-        mma_slice<4, 8, SKIP>(fa, fb, acc, mode);
+        mma_slice<4, 8, SKIP>(fa, fb, acc);
       } else {
-        mma_slice<0, 8, SKIP>(fa, fb, acc, mode);
+        mma_slice<0, 8, SKIP>(fa, fb, acc);
       }
     }
     __syncthreads();
@@ -425,16 +399,44 @@ __device__ __forceinline__ void gemm_tile_loop(const OPP& P, const OPQ& Q, int m
 
 }
 
-// The accumulators of the calling wave's quadrant through the epilogue.
-template <bool SKIP, class EPI>
-__device__ __forceinline__ void store_tile(const v16f (&acc)[2][2], int m0, int n0, int wm, int wn,
-                                           int mode, EPI& epi) {
+template <int WM, int WN, bool SAME, bool SKIP, class OPP, class OPQ, class EPI>
+__device__ __forceinline__ void gemm_tile_impl(const OPP& P, const OPQ& Q, int m0, int n0,
+                                               int kbeg, int kend, EPI& epi, float* smem) {
+  typedef Cfg<WM, WN> C;
+  constexpr bool same = SAME;
+  const int t = threadIdx.x & (C::NT - 1);
+  const int lane = t & 63;
+  const int wave = t >> 6;
+  const int r = lane & 31;
+  const int h = lane >> 5;
+  const int wm = (wave / WN) * 64;
+  const int wn = (wave % WN) * 64;
+  static_assert(!SKIP || (SAME && WM == 1 && WN == 1),
+                "only a 64-wide diagonal tile of a symmetric product has a block to skip");
+
+  v16f acc[2][2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.f;
+
+  // (uniform per workgroup: the tile lies inside the columns that vector loads may fetch)
+  constexpr bool can_vec = offers_vec4<OPP>::value || (!SAME && offers_vec4<OPQ>::value);
+  bool vec = false;
+  if constexpr (can_vec) vec = vec_tile_ok(P, m0, C::TM) && (same || vec_tile_ok(Q, n0, C::TN));
+  if constexpr (can_vec) {
+    if (vec)
+      gemm_tile_loop<WM, WN, SAME, SKIP, true>(P, Q, m0, n0, kbeg, kend, smem, wm, wn, acc);
+  }
+  if (!vec)
+    gemm_tile_loop<WM, WN, SAME, SKIP, false>(P, Q, m0, n0, kbeg, kend, smem, wm, wn, acc);
+
   // A diagonal tile of a symmetric product: the blocks above the tile's diagonal are
   // stored at their mirror position too, the blocks below it were not computed.
-  auto computed = [&](int a, int b) {
-    return !SKIP || (mode == WAVE_DIAG ? a <= b : a == (mode == WAVE_ROW0 ? 0 : 1));
-  };
-  auto mirrored = [&](int a, int b) { return SKIP && computed(a, b) && (wm + 32 * a < wn + 32 * b); };
+  auto computed = [](int a, int b) { return !SKIP || a <= b; };
+  auto mirrored = [](int a, int b) { return SKIP && a < b; };
 
   if constexpr (reading_epilogue<EPI>::value) {
     // C = alpha*acc + beta*C_old: the old values are loaded 32 at a time ahead of the
@@ -482,55 +484,6 @@ __device__ __forceinline__ void store_tile(const v16f (&acc)[2][2], int m0, int 
           if (mirrored(a, b)) epi.store(col, row, acc[a][b][i]);
         }
       }
-}
-
-template <int WM, int WN, bool SAME, bool SKIP, class OPP, class OPQ, class EPI>
-__device__ __forceinline__ void gemm_tile_impl(const OPP& P, const OPQ& Q, int m0, int n0,
-                                               int kbeg, int kend, EPI& epi, float* smem) {
-  typedef Cfg<WM, WN> C;
-  constexpr bool same = SAME;
-  const int t = threadIdx.x & (C::NT - 1);
-  const int lane = t & 63;
-  const int wave = t >> 6;
-  const int r = lane & 31;
-  const int h = lane >> 5;
-  int wm = (wave / WN) * 64;
-  int wn = (wave % WN) * 64;
-  static_assert(SAME || !SKIP, "only a diagonal tile of a symmetric product has blocks to skip");
-  static_assert(!SKIP || (WM == WN && WM <= 2), "skipping is written for 64- and 128-wide tiles");
-  int mode = WAVE_FULL;
-  if (SKIP) {
-    if (wm == wn) {
-      mode = WAVE_DIAG;
-    } else if (wm < wn) {
-      mode = WAVE_ROW0;
-    } else {             // the quadrant below the diagonal: the lower half of the one above
-      mode = WAVE_ROW1;
-      wm = 0;
-      wn = 64;
-    }
-  }
-
-  v16f acc[2][2];
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.f;
-
-  // (uniform per workgroup: the tile lies inside the columns that vector loads may fetch)
-  constexpr bool can_vec = offers_vec4<OPP>::value || (!SAME && offers_vec4<OPQ>::value);
-  bool vec = false;
-  if constexpr (can_vec) vec = vec_tile_ok(P, m0, C::TM) && (same || vec_tile_ok(Q, n0, C::TN));
-  if constexpr (can_vec) {
-    if (vec)
-      gemm_tile_loop<WM, WN, SAME, SKIP, true>(P, Q, m0, n0, kbeg, kend, smem, wm, wn, mode, acc);
-  }
-  if (!vec)
-    gemm_tile_loop<WM, WN, SAME, SKIP, false>(P, Q, m0, n0, kbeg, kend, smem, wm, wn, mode, acc);
-
-  store_tile<SKIP>(acc, m0, n0, wm, wn, mode, epi);
 }
 
 // SKIP_LOWER: a diagonal tile (`same`) leaves out its blocks below the diagonal.

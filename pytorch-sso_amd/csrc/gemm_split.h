@@ -7,6 +7,9 @@
 // rounded rest of the ones before), x = h + m + l, so a product of two floats is nine
 // products of bf16 numbers, each exact in float32:
 //     x y = h h' + (h m' + m h') + (h l' + m m' + l h') + [m l' + l m' + l l'].
+// (An element below 2^-109, 1.5e-33, is that sum only down to 2^-133, the smallest bf16 number: it
+// enters rounded to a multiple of that, so that a product with a large factor keeps 2^-134 / |x|
+// instead of 2^-24.)
 // The bracket is at most 2^-23 and on average 2^-26 of x y, below the rounding of one float32
 // accumulation, and is left out; the other six run as v_mfma_f32_32x32x16_bf16.  The leading
 // products and the five corrections have accumulators of their own: the leading ones are
@@ -15,6 +18,8 @@
 // engine / v_mfma_f32_32x32x2_f32 on the same data):
 //     N(0,1):           K = 128  6.3e-8 / 2.2e-7    K = 4096  4.0e-7 / 1.1e-6    K = 65536  1.7e-6 / 4.6e-6
 //     max(0, N(0,1)):   K = 128  4.4e-8 / 8.6e-8    K = 4096  3.2e-7 / 5.0e-7    K = 65536  1.4e-6 / 2.0e-6
+// and a factor of N(0,1) (either engine): K = 1  2.6e-8 / 2.5e-8, worst element 1.7 / 1.0 times 2^-24;
+// 2  2.6e-8 / 3.1e-8;  4  2.7e-8 / 4.0e-8;  16  3.3e-8 / 7.3e-8;  53  4.7e-8 / 1.3e-7
 // (with all six products in one accumulator the errors are those of the fp32 instruction,
 // and sums of positive terms drift by -1.3e-6 at K = 65536: the accumulation inside the
 // instruction rounds down.)
@@ -351,20 +356,19 @@ __device__ __forceinline__ void static_for(F&& f) {
 // The 32x32 blocks of a tile that one wave computes.
 // FULL: the four blocks of its 64x64 quadrant, block (a, b) = rows a of P against rows b of Q.
 // TRI: a diagonal tile of a symmetric product (P = Q) is symmetric itself; its blocks on and
-// above the diagonal (10 of 16 in a 128-wide tile, 3 of 4 in a 64-wide one) are dealt to the
-// waves three at a time, as products of three fragment rows r0, r1, r2 of the one operand:
+// above the diagonal (10 of 16) are dealt to the four waves three at a time, as products of three
+// fragment rows r0, r1, r2 of the one operand:
 //     block 0 = (r0, r1)    block 1 = (r0, r2)    block 2 = (r1, r1)
-//   waves 0 / 1 of a 128-wide tile: r = (0, 1, 0) / (2, 3, 2), the three blocks of a diagonal
-//   quadrant;  waves 2 / 3: r = (0, 2, 3) / (1, 2, 3), a row of the quadrant above the
-//   diagonal (their block 2 repeats one of wave 1's and is not stored).
+//   waves 0 / 1: r = (0, 1, 0) / (2, 3, 2), the three blocks of a diagonal quadrant;
+//   waves 2 / 3: r = (0, 2, 3) / (1, 2, 3), a row of the quadrant above the diagonal (their block 2
+//   repeats one of wave 1's and is not stored).
 // Every wave runs the same code, and the tile is done in three quarters of the time.
 struct SplitTri {
   int r[3];
   bool last;           // block 2 is this wave's to store
 };
-template <int W>
 __device__ __forceinline__ SplitTri split_tri(int wave) {
-  if (W == 1 || wave == 0) return SplitTri{{0, 1, 0}, true};
+  if (wave == 0) return SplitTri{{0, 1, 0}, true};
   if (wave == 1) return SplitTri{{2, 3, 2}, true};
   return SplitTri{{wave - 2, 2, 3}, false};
 }
@@ -707,14 +711,14 @@ __device__ __forceinline__ void split_tile_full(const OPP& P, const OPQ& Q, int 
 
 // a diagonal tile of a symmetric product: with `both`, the blocks above its diagonal are stored
 // at their mirror positions too
-template <int W, class OP, class STORE>
+template <class OP, class STORE>
 __device__ __forceinline__ void split_tile_tri(const OP& P, int m0, int kbeg, int kend, float* smem,
                                                bool both, const STORE& store) {
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x & (64 * W * W - 1)) >> 6);
-  const SplitTri t = split_tri<W>(wave);
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x & (SplitCfg<2, 2>::NT - 1)) >> 6);
+  const SplitTri t = split_tri(wave);
   const int prow[3] = {32 * t.r[0], 32 * t.r[1], 32 * t.r[2]}, qrow[2] = {0, 0};
   v16f acc[3];
-  split_blocks<W, W, true>(P, P, m0, m0, kbeg, kend, smem, prow, qrow, acc);
+  split_blocks<2, 2, true>(P, P, m0, m0, kbeg, kend, smem, prow, qrow, acc);
   const int row0[3] = {m0 + prow[0], m0 + prow[0], m0 + prow[1]};
   const int col0[3] = {m0 + prow[1], m0 + prow[2], m0 + prow[1]};
   const int above = both ? BLK_BOTH : BLK_PLAIN, on = both ? BLK_UPPER_BOTH : BLK_UPPER;
@@ -732,7 +736,7 @@ __device__ __forceinline__ void split_tile(const OPP& P, const OPQ& Q, int m0, i
   auto store = [&](auto&& put) { put(epi); };
   if constexpr (std::is_same<OPP, OPQ>::value) {
     if (same) {
-      split_tile_tri<2>(P, m0, kbeg, kend, smem, both, store);
+      split_tile_tri(P, m0, kbeg, kend, smem, both, store);
       return;
     }
   }

@@ -19,7 +19,7 @@ __device__ __forceinline__ void syrk_tile(const OP& op, int bi, int bj, int kbeg
       if (unsplit) put(whole);
       else put(part);
     };
-    if (bi == bj) split_tile_tri<W>(op, bi * TS, kbeg, kend, smem, true, store);
+    if (bi == bj) split_tile_tri(op, bi * TS, kbeg, kend, smem, true, store);
     else split_tile_full<W, W>(op, op, bi * TS, bj * TS, kbeg, kend, smem, store);
   } else {
     if (unsplit) gemm_tile_cfg<W, W, true>(op, op, bi * TS, bj * TS, kbeg, kend, bi == bj, whole, smem);
