@@ -675,7 +675,7 @@ static TapOrder make_order(const TapPlanHost& hp, std::vector<unsigned>& entries
 }
 
 // chunks per item of a grouped launch (one-wave 64-wide tiles / four-wave 128-wide tiles);
-// measured flat between 48 and 192
+// factors of a ResNet-50, 32 images: 4.62 / 4.57 / 4.64 ms with 64 / 96 / 128 chunks of 128-wide tiles
 constexpr int TAPS_GROUP_CPS1 = 192, TAPS_GROUP_CPS2 = 96;
 
 static TapsGroupPlan* make_taps_group_plan(int count, const TapsJob* jobs) {

@@ -178,7 +178,8 @@ __global__ __launch_bounds__(256) void conv_planes_kernel(const PlaneJob* __rest
 
 // Items of a grouped launch are dispatched longest first and the launch holds many of
 // them, so an item may be long: about this many 16-deep chunks, which keeps the
-// partial tiles that a split writes and the reduction reads small beside the input.
+// partial tiles that a split writes and the reduction reads small beside the input.  (Factors of a
+// ResNet-50, 32 images: 4.69 / 4.57 / 4.66 ms with 64 / 96 / 128 chunks of 128-wide tiles.)
 constexpr int GROUP_TARGET_CPS_W2 = 96;
 constexpr int GROUP_TARGET_CPS_W1 = 192;
 constexpr int MANY_SPLITS = 16;          // above: the reduction with 16 split lanes
@@ -191,8 +192,8 @@ struct GroupPlan {
 };
 
 // 64-wide tiles (one wave each) up to 192 rows; from there a 128-wide tile has at most a
-// quarter of padding and loads half as many operand elements per matrix instruction
-// (factors of 256 rows: 7 % faster on 128-wide tiles).
+// quarter of padding, and it runs on the bf16 matrix cores (factors of a ResNet-50, 32 images: 4.57 ms,
+// and 5.1 ms with 64-wide tiles up to 256 rows; 128 rows make no difference there).
 constexpr int GROUP_W1_MAX_DIM = 192;
 
 static GroupPlan plan_group(int d, long K, long target) {

@@ -504,20 +504,18 @@ __device__ __forceinline__ bool trail_tile(int T, int row_lo, int row_hi, int lo
 // updates only the remaining rows of that group (nk = 1), and the rows beyond it receive
 // the whole group at once (nk = GROUP_BLOCKS), which cuts the read-modify-write passes over
 // the trailing matrix by that factor (a rank-128 update of a large trailing matrix is
-// bound by memory traffic, not by the matrix cores).  Taller groups run no faster (measured
-// up to 16: the tiles that ride along with a diagonal block are hidden either way) and
-// cost accuracy: the float32 error of the inverse of a 9217^2 factor with condition number
-// 9e2 grows from 2.2e-5 (height 1) over 5.2e-5 (4; scipy's float32 LU inverse: 4.7e-5) to
-// 1.0e-4 (16), because a deeper product accumulates more terms before it meets the
-// entry it nearly cancels.
+// bound by memory traffic, not by the matrix cores).  Taller groups cost the factors of a ResNet-50
+// more than they bring to larger matrices (height 4 / 6 / 8: 3.71 / 3.81 / 3.92 ms; 9217 / 4097 / 4097
+// and smaller 7.44 / 7.32 / 7.39), and accuracy: on the fp32 tile engine the error of the
+// inverse of a 9217^2 factor with condition number 9e2 grew from 2.2e-5 (height 1) over
+// 5.2e-5 (4; scipy's float32 LU inverse: 4.7e-5) to 1.0e-4 (16), because a deeper product
+// accumulates more terms before it meets the entry it nearly cancels.
 constexpr int GROUP_BLOCKS = 4;
 // The last TAIL_BLOCKS diagonal blocks of the largest matrices form one group: the deeper
 // update of the rows beyond a group is a launch that lasts as long as one 512-deep tile
-// (50 us) however few tiles it has, while the rank-128 updates of a short trailing matrix
-// all fit beside the next diagonal block (up to three tiles per compute unit there).
-// (with the tiles packed three to a workgroup: config 3 inversion 4.75 / 4.77 / 4.90 / 5.16 ms
-// with 16 / 24 / 32 / 40; a 3201^2 and a 1601^2 matrix 1.68 / 1.58 / 1.53 / 1.53 ms; three
-// 9217 / 4097 / 4097 matrices 10.12 / 10.03 / 9.95 / 9.92 ms and 10.58 ms with 64)
+// however few tiles it has, while the rank-128 updates of a short trailing matrix
+// fit beside the next diagonal block.  16 / 24 / 32 / 40: the factors of a ResNet-50 3.76 / 3.71 /
+// 4.00 / 4.40 ms, matrices of 9217 / 4097 / 4097 and smaller 7.48 / 7.44 / 7.35 / 7.36.
 constexpr int TAIL_BLOCKS = 24;
 
 __global__ __launch_bounds__(NTHREADS, 2) void potrf_trail_kernel(const MatDesc* table, int kb0,
@@ -979,8 +977,8 @@ __host__ __device__ inline int merge_tiles(int T, int depth) {
 }
 
 // Tile `local` of the merges at `depth`, longest reduction first: a launch lasts at least
-// as long as its longest tile (up to T/2 blocks on ONE compute unit, shared with two other
-// workgroups), so those start first and the launch ends on its one-block tiles.  The
+// as long as its longest tile (up to T/2 blocks on ONE compute unit, shared with another
+// workgroup), so those start first and the launch ends on its one-block tiles.  The
 // reduction of the first product grows with the column of the tile (`fast` = column, the
 // tiles of a column share the Y22 panel), that of the second shrinks with the row (`fast`
 // = row, its tiles share the Y11 panel).  The halves of all segments of a depth differ by
