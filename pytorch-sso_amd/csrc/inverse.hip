@@ -129,8 +129,13 @@ __global__ __launch_bounds__(256) void inv_copy_damp_kernel(const MatDesc* table
 // 128x128 diagonal block: Cholesky (upper) and its inverse, in LDS.
 // ---------------------------------------------------------------------------
 constexpr int DB = 128;          // diagonal block size
-constexpr int DLD = DB + 1;      // LDS leading dimension
-constexpr int DIAG_SMEM_BYTES = 2 * DB * DLD * (int)sizeof(float);
+constexpr int DLD = DB + 4;      // LDS leading dimension (rows of 16-byte pieces)
+// S and Z; what the steps of the strips leave; the A operands of one strip; marks by strip and block
+// column; write items taken
+constexpr int DIAG_STEPS = 4 * 16 * 4;
+constexpr int DIAG_OPS = 16 * 64;
+constexpr int DIAG_MARKS = 4 * 8 * 8;
+constexpr int DIAG_SMEM_BYTES = (2 * DB * DLD + DIAG_STEPS + DIAG_OPS + DIAG_MARKS + 4) * (int)sizeof(float);
 
 __device__ __forceinline__ float lane_value(float v, int src_lane) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), src_lane));
@@ -182,8 +187,10 @@ __device__ __forceinline__ v16f lds_mma32(const lds_f* a, int a_ks, int a_is, co
 // h = lane >> 5) is (row 8*(t/4) + 4*h + t%4, column r), so row c of a block is ONE register
 // (index 4*(c/8) + c%4) in the 32 lanes of half (c/4)%2, lane = column, and rows c, c+1
 // (c even) are neighbouring registers in the same half.
-//   L: the diagonal leaf, a full symmetric 32x32 block (Schur complement of the rows above);
-//   P: the same rows of another 32 columns (a block of the row panel, or of [ . | identity]).
+//   L: the diagonal leaf, a full symmetric 32x32 block (Schur complement of the rows above),
+//      held by the wave that leads the strip;
+//   P: the same rows of another 32 columns (a block of the row panel, or of [ . | identity]),
+//      held by a wave that follows.
 // A step finishes rows c and c+1:  with the 2x2 pivot block [p00 p01; p01 p11] of L,
 //   w0 = L[c] / sqrt(p00),  u01 = p01 / sqrt(p00),  w1 = (L[c+1] - u01 w0) / sqrt(p11 - u01^2)
 // are rows c, c+1 of U (the same combination y0, y1 of P's rows: those rows of the second
@@ -195,10 +202,15 @@ __device__ __forceinline__ v16f lds_mma32(const lds_f* a, int a_ks, int a_is, co
 // v_permlane32_swap moves the second into the other half; apart from that and the three
 // pivot entries (v_readlane) no value changes lanes.  The chain from step to step is
 //   matrix instruction -> pivots -> two 1/sqrt -> w1 -> swap -> matrix instruction.
-// The finished rows go to LDS as they are made, straight from the operand registers
-// (`leaf_rows`: where U_qq goes, or a block of LDS that nothing reads for a wave that only
-// needs the multipliers; `blk_rows`: the second block's rows).  Below its diagonal U_qq is
-// left with rounding noise there; whoever copies it out writes zeros instead.
+// The leading wave does that and nothing else.  It leaves the finished rows in LDS, straight
+// from the operand register, its A operand, and behind them the two 1/sqrt, u01 and a mark; the waves
+// that follow read them, two steps ahead of their use, and end a few steps behind it.
+// (One wave with the leaf and a second block took 280-400 cycles a step: the second block's
+// instructions are not hidden behind the matrix instruction of the same wave.  Measured on one
+// wave: the leading step 170, 210 with what it leaves as one 16-byte store, 186 as it is; the
+// following one 122, and 190 with a matrix instruction of another accumulator in it.)
+// LDS serves the requests of a wave in order, so whoever sees the mark sees the rows.
+// Below its diagonal U_qq is left with rounding noise; whoever copies it out writes zeros instead.
 // `pmin`, `piv`: the smallest pivot so far and all 32 of them, for the caller's check.
 // With P = rows of the panel the strip ends as U[q][*] = U_qq^-T A[q][*] without a
 // triangular solve; with P = [pending | identity] as the rows of U^-T.
@@ -211,64 +223,214 @@ __device__ __forceinline__ float pair_operand(float x0, float x1) {
   return __builtin_bit_cast(float, H ? sw[1] : sw[0]);
 }
 
-template <int C>
-__device__ __forceinline__ void elim_pair(v16f& L, v16f& P, lds_f* leaf_rows, lds_f* blk_rows,
-                                          int r, float& pmin, float (&piv)[32]) {
-  constexpr int T = 4 * (C >> 3) + (C & 3), H = (C >> 2) & 1;
-  const float v0 = L[T], v1 = L[T + 1];
-  const float p00 = lane_value(v0, 32 * H + C);
-  const float p01 = lane_value(v0, 32 * H + C + 1);
-  const float p11 = lane_value(v1, 32 * H + C + 1);
-  const float r0 = __builtin_amdgcn_rsqf(p00);
-  const float u01 = p01 * r0;
-  const float d = fmaf(-u01, u01, p11);
-  const float r1 = __builtin_amdgcn_rsqf(d);
-  const float w0 = v0 * r0;
-  const float w1 = fmaf(-u01, w0, v1) * r1;
-  const float xb = pair_operand<H>(w0, w1);
-  const float xa = r > C + 1 ? -xb : 0.f;
-  if (C < 30) L = __builtin_amdgcn_mfma_f32_32x32x2f32(xa, xb, L, 0, 0, 0);
-  // (nothing below moves in front of that instruction: the second block's work belongs in
-  // the wait for its result)
-  __builtin_amdgcn_sched_barrier(0);
-  const float y0 = P[T] * r0;
-  const float y1 = fmaf(-u01, y0, P[T + 1]) * r1;
-  const float pb = pair_operand<H>(y0, y1);
-  if (C < 30) P = __builtin_amdgcn_mfma_f32_32x32x2f32(xa, pb, P, 0, 0, 0);
-  // the finished rows: the operand registers hold row C in the lanes 0-31 and row C+1 in the
-  // lanes 32-63, so one store writes both (the pointers carry the lane's row and column)
-  leaf_rows[C * DLD] = xb;
-  blk_rows[C * DLD] = pb;
-  pmin = fminf(fminf(pmin, p00), d);
-  piv[C] = p00;
-  piv[C + 1] = d;
-  __builtin_amdgcn_sched_barrier(0);
-}
+// What a step leaves for the waves that follow: {1/sqrt of its two pivots}, {u01, mark}, the mark
+// behind everything else (volatile: in this order, and the loads in front of what they guard)
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef volatile __attribute__((address_space(3))) float lds_vf;
+typedef volatile __attribute__((address_space(3))) v2f lds_vf2;
 
 template <int C>
-__device__ __forceinline__ void elim_from(v16f& L, v16f& P, lds_f* leaf_rows, lds_f* blk_rows,
-                                          int r, float& pmin, float (&piv)[32]) {
+__device__ __forceinline__ void lead_from(v16f& L, lds_vf* rows, lds_vf* ops, lds_vf2* steps, int r,
+                                          float& pmin, float (&piv)[32]) {
   if constexpr (C < 32) {
-    elim_pair<C>(L, P, leaf_rows, blk_rows, r, pmin, piv);
-    elim_from<C + 2>(L, P, leaf_rows, blk_rows, r, pmin, piv);
+    constexpr int T = 4 * (C >> 3) + (C & 3), H = (C >> 2) & 1;
+    const float v0 = L[T], v1 = L[T + 1];
+    const float p00 = lane_value(v0, 32 * H + C);
+    const float p01 = lane_value(v0, 32 * H + C + 1);
+    const float p11 = lane_value(v1, 32 * H + C + 1);
+    const float r0 = __builtin_amdgcn_rsqf(p00);
+    const float u01 = p01 * r0;
+    const float d = fmaf(-u01, u01, p11);
+    const float r1 = __builtin_amdgcn_rsqf(d);
+    const float w0 = v0 * r0;
+    const float w1 = fmaf(-u01, w0, v1) * r1;
+    const float xb = pair_operand<H>(w0, w1);
+    const float xa = r > C + 1 ? -xb : 0.f;
+    if (C < 30) L = __builtin_amdgcn_mfma_f32_32x32x2f32(xa, xb, L, 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    // (the operand register holds row C in the lanes 0-31 and row C+1 in the lanes 32-63: one
+    // store writes both, the pointer carries the lane's row and column)
+    rows[C * DLD] = xb;
+    ops[C / 2 * 64] = xa;
+    steps[C] = v2f{r0, r1};
+    steps[C + 1] = v2f{u01, 1.f};
+    pmin = fminf(fminf(pmin, p00), d);
+    piv[C] = p00;
+    piv[C + 1] = d;
+    __builtin_amdgcn_sched_barrier(0);
+    lead_from<C + 2>(L, rows, ops, steps, r, pmin, piv);
   }
 }
+
+__device__ __forceinline__ bool is_marked(float mark) {
+  return __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, mark)) != 0;
+}
+
+// What a following wave reads of two steps: the mark of the later one first
+struct TwoSteps {
+  v2f m1, s1, m0, s0;
+  float x0, x1;
+  __device__ __forceinline__ void read(const lds_vf* ops, const lds_vf2* steps) {
+    m1 = steps[3];
+    s1 = steps[2];
+    m0 = steps[1];
+    s0 = steps[0];
+    x0 = ops[0];
+    x1 = ops[64];
+  }
+  __device__ __forceinline__ bool ready() const { return is_marked(m1[1]); }
+};
+
+template <int C>
+__device__ __forceinline__ void follow_step(v16f& P, const v2f& s, float u01, float x, lds_vf* rows) {
+  constexpr int T = 4 * (C >> 3) + (C & 3), H = (C >> 2) & 1;
+  const float y0 = P[T] * s[0];
+  const float y1 = fmaf(-u01, y0, P[T + 1]) * s[1];
+  const float pb = pair_operand<H>(y0, y1);
+  if (C < 30) P = __builtin_amdgcn_mfma_f32_32x32x2f32(x, pb, P, 0, 0, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  rows[C * DLD] = pb;
+}
+
+// `ops`, `steps`: the strip's; `rows`: where the rows of P go (the pointer carries the lane's row and
+// column); `marks`: one for every two of its steps
+template <int C>
+__device__ __forceinline__ void follow_from(v16f& P, TwoSteps t, const lds_vf* ops,
+                                            const lds_vf2* steps, lds_vf* rows, lds_vf* marks) {
+  if constexpr (C < 32) {
+    // (the leading wave takes all its steps whatever it finds, and waits for nobody)
+    if (__builtin_expect(!t.ready(), 0)) {
+      do t.read(ops + C / 2 * 64, steps + C);
+      while (!t.ready());
+    }
+    // (a register of a load in flight that nobody uses would be given to the next load, which then
+    // waits for the first)
+    asm volatile("" :: "v"(t.m0));
+    TwoSteps tn = t;
+    if constexpr (C < 28) tn.read(ops + (C + 4) / 2 * 64, steps + C + 4);
+    __builtin_amdgcn_sched_barrier(0);
+    follow_step<C>(P, t.s0, t.m0[0], t.x0, rows);
+    follow_step<C + 2>(P, t.s1, t.m1[0], t.x1, rows);
+    marks[C / 4] = 1.f;
+    __builtin_amdgcn_sched_barrier(0);
+    follow_from<C + 4>(P, tn, ops, steps, rows, marks);
+  }
+}
+
+// What strip q takes from a block of a strip below,  A^T B  with A and B blocks of strip q, while the
+// waves that make their rows are at it: `a`, `b` (with the lane's row and column), two steps at a
+// time behind their marks.  Those waves end, see follow_from.
+struct Rows {
+  const lds_vf *a, *b;
+  const lds_vf *mark_a, *mark_b;
+};
+// PAIRS such products at a time.  The marks are read as one value, by lane, and tested at once.
+template <int PAIRS>
+__device__ __forceinline__ void collect(v16f (&N)[PAIRS], const Rows (&rows)[PAIRS]) {
+  const lds_vf* mark = threadIdx.x & 1 ? rows[0].mark_b : rows[0].mark_a;
+  if (PAIRS == 2 && (threadIdx.x & 2)) mark = threadIdx.x & 1 ? rows[PAIRS - 1].mark_b : rows[PAIRS - 1].mark_a;
+  struct {
+    float mark, a[2][PAIRS], b[2][PAIRS];
+  } t, n;
+  auto read = [&](auto& x, int k) {
+    x.mark = mark[k];
+#pragma unroll
+    for (int i = 0; i < PAIRS; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        x.a[j][i] = rows[i].a[(4 * k + 2 * j) * DLD];
+        x.b[j][i] = rows[i].b[(4 * k + 2 * j) * DLD];
+      }
+  };
+  auto ready = [&](const auto& x) { return __builtin_amdgcn_ballot_w64(__builtin_bit_cast(int, x.mark) == 0) == 0; };
+  read(t, 0);
+#pragma unroll
+  for (int i = 0; i < PAIRS; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) N[i][e] = 0.f;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    if (__builtin_expect(!ready(t), 0)) {
+      do read(t, k);
+      while (!ready(t));
+    }
+    n = t;
+    if (k < 7) read(n, k + 1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int i = 0; i < PAIRS; ++i)
+        N[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(t.a[j][i], t.b[j][i], N[i], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    t = n;
+  }
+}
+
+// Which wave does what in strip q.  Block columns: 1-3 of S (the row panel), 4-7 = 0-3 of Z.
+//   LEAD: the leaf;  FOLLOW c: the block of column c;  COLLECT c: what strip q takes from the block
+//   of column c in strip q+1, which that wave then follows, or leads, with;  HELP: the rest.
+// A SIMD has the waves s, s+4, s+8 and issues one instruction at a time to its matrix core or its
+// vector unit; of a step, the leading wave takes it 160 cycles, a following one 90, a collecting
+// one 70, and a helper 1400 cycles for a block.  So the leading wave has no following one beside
+// it, and every SIMD has about the same to do:
+//   SIMD      0               1                     2                    3
+//   strip 0   lead, C4, H     F1, C1, H             F2, C2, H            F3, C3, F4
+//   strip 1   C4, F4, F5      lead, C5, H (1)       C2, F2, H (2)        C3, F3, H (2 blocks)
+//   strip 2   F4, C4, C5      F6, F5, C6            lead, H, H (2)       F3, C3, H (1)
+//   strip 3   F4, F5          F6, H                 F7, H, H             lead
+enum { ROLE_NONE = 0, ROLE_LEAD = 1, ROLE_FOLLOW = 2, ROLE_COLLECT = 3, ROLE_HELP = 4 };
+constexpr int STRIP_HELPERS = 3;
+struct StripRoles {
+  unsigned long long bits = 0;      // 5 bits a wave
+  static constexpr unsigned long long code(int kind, int c) {
+    return kind == ROLE_LEAD ? 1 : kind == ROLE_HELP ? 2 + c : kind == ROLE_FOLLOW ? 8 + c
+           : kind == ROLE_COLLECT ? 16 + c : 0;
+  }
+  constexpr StripRoles& set(int wave, int kind, int c = 0) {
+    bits |= code(kind, c) << (5 * wave);
+    return *this;
+  }
+};
+constexpr unsigned long long STRIP_ROLES[4] = {
+    StripRoles().set(0, ROLE_LEAD).set(4, ROLE_COLLECT, 4).set(8, ROLE_HELP, 0)
+        .set(1, ROLE_FOLLOW, 1).set(5, ROLE_COLLECT, 1).set(9, ROLE_HELP, 1)
+        .set(2, ROLE_FOLLOW, 2).set(10, ROLE_COLLECT, 2).set(6, ROLE_HELP, 2)
+        .set(3, ROLE_FOLLOW, 3).set(7, ROLE_COLLECT, 3).set(11, ROLE_FOLLOW, 4).bits,
+    StripRoles().set(0, ROLE_COLLECT, 4).set(4, ROLE_FOLLOW, 4).set(8, ROLE_FOLLOW, 5)
+        .set(5, ROLE_LEAD).set(9, ROLE_COLLECT, 5).set(1, ROLE_HELP, 0)
+        .set(2, ROLE_COLLECT, 2).set(10, ROLE_FOLLOW, 2).set(6, ROLE_HELP, 1)
+        .set(3, ROLE_COLLECT, 3).set(7, ROLE_FOLLOW, 3).set(11, ROLE_HELP, 2).bits,
+    StripRoles().set(0, ROLE_FOLLOW, 4).set(4, ROLE_COLLECT, 4).set(8, ROLE_COLLECT, 5)
+        .set(5, ROLE_FOLLOW, 6).set(9, ROLE_FOLLOW, 5).set(1, ROLE_COLLECT, 6)
+        .set(2, ROLE_LEAD).set(6, ROLE_HELP, 0).set(10, ROLE_HELP, 1)
+        .set(3, ROLE_FOLLOW, 3).set(7, ROLE_COLLECT, 3).set(11, ROLE_HELP, 2).bits,
+    StripRoles().set(4, ROLE_FOLLOW, 4).set(8, ROLE_FOLLOW, 5)
+        .set(1, ROLE_FOLLOW, 6).set(5, ROLE_HELP, 0)
+        .set(6, ROLE_FOLLOW, 7).set(2, ROLE_HELP, 1).set(10, ROLE_HELP, 2)
+        .set(7, ROLE_LEAD).bits};
 
 // Factors and inverts diagonal block p of matrix m: one workgroup of DIAG_THREADS threads
 // (12 waves) with DIAG_SMEM_BYTES of LDS at dsm: S, the block (upper triangle and the whole
 // diagonal 32-blocks; finished rows of U replace it strip by strip), and Z, the rows of
 // U_pp^-T.
-// Four strips of 32 rows.  In strip q each of the waves 0-3 holds the leaf (its own copy:
-// the multipliers of a step come from it) and ONE further block of the same rows: a block
-// of the row panel to the right of the leaf (3 - q of them), or a block of the same rows of
-// Z (q + 1 of them, the last one starting as the identity).  That is four blocks in every
-// strip, one per wave, and the inverse Y_pp = Z^T is complete when the last strip is: no back
-// substitution, no doubling.  The updates by finished strips happen in LDS, by the other
-// waves: strip q-1's update of the rows of strip q first (four blocks, waves 4-7: this is
-// on the chain), its update of the rows further down while strip q is eliminated (at most
-// five blocks, waves 4-11); those waves also write the finished rows of strip q-1 to global
-// memory meanwhile, so that only the last strip's are left at the end.
+// Four strips of 32 rows, one barrier behind each.  Strip q has its leaf and four further blocks of
+// the same rows: the blocks of the row panel to the right of the leaf, and the blocks of the
+// same rows of Z (the last one starting as the identity).  The inverse Y_pp = Z^T is complete
+// when the last strip is: no back substitution, no doubling.  What a strip takes from the rows
+// below it goes
+//   to strip q+1 while strip q is eliminated, by the waves that then have those blocks (COLLECT);
+//   to the rows further down, in LDS, by the helping waves.
+// The finished rows of strip q are written to memory during strip q+1, by the waves that are done.
+// Bound by latency and, in the strips, by the issue of a SIMD's matrix core and vector unit, which take
+// turns: the steps of a strip take the leading wave 200 cycles each where nothing else is on its
+// SIMD.  One block alone 21.0 -> 17.1 us, with the pending panel 26.1 -> 21.2 (four waves that each
+// held the leaf and a second block, three barriers a strip, the pending panel on the fp32 instructions, 4-byte
+// accesses to memory); the inverse of a 2305^2 matrix and its Cholesky factor 1333 -> 1160 us.
 constexpr int DIAG_THREADS = 768;
+typedef SplitChunk<DB> PendingGroup;                       // (HALF: 8 k of 128 columns)
+constexpr int PENDING_PLANE = 8 * PendingGroup::HALF;      // 64 k
+static_assert(3 * PENDING_PLANE <= (DB - 32) * DLD * (int)sizeof(float), "half of W lives in the LDS of Z");
 
 // `pending`: the row panel above (block row p-1) has not been applied to this block yet
 // (the launch that holds this workgroup applies it to the rest of block row p meanwhile).
@@ -276,6 +438,11 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
                                            bool pending) {
   lds_f* const S = (lds_f*)dsm;
   lds_f* const Z = S + DB * DLD;
+  lds_f* const steps = Z + DB * DLD;
+  lds_f* const ops = steps + DIAG_STEPS;
+  lds_f* const marks = ops + DIAG_OPS;
+  typedef __attribute__((address_space(3))) int lds_i;
+  lds_i* const taken = (lds_i*)(marks + DIAG_MARKS);
   const int n = m.n;
   const int r0 = p * DB;
   const int nb = min(DB, n - r0);
@@ -283,174 +450,289 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);     // (provably uniform: scalar branches)
   const int lane = t & 63;
   const int r = lane & 31, h = lane >> 5;
-  // the waves that eliminate the strips go first wherever they share a SIMD with the others
-  if (wave < 4) __builtin_amdgcn_s_setprio(3);
+  if (t < DIAG_STEPS) steps[t] = 0.f;
+  if (t < DIAG_MARKS) marks[t] = 0.f;
+  if (t < 4) taken[t] = 0;
 
-  // load the upper triangle; pad with the identity up to 128.  All loads of a thread are
-  // issued before the first is used: one memory round trip for the block.
-  // (raw buffer loads: no 64-bit address per element, and the elements outside the
-  // triangle cost no memory access)
+  // pending: W, tile (p-1, p) of U, all of its 128 rows, in the same round trip as the block; 8
+  // consecutive k of one column a piece, wave by wave
+  constexpr int WGROUPS = (DB * DB / 8 + DIAG_THREADS - 1) / DIAG_THREADS;
+  float w[WGROUPS][8];
+  auto wgroup = [&](int g) { return (wave >> 1) + DIAG_THREADS / DB * g; };      // of 8 k
+
+  // load the upper triangle, by 32-blocks; pad with the identity up to 128.  All loads of a thread
+  // are issued before the first is used: one memory round trip for the block.  (What lies
+  // below the diagonal inside a diagonal 32-block is nobody's value and stays unread.)
   {
     const __amdgpu_buffer_rsrc_t rs = make_rsrc(m.U + (size_t)r0 * n + r0);
-    // (pending: tile (p-1, p) of U, all of its 128 rows, in the same round trip)
     const __amdgpu_buffer_rsrc_t ra = make_rsrc(m.U + ((size_t)r0 - DB) * n + r0);
-    constexpr int PER = (DB * DB + DIAG_THREADS - 1) / DIAG_THREADS;
-    float v[PER], a[PER];
+    constexpr int ROWS = DIAG_THREADS / 32, PER = (DB + ROWS - 1) / ROWS;
+    const int j = 4 * (t & 31);
+    v4f v[PER];
 #pragma unroll
     for (int u = 0; u < PER; ++u) {
-      const int e = u * DIAG_THREADS + t;
-      const int i = e >> 7, j = e & 127;
-      // (the diagonal 32-blocks in full, their lower triangles from the upper one: a strip
-      // reads its leaf as a plain symmetric block)
-      const bool in = i < nb && j < nb && (j >= i || (j >> 5) == (i >> 5));
-      v[u] = buffer_load(rs, in ? (unsigned)(min(i, j) * n + max(i, j)) * 4u : INV_M);
-      if (pending) a[u] = buffer_load(ra, (i < DB && j < nb) ? (unsigned)(i * n + j) * 4u : INV_M);
+      const int i = u * ROWS + (t >> 5);
+      const unsigned at = (unsigned)(i * n + j) * 4u;
+      const bool in = i < nb && j >= (i & ~31);
+      if (nb - j >= 4 || nb <= j) {
+        v[u] = buffer_load4(rs, in && j < nb ? at : INV_M);
+      } else {
+        // (the last columns of the matrix: nothing is read behind its end)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[u][e] = buffer_load(rs, in && j + e < nb ? at + 4 * e : INV_M);
+      }
+    }
+    if (pending) {
+      const unsigned col = t % DB < nb ? 4u * (t % DB) : INV_M;
+#pragma unroll
+      for (int g = 0; g < WGROUPS; ++g)
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          w[g][k] = buffer_load_at(ra, wgroup(g) < DB / 8 ? col : INV_M, 4u * n * (8 * wgroup(g) + k));
     }
 #pragma unroll
     for (int u = 0; u < PER; ++u) {
-      const int e = u * DIAG_THREADS + t;
-      if (e >= DB * DB) break;
-      const int i = e >> 7, j = e & 127;
-      const bool in = i < nb && j < nb && (j >= i || (j >> 5) == (i >> 5));
-      const bool pad = (i >= nb || j >= nb) && i == j;
-      S[i * DLD + j] = in ? v[u] : (pad ? 1.f : 0.f);
-      if (pending) Z[i * DLD + j] = a[u];
+      const int i = u * ROWS + (t >> 5);
+      if (i >= DB) break;
+      if (i >= nb) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[u][e] = i == j + e ? 1.f : 0.f;
+      }
+      *(lds_f4*)(S + i * DLD + j) = v[u];
     }
   }
-  __syncthreads();
-  // S -= W^T W, W = tile (p-1, p) of U (in Z for now), 128 deep, by 32x32 blocks: the four
-  // blocks of the first strip's rows now (waves 4-7, one per SIMD), the other six while
-  // that strip is eliminated (it writes Z in the columns of its own block only, which
-  // those six do not read; later strips find W spent)
-  auto pending_block = [&](int blk) {
-    int bi, bj;
-    upper_tile(blk, 4, bi, bj);
-    const v16f acc = lds_mma32(Z + 32 * bi, DLD, 1, Z + 32 * bj, DLD, 1, DB);
-    lds_f* const c = S + (32 * bi + 4 * h) * DLD + 32 * bj + r;
-    float old[16];
+  // S -= W^T W, split into bf16 parts as in gemm_split.h, half of the reduction after the other in
+  // the LDS of Z, a 32x32 block of S on each of ten waves; the waves 0-3 have the blocks that they
+  // start the first strip with, and do not wait for the others.
+  if (pending) {
+    v16f acc, cor;
 #pragma unroll
-    for (int e = 0; e < 16; ++e) old[e] = c[(8 * (e >> 2) + (e & 3)) * DLD];
+    for (int e = 0; e < 16; ++e) acc[e] = cor[e] = 0.f;
+    // (behind the first 32 rows of Z, which the first strip writes)
+    lds_c* const planes = (lds_c*)(Z + 32 * DLD);
+    int bi = 0, bj = 0;
+    if (wave < 10) upper_tile(wave, 4, bi, bj);
+    v4u ph[WGROUPS], pm[WGROUPS], pl[WGROUPS];
+    // the pieces of one half of the reduction, split (the second half's under the first's products)
+    auto split_half = [&](int half) {
 #pragma unroll
-    for (int e = 0; e < 16; ++e) c[(8 * (e >> 2) + (e & 3)) * DLD] = old[e] - acc[e];
-  };
-  if (pending && wave >= 4 && wave < 8) pending_block(wave - 4);
-  // (the loop over the strips starts with a barrier)
+      for (int g = 0; g < WGROUPS; ++g) {
+        if (wgroup(g) >> 3 != half) continue;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          unsigned x, y, z;
+          split_pair(w[g][2 * k], w[g][2 * k + 1], x, y, z);
+          ph[g][k] = x;
+          pm[g][k] = y;
+          pl[g][k] = z;
+        }
+      }
+    };
+    if (wave < 4) __builtin_amdgcn_s_setprio(3);
+    split_half(0);
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      if (half) __syncthreads();          // (the first half has been read)
+#pragma unroll
+      for (int g = 0; g < WGROUPS; ++g) {
+        if (wgroup(g) >> 3 != half) continue;
+        lds_c* const at = planes + (wgroup(g) & 7) * PendingGroup::HALF + (t % DB) * 16;
+        *(lds_u4*)at = ph[g];
+        *(lds_u4*)(at + PENDING_PLANE) = pm[g];
+        *(lds_u4*)(at + 2 * PENDING_PLANE) = pl[g];
+      }
+      __syncthreads();
+      if (wave < 10) {
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+          v8bf a[3], b[3];
+#pragma unroll
+          for (int part = 0; part < 3; ++part) {
+            const lds_c* const at = planes + part * PENDING_PLANE + (2 * ks + h) * PendingGroup::HALF + r * 16;
+            a[part] = __builtin_bit_cast(v8bf, *(const lds_u4*)(at + 32 * bi * 16));
+            b[part] = __builtin_bit_cast(v8bf, *(const lds_u4*)(at + 32 * bj * 16));
+          }
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[0], acc, 0, 0, 0);
+          cor = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[1], cor, 0, 0, 0);
+          cor = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[0], cor, 0, 0, 0);
+          cor = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[1], cor, 0, 0, 0);
+          cor = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[2], cor, 0, 0, 0);
+          cor = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2], b[0], cor, 0, 0, 0);
+        }
+      }
+      if (half == 0) split_half(1);
+    }
+    if (wave < 10) {
+      add_corrections(acc, cor);
+      lds_f* const at = S + (32 * bi + 4 * h) * DLD + 32 * bj + r;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) at[(8 * (e >> 2) + (e & 3)) * DLD] -= acc[e];
+    }
+  } else {
+    __syncthreads();
+  }
+  v16f N[1];           // what the strip above takes from this wave's block
+#pragma unroll
+  for (int e = 0; e < 16; ++e) N[0][e] = 0.f;
 
   typedef __attribute__((address_space(1))) float global_f;
+  typedef __attribute__((address_space(1), aligned(4))) v4f global_f4;
   global_f* const gU = (global_f*)(m.U + (size_t)r0 * n + r0);
   global_f* const gY = (global_f*)(m.Y + (size_t)r0 * n + r0);
-  // rows [32 qs, 32 qs + 32) of U and the same columns of Y = Z^T, by `nthr` threads
-  auto write_strip = [&](int qs, int tid, int nthr) {
-    for (int e0 = 0; e0 < 32 * DB; e0 += 8 * nthr) {
-      float u[8], y[8];
+  // rows [32 qs, 32 qs + 32) of U and the same columns of Y = Z^T, a sixteenth of them
+  constexpr int WRITE_ITEMS = 16;
+  auto write_item = [&](int qs, int item) {
+    const int e = 64 * item + lane;
+    const int iu = 32 * qs + (e >> 5), ju = 4 * (e & 31);      // U[iu][ju ...]
+    const int iy = e >> 3, jy = 32 * qs + 4 * (e & 7);         // Y[iy][jy ...] = Z[jy ...][iy]
+    v4f u = *(const lds_f4*)(S + iu * DLD + ju), y;
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const int e = min(e0 + k * nthr + tid, 32 * DB - 1);
-        const int iu = 32 * qs + (e >> 7), ju = e & 127;      // U[iu][ju]
-        const int iy = e >> 5, jy = 32 * qs + (e & 31);       // Y[iy][jy] = Z[jy][iy]
-        u[k] = iu <= ju ? S[iu * DLD + ju] : 0.f;
-        y[k] = iy <= jy ? Z[jy * DLD + iy] : 0.f;
-      }
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const int e = e0 + k * nthr + tid;
-        if (e >= 32 * DB) break;
-        const int iu = 32 * qs + (e >> 7), ju = e & 127;
-        const int iy = e >> 5, jy = 32 * qs + (e & 31);
-        if (iu < nb && ju < nb) gU[iu * n + ju] = u[k];
-        if (iy < nb && jy < nb) gY[iy * n + jy] = y[k];
-      }
+    for (int i = 0; i < 4; ++i) {
+      y[i] = Z[(jy + i) * DLD + iy];
+      u[i] = iu <= ju + i ? u[i] : 0.f;
+      y[i] = iy <= jy + i ? y[i] : 0.f;
     }
+    auto put = [&](global_f* row, int col, const v4f& x) {
+      if (col + 4 <= nb) {
+        *(global_f4*)(row + col) = x;
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (col + i < nb) row[col + i] = x[i];
+      }
+    };
+    if (iu < nb) put(gU + iu * n, ju, u);
+    if (iy < nb) put(gY + iy * n, jy, y);
   };
 
   const int nq = (nb + 31) / 32;
-  // Strip qs's update of block row i, by `nw` of the waves from 4 on, block by block in LDS
-  // (item k of the row goes to wave 4 + (first + k) % nw):
-  //   S(i, j) -= U[qs][i]^T U[qs][j]  (i <= j),     Z(i, s) -= U[qs][i]^T Z[qs][s]  (s <= qs)
-  auto update_row = [&](int qs, int i, int first, int nw) {
-    const lds_f* const above = S + 32 * qs * DLD;
-    const lds_f* const zabove = Z + 32 * qs * DLD;
-    for (int k = 0; k < nq - i + qs + 1; ++k) {
-      if ((first + k) % nw != wave - 4) continue;
-      const bool in_s = k < nq - i;
-      const int col = in_s ? i + k : k - (nq - i);         // block column of S, or of Z
-      const v16f acc = lds_mma32(above + 32 * i, DLD, 1, (in_s ? above : zabove) + 32 * col,
-                                 DLD, 1, 32);
-      lds_f* const c = (in_s ? S : Z) + (32 * i + 4 * h) * DLD + 32 * col + r;
-      // (a block of Z below the diagonal starts at zero: its first update, by the strip of
-      // its column, finds it uninitialised)
-      const bool fresh = !in_s && col == qs;
-      float old[16];
-#pragma unroll
-      for (int e = 0; e < 16; ++e) old[e] = fresh ? 0.f : c[(8 * (e >> 2) + (e & 3)) * DLD];
-#pragma unroll
-      for (int e = 0; e < 16; ++e) c[(8 * (e >> 2) + (e & 3)) * DLD] = old[e] - acc[e];
-    }
-    return nq - i + qs + 1;
+  // Element (8*(e/4) + 4h + e%4, r) of block (i, col) of S, or of Z
+  auto block_at = [&](bool in_s, int i, int col) {
+    return (in_s ? S : Z) + (32 * i + 4 * h) * DLD + 32 * col + r;
   };
   for (int q = 0; q < nq; ++q) {
     const int c0 = 32 * q;
-    const int rest = nq - q - 1;       // 32-blocks of the row panel to the right of the leaf
-    const bool strip_wave = wave < 4 && wave < nq;
-    const bool panel = wave < rest;    // this wave's second block: panel block jb, or block s
-    const int jb = q + 1 + wave;       // of the rows of Z
-    const int s = wave - rest;
-    // the rows of this strip meet the update by the strip above (nq blocks, one per wave)
-    if (wave >= 4 && q > 0) update_row(q - 1, q, 0, 4);
-    __syncthreads();
-    if (wave < 4) {
-      if (strip_wave) {
-        v16f L, P;
-        const lds_f* const lsrc = S + (c0 + 4 * h) * DLD + c0 + r;
-        const lds_f* const psrc =
-            (panel ? S + c0 * DLD + 32 * jb : Z + c0 * DLD + 32 * s) + 4 * h * DLD + r;
+    const unsigned long long roles = q == 0 ? STRIP_ROLES[0] : q == 1 ? STRIP_ROLES[1]
+                                   : q == 2 ? STRIP_ROLES[2] : STRIP_ROLES[3];
+    const int code = (int)(roles >> (5 * wave)) & 31;
+    const int c = code & 7;
+    const bool in_s = c < 4;
+    const bool there = in_s ? c < nq : c - 4 <= q;        // (a matrix may end in this block)
+    // first row of this strip in block column k, with the lane's row and column
+    auto rows_at = [&](int k) {
+      return (lds_vf*)((k < 4 ? S : Z) + (c0 + h) * DLD + 32 * (k & 3) + r);
+    };
+    auto marks_at = [&](int k) { return (lds_vf*)(marks + (8 * q + k) * 8); };
+    lds_vf2* const step = (lds_vf2*)(steps + 64 * q);
+    lds_vf* const op = (lds_vf*)(ops + lane);
+    if (code == 1) {
+      __builtin_amdgcn_s_setprio(3);
+      // (the lane's column made opaque, so that the lane masks derived from it are computed
+      // where they are used instead of being kept, and spilled, across the loop over the strips)
+      int rr = r;
+      asm volatile("" : "+v"(rr));
+      v16f L;
+      // (the leaf in full, what lies below its diagonal from above it)
+      const lds_f* const src = S + c0 * DLD + c0;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) L[e] = lsrc[(8 * (e >> 2) + (e & 3)) * DLD];
-        if (panel || s < q) {
+      for (int e = 0; e < 16; ++e) {
+        const int row = 8 * (e >> 2) + 4 * h + (e & 3);
+        L[e] = src[row <= rr ? row * DLD + rr : rr * DLD + row] - N[0][e];
+      }
+      float pmin = 1.f, piv[32];
+      lead_from<0>(L, rows_at(q), op, step, rr, pmin, piv);
+      // LAPACK's info: the first pivot that is not positive.  A NaN anywhere in the leaf
+      // reaches a pivot and from there every later one, so the last pivot stands for them.
+      if (!(pmin > 0.f) || !(piv[31] > 0.f)) {
+        int bad = 0;
 #pragma unroll
-          for (int e = 0; e < 16; ++e) P[e] = psrc[(8 * (e >> 2) + (e & 3)) * DLD];
-        } else {
+        for (int i = 31; i >= 0; --i)
+          if (!(piv[i] > 0.f)) bad = r0 + c0 + i + 1;
+        int* const out = info + m.out;
+        if (lane == 0 && *out == 0) *out = bad;
+      }
+    } else if (code >= 16) {
+      __builtin_amdgcn_s_setprio(1);
+      if (there && q + 1 < nq) {
+        const Rows from[1] = {{rows_at(q + 1), rows_at(c), marks_at(q + 1), marks_at(c)}};
+        collect<1>(N, from);
+      }
+    } else if (code >= 8) {
+      __builtin_amdgcn_s_setprio(2);
+      if (there) {
+        v16f P;
+        if (!in_s && c - 4 == q) {
 #pragma unroll
           for (int e = 0; e < 16; ++e) P[e] = 8 * (e >> 2) + 4 * h + (e & 3) == r ? 1.f : 0.f;
-        }
-        // (block (3, 0) of S, below its diagonal, is never used; the lane's column made
-        // opaque per strip, so that the lane masks derived from it are computed where they
-        // are used instead of being kept, and spilled, across the loop over the strips)
-        int rr = r;
-        asm volatile("" : "+v"(rr));
-        lds_f* const leaf_rows = (wave == 0 ? S + c0 * DLD + c0 : S + 96 * DLD) + h * DLD + r;
-        lds_f* const blk_rows = (panel ? S + c0 * DLD + 32 * jb : Z + c0 * DLD + 32 * s) + h * DLD + r;
-        float pmin = 1.f, piv[32];
-        // every wave has its copy of the leaf in registers before wave 0 writes U_qq over it
-        // (the waves 4-7 and the idle ones pass the same barrier below)
-        __syncthreads();
-        elim_from<0>(L, P, leaf_rows, blk_rows, rr, pmin, piv);
-        // LAPACK's info: the first pivot that is not positive.  A NaN anywhere in the leaf
-        // reaches a pivot and from there every later one, so the last pivot stands for them.
-        if (wave == 0 && (!(pmin > 0.f) || !(piv[31] > 0.f))) {
-          int bad = 0;
+        } else {
+          // (a block of Z below the diagonal starts at zero: the strip of its column is the
+          // first to update it, and finds it uninitialised)
+          const bool fresh = !in_s && c - 4 == q - 1;
+          const lds_f* const src = block_at(in_s, q, c & 3);
 #pragma unroll
-          for (int c = 31; c >= 0; --c)
-            if (!(piv[c] > 0.f)) bad = r0 + c0 + c + 1;
-          int* const out = info + m.out;
-          if (lane == 0 && *out == 0) *out = bad;
+          for (int e = 0; e < 16; ++e)
+            P[e] = (fresh ? 0.f : src[(8 * (e >> 2) + (e & 3)) * DLD]) - N[0][e];
         }
-      } else {
-        __syncthreads();
+        TwoSteps none;
+        none.m1 = none.s1 = none.m0 = none.s0 = v2f{0.f, 0.f};
+        none.x0 = none.x1 = 0.f;
+        follow_from<0>(P, none, op, step, rows_at(c), marks_at(c));
       }
-    } else {
-      __syncthreads();
-      // meanwhile: the strip above's update of the rows further down, and its rows to memory
-      if (q == 0 && pending && wave < 10) pending_block(wave);      // blocks 4..9
-      if (q > 0) {
-      int first = 0;
-      for (int i = q + 1; i < nq; ++i) first += update_row(q - 1, i, first, 8);
-      write_strip(q - 1, t - 256, DIAG_THREADS - 256);
+    } else if (code >= 2) {
+      __builtin_amdgcn_s_setprio(0);
+      // what this strip takes from the rows further down:  block (i, i), (i, i+1), ... of S and
+      // (i, 0), ... (i, q) of Z for the block rows i > q + 1; at most five blocks, two to a wave
+      int found = 0, at_i[2] = {0, 0}, at_c[2] = {0, 0}, k = 0;
+      for (int i = q + 2; i < nq; ++i)
+        for (int b = 0; b < nq - i + q + 1; ++b, ++k)
+          if (k % STRIP_HELPERS == code - 2) {
+            at_i[1] = i;
+            at_c[1] = b < nq - i ? i + b : 4 + b - (nq - i);
+            if (found == 0) at_i[0] = at_i[1], at_c[0] = at_c[1];
+            ++found;
+          }
+      auto rows_of = [&](int f) {
+        return Rows{rows_at(at_i[f]), rows_at(at_c[f]), marks_at(at_i[f]), marks_at(at_c[f])};
+      };
+      auto apply = [&](int f, const v16f& x) {
+        lds_f* const at = block_at(at_c[f] < 4, at_i[f], at_c[f] & 3);
+        // (a block of Z below the diagonal starts at zero: the strip of its column is the
+        // first to update it, and finds it uninitialised)
+        const bool fresh = at_c[f] == 4 + q;
+        float old[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) old[e] = fresh ? 0.f : at[(8 * (e >> 2) + (e & 3)) * DLD];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) at[(8 * (e >> 2) + (e & 3)) * DLD] = old[e] - x[e];
+      };
+      if (found == 2) {
+        v16f X[2];
+        const Rows from[2] = {rows_of(0), rows_of(1)};
+        collect<2>(X, from);
+        apply(0, X[0]);
+        apply(1, X[1]);
+      } else if (found == 1) {
+        v16f X[1];
+        const Rows from[1] = {rows_of(0)};
+        collect<1>(X, from);
+        apply(0, X[0]);
+      }
+    }
+    // the rows of the strip above to memory, by whoever is done
+    if (q > 0) {
+      for (;;) {
+        int item = 0;
+        if (lane == 0)
+          item = __hip_atomic_fetch_add(taken + q, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        item = __builtin_amdgcn_readfirstlane(item);
+        if (item >= WRITE_ITEMS) break;
+        write_item(q - 1, item);
       }
     }
     __syncthreads();
   }
-  write_strip(nq - 1, t, DIAG_THREADS);
+  __builtin_amdgcn_s_setprio(0);
+  for (int item = wave; item < WRITE_ITEMS; item += DIAG_THREADS / 64) write_item(nq - 1, item);
 }
 
 __global__ __launch_bounds__(DIAG_THREADS) void potrf_diag_kernel(const MatDesc* table, int p,
@@ -1580,9 +1862,9 @@ int kfac_damped_inverse_batched_static(int count, const int* dims, const float* 
 double kfac_inverse_executed_flops(int count, const int* dims, const int* factored) {
   if (count <= 0 || !dims) return 0.;
   const double B = 2. * DB * DB * DB;       // one 128-deep step of a 128 x 128 tile
-  // diagonal block: per strip 4 waves x 15 rank-2 steps x 2 blocks, the updates by finished
-  // strips (12 + 8 blocks, 32 deep), the pending panel (10 blocks, 128 deep)
-  const double diag = 4096. * (4 * 120 + 20 * 16 + 10 * 64);
+  // diagonal block: per strip 15 rank-2 steps of five blocks, the updates by finished strips
+  // (20 blocks, 32 deep), the pending panel (10 blocks, 128 deep)
+  const double diag = 4096. * (4 * 75 + 20 * 16 + 10 * 64);
   double total = 0.;
   std::vector<int> Ts(count);
   for (int i = 0; i < count; ++i) Ts[i] = cdiv(dims[i], DB);
