@@ -65,7 +65,7 @@ __global__ void inv_setup_kernel(DescChunk chunk, MatDesc* table, int offset, in
 // trace of src (one workgroup per matrix)
 __global__ __launch_bounds__(256) void inv_trace_kernel(MatDesc* table) {
   __shared__ float red[256];
-  MatDesc& m = table[blockIdx.x];
+  MatDesc m = chunk.d[blockIdx.x];
   const int n = m.n;
   float s = 0.f;
   for (int i = threadIdx.x; i < n; i += 256) s += m.src[(size_t)i * n + i];
@@ -324,44 +324,49 @@ struct Rows {
   const lds_vf *a, *b;
   const lds_vf *mark_a, *mark_b;
 };
-// PAIRS such products at a time.  The marks are read as one value, by lane, and tested at once.
-template <int PAIRS>
-__device__ __forceinline__ void collect(v16f (&N)[PAIRS], const Rows (&rows)[PAIRS]) {
-  const lds_vf* mark = threadIdx.x & 1 ? rows[0].mark_b : rows[0].mark_a;
-  if (PAIRS == 2 && (threadIdx.x & 2)) mark = threadIdx.x & 1 ? rows[PAIRS - 1].mark_b : rows[PAIRS - 1].mark_a;
-  struct {
-    float mark, a[2][PAIRS], b[2][PAIRS];
-  } t, n;
-  auto read = [&](auto& x, int k) {
-    x.mark = mark[k];
-#pragma unroll
-    for (int i = 0; i < PAIRS; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        x.a[j][i] = rows[i].a[(4 * k + 2 * j) * DLD];
-        x.b[j][i] = rows[i].b[(4 * k + 2 * j) * DLD];
-      }
+// One such product, or (TWO) two at a time.  The marks are read as one value, by lane, and tested
+// at once.
+template <bool TWO>
+__device__ __forceinline__ void collect(v16f& N, const Rows r0, v16f& M, const Rows r1) {
+  const lds_vf* mark = threadIdx.x & 1 ? r0.mark_b : r0.mark_a;
+  if (TWO && (threadIdx.x & 2)) mark = threadIdx.x & 1 ? r1.mark_b : r1.mark_a;
+  struct Step {
+    float mark, a0, a1, b0, b1, c0, c1, d0, d1;
   };
-  auto ready = [&](const auto& x) { return __builtin_amdgcn_ballot_w64(__builtin_bit_cast(int, x.mark) == 0) == 0; };
-  read(t, 0);
+  auto read = [&](int k) {
+    Step x;
+    const int at = 4 * k * DLD;
+    x.mark = mark[k];
+    x.a0 = r0.a[at];
+    x.b0 = r0.b[at];
+    x.a1 = r0.a[at + 2 * DLD];
+    x.b1 = r0.b[at + 2 * DLD];
+    x.c0 = x.c1 = x.d0 = x.d1 = 0.f;
+    if (TWO) {
+      x.c0 = r1.a[at];
+      x.d0 = r1.b[at];
+      x.c1 = r1.a[at + 2 * DLD];
+      x.d1 = r1.b[at + 2 * DLD];
+    }
+    return x;
+  };
+  auto ready = [&](const Step& x) { return __builtin_amdgcn_ballot_w64(__builtin_bit_cast(int, x.mark) == 0) == 0; };
+  Step t = read(0);
 #pragma unroll
-  for (int i = 0; i < PAIRS; ++i)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) N[i][e] = 0.f;
+  for (int e = 0; e < 16; ++e) N[e] = 0.f;
+  if (TWO) M = N;
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
     if (__builtin_expect(!ready(t), 0)) {
-      do read(t, k);
+      do t = read(k);
       while (!ready(t));
     }
-    n = t;
-    if (k < 7) read(n, k + 1);
+    const Step n = k < 7 ? read(k + 1) : t;
     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int i = 0; i < PAIRS; ++i)
-        N[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(t.a[j][i], t.b[j][i], N[i], 0, 0, 0);
+    N = __builtin_amdgcn_mfma_f32_32x32x2f32(t.a0, t.b0, N, 0, 0, 0);
+    if (TWO) M = __builtin_amdgcn_mfma_f32_32x32x2f32(t.c0, t.d0, M, 0, 0, 0);
+    N = __builtin_amdgcn_mfma_f32_32x32x2f32(t.a1, t.b1, N, 0, 0, 0);
+    if (TWO) M = __builtin_amdgcn_mfma_f32_32x32x2f32(t.c1, t.d1, M, 0, 0, 0);
     __builtin_amdgcn_sched_barrier(0);
     t = n;
   }
@@ -571,9 +576,9 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
   } else {
     __syncthreads();
   }
-  v16f N[1];           // what the strip above takes from this wave's block
+  v16f N;              // what the strip above takes from this wave's block
 #pragma unroll
-  for (int e = 0; e < 16; ++e) N[0][e] = 0.f;
+  for (int e = 0; e < 16; ++e) N[e] = 0.f;
 
   typedef __attribute__((address_space(1))) float global_f;
   typedef __attribute__((address_space(1), aligned(4))) v4f global_f4;
@@ -637,7 +642,7 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const int row = 8 * (e >> 2) + 4 * h + (e & 3);
-        L[e] = src[row <= rr ? row * DLD + rr : rr * DLD + row] - N[0][e];
+        L[e] = src[row <= rr ? row * DLD + rr : rr * DLD + row] - N[e];
       }
       float pmin = 1.f, piv[32];
       lead_from<0>(L, rows_at(q), op, step, rr, pmin, piv);
@@ -653,10 +658,8 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
       }
     } else if (code >= 16) {
       __builtin_amdgcn_s_setprio(1);
-      if (there && q + 1 < nq) {
-        const Rows from[1] = {{rows_at(q + 1), rows_at(c), marks_at(q + 1), marks_at(c)}};
-        collect<1>(N, from);
-      }
+      const Rows from{rows_at(q + 1), rows_at(c), marks_at(q + 1), marks_at(c)};
+      if (there && q + 1 < nq) collect<false>(N, from, N, from);
     } else if (code >= 8) {
       __builtin_amdgcn_s_setprio(2);
       if (there) {
@@ -671,7 +674,7 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
           const lds_f* const src = block_at(in_s, q, c & 3);
 #pragma unroll
           for (int e = 0; e < 16; ++e)
-            P[e] = (fresh ? 0.f : src[(8 * (e >> 2) + (e & 3)) * DLD]) - N[0][e];
+            P[e] = (fresh ? 0.f : src[(8 * (e >> 2) + (e & 3)) * DLD]) - N[e];
         }
         TwoSteps none;
         none.m1 = none.s1 = none.m0 = none.s0 = v2f{0.f, 0.f};
@@ -682,23 +685,24 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
       __builtin_amdgcn_s_setprio(0);
       // what this strip takes from the rows further down:  block (i, i), (i, i+1), ... of S and
       // (i, 0), ... (i, q) of Z for the block rows i > q + 1; at most five blocks, two to a wave
-      int found = 0, at_i[2] = {0, 0}, at_c[2] = {0, 0}, k = 0;
+      int found = 0, i0 = 0, k0 = 0, i1 = 0, k1 = 0, k = 0;
       for (int i = q + 2; i < nq; ++i)
         for (int b = 0; b < nq - i + q + 1; ++b, ++k)
           if (k % STRIP_HELPERS == code - 2) {
-            at_i[1] = i;
-            at_c[1] = b < nq - i ? i + b : 4 + b - (nq - i);
-            if (found == 0) at_i[0] = at_i[1], at_c[0] = at_c[1];
+            i1 = i;
+            k1 = b < nq - i ? i + b : 4 + b - (nq - i);
+            i0 = found ? i0 : i1;
+            k0 = found ? k0 : k1;
             ++found;
           }
-      auto rows_of = [&](int f) {
-        return Rows{rows_at(at_i[f]), rows_at(at_c[f]), marks_at(at_i[f]), marks_at(at_c[f])};
+      auto rows_of = [&](int i, int col) {
+        return Rows{rows_at(i), rows_at(col), marks_at(i), marks_at(col)};
       };
-      auto apply = [&](int f, const v16f& x) {
-        lds_f* const at = block_at(at_c[f] < 4, at_i[f], at_c[f] & 3);
+      auto apply = [&](int i, int col, const v16f& x) {
+        lds_f* const at = block_at(col < 4, i, col & 3);
         // (a block of Z below the diagonal starts at zero: the strip of its column is the
         // first to update it, and finds it uninitialised)
-        const bool fresh = at_c[f] == 4 + q;
+        const bool fresh = col == 4 + q;
         float old[16];
 #pragma unroll
         for (int e = 0; e < 16; ++e) old[e] = fresh ? 0.f : at[(8 * (e >> 2) + (e & 3)) * DLD];
@@ -706,16 +710,14 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
         for (int e = 0; e < 16; ++e) at[(8 * (e >> 2) + (e & 3)) * DLD] = old[e] - x[e];
       };
       if (found == 2) {
-        v16f X[2];
-        const Rows from[2] = {rows_of(0), rows_of(1)};
-        collect<2>(X, from);
-        apply(0, X[0]);
-        apply(1, X[1]);
+        v16f x, y;
+        collect<true>(x, rows_of(i0, k0), y, rows_of(i1, k1));
+        apply(i0, k0, x);
+        apply(i1, k1, y);
       } else if (found == 1) {
-        v16f X[1];
-        const Rows from[1] = {rows_of(0)};
-        collect<1>(X, from);
-        apply(0, X[0]);
+        v16f x;
+        collect<false>(x, rows_of(i0, k0), x, rows_of(i0, k0));
+        apply(i0, k0, x);
       }
     }
     // the rows of the strip above to memory, by whoever is done
