@@ -18,241 +18,165 @@ struct VecDesc {
   float s0, s1, s2, s3;
 };
 
-constexpr int VEC_CHUNK = 64;
-struct VecChunk {
-  VecDesc d[VEC_CHUNK];
+// A list of tensors travels as a kernel argument, with the first workgroup of each: one launch per
+// call and no table in memory.  (A launch that writes a table and one that reads it, twice where
+// some tensors cannot be accessed by 16 bytes: a VOGN step of a 784-1000-1000-10 network spent 45 of
+// its 225 launches on tables.)  The argument's size costs host time, so short lists have a short one.
+constexpr int VEC_SHORT = 8, VEC_LONG = 64;
+template <int N>
+struct VecList {
+  VecDesc d[N];
+  int first[N + 1];
+  int n;
 };
-
-__global__ void vec_setup_kernel(VecChunk chunk, VecDesc* table, int offset, int count) {
-  const int i = threadIdx.x;
-  if (i < count) table[offset + i] = chunk.d[i];
-}
+static_assert(sizeof(VecList<VEC_LONG>) <= 4096, "kernel arguments");
 
 enum { OP_AXPBY = 0, OP_DIAG_INV = 1, OP_MUL = 2, OP_SGD = 3, OP_SQRT = 4, OP_MAX = 5, OP_ADDCMUL = 6 };
 
 constexpr int EW_THREADS = 256;
-constexpr int EW_PER_THREAD = 4;
-constexpr int EW_BLOCK = EW_THREADS * EW_PER_THREAD;
-
-// Each thread handles EW_PER_THREAD elements: all loads first, then the
-// arithmetic, then all stores.  (Load/store pairs issued one element at a time
-// would each wait for their own load: a store may alias the next load, so the
-// compiler keeps them in order.)
+// accesses per thread and tensor in flight
 template <int OP>
-__global__ __launch_bounds__(EW_THREADS) void vec_kernel(const VecDesc* table) {
-  const VecDesc m = table[blockIdx.y];
-  const long nblocks = (m.numel + EW_BLOCK - 1) / EW_BLOCK;
-  constexpr bool USES_B = OP == OP_AXPBY || OP == OP_MUL || OP == OP_SGD || OP == OP_MAX ||
-                          OP == OP_ADDCMUL;
-  constexpr bool USES_C = OP == OP_SGD || OP == OP_ADDCMUL;
-  for (long blk = blockIdx.x; blk < nblocks; blk += gridDim.x) {
-    const long base = blk * EW_BLOCK + threadIdx.x;
-    float a[EW_PER_THREAD], b[EW_PER_THREAD], c[EW_PER_THREAD];
-#pragma unroll
-    for (int k = 0; k < EW_PER_THREAD; ++k) {
-      const long i = base + (long)k * EW_THREADS;
-      const bool in = i < m.numel;
-      a[k] = in ? m.a[i] : 0.f;
-      b[k] = 0.f;
-      c[k] = 0.f;
-      if (USES_B && in && !(OP == OP_AXPBY && m.s1 == 0.f)) b[k] = m.b[i];
-      if (USES_C && in && !(OP == OP_SGD && m.s1 == 0.f)) c[k] = m.c[i];
+__host__ __device__ constexpr int ew_in_flight(bool vec) {
+  return vec && (OP == OP_SGD || OP == OP_ADDCMUL) ? 2 : 4;
+}
+template <int OP>
+__host__ __device__ constexpr int ew_block(bool vec) {
+  return EW_THREADS * ew_in_flight<OP>(vec) * (vec ? 4 : 1);
+}
+
+// One element: a, b, c are the values read, and what is written back where the operation does so.
+template <int OP>
+__device__ __forceinline__ void vec_op(const VecDesc& m, float& a, float& b, float& c) {
+  if (OP == OP_AXPBY) {
+    // b = s0 * a + s1 * b     (s1 == 0: b is not read)
+    b = m.s1 != 0.f ? m.s0 * a + m.s1 * b : m.s0 * a;
+  } else if (OP == OP_DIAG_INV) {
+    // b = 1 / ((s1 ? sqrt(a) : a) + s0)
+    const float v = m.s1 != 0.f ? sqrtf(a) : a;
+    b = 1.f / (v + m.s0);
+  } else if (OP == OP_MUL) {
+    b = b * a;
+  } else if (OP == OP_SQRT) {
+    b = sqrtf(a);
+  } else if (OP == OP_MAX) {
+    b = fmaxf(a, b);
+  } else if (OP == OP_ADDCMUL) {
+    // b = a + s0 * b * c     (a = mean, b = noise in / parameter out, c = std)
+    b = fmaf(m.s0 * b, c, a);
+  } else {
+    // a = param, b = grad, c = momentum buffer; s0 = lr, s1 = momentum, s2 = weight decay
+    float g = b;
+    if (m.s2 != 0.f) g += m.s2 * a;
+    if (m.s1 != 0.f) {
+      g = m.s1 * c + g;
+      c = g;
     }
+    b = g;
+    a = a - m.s0 * g;
+  }
+}
+
+template <int OP>
+__device__ __forceinline__ void vec_op(const VecDesc& m, float4& a, float4& b, float4& c) {
+  vec_op<OP>(m, a.x, b.x, c.x);
+  vec_op<OP>(m, a.y, b.y, c.y);
+  vec_op<OP>(m, a.z, b.z, c.z);
+  vec_op<OP>(m, a.w, b.w, c.w);
+}
+
+// All loads of a thread first, then the arithmetic, then all stores.  (Load/store pairs issued
+// one at a time would each wait for their own load: a store may alias the next load, so the
+// compiler keeps them in order.)
+template <int OP, class V>
+__device__ __forceinline__ void vec_tensor(const VecDesc& m, int local, int blocks) {
+  constexpr int K = ew_in_flight<OP>(sizeof(V) == 16), STEP = K * EW_THREADS;
+  const bool read_b = OP == OP_MUL || OP == OP_SGD || OP == OP_MAX || OP == OP_ADDCMUL ||
+                      (OP == OP_AXPBY && m.s1 != 0.f);
+  const bool read_c = OP == OP_ADDCMUL || (OP == OP_SGD && m.s1 != 0.f);
+  V* const pa = reinterpret_cast<V*>(m.a);
+  V* const pb = reinterpret_cast<V*>(m.b);
+  V* const pc = reinterpret_cast<V*>(m.c);
+  const long n = m.numel / (long)(sizeof(V) / 4);
+  for (long i0 = (long)local * STEP + threadIdx.x; i0 < n; i0 += (long)blocks * STEP) {
+    V a[K], b[K], c[K];
 #pragma unroll
-    for (int k = 0; k < EW_PER_THREAD; ++k) {
-      const long i = base + (long)k * EW_THREADS;
-      if (i >= m.numel) continue;
-      if (OP == OP_AXPBY) {
-        // b = s0 * a + s1 * b     (s1 == 0: b is not read)
-        float v = m.s0 * a[k];
-        if (m.s1 != 0.f) v += m.s1 * b[k];
-        m.b[i] = v;
-      } else if (OP == OP_DIAG_INV) {
-        // b = 1 / ((s1 ? sqrt(a) : a) + s0)
-        float v = a[k];
-        if (m.s1 != 0.f) v = sqrtf(v);
-        m.b[i] = 1.f / (v + m.s0);
-      } else if (OP == OP_MUL) {
-        m.b[i] = b[k] * a[k];                       // b *= a
-      } else if (OP == OP_SQRT) {
-        m.b[i] = sqrtf(a[k]);
-      } else if (OP == OP_MAX) {
-        m.b[i] = fmaxf(a[k], b[k]);
-      } else if (OP == OP_ADDCMUL) {
-        // b = a + s0 * b * c     (a = mean, b = noise in / parameter out, c = std)
-        m.b[i] = fmaf(m.s0 * b[k], c[k], a[k]);
-      } else {
-        // a = param, b = grad, c = momentum buffer; s0 = lr, s1 = momentum, s2 = weight decay
-        float g = b[k];
-        const float p = a[k];
-        if (m.s2 != 0.f) g += m.s2 * p;
-        if (m.s1 != 0.f) {
-          g = m.s1 * c[k] + g;
-          m.c[i] = g;
-        }
-        m.b[i] = g;
-        m.a[i] = p - m.s0 * g;
+    for (int k = 0; k < K; ++k) {
+      const long i = i0 + k * EW_THREADS;
+      a[k] = b[k] = c[k] = V{};
+      if (i < n) {
+        a[k] = pa[i];
+        if (read_b) b[k] = pb[i];
+        if (read_c) c[k] = pc[i];
       }
     }
-  }
-}
-
-// y = s0*x + s1*y on float4 (all pointers 16-byte aligned, numel % 4 == 0): the
-// running average of the factors moves the most bytes of all tails.  Four float4
-// per thread and iteration, loads ahead of stores.
-__global__ __launch_bounds__(EW_THREADS) void axpby4_kernel(const VecDesc* table) {
-  const VecDesc m = table[blockIdx.y];
-  const long n4 = m.numel >> 2;
-  const float4* x = reinterpret_cast<const float4*>(m.a);
-  float4* y = reinterpret_cast<float4*>(m.b);
-  const long stride = (long)gridDim.x * EW_THREADS;
-  const bool rd = m.s1 != 0.f;
-  for (long i0 = (long)blockIdx.x * EW_THREADS + threadIdx.x; i0 < n4; i0 += 4 * stride) {
-    float4 a[4], b[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const long i = i0 + k * stride;
-      a[k] = i < n4 ? x[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-      b[k] = (rd && i < n4) ? y[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const long i = i0 + k * stride;
-      if (i < n4) {
-        float4 o;
-        o.x = m.s0 * a[k].x + m.s1 * b[k].x;
-        o.y = m.s0 * a[k].y + m.s1 * b[k].y;
-        o.z = m.s0 * a[k].z + m.s1 * b[k].z;
-        o.w = m.s0 * a[k].w + m.s1 * b[k].w;
-        y[i] = o;
-      }
+    for (int k = 0; k < K; ++k) {
+      const long i = i0 + k * EW_THREADS;
+      if (i >= n) break;
+      vec_op<OP>(m, a[k], b[k], c[k]);
+      if (OP == OP_SGD && read_c) pc[i] = c[k];
+      pb[i] = b[k];
+      if (OP == OP_SGD) pa[i] = a[k];
     }
   }
 }
 
-// The fused update on float4 (all pointers 16-byte aligned, numel % 4 == 0): a = param,
-// b = grad, c = momentum buffer; s0 = lr, s1 = momentum, s2 = weight decay.  Two float4
-// of each tensor per thread and iteration, loads ahead of stores.
-__device__ __forceinline__ float sgd_one(float p, float g, float c, const VecDesc& m, float& buf) {
-  if (m.s2 != 0.f) g += m.s2 * p;
-  if (m.s1 != 0.f) {
-    g = m.s1 * c + g;
-    buf = g;
-  }
-  return g;
+// all pointers of a tensor 16-byte aligned and its size a multiple of 4
+__host__ __device__ inline bool ew_vec(const VecDesc& d) {
+  return (((uintptr_t)d.a | (uintptr_t)d.b | (uintptr_t)d.c) & 15) == 0 && (d.numel & 3) == 0;
 }
 
-__global__ __launch_bounds__(EW_THREADS) void sgd4_kernel(const VecDesc* table) {
-  const VecDesc m = table[blockIdx.y];
-  const long n4 = m.numel >> 2;
-  float4* pa = reinterpret_cast<float4*>(m.a);
-  float4* pb = reinterpret_cast<float4*>(m.b);
-  float4* pc = reinterpret_cast<float4*>(m.c);
-  const long stride = (long)gridDim.x * EW_THREADS;
-  const bool mom = m.s1 != 0.f;
-  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-  for (long i0 = (long)blockIdx.x * EW_THREADS + threadIdx.x; i0 < n4; i0 += 2 * stride) {
-    float4 a[2], b[2], c[2];
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const long i = i0 + k * stride;
-      const bool in = i < n4;
-      a[k] = in ? pa[i] : zero;
-      b[k] = in ? pb[i] : zero;
-      c[k] = (in && mom) ? pc[i] : zero;
-    }
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const long i = i0 + k * stride;
-      if (i >= n4) continue;
-      float4 g, buf = c[k];
-      g.x = sgd_one(a[k].x, b[k].x, c[k].x, m, buf.x);
-      g.y = sgd_one(a[k].y, b[k].y, c[k].y, m, buf.y);
-      g.z = sgd_one(a[k].z, b[k].z, c[k].z, m, buf.z);
-      g.w = sgd_one(a[k].w, b[k].w, c[k].w, m, buf.w);
-      if (mom) pc[i] = buf;
-      pb[i] = g;
-      pa[i] = make_float4(a[k].x - m.s0 * g.x, a[k].y - m.s0 * g.y, a[k].z - m.s0 * g.z,
-                          a[k].w - m.s0 * g.w);
-    }
+template <int OP, int N>
+__global__ __launch_bounds__(EW_THREADS) void vec_kernel(const VecList<N> list) {
+  int j = 0, end = list.n;
+  while (end - j > 1) {
+    const int mid = (j + end) >> 1;
+    if (list.first[mid] <= (int)blockIdx.x) j = mid; else end = mid;
   }
+  const VecDesc m = list.d[j];
+  const int local = blockIdx.x - list.first[j], blocks = list.first[j + 1] - list.first[j];
+  if (ew_vec(m))
+    vec_tensor<OP, float4>(m, local, blocks);
+  else
+    vec_tensor<OP, float>(m, local, blocks);
 }
 
 static size_t vec_workspace(int count) { return (size_t)count * sizeof(VecDesc); }
 
-static long upload_table(const std::vector<VecDesc>& descs, VecDesc* table, long per_block,
-                         hipStream_t stream);
+// Workgroups of a tensor: one per block of elements, up to a share of this many (a large
+// tensor's walk it in strides).
+constexpr long EW_MAX_BLOCKS = 8192;
 
-// the running average: float4 kernel for the tensors that allow it, scalar for the rest
-static int run_axpby(std::vector<VecDesc>& descs, void* workspace, size_t workspace_bytes,
-                     hipStream_t stream) {
-  const int count = (int)descs.size();
-  if (count == 0) return KFAC_OK;
-  if (!workspace || workspace_bytes < vec_workspace(count)) return KFAC_ERR_WORKSPACE;
-  std::vector<VecDesc> v4, sc;
-  for (const VecDesc& d : descs) {
-    const bool aligned = (((uintptr_t)d.a | (uintptr_t)d.b) & 15) == 0 && (d.numel & 3) == 0;
-    (aligned ? v4 : sc).push_back(d);
+template <int OP, int N>
+static void launch_vec(const VecDesc* d, int count, long max_blocks, hipStream_t stream) {
+  VecList<N> list;
+  list.n = count;
+  list.first[0] = 0;
+  for (int k = 0; k < count; ++k) {
+    list.d[k] = d[k];
+    const long per_block = ew_block<OP>(ew_vec(d[k]));
+    const long blocks = (d[k].numel + per_block - 1) / per_block;
+    list.first[k + 1] = list.first[k] + (int)std::min(blocks, max_blocks);
   }
-  VecDesc* table = (VecDesc*)workspace;
-  if (!v4.empty()) {
-    const long maxblocks = upload_table(v4, table, 4L * EW_THREADS * 4, stream);
-    long gx = std::max<long>(64, 8192 / (long)v4.size());
-    gx = std::min(gx, maxblocks);
-    hipLaunchKernelGGL(axpby4_kernel, dim3((unsigned)gx, (unsigned)v4.size()), dim3(EW_THREADS), 0,
-                       stream, table);
-  }
-  if (!sc.empty()) {
-    VecDesc* t2 = table + v4.size();
-    const long maxblocks = upload_table(sc, t2, EW_BLOCK, stream);
-    long gx = std::max<long>(64, 4096 / (long)sc.size());
-    gx = std::min(gx, maxblocks);
-    hipLaunchKernelGGL((vec_kernel<OP_AXPBY>), dim3((unsigned)gx, (unsigned)sc.size()),
-                       dim3(EW_THREADS), 0, stream, t2);
-  }
-  return launch_status();
+  hipLaunchKernelGGL((vec_kernel<OP, N>), dim3((unsigned)list.first[count]), dim3(EW_THREADS), 0,
+                     stream, list);
 }
 
-// copies the descriptors to the device table; returns the block count of the largest tensor
-static long upload_table(const std::vector<VecDesc>& descs, VecDesc* table, long per_block,
-                         hipStream_t stream) {
-  const int count = (int)descs.size();
-  long maxblocks = 1;
-  for (int s0 = 0; s0 < count; s0 += VEC_CHUNK) {
-    VecChunk chunk;
-    const int cnt = std::min(VEC_CHUNK, count - s0);
-    for (int k = 0; k < cnt; ++k) {
-      chunk.d[k] = descs[s0 + k];
-      maxblocks = std::max(maxblocks, (descs[s0 + k].numel + per_block - 1) / per_block);
-    }
-    hipLaunchKernelGGL(vec_setup_kernel, dim3(1), dim3(VEC_CHUNK), 0, stream, chunk, table, s0,
-                       cnt);
-  }
-  return maxblocks;
-}
-
+// (the workspace is not needed any more; callers go on bringing it)
 template <int OP>
-static int run_vec(std::vector<VecDesc>& descs, void* workspace, size_t workspace_bytes,
+static int run_vec(const std::vector<VecDesc>& descs, void* workspace, size_t workspace_bytes,
                    hipStream_t stream) {
   const int count = (int)descs.size();
   if (count == 0) return KFAC_OK;
   if (!workspace || workspace_bytes < vec_workspace(count)) return KFAC_ERR_WORKSPACE;
-  VecDesc* table = (VecDesc*)workspace;
-  long maxblocks = 1;
-  for (int s0 = 0; s0 < count; s0 += VEC_CHUNK) {
-    VecChunk chunk;
-    const int cnt = std::min(VEC_CHUNK, count - s0);
-    for (int k = 0; k < cnt; ++k) {
-      chunk.d[k] = descs[s0 + k];
-      maxblocks = std::max(maxblocks, (descs[s0 + k].numel + EW_BLOCK - 1) / EW_BLOCK);
-    }
-    hipLaunchKernelGGL(vec_setup_kernel, dim3(1), dim3(VEC_CHUNK), 0, stream, chunk, table, s0,
-                       cnt);
+  const long max_blocks = std::max<long>(64, EW_MAX_BLOCKS / count);
+  for (int s0 = 0; s0 < count; s0 += VEC_LONG) {
+    const int cnt = std::min(VEC_LONG, count - s0);
+    if (cnt <= VEC_SHORT)
+      launch_vec<OP, VEC_SHORT>(descs.data() + s0, cnt, max_blocks, stream);
+    else
+      launch_vec<OP, VEC_LONG>(descs.data() + s0, cnt, max_blocks, stream);
   }
-  long gx = std::max<long>(64, 4096 / count);
-  gx = std::min(gx, maxblocks);
-  hipLaunchKernelGGL((vec_kernel<OP>), dim3((unsigned)gx, count), dim3(EW_THREADS), 0, stream,
-                     table);
   return launch_status();
 }
 
@@ -586,7 +510,7 @@ int kfac_axpby_batched(int count, const int64_t* numel, const float* const* x, f
     if (numel[i] <= 0 || !x[i] || !y[i]) return KFAC_ERR_ARG;
     d[i] = VecDesc{(float*)x[i], y[i], nullptr, (long)numel[i], a, b, 0.f, 0.f};
   }
-  return run_axpby(d, workspace, workspace_bytes, (hipStream_t)stream);
+  return run_vec<OP_AXPBY>(d, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 int kfac_diag_inverse_batched(int count, const int64_t* numel, const float* const* ema,
@@ -664,32 +588,7 @@ int kfac_sgd_update_batched(int count, const int64_t* numel, float* const* param
     d[i] = VecDesc{param[i], grad[i], momentum_buf ? momentum_buf[i] : nullptr, (long)numel[i],
                    lr[i], momentum[i], weight_decay[i], 0.f};
   }
-  // float4 kernel for the tensors that allow it (the weights), scalar for the rest
-  if (count == 0) return KFAC_OK;
-  if (!workspace || workspace_bytes < vec_workspace(count)) return KFAC_ERR_WORKSPACE;
-  std::vector<VecDesc> v4, sc;
-  for (const VecDesc& e : d) {
-    const bool aligned =
-        (((uintptr_t)e.a | (uintptr_t)e.b | (uintptr_t)e.c) & 15) == 0 && (e.numel & 3) == 0;
-    (aligned ? v4 : sc).push_back(e);
-  }
-  VecDesc* table = (VecDesc*)workspace;
-  if (!v4.empty()) {
-    const long maxblocks = upload_table(v4, table, 4L * EW_THREADS * 2, (hipStream_t)stream);
-    long gx = std::max<long>(64, 8192 / (long)v4.size());
-    gx = std::min(gx, maxblocks);
-    hipLaunchKernelGGL(sgd4_kernel, dim3((unsigned)gx, (unsigned)v4.size()), dim3(EW_THREADS), 0,
-                       (hipStream_t)stream, table);
-  }
-  if (!sc.empty()) {
-    VecDesc* t2 = table + v4.size();
-    const long maxblocks = upload_table(sc, t2, EW_BLOCK, (hipStream_t)stream);
-    long gx = std::max<long>(64, 4096 / (long)sc.size());
-    gx = std::min(gx, maxblocks);
-    hipLaunchKernelGGL((vec_kernel<OP_SGD>), dim3((unsigned)gx, (unsigned)sc.size()),
-                       dim3(EW_THREADS), 0, (hipStream_t)stream, t2);
-  }
-  return launch_status();
+  return run_vec<OP_SGD>(d, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 static void launch_rowsq(const float* x, int64_t rows, int channels, int len, const float* scale,

@@ -62,8 +62,8 @@ __global__ void inv_setup_kernel(DescChunk chunk, MatDesc* table, int offset, in
   if (i < count) table[offset + i] = chunk.d[i];
 }
 
-// trace of src (one workgroup per matrix)
-__global__ __launch_bounds__(256) void inv_trace_kernel(MatDesc* table) {
+// the same, with the trace of src (one workgroup per matrix)
+__global__ __launch_bounds__(256) void inv_trace_kernel(const DescChunk chunk, MatDesc* table, int offset) {
   __shared__ float red[256];
   MatDesc m = chunk.d[blockIdx.x];
   const int n = m.n;
@@ -75,7 +75,10 @@ __global__ __launch_bounds__(256) void inv_trace_kernel(MatDesc* table) {
     if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
     __syncthreads();
   }
-  if (threadIdx.x == 0) m.trace = red[0];
+  if (threadIdx.x == 0) {
+    m.trace = red[0];
+    table[offset + blockIdx.x] = m;
+  }
 }
 
 __device__ __forceinline__ float effective_damp(const MatDesc* table, const MatDesc& m) {
@@ -1573,6 +1576,8 @@ static int run_batched(std::vector<HostMat>& mats, int mode, int* info, void* wo
   size_t yoff = 0;
   int Tmax = 0;
   std::vector<int> Ts(nmat);
+  bool any_pi = false;
+  for (auto& h : mats) any_pi |= h.partner >= 0;
   for (int s0 = 0; s0 < nmat; s0 += SETUP_CHUNK) {
     DescChunk chunk;
     const int cnt = std::min(SETUP_CHUNK, nmat - s0);
@@ -1599,8 +1604,10 @@ static int run_batched(std::vector<HostMat>& mats, int mode, int* info, void* wo
       Ts[s0 + k] = d.T;
       Tmax = std::max(Tmax, d.T);
     }
-    hipLaunchKernelGGL(inv_setup_kernel, dim3(1), dim3(SETUP_CHUNK), 0, stream, chunk, table, s0,
-                       cnt);
+    if (any_pi)
+      hipLaunchKernelGGL(inv_trace_kernel, dim3(cnt), dim3(256), 0, stream, chunk, table, s0);
+    else
+      hipLaunchKernelGGL(inv_setup_kernel, dim3(1), dim3(SETUP_CHUNK), 0, stream, chunk, table, s0, cnt);
   }
   auto active = [&](int minT) {   // matrices with T >= minT (a prefix of the sorted table)
     int c = 0;
@@ -1628,9 +1635,6 @@ static int run_batched(std::vector<HostMat>& mats, int mode, int* info, void* wo
     for_matrices(count, [&](int s) { return items(Ts[s]); }, launch);
   };
 
-  bool any_pi = false;
-  for (auto& h : mats) any_pi |= h.partner >= 0;
-  if (any_pi) hipLaunchKernelGGL(inv_trace_kernel, dim3(nmat), dim3(256), 0, stream, table);
   for_worklists(nmat, [](int T) { return COPY_PARTS * T * (T + 1) / 2; },
                 [&](const WorkList& wl, int grid) {
     hipLaunchKernelGGL(inv_copy_damp_kernel, dim3(grid), dim3(256), 0, stream, table, info, wl);
