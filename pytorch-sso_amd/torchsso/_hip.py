@@ -12,6 +12,11 @@ import threading
 
 import torch
 
+try:
+    from torchsso import _host
+except ImportError:          # (not built: `load` says so)
+    _host = None
+
 _LIB_NAME = 'libkfac_hip.so'
 _lib = None
 _lock = threading.Lock()
@@ -134,18 +139,32 @@ def f32_array(values):
     return (ctypes.c_float * len(values))(*[float(v) for v in values])
 
 
+def ints(values):
+    """int32 values as the C ABI takes them (packed natively; the caller passes them on at once)."""
+    return _host.ints(values) if _host is not None else int_array(values)
+
+
+def floats(values):
+    return _host.floats(values) if _host is not None else f32_array(values)
+
+
+def numels(tensors):
+    """Element counts (int64) of a list of tensors."""
+    packed = None if _host is None else _host.numels(tensors)
+    return i64_array([t.numel() for t in tensors]) if packed is None else packed
+
+
 def ptr_array(tensors, what='tensor', allow_none=False):
     """Host array of device addresses (0 for None when allowed)."""
-    f32 = torch.float32
+    packed = None if _host is None else _host.pointers(tensors, allow_none)
+    if packed is not None:
+        return packed
     out = []
     for i, t in enumerate(tensors):
         if t is None:
             if not allow_none:
                 raise KfacHipError('%s %d is None' % (what, i))
             out.append(None)
-        # (dev_ptr's conditions; its message is put together only where one fails)
-        elif isinstance(t, torch.Tensor) and t.is_cuda and t.dtype is f32 and t.is_contiguous():
-            out.append(t.data_ptr())
         else:
             out.append(dev_ptr(t, '%s %d' % (what, i)))
     return (ctypes.c_void_p * len(out))(*out)
@@ -164,10 +183,11 @@ def load():
         if _lib is not None:
             return _lib
         path = lib_path()
-        if not os.path.exists(path):
+        if not os.path.exists(path) or _host is None:
             raise KfacHipError(
                 '%s is not built: run `python pytorch-sso_amd/build_ext.py` '
-                '(there is no CPU or PyTorch fallback for the K-FAC kernels)' % path)
+                '(there is no CPU or PyTorch fallback for the K-FAC kernels)'
+                % (path if not os.path.exists(path) else 'torchsso/_host.so'))
         lib = ctypes.CDLL(path)
         for name, (res, args) in _SIGNATURES.items():
             fn = getattr(lib, name)
@@ -184,6 +204,9 @@ def check(status, what):
 
 def dev_ptr(t, what='tensor'):
     """Device address of a contiguous fp32 HIP tensor (loud otherwise)."""
+    address = None if _host is None else _host.pointer(t)
+    if address is not None:
+        return address
     if not isinstance(t, torch.Tensor):
         raise KfacHipError('%s: expected a torch.Tensor' % what)
     if not t.is_cuda:
@@ -204,6 +227,12 @@ def stream_ptr(device=None, stream=None):
     if index is None:
         return torch.cuda.current_stream(device).cuda_stream
     return torch._C._cuda_getCurrentRawStream(index)     # (no Stream object around the handle)
+
+
+def order_streams(index, waiting, waited):
+    """What the stream `waiting` of device `index` is given from now on runs behind what the
+    stream `waited` (both torch.cuda.Stream) holds now."""
+    _host.order(index, waiting.cuda_stream, waited.cuda_stream)
 
 
 _all_workspaces = []     # the `bufs` dict of every thread's _Workspace

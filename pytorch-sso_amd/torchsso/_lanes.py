@@ -38,6 +38,8 @@ import threading
 
 import torch
 
+from torchsso import _hip, _ops
+
 _count = 2
 _mode = 'grouped'
 _lock = threading.Lock()
@@ -195,8 +197,18 @@ def deferred_count():
         return sum(len(q.items) + len(q.bn) for q in _deferred.values())
 
 
-def _run_deferred(only=None, bn_only=False):
-    from torchsso import _ops
+_events = []       # events of engine calls that are done with, for the next ones
+
+
+def _drop(held):
+    """(under the lock) the calls in `held` keep nothing alive any more"""
+    if len(_events) < 64:
+        _events.extend(done for done, _, _ in held)
+
+
+def _run_deferred(only=None, bn_only=False, reader=False):
+    """Hands what is queued to the engine.  `reader`: the current stream is about to be made to wait
+    for the products anyway."""
     with _lock:
         todo = []
         for i, q in _deferred.items():
@@ -210,17 +222,17 @@ def _run_deferred(only=None, bn_only=False):
                 _deferred[i] = _Queue()
     for i, items, bn in todo:
         device = torch.device('cuda', i)
-        cur = torch.cuda.current_stream(i)
+        cur = _current_stream(i)
         if bn:
             # the BatchNorm reductions stay on the caller's stream (one launch for all queued
             # layers): they are bound by memory and run beside the factor products of the
             # side streams; whoever reads their outputs does so on this stream, behind them
             waited = []
             for job, st in bn:
-                if st != cur:
+                if st is not cur and st != cur:
                     if st not in waited:
                         waited.append(st)
-                        cur.wait_stream(st)
+                        _hip.order_streams(i, cur, st)
                     for t in (job[0], job[2]) + tuple(job[4:]):
                         if t is not None:
                             t.record_stream(cur)
@@ -228,14 +240,16 @@ def _run_deferred(only=None, bn_only=False):
         if not items:
             continue
         side = None
-        if _count > 0:
-            # the engine call goes to a side stream (the calls of a pass take turns), so
-            # that it runs beside whatever the caller's stream does next
+        # the engine call goes to a side stream (the calls of a pass take turns), so that it runs
+        # beside whatever the caller's stream does next; a reader's stream does nothing before
+        # the call is done, unless it has BatchNorm reductions to run, and takes the call itself: no
+        # event forward and back (a fully connected network's step: 30 us of host time)
+        if _count > 0 and (bn or not reader):
             _, lst = _lane_streams(device)
             with _lock:
                 lane = _calls.get(i, 0) % _count
                 _calls[i] = _calls.get(i, 0) + 1
-            side, fork = lst[lane]
+            side = lst[lane][0]
             if side == cur:
                 side = None
         target = cur if side is None else side
@@ -243,7 +257,7 @@ def _run_deferred(only=None, bn_only=False):
         # has run what it held at the time of the hook (all of it, to keep this simple)
         others = []
         for _, keep, st in items:
-            if st != cur:
+            if st is not cur and st != cur:
                 if st not in others and st != target:
                     others.append(st)
                 for t in keep:
@@ -251,21 +265,22 @@ def _run_deferred(only=None, bn_only=False):
                         t.record_stream(target)
         jobs = [job for job, _, _ in items]
         if side is not None:
-            with _lock:
-                fork.record(cur)
-                side.wait_event(fork)
-                # a call still in flight on ANOTHER side stream that writes a buffer this
-                # call reads or adds to (factors accumulated over MC samples): wait for it
+            _hip.order_streams(i, side, cur)
+        with _lock:
+            # a call still in flight on ANOTHER side stream that writes a buffer this
+            # call reads or adds to (factors accumulated over MC samples): wait for it
+            held = _inflight.get(i)
+            if held:
                 touched = set()
                 for job in jobs:
                     touched.add(job.C)
                     if job.C_prev:
                         touched.add(job.C_prev)
-                for done, _, written in _inflight.get(i, []):
+                for done, _, written in held:
                     if not touched.isdisjoint(written):
-                        side.wait_event(done)
+                        target.wait_event(done)
         for st in others:
-            target.wait_stream(st)
+            _hip.order_streams(i, target, st)
         # (the call's workspace is the cached scratch of the stream it runs on; a pass under
         # no_grad leaves its inputs referenced in the queue, or in `_inflight`, until the
         # next flush or join)
@@ -273,10 +288,13 @@ def _run_deferred(only=None, bn_only=False):
         if side is not None:
             # the tensors stay referenced until the caller's stream has been made to wait
             # for the side stream (join), or until the side stream is seen to have passed
-            done = torch.cuda.Event()
-            done.record(side)
             with _lock:
-                held = [h for h in _inflight.get(i, []) if not h[0].query()]
+                done = _events.pop() if _events else torch.cuda.Event()
+                done.record(side)
+                held, past = [], []
+                for h in _inflight.get(i, ()):
+                    (past if h[0].query() else held).append(h)
+                _drop(past)
                 held.append((done, items, set(job.C for job in jobs)))
                 _inflight[i] = held
                 _pending.setdefault(i, set()).add(lane)
@@ -339,8 +357,8 @@ def curvature_stream(device, k=0):
 def join(device=None):
     """The current stream of `device` (all devices if None) waits for the factor
     products enqueued so far."""
-    if _deferred:
-        _run_deferred(None if device is None or device.index is None else device.index)
+    if any(q.items or q.bn for q in list(_deferred.values())):
+        _run_deferred(None if device is None or device.index is None else device.index, reader=True)
     if not _pending:
         return
     with _lock:
@@ -349,9 +367,9 @@ def join(device=None):
         for i, _ in todo:
             _pending[i].clear()
     for i, lanes in todo:
-        cur = torch.cuda.current_stream(i)
+        cur = _current_stream(i)
         for lane in lanes:
-            cur.wait_stream(_streams[i][lane][0])
+            _hip.order_streams(i, cur, _streams[i][lane][0])
         with _lock:
             held = _inflight.pop(i, None) or []
         # What these calls read may be freed from here on, and the allocator hands a freed
@@ -360,9 +378,11 @@ def join(device=None):
         for done, items, _ in held:
             waited = []
             for _, _, st in items:
-                if st != cur and st not in waited:
+                if st is not cur and st != cur and st not in waited:
                     waited.append(st)
                     st.wait_event(done)
+        with _lock:
+            _drop(held)
 
 
 def _at_exit():
@@ -384,6 +404,7 @@ def _at_exit():
     _streams.clear()
     _deferred.clear()
     _inflight.clear()
+    _events.clear()
 
 
 atexit.register(_at_exit)

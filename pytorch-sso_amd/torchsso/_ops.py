@@ -3,6 +3,8 @@
 Each wrapper checks shapes on the host before anything is launched, brings the
 scratch the entry point asks for, and enqueues on torch's current stream.
 """
+import ctypes
+
 import torch
 
 from torchsso import _hip
@@ -150,6 +152,8 @@ def factor_job(kind, x, alpha, out, beta=0., prev=None, add_bias=False, kernel_s
 
 def factor_job_update(job, x, alpha, out, beta=0., prev=None):
     """Points an existing job (same kind, shapes and geometry) at new tensors."""
+    if _hip._host is not None and _hip._host.update_job(ctypes.addressof(job), x, out, prev, alpha, beta):
+        return
     if beta != 0 and prev is None:
         prev = out
     job.x = _hip.dev_ptr(x, 'input')
@@ -174,7 +178,7 @@ def factor_grouped(jobs, device, stream=None):
     lib = _hip.load()
     if len(jobs) == 0:
         return
-    arr = (_hip.FactorJob * len(jobs))(*jobs)
+    arr = _hip._host.jobs([ctypes.addressof(job) for job in jobs])
     ws, ws_bytes = _hip.workspace(device, lib.kfac_factor_grouped_workspace_bytes(len(jobs), arr),
                                   stream)
     st = lib.kfac_factor_grouped(len(jobs), arr, _ws_ptr(ws), ws_bytes,
@@ -224,10 +228,10 @@ def pi_damped_inverse_batched(As, Gs, dampings, A_invs=None, G_invs=None, info=N
     dims = []
     for a, g in zip(dA, dG):
         dims += [a, g]
-    ws, ws_bytes = _hip.workspace(dev, lib.kfac_inverse_workspace_bytes(len(dims), _hip.int_array(dims)))
+    ws, ws_bytes = _hip.workspace(dev, lib.kfac_inverse_workspace_bytes(len(dims), _hip.ints(dims)))
     st = lib.kfac_pi_damped_inverse_batched(
-        layers, _hip.int_array(dA), _hip.int_array(dG), _hip.ptr_array(As, 'A'),
-        _hip.ptr_array(Gs, 'G'), _hip.f32_array(dampings), _hip.ptr_array(A_invs, 'A_inv'),
+        layers, _hip.ints(dA), _hip.ints(dG), _hip.ptr_array(As, 'A'),
+        _hip.ptr_array(Gs, 'G'), _hip.floats(dampings), _hip.ptr_array(A_invs, 'A_inv'),
         _hip.ptr_array(G_invs, 'G_inv'), info.data_ptr(), _ws_ptr(ws), ws_bytes,
         _hip.stream_ptr(dev))
     _hip.check(st, 'kfac_pi_damped_inverse_batched')
@@ -254,10 +258,10 @@ def _pi_inverse_two_outputs(entry, As, Gs, dampings, A_invs, G_invs, A_others, G
     dims = []
     for a, g in zip(dA, dG):
         dims += [a, g]
-    ws, ws_bytes = _hip.workspace(dev, lib.kfac_inverse_workspace_bytes(len(dims), _hip.int_array(dims)))
+    ws, ws_bytes = _hip.workspace(dev, lib.kfac_inverse_workspace_bytes(len(dims), _hip.ints(dims)))
     st = getattr(lib, entry)(
-        layers, _hip.int_array(dA), _hip.int_array(dG), _hip.ptr_array(As, 'A'),
-        _hip.ptr_array(Gs, 'G'), _hip.f32_array(dampings), _hip.ptr_array(A_invs, 'A_inv', True),
+        layers, _hip.ints(dA), _hip.ints(dG), _hip.ptr_array(As, 'A'),
+        _hip.ptr_array(Gs, 'G'), _hip.floats(dampings), _hip.ptr_array(A_invs, 'A_inv', True),
         _hip.ptr_array(G_invs, 'G_inv', True), _hip.ptr_array(A_others, 'A output', True),
         _hip.ptr_array(G_others, 'G output', True), info.data_ptr(), _ws_ptr(ws), ws_bytes,
         _hip.stream_ptr(dev))
@@ -300,8 +304,8 @@ def precondition_factored_batched(G_ops, A_ops, grad_ws, grad_bs, g_factored=Non
     _square_dims(G_ops, 'G operand')
     _square_dims(A_ops, 'A operand')
     dG, dA = _kron_dims(G_ops, A_ops, grad_ws, grad_bs, 'precondition')
-    dGa, dAa = _hip.int_array(dG), _hip.int_array(dA)
-    flags = [None if f is None else _hip.int_array([int(bool(v)) for v in f])
+    dGa, dAa = _hip.ints(dG), _hip.ints(dA)
+    flags = [None if f is None else _hip.ints([int(bool(v)) for v in f])
              for f in (g_factored, a_factored)]
     ws, ws_bytes = _hip.workspace(dev, lib.kfac_precondition_factored_workspace_bytes(layers, dGa, dAa))
     st = lib.kfac_precondition_factored_batched(
@@ -323,10 +327,10 @@ def damped_inverse_batched(mats, damps=None, outs=None, info=None):
         outs = [torch.empty_like(m) for m in mats]
     if info is None:
         info = torch.empty(count, dtype=torch.int32, device=dev)
-    ws, ws_bytes = _hip.workspace(dev, lib.kfac_inverse_workspace_bytes(count, _hip.int_array(dims)))
+    ws, ws_bytes = _hip.workspace(dev, lib.kfac_inverse_workspace_bytes(count, _hip.ints(dims)))
     st = lib.kfac_damped_inverse_batched(
-        count, _hip.int_array(dims), _hip.ptr_array(mats, 'matrix'),
-        None if damps is None else _hip.f32_array(damps), _hip.ptr_array(outs, 'inverse'),
+        count, _hip.ints(dims), _hip.ptr_array(mats, 'matrix'),
+        None if damps is None else _hip.floats(damps), _hip.ptr_array(outs, 'inverse'),
         info.data_ptr(), _ws_ptr(ws), ws_bytes, _hip.stream_ptr(dev))
     _hip.check(st, 'kfac_damped_inverse_batched')
     return outs, info
@@ -344,9 +348,9 @@ def cholesky_upper_batched(mats, outs=None, info=None):
         outs = [torch.empty_like(m) for m in mats]
     if info is None:
         info = torch.empty(count, dtype=torch.int32, device=dev)
-    ws, ws_bytes = _hip.workspace(dev, lib.kfac_inverse_workspace_bytes(count, _hip.int_array(dims)))
+    ws, ws_bytes = _hip.workspace(dev, lib.kfac_inverse_workspace_bytes(count, _hip.ints(dims)))
     st = lib.kfac_cholesky_upper_batched(
-        count, _hip.int_array(dims), _hip.ptr_array(mats, 'matrix'), _hip.ptr_array(outs, 'factor'),
+        count, _hip.ints(dims), _hip.ptr_array(mats, 'matrix'), _hip.ptr_array(outs, 'factor'),
         info.data_ptr(), _ws_ptr(ws), ws_bytes, _hip.stream_ptr(dev))
     _hip.check(st, 'kfac_cholesky_upper_batched')
     return outs, info
@@ -378,7 +382,7 @@ def precondition_batched(G_invs, A_invs, grad_ws, grad_bs):
     _square_dims(G_invs, 'G_inv')
     _square_dims(A_invs, 'A_inv')
     dG, dA = _kron_dims(G_invs, A_invs, grad_ws, grad_bs, 'precondition')
-    dGa, dAa = _hip.int_array(dG), _hip.int_array(dA)
+    dGa, dAa = _hip.ints(dG), _hip.ints(dA)
     ws, ws_bytes = _hip.workspace(dev, lib.kfac_precondition_workspace_bytes(layers, dGa, dAa))
     st = lib.kfac_precondition_batched(
         layers, dGa, dAa, _hip.ptr_array(G_invs, 'G_inv'), _hip.ptr_array(A_invs, 'A_inv'),
@@ -401,7 +405,7 @@ def sample_batched(U_Gs, U_As, noises, mean_ws, mean_bs, param_ws, param_bs, std
         if tuple(e.shape) != (dG[l], dA[l]):
             raise _hip.KfacHipError('noise %d has shape %s, expected (%d, %d)'
                                     % (l, tuple(e.shape), dG[l], dA[l]))
-    dGa, dAa = _hip.int_array(dG), _hip.int_array(dA)
+    dGa, dAa = _hip.ints(dG), _hip.ints(dA)
     ws, ws_bytes = _hip.workspace(dev, lib.kfac_precondition_workspace_bytes(layers, dGa, dAa))
     st = lib.kfac_sample_batched(
         layers, dGa, dAa, _hip.ptr_array(U_Gs, 'U_G'), _hip.ptr_array(U_As, 'U_A'),
@@ -412,17 +416,22 @@ def sample_batched(U_Gs, U_As, noises, mean_ws, mean_bs, param_ws, param_bs, std
     _hip.check(st, 'kfac_sample_batched')
 
 
-def _vec_args(lib, tensors):
+def _vec_args(lib, tensors, numel=None):
     dev = tensors[0].device
-    numel = _hip.i64_array([t.numel() for t in tensors])
+    if numel is None:
+        numel = _hip.numels(tensors)
     ws, ws_bytes = _hip.workspace(dev, lib.kfac_vector_workspace_bytes(len(tensors)))
     return dev, numel, ws, ws_bytes
 
 
 def _check_same_numel(xs, ys, what):
-    for i, (x, y) in enumerate(zip(xs, ys)):
-        if x.numel() != y.numel():
-            raise _hip.KfacHipError('%s %d: %d vs %d elements' % (what, i, x.numel(), y.numel()))
+    """The element counts of xs, which those of ys have to match."""
+    numel, others = _hip.numels(xs), _hip.numels(ys)
+    if numel != others or not isinstance(numel, bytes):
+        for i, (x, y) in enumerate(zip(xs, ys)):
+            if x.numel() != y.numel():
+                raise _hip.KfacHipError('%s %d: %d vs %d elements' % (what, i, x.numel(), y.numel()))
+    return numel
 
 
 def axpby_batched(xs, ys, a, b):
@@ -430,8 +439,8 @@ def axpby_batched(xs, ys, a, b):
     lib = _hip.load()
     if len(xs) == 0:
         return
-    _check_same_numel(xs, ys, 'axpby')
-    dev, numel, ws, ws_bytes = _vec_args(lib, xs)
+    numel = _check_same_numel(xs, ys, 'axpby')
+    dev, numel, ws, ws_bytes = _vec_args(lib, xs, numel)
     st = lib.kfac_axpby_batched(len(xs), numel, _hip.ptr_array(xs, 'x'), _hip.ptr_array(ys, 'y'),
                                 float(a), float(b), _ws_ptr(ws), ws_bytes, _hip.stream_ptr(dev))
     _hip.check(st, 'kfac_axpby_batched')
@@ -441,10 +450,10 @@ def diag_inverse_batched(emas, invs, dampings, use_sqrt):
     lib = _hip.load()
     if len(emas) == 0:
         return
-    _check_same_numel(emas, invs, 'diag inverse')
-    dev, numel, ws, ws_bytes = _vec_args(lib, emas)
+    numel = _check_same_numel(emas, invs, 'diag inverse')
+    dev, numel, ws, ws_bytes = _vec_args(lib, emas, numel)
     st = lib.kfac_diag_inverse_batched(len(emas), numel, _hip.ptr_array(emas, 'ema'),
-                                       _hip.ptr_array(invs, 'inv'), _hip.f32_array(dampings),
+                                       _hip.ptr_array(invs, 'inv'), _hip.floats(dampings),
                                        int(bool(use_sqrt)), _ws_ptr(ws), ws_bytes,
                                        _hip.stream_ptr(dev))
     _hip.check(st, 'kfac_diag_inverse_batched')
@@ -454,8 +463,8 @@ def diag_precondition_batched(invs, grads):
     lib = _hip.load()
     if len(invs) == 0:
         return
-    _check_same_numel(invs, grads, 'diag precondition')
-    dev, numel, ws, ws_bytes = _vec_args(lib, invs)
+    numel = _check_same_numel(invs, grads, 'diag precondition')
+    dev, numel, ws, ws_bytes = _vec_args(lib, invs, numel)
     st = lib.kfac_diag_precondition_batched(len(invs), numel, _hip.ptr_array(invs, 'inv'),
                                             _hip.ptr_array(grads, 'grad'), _ws_ptr(ws), ws_bytes,
                                             _hip.stream_ptr(dev))
@@ -467,8 +476,8 @@ def sqrt_batched(xs, ys):
     lib = _hip.load()
     if len(xs) == 0:
         return
-    _check_same_numel(xs, ys, 'sqrt')
-    dev, numel, ws, ws_bytes = _vec_args(lib, xs)
+    numel = _check_same_numel(xs, ys, 'sqrt')
+    dev, numel, ws, ws_bytes = _vec_args(lib, xs, numel)
     st = lib.kfac_sqrt_batched(len(xs), numel, _hip.ptr_array(xs, 'x'), _hip.ptr_array(ys, 'y'),
                                _ws_ptr(ws), ws_bytes, _hip.stream_ptr(dev))
     _hip.check(st, 'kfac_sqrt_batched')
@@ -479,8 +488,8 @@ def max_batched(xs, ys):
     lib = _hip.load()
     if len(xs) == 0:
         return
-    _check_same_numel(xs, ys, 'max')
-    dev, numel, ws, ws_bytes = _vec_args(lib, xs)
+    numel = _check_same_numel(xs, ys, 'max')
+    dev, numel, ws, ws_bytes = _vec_args(lib, xs, numel)
     st = lib.kfac_max_batched(len(xs), numel, _hip.ptr_array(xs, 'x'), _hip.ptr_array(ys, 'y'),
                               _ws_ptr(ws), ws_bytes, _hip.stream_ptr(dev))
     _hip.check(st, 'kfac_max_batched')
@@ -497,7 +506,7 @@ def diag_sample_batched(means, stds, noise_to_params, std_scales):
     st = lib.kfac_diag_sample_batched(len(means), numel, _hip.ptr_array(means, 'mean'),
                                       _hip.ptr_array(stds, 'std'),
                                       _hip.ptr_array(noise_to_params, 'param'),
-                                      _hip.f32_array(std_scales), _ws_ptr(ws), ws_bytes,
+                                      _hip.floats(std_scales), _ws_ptr(ws), ws_bytes,
                                       _hip.stream_ptr(dev))
     _hip.check(st, 'kfac_diag_sample_batched')
 
@@ -551,15 +560,15 @@ def sgd_update_batched(params, grads, bufs, lrs, momenta, weight_decays):
     lib = _hip.load()
     if len(params) == 0:
         return
-    _check_same_numel(params, grads, 'update')
+    numel = _check_same_numel(params, grads, 'update')
     for i, (p, buf, m) in enumerate(zip(params, bufs, momenta)):
         if m != 0 and (buf is None or buf.numel() != p.numel()):
             raise _hip.KfacHipError('update %d: momentum buffer missing or of wrong size' % i)
-    dev, numel, ws, ws_bytes = _vec_args(lib, params)
+    dev, numel, ws, ws_bytes = _vec_args(lib, params, numel)
     st = lib.kfac_sgd_update_batched(
         len(params), numel, _hip.ptr_array(params, 'param'), _hip.ptr_array(grads, 'grad'),
-        _hip.ptr_array(bufs, 'momentum buffer', True), _hip.f32_array(lrs),
-        _hip.f32_array(momenta), _hip.f32_array(weight_decays), _ws_ptr(ws), ws_bytes,
+        _hip.ptr_array(bufs, 'momentum buffer', True), _hip.floats(lrs),
+        _hip.floats(momenta), _hip.floats(weight_decays), _ws_ptr(ws), ws_bytes,
         _hip.stream_ptr(dev))
     _hip.check(st, 'kfac_sgd_update_batched')
 
@@ -646,8 +655,8 @@ def bn_diag_cov_batched(jobs, device, stream=None):
     count = len(jobs)
     ws, ws_bytes = _hip.workspace(device, lib.kfac_bn_diag_cov_batched_workspace_bytes(count), stream)
     st = lib.kfac_bn_diag_cov_batched(
-        count, _hip.ptr_array(gs, 'grad_output'), _hip.int_array(ns), _hip.int_array(cs),
-        _hip.int_array(ls), _hip.ptr_array(sxs, 'sx'), _hip.f32_array(alphas),
+        count, _hip.ptr_array(gs, 'grad_output'), _hip.ints(ns), _hip.ints(cs),
+        _hip.ints(ls), _hip.ptr_array(sxs, 'sx'), _hip.floats(alphas),
         _hip.ptr_array(ws_, 'w_curv'), _hip.ptr_array(bs, 'b_curv', allow_none=True),
         _ws_ptr(ws), ws_bytes, _hip.stream_ptr(device, stream))
     _hip.check(st, 'kfac_bn_diag_cov_batched')
@@ -712,7 +721,7 @@ def _pack_call(arrays, buf, offset, unpack):
     ws, ws_bytes = _hip.workspace(dev, lib.kfac_pack_workspace_bytes(len(tensors)))
     fn = lib.kfac_unpack_batched if unpack else lib.kfac_pack_batched
     st = fn(len(tensors), _hip.ptr_array(tensors, 'array'), _hip.i64_array(numel),
-            _hip.int_array(dims), _hip.int_array(flags), _hip.dev_ptr(buf, 'buffer'), int(offset),
+            _hip.ints(dims), _hip.ints(flags), _hip.dev_ptr(buf, 'buffer'), int(offset),
             _ws_ptr(ws), ws_bytes, _hip.stream_ptr(dev))
     _hip.check(st, 'kfac_unpack_batched' if unpack else 'kfac_pack_batched')
     return offset + total

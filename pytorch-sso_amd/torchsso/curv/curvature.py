@@ -604,8 +604,8 @@ def update_inv_all(curvs, with_std=()):
             _, _, info = _ops.pi_damped_inverse_batched(*args, column(0, 0), column(0, 1))
             for c in kron:
                 c._info_reversed = False
-        for i, c in enumerate(kron):
-            c.info = info[2 * i:2 * i + 2]
+        for c, status in zip(kron, info.view(-1, 2).unbind()):
+            c.info = status
     if diag:
         by_sqrt = {False: ([], [], []), True: ([], [], [])}
         for c in diag:
@@ -756,16 +756,18 @@ def _chain_split(pairs):
     """The (curvature, params) pairs in the classes of `chain_classes`, or None."""
     if two_stream_min_dim is None or len(pairs) < 2:
         return None
-    dims, devices = [], set()
+    dims, first = [], pairs[0][1][0].get_device()
+    if first < 0:
+        return None
     for c, params in pairs:
         w = params[0]
-        if not w.is_cuda:
+        if w.get_device() != first:          # (on the host, or on another device)
             return None
-        devices.add(w.device)
-        dims.append(max(w.shape[0], w[0].numel() + (1 if c.bias else 0))
-                    if c.kind == 'kron' else 0)
-    if len(devices) != 1:
-        return None
+        if c.kind == 'kron':
+            rows = w.shape[0]
+            dims.append(max(rows, w.numel() // rows + (1 if c.bias else 0)))
+        else:
+            dims.append(0)
     classes = chain_classes(dims, two_stream_min_dim, curvature_streams_max)
     return None if classes is None else [[pairs[i] for i in cls] for cls in classes]
 

@@ -266,7 +266,7 @@ class SecondOrderOptimizer(Optimizer):
         accs, datas = [], []
         for group in self.param_groups:
             accs.append(group['acc_grads'])
-            datas.append([p.grad.data for p in group['params']])
+            datas.append([p.grad for p in group['params']])
             curv = group['curv']
             if curv is not None and getattr(curv, '_acc_into', None) is None:
                 accs.append(group['acc_curv'])

@@ -50,7 +50,7 @@ def class_probabilities(output):
 
 
 def _running_sum(total, value, weight):
-    return value * weight if total is None else total + value * weight
+    return value * weight if total is None else torch.add(total, value, alpha=weight)
 
 
 class VIOptimizer(SecondOrderOptimizer):

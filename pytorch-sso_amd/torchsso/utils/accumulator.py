@@ -56,7 +56,7 @@ class TensorAccumulator(object):
             if not as_list[0].is_cuda:
                 acc.update(data, scale)
                 continue
-            src = [d.detach().contiguous() for d in as_list]
+            src = [d if d.is_contiguous() else d.detach().contiguous() for d in as_list]
             have = acc._accumulation
             if have is None:
                 new = [d.new_empty(d.shape) for d in src]
