@@ -18,7 +18,7 @@ bool enable_large_lds(const void* kernel, int bytes);
 
 #define KFAC_LAUNCH_TILE2(kernel, grid, stream, ...)                                         \
   do {                                                                                       \
-    constexpr int lds_bytes_ = kfac::SplitCfg<2, 2>::SMEM_BYTES;                           \
+    constexpr int lds_bytes_ = kfac::SplitCfg<2>::SMEM_BYTES;                           \
     if (kfac::enable_large_lds((const void*)(kernel), lds_bytes_))                           \
       hipLaunchKernelGGL((kernel), (grid), dim3(kfac::NTHREADS), lds_bytes_, (stream),       \
                          __VA_ARGS__);                                                       \
@@ -78,24 +78,28 @@ inline int piece_blocks(long work, int longest) {
 }
 
 // Chunks per item of a launch of factor products that hold `units` (tile, chunk) pairs, on tiles
-// of w x w waves: `dflt` where the launch holds plenty of items at that length, shorter items
-// where it would not fill the chip: twice with workgroups of one wave (8 per CU are resident), 1.5
-// times with those of four (output gradients of 32 images of 2048x7x7 / 1024x13x13 / 256x56x56 in
-// 1.5 / 2 / 3 rounds: 79 / 87 / 98, 69 / 73 / 82, 73 / 78 / 91 us), or once where that would take
-// items of less than 8 chunks (a strided pointwise layer, 256 rows, 588 items of 8 chunks 64 us,
-// one round of 10 chunks 54).
-inline long group_item_chunks(int w, double units, long dflt) {
-  const double resident = w == 1 ? 2048. : RESIDENT_TILES;
-  long t = (long)(units / ((w == 1 ? 2. : 1.5) * resident));
+// 64 w wide: `dflt` where the launch holds plenty of items at that length, shorter items where it
+// would not fill the chip.  128-wide tiles: 1.5 times (output gradients of 32 images of 2048x7x7 /
+// 1024x13x13 / 256x56x56 in 1.5 / 2 / 3 rounds: 79 / 87 / 98, 69 / 73 / 82, 73 / 78 / 91 us), or once
+// where that would take items of less than 8 chunks (a strided pointwise layer, 256 rows, 588 items
+// of 8 chunks 64 us, one round of 10 chunks 54).  64-wide tiles: once, with as many items as are resident
+// (`resident_small`: five workgroups per CU; correlations, whose strips are short items, six).
+// Output gradients of 32 images of 64x112x112 / six of 64x56x56 / 128x56x56 with 768, 1280, 1536 and
+// 4096 items: 39 41 46 60 / 43 45 49 68 / 31 35 36 39 us; 3x3 inputs of 64x56x56, one layer / three, in
+// 1280, 1536, 4096: 142 135 166 / 334 323 319; the stem of a ResNet-50 with 768 ... 4096: 181 168 162 170.
+constexpr double RESIDENT_SMALL = 1280., RESIDENT_SMALL_CORR = 1536.;
+inline long group_item_chunks(int w, double units, long dflt, double resident_small = RESIDENT_SMALL) {
+  const double resident = w == 1 ? resident_small : RESIDENT_TILES;
+  long t = (long)(units / ((w == 1 ? 1. : 1.5) * resident));
   if (t < 8) t = w == 1 ? 8 : std::max(8L, (long)(units / resident) + 1);
   return std::min(t, dflt);
 }
 
 // Tiles' worth of MFMA work in the T(T+1)/2 upper tiles of a symmetric product with T tiles
-// per side: of the 32x32 blocks of a diagonal tile a 128-wide one of four waves computes 12 of 16
-// (three each, split_tile_tri), a 64-wide one of one wave 3 of 4.
-inline double syrk_tile_units(int T) {
-  return (double)T * (T - 1) / 2 + T * (3. / 4.);
+// per side, 64 w wide: of the 32x32 blocks of a diagonal tile the four waves compute 12 of 16 where it is
+// 128 wide (three each, split_tile_tri), all four where it is 64 wide.
+inline double syrk_tile_units(int T, int w) {
+  return (double)T * (T - 1) / 2 + T * (w == 1 ? 1. : 3. / 4.);
 }
 
 inline int launch_status() {

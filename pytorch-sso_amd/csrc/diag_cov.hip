@@ -48,7 +48,6 @@ __global__ __launch_bounds__(NTHREADS, 2) void diag_linear_kernel(const float* g
 
 // sum of squares of the accumulators over the calls of the tile engine
 struct EpiSquares {
-  static constexpr bool indexed = true;
   float sq[64];
   __device__ __forceinline__ void store_at(int idx, float v) { sq[idx] = fmaf(v, v, sq[idx]); }
 };
@@ -57,6 +56,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void diag_conv_kernel(
     const float* g, const float* x, int n, int cout, int c, int H, int Wd, int kh, int kw, int sh,
     int sw, int ph, int pw, int dh, int dw, int OH, int OW, int samples_per_split, int splits,
     float alpha, float* out, float* ws) {
+  static_assert(SMEM_FLOATS * 4 <= SplitCfg<2>::SMEM_BYTES, "the launch gives these tiles that much");
   extern __shared__ __attribute__((aligned(16))) float smem[];
   const int ckk = c * kh * kw;
   const int L = OH * OW;
@@ -71,7 +71,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void diag_conv_kernel(
   for (int b = b0; b < b1; ++b) {
     DenseMK P{g + (size_t)b * cout * L, L, cout};
     const ConvA Q(Q0, x + (size_t)b * c * H * Wd);
-    gemm_tile(P, Q, m0, n0, 0, L, false, epi, smem);
+    gemm_tile(P, Q, m0, n0, 0, L, epi, smem);
   }
   float* dst = splits == 1 ? out : ws + (size_t)split * cout * ckk;
   const float scale = splits == 1 ? alpha : 1.f;
@@ -82,7 +82,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void diag_conv_kernel(
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         int row, col;
-        acc_coords<2, 2>(m0, n0, a, bb, i, row, col);
+        acc_coords(m0, n0, a, bb, i, row, col);
         if (row < cout && col < ckk)
           dst[(size_t)row * ckk + col] = scale * epi.sq[(a * 2 + bb) * 16 + i];
       }

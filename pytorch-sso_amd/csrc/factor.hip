@@ -65,30 +65,33 @@ void upload_table(const void* host, size_t bytes, void* dev, hipStream_t stream)
 }
 
 // Tile configuration and k-split of a symmetric d x d product reduced over K:
-// 64-wide single-wave tiles for small factors (a 128-wide tile would be mostly
-// padding), 128-wide tiles otherwise; enough k-splits to put about 8 waves on
-// every SIMD, each split at least 128 deep.
+// 64-wide tiles for small factors (a 128-wide tile would be mostly padding), 128-wide
+// tiles otherwise; enough k-splits to fill the chip, each split at least 128 deep.
 struct SyrkPlan {
-  int w;        // waves per tile side: 1 -> 64x64 tiles, 2 -> 128x128
+  int w;        // 1 -> 64x64 tiles, 2 -> 128x128
   int ts;       // tile size
   int T;        // tiles per side
   int ntiles;   // upper-triangular tiles
   int splits;
-  int cps;      // chunks (of the configuration's KC) per split
+  int cps;      // chunks (of KC) per split
 };
 
 static SyrkPlan plan_syrk(int d, long K) {
   SyrkPlan p;
-  p.w = d <= 256 ? 1 : 2;
+  // 64-wide tiles up to 192 rows, and to 256 where the reduction is short: of 200 rows over 4096 / 16384 /
+  // 32768 / 60000 / 100000 terms 13.1 / 22.7 / 30.4 / 45.6 / 64.8 us, on 128-wide tiles 18.1 / 26.4 / 31.0 / 41.0 /
+  // 55.5; of 256 over the same 13.8 / 23.7 / 31.5 / 48.4 / 69.1 and 19.1 / 28.2 / 34.5 / 45.9 / 61.9.
+  p.w = d <= 192 || (d <= 256 && K <= 32768) ? 1 : 2;
   p.ts = 64 * p.w;
   p.T = cdiv(d, p.ts);
   p.ntiles = p.T * (p.T + 1) / 2;
-  const int kc = p.w == 1 ? Cfg<1, 1>::KC : Cfg<2, 2>::KC;
-  const long nchunks = (K + kc - 1) / kc;
-  const long target = 2048 / (p.w * p.w);
+  const long nchunks = (K + KC - 1) / KC;
+  // (64-wide: 32 images of 64x112x112 in 1280 / 1536 / 2048 workgroups 39.5 / 42.7 / 46.4 us, of the
+  // 3x224x224 of a 7x7 stem 244 / 222 / 221)
+  const long target = p.w == 1 ? 1536 : 512;
   long splits = target / p.ntiles;
   if (splits < 1) splits = 1;
-  const long min_chunks = 128 / kc;      // each split at least 128 deep
+  const long min_chunks = 128 / KC;      // each split at least 128 deep
   const long max_splits = nchunks / min_chunks > 0 ? nchunks / min_chunks : 1;
   if (splits > max_splits) splits = max_splits;
   long cps = (nchunks + splits - 1) / splits;
@@ -127,31 +130,21 @@ static SyrkPlan plan_syrk(int d, long K) {
   return p;
 }
 
-// Index positions of an image of `hw` terms in a product in runs: 128-wide tiles take padded runs
-// (padded_run), also in products of their own: 8 images of 600x3x3 / 32 of 512x3x3 / 32 of
-// 2048x7x7 / 32 of 384x55x55 unpadded 21.2 / 24.1 / 71.3 / 122.7 us, padded 18.3 / 19.0 / 64.4 /
-// 108.2 (on the fp32 tile engine, which does not care about runs: 18.9 / 22.8 / 92.5 / 171.0).
-static int syrk_positions(int d, int64_t terms, int hw) {
-  return plan_syrk(d, (long)terms).w == 2 ? padded_run(hw) : hw;
-}
-
 // The plan of `terms` terms carried over to the `positions` that they take up: no more splits,
 // so that the scratch is that of kfac_factor_workspace_bytes(d, terms).
 static SyrkPlan stretch_plan(SyrkPlan p, int64_t positions) {
-  const int kc = p.w == 1 ? Cfg<1, 1>::KC : Cfg<2, 2>::KC;
-  const long nchunks = (long)((positions + kc - 1) / kc);
+  const long nchunks = (long)((positions + KC - 1) / KC);
   p.cps = (int)((nchunks + p.splits - 1) / p.splits);
   p.splits = (int)((nchunks + p.cps - 1) / p.cps);
   return p;
 }
 
 template <class OP, int W>
-__global__ __launch_bounds__(64 * W * W, W == 2 ? 2 : 1) void syrk_kernel(OP op, int d, int K, int T, int ntiles,
+__global__ __launch_bounds__(256, W == 2 ? 2 : 3) void syrk_kernel(OP op, int d, int K, int T, int ntiles,
                                                           int splits, int chunks_per_split,
                                                           float* C, const float* Cin,
                                                           float alpha, float beta, float* ws) {
   constexpr int TS = 64 * W;
-  constexpr int KC = Cfg<W, W>::KC;
   extern __shared__ __attribute__((aligned(16))) float smem[];
   // work item = (split, tile), tile fastest: the tiles of one split read the
   // same rows of the input, so they are kept on one XCD
@@ -192,7 +185,7 @@ static void launch_syrk_cfg(const OP& op, const SyrkPlan& p, int d, int64_t K, f
   constexpr int TS = 64 * W;
   constexpr int lds_bytes = syrk_lds_bytes<W>();
   if (!enable_large_lds((const void*)syrk_kernel<OP, W>, lds_bytes)) return;
-  hipLaunchKernelGGL((syrk_kernel<OP, W>), dim3(p.ntiles, p.splits), dim3(64 * W * W), lds_bytes,
+  hipLaunchKernelGGL((syrk_kernel<OP, W>), dim3(p.ntiles, p.splits), dim3(256), lds_bytes,
                      stream, op, d, (int)K, p.T, p.ntiles, p.splits, p.cps, C, Cin, alpha, beta,
                      (float*)workspace);
   if (p.splits > 16) {
@@ -249,9 +242,8 @@ static int64_t slice_len(int64_t total, int64_t elems_per_unit) {
 // tile leaves out its 32x32 blocks below the diagonal.
 static double syrk_executed_flops(int d, int64_t terms, int64_t K) {
   const SyrkPlan p = plan_syrk(d, (long)terms);
-  const int kc = p.w == 1 ? Cfg<1, 1>::KC : Cfg<2, 2>::KC;
-  const double chunks = (double)((K + kc - 1) / kc);
-  return syrk_tile_units(p.T) * chunks * kc * 2.0 * p.ts * p.ts;
+  const double chunks = (double)((K + KC - 1) / KC);
+  return syrk_tile_units(p.T, p.w) * chunks * KC * 2.0 * p.ts * p.ts;
 }
 
 double kfac_factor_executed_flops(int d, int64_t K) {
@@ -276,7 +268,7 @@ double kfac_factor_conv_a_executed_flops(int n, int c, int H, int W, int kh, int
     const int cnt = (int)(n - n0 < step ? n - n0 : step);
     if (kh == 1 && kw == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0 && !add_bias) {
       const int64_t terms = (int64_t)cnt * H * W;
-      total += syrk_executed_flops(d, terms, (int64_t)cnt * syrk_positions(d, terms, H * W));
+      total += syrk_executed_flops(d, terms, (int64_t)cnt * padded_run(H * W));
       continue;
     }
     if (conv_a_taps_applicable(c, kh, kw, sh, sw, add_bias)) {
@@ -359,7 +351,7 @@ int kfac_factor_conv_a(const float* x, int n, int c, int H, int W, int kh, int k
     if (kh == 1 && kw == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0 && !add_bias) {
       // a pointwise convolution: M is the input itself, viewed as [c, n*H*W]
       const int64_t terms = (int64_t)cnt * H * W;
-      const int positions = syrk_positions(d, terms, H * W);
+      const int positions = padded_run(H * W);
       ConvG op{x + n0 * image, c, H * W, positions};
       const int st = launch_syrk(op, d, terms, (int64_t)cnt * positions, alpha, bslice, prev, C,
                                  workspace, workspace_bytes, (hipStream_t)stream);
@@ -392,7 +384,7 @@ int kfac_factor_conv_g(const float* g, int n, int c, int h, int w, float alpha, 
   for (int64_t n0 = 0; n0 < n; n0 += step) {
     const int cnt = (int)(n - n0 < step ? n - n0 : step);
     const int64_t terms = (int64_t)cnt * h * w;
-    const int positions = syrk_positions(c, terms, h * w);
+    const int positions = padded_run(h * w);
     ConvG op{g + n0 * image, c, h * w, positions};
     const int st = launch_syrk(op, c, terms, (int64_t)cnt * positions, alpha, n0 == 0 ? beta : 1.f,
                                n0 == 0 ? C_prev : nullptr, C, workspace, workspace_bytes,

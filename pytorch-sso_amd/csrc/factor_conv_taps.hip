@@ -41,7 +41,7 @@ struct ShiftX {
   static constexpr bool pads_runs = true;
   const float* p;
   int C, H, W, u0, v0, hh, ww;     // u0, v0 already include the displacement
-  int wwp;                         // index positions of a row (row_positions)
+  int wwp;                         // index positions of a row (padded_run)
   FastDiv by_area, by_ww;          // divisions by hh * wwp and by wwp
   struct MS { unsigned off; };
   struct KS { unsigned off; };
@@ -78,21 +78,18 @@ struct ShiftX {
   }
 };
 
-// Index positions of a row of a rectangle: padded (padded_run) for 128-wide tiles.
-__host__ __device__ inline int row_positions(int ww, int w) { return w == 2 ? padded_run(ww) : ww; }
-
 // Time of a chunk of a job against one in runs of at least 4.  Rows of up to three positions (the
 // strips beside the left and right edge) are loaded element by element, every lane of a load in a
 // line of its own: on 128-wide tiles such a chunk lasts several times as long, and a plan that
 // counts it as one ends with the few items of those strips.  Factor of 32 images of 128x56x56 /
 // 256x14x14 / 64 of 128x14x14, one product: 667 / 190 / 110 us counted as 1, 349 / 125 / 76 as 5,
 // 331 / 117 / 71 as 6, 302 / 112 / 71 as 8 (but 32 of 512x9x9, where every job is short: 207 / 210 /
-// 209 / 224).  The 64-wide tiles load everything element by element.
+// 209 / 224).
 constexpr int SHORT_RUN_COST = 6;
-static int chunk_cost(int ww, int w) { return w == 2 && ww < 4 ? SHORT_RUN_COST : 1; }
+static int chunk_cost(int ww) { return ww < 4 ? SHORT_RUN_COST : 1; }
 
 struct JobDesc {
-  short u0, v0, hh, ww;    // rectangle of the first factor; the reduction runs over its rows (row_positions)
+  short u0, v0, hh, ww;    // rectangle of the first factor; the reduction runs over its rows (padded_run)
   short dy, dx;            // displacement of the second factor
   short splits;            // k-splits
   unsigned char sh_area, sh_ww;   // shifts of the two FastDiv of a ShiftX
@@ -126,10 +123,9 @@ __device__ __forceinline__ void corr_product(const float* x, int nimg, int C, in
                                              const TapPlanDev& plan, int tiles_side, float* ws,
                                              int j, int split, int tile, float* smem) {
   constexpr int TS = 64 * W;
-  constexpr int KC = Cfg<W, W>::KC;
   const JobDesc jd = plan.jobs[j];
   const int bi = tile / tiles_side, bj = tile - bi * tiles_side;
-  const int wwp = row_positions(jd.ww, W);
+  const int wwp = padded_run(jd.ww);
   const int K = nimg * jd.hh * wwp;
   const int kbeg = split * jd.cps * KC;
   int kend = kbeg + jd.cps * KC;
@@ -142,10 +138,7 @@ __device__ __forceinline__ void corr_product(const float* x, int nimg, int C, in
   ShiftX P{x, C, H, Wd, jd.u0, jd.v0, jd.hh, jd.ww, wwp, by_area, by_ww};
   ShiftX Q{x, C, H, Wd, jd.u0 + jd.dy, jd.v0 + jd.dx, jd.hh, jd.ww, wwp, by_area, by_ww};
   EpiStore epi{ws + (size_t)(jd.part0 + split) * C * C, C, C, C, 1.f, 0.f, false};
-  if constexpr (W == 2)
-    split_tile(P, Q, bi * TS, bj * TS, kbeg, kend, false, epi, smem);
-  else
-    gemm_tile_cfg<W, W>(P, Q, bi * TS, bj * TS, kbeg, kend, false, epi, smem);
+  split_tile_full<W>(P, Q, bi * TS, bj * TS, kbeg, kend, smem, [&](auto&& put) { put(epi); });
 }
 
 // work item `item` of one layer's plan -> (job, split, tile), job by job
@@ -163,7 +156,7 @@ __device__ __forceinline__ void corr_item(const float* x, int nimg, int C, int H
 }
 
 template <int W>
-__global__ __launch_bounds__(64 * W * W, W == 2 ? 2 : 1) void corr_kernel(
+__global__ __launch_bounds__(256, W == 2 ? 2 : 3) void corr_kernel(
     const float* x, int nimg, int C, int H, int Wd, const TapPlanDev plan, int tiles_side,
     float* ws) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
@@ -209,7 +202,7 @@ __device__ __forceinline__ int find_layer(const int* __restrict__ cum, int n, in
 
 // the correlation items of all layers of one tile size in one launch
 template <int W>
-__global__ __launch_bounds__(64 * W * W, W == 2 ? 2 : 1) void corr_grouped_kernel(
+__global__ __launch_bounds__(256, W == 2 ? 2 : 3) void corr_grouped_kernel(
     const TapLayer* __restrict__ layers, const TapPlanDev* __restrict__ plans,
     const TapOrder* __restrict__ order, const unsigned* __restrict__ entries,
     const int* __restrict__ index, const int* __restrict__ cum, int nlayers) {
@@ -499,7 +492,7 @@ static TapPlanHost plan_taps(int n, int c, int H, int Wd, int kh, int kw, int ph
             jd.v0 = (short)ax.pieces[px].lo;
             jd.ww = (short)(ax.pieces[px].hi - ax.pieces[px].lo);
             jd.dx = (short)ax.pieces[px].delta;
-            const int wwp = row_positions(jd.ww, hp.w);
+            const int wwp = padded_run(jd.ww);
             const FastDiv fa((unsigned)(jd.hh * wwp)), fw((unsigned)wwp);
             jd.m_area = fa.m;
             jd.sh_area = (unsigned char)fa.sh;
@@ -516,17 +509,17 @@ static TapPlanHost plan_taps(int n, int c, int H, int Wd, int kh, int kw, int ph
   const int ts = 64 * hp.w;
   hp.tiles_side = cdiv(c, ts);
   const int ntiles = hp.tiles_side * hp.tiles_side;
-  const int kc = hp.w == 1 ? Cfg<1, 1>::KC : Cfg<2, 2>::KC;
-  auto job_k = [&](const JobDesc& jd) { return (long)n * jd.hh * row_positions(jd.ww, hp.w); };
+  auto job_k = [&](const JobDesc& jd) { return (long)n * jd.hh * padded_run(jd.ww); };
   // (in chunks in runs)
-  auto job_work = [&](const JobDesc& jd) { return (job_k(jd) + kc - 1) / kc * chunk_cost(jd.ww, hp.w); };
+  auto job_work = [&](const JobDesc& jd) { return (job_k(jd) + KC - 1) / KC * chunk_cost(jd.ww); };
   double total = 0;
   for (int j = 0; j < pd.njobs; ++j) total += (double)job_work(pd.jobs[j]);
   // All workgroups of a launch that fits the chip are resident at once (RESIDENT_TILES) and share
   // the matrix cores of their CU, so the launch lasts as long as the fullest CU: about one full
   // round of items of one duration.  (A target of 440 / 480 / 512 items, as above: 341 / 348 /
   // 331, 121 / 125 / 117 and 74 / 76 / 71 us; 700, of the time when three workgroups fitted a
-  // CU: 310 / 140 / 88.)  The one-wave workgroups (8 per CU) do best at 1.5 rounds.
+  // CU: 310 / 140 / 88.)  64-wide tiles: 32 images of 64x56x56 / 64x28x28, 64 of 64x14x14 with 1280 /
+  // 1536 / 2560 / 3072 items 140 131 134 133 / 62 59 69 67 / 48 46 46 46 us.
   // Where the splits of the jobs, rounded to whole ones, make a good deal more than one round all the
   // same (9 tiles and more to a job), shorter items end more evenly: 39 images of 400x16x16, 672
   // items 518 us, 880 462; 2 of 324x52x52, 612 and 846, 208 and 188; but 32 of 512x7x7 180 and 189,
@@ -536,12 +529,12 @@ static TapPlanHost plan_taps(int n, int c, int H, int Wd, int kh, int kw, int ph
     int item = 0, part = 0;
     for (int j = 0; j < pd.njobs; ++j) {
       JobDesc& jd = pd.jobs[j];
-      const long nchunks = (job_k(jd) + kc - 1) / kc;
+      const long nchunks = (job_k(jd) + KC - 1) / KC;
       const long work = job_work(jd);
       long splits = group_cps > 0 ? (work + group_cps / 2) / group_cps
                                   : (long)(target_items * ((double)work / total) / ntiles + 0.5);
       // (an item lasts as long as 128 steps in runs, at least, and is a chunk, at least)
-      const long max_splits = std::max<long>(1, std::min(nchunks, work / (128 / kc)));
+      const long max_splits = std::max<long>(1, std::min(nchunks, work / (128 / KC)));
       splits = std::max<long>(1, std::min(std::min(splits, max_splits), 4096L));
       long cps = (nchunks + splits - 1) / splits;
       splits = (nchunks + cps - 1) / cps;
@@ -555,7 +548,7 @@ static TapPlanHost plan_taps(int n, int c, int H, int Wd, int kh, int kw, int ph
     hp.items = item;
     return part;
   };
-  int part = deal(hp.w == 1 ? 3072.0 : (double)RESIDENT_TILES);
+  int part = deal(hp.w == 1 ? RESIDENT_SMALL_CORR : (double)RESIDENT_TILES);
   if (hp.w == 2 && group_cps == 0 && hp.items > ROUND_LIMIT) part = deal(LONG_ROUND);
   for (int j = pd.njobs; j < MAX_JOBS; ++j) pd.item0[j] = INT_MAX;
   hp.partial_floats = (size_t)(part + pd.npairs) * c * c;     // partials, then the block sums
@@ -579,13 +572,12 @@ size_t conv_a_taps_workspace(int n, int c, int H, int W, int kh, int kw, int ph,
 // (job, split, tile) work item.
 static double plan_executed_flops(const TapPlanHost& hp, int n) {
   const int ts = 64 * hp.w;
-  const int kc = hp.w == 1 ? Cfg<1, 1>::KC : Cfg<2, 2>::KC;
   const double ntiles = (double)hp.tiles_side * hp.tiles_side;
   double total = 0.;
   for (int j = 0; j < hp.dev.njobs; ++j) {
     const JobDesc& jd = hp.dev.jobs[j];
-    const long K = (long)n * jd.hh * row_positions(jd.ww, hp.w);
-    total += ntiles * (double)((K + kc - 1) / kc) * kc * 2.0 * ts * ts;
+    const long K = (long)n * jd.hh * padded_run(jd.ww);
+    total += ntiles * (double)((K + KC - 1) / KC) * KC * 2.0 * ts * ts;
   }
   return total;
 }
@@ -608,12 +600,12 @@ int conv_a_taps(const float* x, int n, int c, int H, int W, int kh, int kw, int 
   float* B = ws + hp.sum_offset;
   const int T = kh * kw;
   if (hp.w == 1) {
-    constexpr int lds = Cfg<1, 1>::SMEM_FLOATS * (int)sizeof(float);
+    constexpr int lds = SplitCfg<1>::SMEM_BYTES;
     if (!enable_large_lds((const void*)corr_kernel<1>, lds)) return KFAC_ERR_LAUNCH;
-    hipLaunchKernelGGL(corr_kernel<1>, dim3(hp.items), dim3(64), lds, stream, x, n, c, H, W,
+    hipLaunchKernelGGL(corr_kernel<1>, dim3(hp.items), dim3(256), lds, stream, x, n, c, H, W,
                        hp.dev, hp.tiles_side, ws);
   } else {
-    constexpr int lds = SplitCfg<2, 2>::SMEM_BYTES;
+    constexpr int lds = SplitCfg<2>::SMEM_BYTES;
     if (!enable_large_lds((const void*)corr_kernel<2>, lds)) return KFAC_ERR_LAUNCH;
     hipLaunchKernelGGL(corr_kernel<2>, dim3(hp.items), dim3(256), lds, stream, x, n, c, H, W,
                        hp.dev, hp.tiles_side, ws);
@@ -674,7 +666,7 @@ static TapOrder make_order(const TapPlanHost& hp, std::vector<unsigned>& entries
   return o;
 }
 
-// chunks per item of a grouped launch (one-wave 64-wide tiles / four-wave 128-wide tiles);
+// chunks per item of a grouped launch (64-wide / 128-wide tiles);
 // factors of a ResNet-50, 32 images: 4.62 / 4.57 / 4.64 ms with 64 / 96 / 128 chunks of 128-wide tiles
 constexpr int TAPS_GROUP_CPS1 = 192, TAPS_GROUP_CPS2 = 96;
 
@@ -696,7 +688,8 @@ static TapsGroupPlan* make_taps_group_plan(int count, const TapsJob* jobs) {
   }
   int group_cps[2];
   for (int w = 0; w < 2; ++w) {
-    group_cps[w] = (int)group_item_chunks(w + 1, units[w], w == 0 ? TAPS_GROUP_CPS1 : TAPS_GROUP_CPS2);
+    group_cps[w] = (int)group_item_chunks(w + 1, units[w], w == 0 ? TAPS_GROUP_CPS1 : TAPS_GROUP_CPS2,
+                                          RESIDENT_SMALL_CORR);
   }
   for (int i = 0; i < count; ++i) {
     const TapsJob& j = jobs[i];
@@ -834,16 +827,16 @@ int conv_a_taps_grouped(int count, const TapsJob* jobs, void* workspace, size_t 
   const TapOrder* dord = (const TapOrder*)(table + gp.orders_off);
   const unsigned* dent = (const unsigned*)(table + gp.entries_off);
   if (!gp.members[1].empty()) {
-    constexpr int lds = SplitCfg<2, 2>::SMEM_BYTES;
+    constexpr int lds = SplitCfg<2>::SMEM_BYTES;
     if (!enable_large_lds((const void*)corr_grouped_kernel<2>, lds)) return KFAC_ERR_LAUNCH;
     hipLaunchKernelGGL(corr_grouped_kernel<2>, dim3(gp.cum_corr[1].back()), dim3(256), lds, stream,
                        dl, dp, dord, dent, (const int*)(table + gp.index_off[1]),
                        (const int*)(table + gp.cum_corr_off[1]), (int)gp.members[1].size());
   }
   if (!gp.members[0].empty()) {
-    constexpr int lds = Cfg<1, 1>::SMEM_FLOATS * (int)sizeof(float);
+    constexpr int lds = SplitCfg<1>::SMEM_BYTES;
     if (!enable_large_lds((const void*)corr_grouped_kernel<1>, lds)) return KFAC_ERR_LAUNCH;
-    hipLaunchKernelGGL(corr_grouped_kernel<1>, dim3(gp.cum_corr[0].back()), dim3(64), lds, stream,
+    hipLaunchKernelGGL(corr_grouped_kernel<1>, dim3(gp.cum_corr[0].back()), dim3(256), lds, stream,
                        dl, dp, dord, dent, (const int*)(table + gp.index_off[0]),
                        (const int*)(table + gp.cum_corr_off[0]), (int)gp.members[0].size());
   }

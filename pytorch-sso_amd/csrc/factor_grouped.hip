@@ -66,10 +66,9 @@ __device__ __forceinline__ int find_job(const int* __restrict__ cum, int njobs, 
 }
 
 template <class OP, int W>
-__global__ __launch_bounds__(64 * W * W, W == 2 ? 2 : 1) void syrk_grouped_kernel(
+__global__ __launch_bounds__(256, W == 2 ? 2 : 3) void syrk_grouped_kernel(
     const SyJob<OP>* __restrict__ jobs, const int* __restrict__ cum, int njobs) {
   constexpr int TS = 64 * W;
-  constexpr int KC = Cfg<W, W>::KC;
   extern __shared__ __attribute__((aligned(16))) float smem[];
   const int g = blockIdx.x;
   const int j = find_job(cum, njobs, g);
@@ -191,7 +190,7 @@ struct GroupPlan {
   }
 };
 
-// 64-wide tiles (one wave each) up to 192 rows; from there a 128-wide tile has at most a
+// 64-wide tiles up to 192 rows; from there a 128-wide tile has at most a
 // quarter of padding, and it runs on the bf16 matrix cores (factors of a ResNet-50, 32 images: 4.57 ms,
 // and 5.1 ms with 64-wide tiles up to 256 rows; 128 rows make no difference there).
 constexpr int GROUP_W1_MAX_DIM = 192;
@@ -293,7 +292,7 @@ static Classified classify(const kfac_factor_job& j) {
   Classified c = classify_shape(j);
   if (c.path != P_CONVG && c.path != P_CONVP) return c;
   const int run = c.path == P_CONVG ? j.H * j.W : c.OH * c.OW;
-  c.positions = c.d > GROUP_W1_MAX_DIM ? padded_run(run) : run;
+  c.positions = padded_run(run);
   c.K = (long)j.rows * c.positions;
   return c;
 }
@@ -413,7 +412,7 @@ static GroupedPlan make_plan(int count, const kfac_factor_job* jobs) {
         else if (p.splits > 1)
           gp.reduce_tile[w].push_back(i);
         gp.executed_flops +=
-            syrk_tile_units(p.T) * (double)((c.K + 15) / 16) * 16 * 2.0 * p.ts * p.ts;
+            syrk_tile_units(p.T, p.w) * (double)((c.K + 15) / 16) * 16 * 2.0 * p.ts * p.ts;
       }
     }
   for (int path = 0; path < SYRK_PATHS; ++path)
@@ -648,7 +647,7 @@ static bool launch_syrk_group(const Launch& l, char* table, hipStream_t stream) 
   if (l.njobs == 0) return true;
   constexpr int lds_bytes = syrk_lds_bytes<W>();
   if (!enable_large_lds((const void*)syrk_grouped_kernel<OP, W>, lds_bytes)) return false;
-  hipLaunchKernelGGL((syrk_grouped_kernel<OP, W>), dim3(l.items), dim3(64 * W * W), lds_bytes,
+  hipLaunchKernelGGL((syrk_grouped_kernel<OP, W>), dim3(l.items), dim3(256), lds_bytes,
                      stream, (const SyJob<OP>*)(table + l.jobs_off),
                      (const int*)(table + l.cum_off), l.njobs);
   return true;

@@ -56,15 +56,59 @@ struct SplitChunk {
   static constexpr int BYTES = 3 * PLANE;
 };
 
-template <int WM, int WN>
+// The 32x32 blocks of a tile that one wave computes, and from which fragment rows (of 32) of the
+// operands.  TM x TN: the tile; NT: its threads; NB blocks a wave, block B = fragment row a(B) of P
+// against row b(B) of Q (SAME: of P: a diagonal tile of a symmetric product, of which only P is
+// staged); PF / QF fragment rows a wave.
+// SplitTile: four waves, each a 64x64 quadrant of 128x128.
+struct SplitTile {
+  static constexpr int TM = 128, TN = 128, NT = 256, NB = 4, PF = 2, QF = 2;
+  static constexpr bool SAME = false;
+  static constexpr int a(int B) { return B >> 1; }
+  static constexpr int b(int B) { return B & 1; }
+};
+// SplitDiag: a 128x128 diagonal tile is symmetric itself; its blocks on and above the diagonal
+// (10 of 16) are dealt to the four waves three at a time, as products of three fragment rows
+// r0, r1, r2 of the one operand:
+//     block 0 = (r0, r1)    block 1 = (r0, r2)    block 2 = (r1, r1)
+//   waves 0 / 1: r = (0, 1, 0) / (2, 3, 2), the three blocks of a diagonal quadrant;
+//   waves 2 / 3: r = (0, 2, 3) / (1, 2, 3), a row of the quadrant above the diagonal (their block 2
+//   repeats one of wave 1's and is not stored).
+// Every wave runs the same code, and the tile is done in three quarters of the time.
+struct SplitDiag {
+  static constexpr int TM = 128, TN = 128, NT = 256, NB = 3, PF = 3, QF = 0;
+  static constexpr bool SAME = true;
+  static constexpr int a(int B) { return B == 2 ? 1 : 0; }
+  static constexpr int b(int B) { return B == 1 ? 2 : 1; }
+};
+// SmallTile, SmallDiag: 64x64, a block on each of four waves (of a diagonal tile three blocks are
+// stored).  A chunk is short work for a wave (6 matrix instructions), so what bounds these is the barrier and
+// the loads of each chunk, and workgroups in flight hide them: five to a CU at 100 registers.  (One wave
+// with the four blocks does with two thirds of the LDS reads, but needs 330 registers.)  On the fp32
+// matrix instructions, a wave to a tile, / here: output gradients of 32 images of 64x112x112 69 / 39 us,
+// 128x56x56 54 / 35, six layers of 64x56x56 82 / 45, of 160x13x13 23 / 18; 3x3 inputs of 64x56x56, three
+// layers, 480 / 319, the 3x224x224 of a 7x7 stem 261 / 162; 4096 rows of 100 28 / 15.
+struct SmallTile {
+  static constexpr int TM = 64, TN = 64, NT = 256, NB = 1, PF = 1, QF = 1;
+  static constexpr bool SAME = false;
+  static constexpr int a(int) { return 0; }
+  static constexpr int b(int) { return 0; }
+};
+struct SmallDiag {
+  static constexpr int TM = 64, TN = 64, NT = 256, NB = 1, PF = 2, QF = 0;
+  static constexpr bool SAME = true;
+  static constexpr int a(int) { return 0; }
+  static constexpr int b(int) { return 1; }
+};
+
+// tiles 64 W wide
+template <int W>
 struct SplitCfg {
-  static constexpr int TM = 64 * WM;
-  static constexpr int TN = 64 * WN;
-  static constexpr int NT = 64 * WM * WN;
-  static constexpr int KC = 16;
-  static constexpr int STAGE = SplitChunk<TM>::BYTES + SplitChunk<TN>::BYTES;
+  static constexpr int TS = 64 * W;
+  static constexpr int NT = NTHREADS;
+  static constexpr int STAGE = 2 * SplitChunk<TS>::BYTES;
   static constexpr int VOTES = 2 * STAGE;                // a word per wave (split_blocks)
-  static constexpr int SMEM_BYTES = VOTES + 4 * WM * WN;
+  static constexpr int SMEM_BYTES = VOTES + 4 * (NT / 64);
 };
 
 __device__ __forceinline__ unsigned pack_bf16(float a, float b) {
@@ -129,7 +173,9 @@ struct KRun {
 enum { ANY_K = 0, FAST_K = 1, PADDED_K = 2 };
 
 // Index positions of a run of `run` elements: a multiple of 4 wherever a group of 4 fits into it.
-// (A run of 5 is 60 % more work and still faster: correlations of 512 channels of 7x7, rows of 5,
+// (A run of 5 is 60 % more work and still faster, as correlations and as products: 8 images of 600x3x3 /
+// 32 of 512x3x3 / 2048x7x7 / 384x55x55 unpadded 21.2 / 24.1 / 71.3 / 122.7 us, padded 18.3 / 19.0 /
+// 64.4 / 108.2; correlations of 512 channels of 7x7, rows of 5,
 // 211 us unpadded, 201 padded; 9x9, rows of 7, 265 / 234; 128 channels of 56x56, rows of 54,
 // 527 / 489; 28x28, rows of 26, 177 / 170.)
 __host__ __device__ inline int padded_run(int run) {
@@ -146,16 +192,19 @@ struct has_padded_runs<OP, std::enable_if_t<OP::pads_runs>> : std::true_type {};
 template <class OP, int ROWS, int NT, int LAYOUT = OP::layout>
 struct SplitStager;
 
-// Consecutive m contiguous: a thread takes 8 consecutive k of one column.
+// Consecutive m contiguous: a thread takes 8 consecutive k of one column (4 where there are more
+// threads than that).
 template <class OP, int ROWS, int NT>
 struct SplitStager<OP, ROWS, NT, KM> {
-  static constexpr int NI = ROWS * 2 / NT;
-  static constexpr int PIECES = 4 * NI;
-  static_assert(ROWS * 2 % NT == 0 && ROWS % 64 == 0, "a wave's lanes share their k");
+  static constexpr int KPT = ROWS * 2 >= NT ? 8 : 4;
+  static constexpr int NI = ROWS * (16 / KPT) / NT;
+  static constexpr int PIECES = KPT / 2 * NI;
+  static_assert(ROWS * (16 / KPT) % NT == 0 && ROWS % 64 == 0, "a wave's lanes share their k");
+  typedef unsigned Part __attribute__((ext_vector_type(KPT / 2)));
   typename OP::MS ms[NI];
-  float regs[2][NI][8];
-  unsigned ones[2];          // bit 8i + j: element j of column i is the constant 1
-  v4u ph, pm, pl;            // the column being split
+  float regs[2][NI][KPT];
+  unsigned ones[2];          // bit KPT i + j: element j of column i is the constant 1
+  Part ph, pm, pl;           // the column being split
 
   static __device__ __forceinline__ int tid() { return threadIdx.x & (NT - 1); }
   static __device__ __forceinline__ int kgroup(int i) {
@@ -172,11 +221,11 @@ struct SplitStager<OP, ROWS, NT, KM> {
   template <int SET, class OTHER>
   __device__ __forceinline__ void take_k(const OP&, const OP&, const OTHER&) {}
   // a chunk inside the k range of a `fast` tile, load by load
-  static constexpr int LOADS = 8 * NI;
+  static constexpr int LOADS = KPT * NI;
   template <int SET, int LOAD, int MODE, bool KNOWN>
   __device__ __forceinline__ void fetch_load(const OP& op, int k0) {
-    constexpr int i = LOAD / 8, j = LOAD % 8;
-    regs[SET][i][j] = buffer_load_at(op.rsrc(), ms[i].off, (k0 + 8 * kgroup(i) + j) * op.kstride());
+    constexpr int i = LOAD / KPT, j = LOAD % KPT;
+    regs[SET][i][j] = buffer_load_at(op.rsrc(), ms[i].off, (k0 + KPT * kgroup(i) + j) * op.kstride());
   }
   // any chunk
   template <int SET>
@@ -184,16 +233,16 @@ struct SplitStager<OP, ROWS, NT, KM> {
     unsigned one = 0;
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      const int k = k0 + 8 * kgroup(i);
+      const int k = k0 + KPT * kgroup(i);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
+      for (int j = 0; j < KPT; ++j) {
         // (k is the same for all lanes: its offset is a scalar)
         const bool in = k + j < kend;
         const unsigned at = in ? (k + j) : 0;
         regs[SET][i][j] = buffer_load_at(op.rsrc(), in ? ms[i].off : INV_M, at * op.kstride());
         if (op.second())
           regs[SET][i][j] += buffer_load_at(op.rsrc2(), in ? ms[i].off2 : INV_M, at * 4u);
-        one |= (unsigned)(op.is_one(ms[i]) && in) << (8 * i + j);
+        one |= (unsigned)(op.is_one(ms[i]) && in) << (KPT * i + j);
       }
     }
     ones[SET] = one;
@@ -201,11 +250,11 @@ struct SplitStager<OP, ROWS, NT, KM> {
   template <int SET, int PIECE, int MODE, bool SCALED = false>
   __device__ __forceinline__ void commit(lds_c* chunk, float scale = 1.f) {
     typedef SplitChunk<ROWS> L;
-    constexpr int i = PIECE / 4, j = PIECE % 4;
+    constexpr int i = PIECE / (KPT / 2), j = PIECE % (KPT / 2);
     float v[2] = {regs[SET][i][2 * j], regs[SET][i][2 * j + 1]};
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
-      if (MODE == ANY_K) v[e] = ((ones[SET] >> (8 * i + 2 * j + e)) & 1u) ? 1.f : v[e];
+      if (MODE == ANY_K) v[e] = ((ones[SET] >> (KPT * i + 2 * j + e)) & 1u) ? 1.f : v[e];
       if (squares_elements<OP>::value) v[e] *= v[e];
       if (SCALED) v[e] *= scale;
     }
@@ -214,11 +263,13 @@ struct SplitStager<OP, ROWS, NT, KM> {
     ph[j] = h;
     pm[j] = m;
     pl[j] = l;
-    if (j == 3) {
-      lds_c* const at = chunk + kgroup(i) * L::HALF + ((tid() + NT * i) & (ROWS - 1)) * 16;
-      *(lds_u4*)at = ph;
-      *(lds_u4*)(at + L::PLANE) = pm;
-      *(lds_u4*)(at + 2 * L::PLANE) = pl;
+    if (j == KPT / 2 - 1) {
+      typedef __attribute__((address_space(3))) Part lds_part;
+      const int k = KPT * kgroup(i);
+      lds_c* const at = chunk + k / 8 * L::HALF + ((tid() + NT * i) & (ROWS - 1)) * 16 + k % 8 * 2;
+      *(lds_part*)at = ph;
+      *(lds_part*)(at + L::PLANE) = pm;
+      *(lds_part*)(at + 2 * L::PLANE) = pl;
     }
   }
 };
@@ -353,16 +404,6 @@ __device__ __forceinline__ void static_for(F&& f) {
   }
 }
 
-// The 32x32 blocks of a tile that one wave computes.
-// FULL: the four blocks of its 64x64 quadrant, block (a, b) = rows a of P against rows b of Q.
-// TRI: a diagonal tile of a symmetric product (P = Q) is symmetric itself; its blocks on and
-// above the diagonal (10 of 16) are dealt to the four waves three at a time, as products of three
-// fragment rows r0, r1, r2 of the one operand:
-//     block 0 = (r0, r1)    block 1 = (r0, r2)    block 2 = (r1, r1)
-//   waves 0 / 1: r = (0, 1, 0) / (2, 3, 2), the three blocks of a diagonal quadrant;
-//   waves 2 / 3: r = (0, 2, 3) / (1, 2, 3), a row of the quadrant above the diagonal (their block 2
-//   repeats one of wave 1's and is not stored).
-// Every wave runs the same code, and the tile is done in three quarters of the time.
 struct SplitTri {
   int r[3];
   bool last;           // block 2 is this wave's to store
@@ -373,40 +414,40 @@ __device__ __forceinline__ SplitTri split_tri(int wave) {
   return SplitTri{{wave - 2, 2, 3}, false};
 }
 
-// fragments of one chunk: [h, m, l][row]; a FULL wave keeps P's two rows and Q's two
-template <bool TRI>
+// fragments of one chunk: [h, m, l][row]
+template <class TILE>
 struct SplitFrags {
-  v8bf p[3][TRI ? 3 : 2];
-  v8bf q[3][TRI ? 1 : 2];
+  v8bf p[3][TILE::PF];
+  v8bf q[3][TILE::QF > 0 ? TILE::QF : 1];
 };
 
-// product PR of the six (in the order h h', h m', m h', m m', h l', l h') for block B
-template <bool TRI, int PR, int B>
-__device__ __forceinline__ void split_product(const SplitFrags<TRI>& fr, v16f& sum) {
-  constexpr int PA = PR == 2 || PR == 3 ? 1 : PR == 5 ? 2 : 0;
-  constexpr int PB = PR == 1 || PR == 3 ? 1 : PR == 4 ? 2 : 0;
-  v8bf a, b;
-  if constexpr (TRI) {
-    a = fr.p[PA][B == 2 ? 1 : 0];
-    b = fr.p[PB][B == 1 ? 2 : 1];
-  } else {
-    a = fr.p[PA][B >> 1];
-    b = fr.q[PB][B & 1];
-  }
+// product PR of the six (in the order h h', h m', m h', m m', h l', l h'; then m l', l m') for block B
+template <class TILE, int PR, int B>
+__device__ __forceinline__ void split_product(const SplitFrags<TILE>& fr, v16f& sum) {
+  constexpr int PA = PR == 2 || PR == 3 || PR == 6 ? 1 : PR == 5 || PR == 7 ? 2 : 0;
+  constexpr int PB = PR == 1 || PR == 3 || PR == 7 ? 1 : PR == 4 || PR == 6 ? 2 : 0;
+  const v8bf a = fr.p[PA][TILE::a(B)];
+  v8bf b;
+  if constexpr (TILE::SAME) b = fr.p[PB][TILE::b(B)];
+  else b = fr.q[PB][TILE::b(B)];
   sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, sum, 0, 0, 0);
 }
 
+// the fragment rows of a wave, as rows of the tile
+struct SplitRows {
+  int p[3], q[2];
+};
+
 // Accumulates C = P Q over [kbeg, kend) into the wave's blocks (leading products in acc, the
-// corrections in cor).  prow / qrow: the tile rows of its fragments (TRI: prow only).
-template <int WM, int WN, bool TRI, int MODE, class OPP, class OPQ>
+// corrections in cor).
+template <class C, int MODE, class OPP, class OPQ>
 __device__ __forceinline__ void split_tile_loop(const OPP& P, const OPQ& Q, int m0, int n0, int kbeg,
-                                                int kend, lds_c* sm, const int (&prow)[3],
-                                                const int (&qrow)[2], v16f (&acc)[TRI ? 3 : 4],
-                                                v16f (&cor)[TRI ? 3 : 4]) {
-  typedef SplitCfg<WM, WN> C;
-  constexpr int KC = C::KC;
+                                                int kend, lds_c* sm, const SplitRows& rows,
+                                                v16f (&acc)[C::NB], v16f (&cor)[C::NB]) {
+  constexpr bool TRI = C::SAME;
+  constexpr int STAGE = SplitCfg<C::TM / 64>::STAGE;
   constexpr int QOFF = SplitChunk<C::TM>::BYTES;
-  constexpr int NB = TRI ? 3 : 4;
+  constexpr int NB = C::NB;
   const int lane = threadIdx.x & 63;
   typedef SplitStager<OPP, C::TM, C::NT> SP;
   typedef SplitStager<OPQ, C::TN, C::NT> SQ;
@@ -443,16 +484,14 @@ __device__ __forceinline__ void split_tile_loop(const OPP& P, const OPQ& Q, int 
     else
       sq.template commit<SET, X - SP::PIECES, MODE>(stage + QOFF);
   };
-  SplitFrags<TRI> fr[2];
+  SplitFrags<C> fr[2];
   auto load_frags = [&](auto set_, auto plane_) {
     constexpr int SET = decltype(set_)::value, PL = decltype(plane_)::value;
-    const lds_c* const tp = sm + SET * C::STAGE;
+    const lds_c* const tp = sm + SET * STAGE;
 #pragma unroll
-    for (int i = 0; i < (TRI ? 3 : 2); ++i) fr[SET].p[PL][i] = load_frag<C::TM>(tp, prow[i], lane, PL);
-    if (!TRI) {
+    for (int i = 0; i < C::PF; ++i) fr[SET].p[PL][i] = load_frag<C::TM>(tp, rows.p[i], lane, PL);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) fr[SET].q[PL][i] = load_frag<C::TN>(tp + QOFF, qrow[i], lane, PL);
-    }
+    for (int i = 0; i < C::QF; ++i) fr[SET].q[PL][i] = load_frag<C::TN>(tp + QOFF, rows.q[i], lane, PL);
   };
   constexpr std::integral_constant<int, 0> S0{};
   constexpr std::integral_constant<int, 1> S1{};
@@ -472,7 +511,7 @@ __device__ __forceinline__ void split_tile_loop(const OPP& P, const OPQ& Q, int 
   auto step = [&](auto set_, auto full_, int c) {
     constexpr int SET = decltype(set_)::value;
     constexpr bool FULL = decltype(full_)::value;
-    lds_c* const next = sm + (SET ^ 1) * C::STAGE;
+    lds_c* const next = sm + (SET ^ 1) * STAGE;
     load_frags(set_, std::integral_constant<int, 1>{});
     load_frags(set_, std::integral_constant<int, 2>{});
     if (!FULL) fetch(set_, c + 2);
@@ -487,7 +526,7 @@ __device__ __forceinline__ void split_tile_loop(const OPP& P, const OPQ& Q, int 
       static_for<NB>([&](auto blk_) {
         constexpr int B = decltype(blk_)::value;
         constexpr int IDX = PR * NB + B;
-        split_product<TRI, PR, B>(fr[SET], PR == 0 ? acc[B] : cor[B]);
+        split_product<C, PR, B>(fr[SET], PR == 0 ? acc[B] : cor[B]);
         if constexpr (PR < 4) {
           constexpr int LAST = 4 * NB;
           constexpr int l0 = IDX * LOADS / LAST, l1 = (IDX + 1) * LOADS / LAST;
@@ -526,14 +565,17 @@ __device__ __forceinline__ void split_tile_loop(const OPP& P, const OPQ& Q, int 
 // loop has a third of the code and no chunk past the end.  Factor of 16 rows of 300 / 48 of 1000 /
 // 8 of 5000: 12.1 / 15.7 / 57.5 us by the loop above, 9.8 / 14.1 / 52.7 by this one (9.4 / 13.3 /
 // 51.8 on the fp32 tile engine); 64 rows of 512: 16.1 / 16.7.
+// The 64-wide tiles, which replaced fp32 instructions, take the two largest of the products left out as well:
+// in sums of one or two terms those are as large as a float32 sum's own roundings (relative 2-norm
+// of the factor of 1 / 2 rows of 17 ... 192: 2.51e-8 / 2.63e-8 without, 2.47e-8 / 2.59e-8
+// with them, 2.47e-8 / 3.10e-8 by the fp32 ones).
 constexpr int SHORT_K = 48;
-template <int WM, int WN, bool TRI, class OPP, class OPQ>
+template <class C, class OPP, class OPQ>
 __device__ __forceinline__ void split_tile_rolled(const OPP& P, const OPQ& Q, int m0, int n0, int kbeg,
-                                                  int kend, lds_c* sm, const int (&prow)[3],
-                                                  const int (&qrow)[2], float scale,
-                                                  v16f (&acc)[TRI ? 3 : 4], v16f (&cor)[TRI ? 3 : 4]) {
-  typedef SplitCfg<WM, WN> C;
-  constexpr int KC = C::KC;
+                                                  int kend, lds_c* sm, const SplitRows& rows, float scale,
+                                                  v16f (&acc)[C::NB], v16f (&cor)[C::NB]) {
+  constexpr bool TRI = C::SAME;
+  constexpr int STAGE = SplitCfg<C::TM / 64>::STAGE;
   constexpr int QOFF = SplitChunk<C::TM>::BYTES;
   const int lane = threadIdx.x & 63;
   typedef SplitStager<OPP, C::TM, C::NT> SP;
@@ -548,7 +590,7 @@ __device__ __forceinline__ void split_tile_rolled(const OPP& P, const OPQ& Q, in
 #pragma unroll 1
   for (int k0 = kbeg; k0 < kend; k0 += KC) {
     lds_c* const at = sm + stage;
-    stage ^= C::STAGE;
+    stage ^= STAGE;
     static_for<SP::PIECES>(
         [&](auto x) { sp.template commit<0, decltype(x)::value, ANY_K, true>(at, scale); });
     if (!TRI)
@@ -559,21 +601,19 @@ __device__ __forceinline__ void split_tile_rolled(const OPP& P, const OPQ& Q, in
       if (!TRI) sq.template fetch<0>(Q, k0 + KC, kend);
     }
     __syncthreads();       // (every wave is done with the chunk before this one: its stage is free)
-    SplitFrags<TRI> fr;
+    SplitFrags<C> fr;
 #pragma unroll
     for (int pl = 0; pl < 3; ++pl) {
 #pragma unroll
-      for (int i = 0; i < (TRI ? 3 : 2); ++i) fr.p[pl][i] = load_frag<C::TM>(at, prow[i], lane, pl);
-      if (!TRI) {
+      for (int i = 0; i < C::PF; ++i) fr.p[pl][i] = load_frag<C::TM>(at, rows.p[i], lane, pl);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) fr.q[pl][i] = load_frag<C::TN>(at + QOFF, qrow[i], lane, pl);
-      }
+      for (int i = 0; i < C::QF; ++i) fr.q[pl][i] = load_frag<C::TN>(at + QOFF, rows.q[i], lane, pl);
     }
-    static_for<6>([&](auto prod_) {
+    static_for<C::NB == 1 ? 8 : 6>([&](auto prod_) {
       constexpr int PR = decltype(prod_)::value;
-      static_for<(TRI ? 3 : 4)>([&](auto blk_) {
+      static_for<C::NB>([&](auto blk_) {
         constexpr int B = decltype(blk_)::value;
-        split_product<TRI, PR, B>(fr, PR == 0 ? acc[B] : cor[B]);
+        split_product<C, PR, B>(fr, PR == 0 ? acc[B] : cor[B]);
       });
     });
   }
@@ -587,15 +627,15 @@ __device__ __forceinline__ void split_tile_rolled(const OPP& P, const OPQ& Q, in
 // from halves of the elements, and the sums taken four times: what is finite then, is what a
 // float32 sum gives, and what is not, is not there either.  (Half of an element is exact, but for
 // a last bit of 2^-149.)  The waves vote across the barrier that ends a tile anyway.
-template <int WM, int WN, bool TRI, class OPP, class OPQ>
+template <class C, class OPP, class OPQ>
 __device__ __forceinline__ void split_blocks(const OPP& P, const OPQ& Q, int m0, int n0, int kbeg,
-                                             int kend, float* smem, const int (&prow)[3],
-                                             const int (&qrow)[2], v16f (&acc)[TRI ? 3 : 4]) {
-  typedef SplitCfg<WM, WN> C;
-  constexpr int NB = TRI ? 3 : 4;
+                                             int kend, float* smem, const SplitRows& rows,
+                                             v16f (&acc)[C::NB]) {
+  constexpr bool TRI = C::SAME;
+  constexpr int NB = C::NB;
   v16f cor[NB];
   lds_c* const sm = (lds_c*)smem;
-  lds_u* const votes = (lds_u*)(sm + C::VOTES);
+  lds_u* const votes = (lds_u*)(sm + SplitCfg<C::TM / 64>::VOTES);
   const int wave = (int)(threadIdx.x & (C::NT - 1)) >> 6;
   // (uniform per workgroup; operands in padded runs are two of a kind)
   const int mode = SplitStager<OPP, C::TM, C::NT>::fast(P, m0);
@@ -609,14 +649,14 @@ __device__ __forceinline__ void split_blocks(const OPP& P, const OPQ& Q, int m0,
   clear();
   if (kend <= kbeg) return;
   if (kend - kbeg <= SHORT_K) {
-    split_tile_rolled<WM, WN, TRI>(P, Q, m0, n0, kbeg, kend, sm, prow, qrow, 1.f, acc, cor);
+    split_tile_rolled<C>(P, Q, m0, n0, kbeg, kend, sm, rows, 1.f, acc, cor);
   } else if (mode == FAST_K && qmode == FAST_K) {
-    split_tile_loop<WM, WN, TRI, FAST_K>(P, Q, m0, n0, kbeg, kend, sm, prow, qrow, acc, cor);
+    split_tile_loop<C, FAST_K>(P, Q, m0, n0, kbeg, kend, sm, rows, acc, cor);
   } else if (has_padded_runs<OPP>::value && mode == PADDED_K) {
     if constexpr (has_padded_runs<OPP>::value)
-      split_tile_loop<WM, WN, TRI, PADDED_K>(P, Q, m0, n0, kbeg, kend, sm, prow, qrow, acc, cor);
+      split_tile_loop<C, PADDED_K>(P, Q, m0, n0, kbeg, kend, sm, rows, acc, cor);
   } else {
-    split_tile_loop<WM, WN, TRI, ANY_K>(P, Q, m0, n0, kbeg, kend, sm, prow, qrow, acc, cor);
+    split_tile_loop<C, ANY_K>(P, Q, m0, n0, kbeg, kend, sm, rows, acc, cor);
   }
   // (0 times a sum that is not finite is NaN; the third part of an element with an infinite leading
   // part is NaN, and so are all the corrections that it enters)
@@ -635,7 +675,7 @@ __device__ __forceinline__ void split_blocks(const OPP& P, const OPQ& Q, int m0,
   for (int w = 0; w < C::NT / 64; ++w) any |= votes[w];
   if (__builtin_expect(__builtin_amdgcn_readfirstlane((int)any) != 0, 0)) {
     clear();
-    split_tile_rolled<WM, WN, TRI>(P, Q, m0, n0, kbeg, kend, sm, prow, qrow, 0.5f, acc, cor);
+    split_tile_rolled<C>(P, Q, m0, n0, kbeg, kend, sm, rows, 0.5f, acc, cor);
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
       add_corrections(acc[b], cor[b]);
@@ -694,36 +734,51 @@ __device__ __forceinline__ void store_blocks(const v16f (&acc)[NB], const int (&
       put(b, [&](int i, int row, int col) { epi.store(row, col, acc[b][i]); });
 }
 
-// a tile of a product of two operands
-template <int WM, int WN, class OPP, class OPQ, class STORE>
+// a tile of a product of two operands, 64 W wide
+template <int W, class OPP, class OPQ, class STORE>
 __device__ __forceinline__ void split_tile_full(const OPP& P, const OPQ& Q, int m0, int n0, int kbeg,
                                                 int kend, float* smem, const STORE& store) {
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x & (64 * WM * WN - 1)) >> 6);
-  const int wm = (wave / WN) * 64, wn = (wave % WN) * 64;
-  const int prow[3] = {wm, wm + 32, 0}, qrow[2] = {wn, wn + 32};
-  v16f acc[4];
-  split_blocks<WM, WN, false>(P, Q, m0, n0, kbeg, kend, smem, prow, qrow, acc);
-  const int row0[4] = {m0 + wm, m0 + wm, m0 + wm + 32, m0 + wm + 32};
-  const int col0[4] = {n0 + wn, n0 + wn + 32, n0 + wn, n0 + wn + 32};
-  const int what[4] = {BLK_PLAIN, BLK_PLAIN, BLK_PLAIN, BLK_PLAIN};
-  store([&](const auto& epi) { store_blocks<4>(acc, row0, col0, what, epi); });
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x & (SplitCfg<W>::NT - 1)) >> 6);
+  const int wm = (wave >> 1) * 32 * W, wn = (wave & 1) * 32 * W;
+  if constexpr (W == 1) {
+    v16f acc[1];
+    split_blocks<SmallTile>(P, Q, m0, n0, kbeg, kend, smem, SplitRows{{wm}, {wn}}, acc);
+    const int row0[1] = {m0 + wm}, col0[1] = {n0 + wn}, what[1] = {BLK_PLAIN};
+    store([&](const auto& epi) { store_blocks<1>(acc, row0, col0, what, epi); });
+  } else {
+    v16f acc[4];
+    split_blocks<SplitTile>(P, Q, m0, n0, kbeg, kend, smem, SplitRows{{wm, wm + 32}, {wn, wn + 32}}, acc);
+    const int row0[4] = {m0 + wm, m0 + wm, m0 + wm + 32, m0 + wm + 32};
+    const int col0[4] = {n0 + wn, n0 + wn + 32, n0 + wn, n0 + wn + 32};
+    const int what[4] = {BLK_PLAIN, BLK_PLAIN, BLK_PLAIN, BLK_PLAIN};
+    store([&](const auto& epi) { store_blocks<4>(acc, row0, col0, what, epi); });
+  }
 }
 
 // a diagonal tile of a symmetric product: with `both`, the blocks above its diagonal are stored
 // at their mirror positions too
-template <class OP, class STORE>
+template <int W, class OP, class STORE>
 __device__ __forceinline__ void split_tile_tri(const OP& P, int m0, int kbeg, int kend, float* smem,
                                                bool both, const STORE& store) {
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x & (SplitCfg<2, 2>::NT - 1)) >> 6);
-  const SplitTri t = split_tri(wave);
-  const int prow[3] = {32 * t.r[0], 32 * t.r[1], 32 * t.r[2]}, qrow[2] = {0, 0};
-  v16f acc[3];
-  split_blocks<2, 2, true>(P, P, m0, m0, kbeg, kend, smem, prow, qrow, acc);
-  const int row0[3] = {m0 + prow[0], m0 + prow[0], m0 + prow[1]};
-  const int col0[3] = {m0 + prow[1], m0 + prow[2], m0 + prow[1]};
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x & (SplitCfg<W>::NT - 1)) >> 6);
   const int above = both ? BLK_BOTH : BLK_PLAIN, on = both ? BLK_UPPER_BOTH : BLK_UPPER;
-  const int what[3] = {above, t.r[0] == t.r[2] ? on : above, t.last ? on : BLK_NONE};
-  store([&](const auto& epi) { store_blocks<3>(acc, row0, col0, what, epi); });
+  if constexpr (W == 1) {
+    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+    v16f acc[1];
+    split_blocks<SmallDiag>(P, P, m0, m0, kbeg, kend, smem, SplitRows{{wm, wn}, {}}, acc);
+    const int row0[1] = {m0 + wm}, col0[1] = {m0 + wn};
+    const int what[1] = {wm == wn ? on : wm < wn ? above : (int)BLK_NONE};
+    store([&](const auto& epi) { store_blocks<1>(acc, row0, col0, what, epi); });
+  } else {
+    const SplitTri t = split_tri(wave);
+    const int r0 = 32 * t.r[0], r1 = 32 * t.r[1], r2 = 32 * t.r[2];
+    v16f acc[3];
+    split_blocks<SplitDiag>(P, P, m0, m0, kbeg, kend, smem, SplitRows{{r0, r1, r2}, {}}, acc);
+    const int row0[3] = {m0 + r0, m0 + r0, m0 + r1};
+    const int col0[3] = {m0 + r1, m0 + r2, m0 + r1};
+    const int what[3] = {above, t.r[0] == t.r[2] ? on : above, t.last ? on : (int)BLK_NONE};
+    store([&](const auto& epi) { store_blocks<3>(acc, row0, col0, what, epi); });
+  }
 }
 
 // The tile (m0, n0) of the product, 128x128 on 256 threads; `same`: P and Q describe the same
@@ -736,11 +791,11 @@ __device__ __forceinline__ void split_tile(const OPP& P, const OPQ& Q, int m0, i
   auto store = [&](auto&& put) { put(epi); };
   if constexpr (std::is_same<OPP, OPQ>::value) {
     if (same) {
-      split_tile_tri(P, m0, kbeg, kend, smem, both, store);
+      split_tile_tri<2>(P, m0, kbeg, kend, smem, both, store);
       return;
     }
   }
-  split_tile_full<2, 2>(P, Q, m0, n0, kbeg, kend, smem, store);
+  split_tile_full<2>(P, Q, m0, n0, kbeg, kend, smem, store);
 }
 
 }  // namespace kfac

@@ -41,7 +41,6 @@ __device__ __forceinline__ unsigned k_offset_or_invalid(unsigned off, bool valid
 struct DenseKM {
   static constexpr int layout = KM;
   static constexpr bool has_second = true;
-  static constexpr bool vec4 = true;
   // (the columns in memory; the optional last one is not)
   __device__ __forceinline__ int vec_cols() const { return extra ? M - 1 : M; }
   // (bytes from one k to the next)

@@ -6,29 +6,22 @@
 namespace kfac {
 
 // Tile (bi <= bj) of P^T P over one k-split: into C through `whole` where the reduction is not
-// split, else as a raw partial.  128-wide tiles run on the bf16 matrix cores (gemm_split.h),
-// 64-wide ones, a wave each, on the fp32 ones: split on its way into LDS, an operand element
-// of a 64-wide tile costs as many vector instructions as it saves matrix instructions.
+// split, else as a raw partial.  On the bf16 matrix cores (gemm_split.h).
 template <int W, class OP>
 __device__ __forceinline__ void syrk_tile(const OP& op, int bi, int bj, int kbeg, int kend,
                                           bool unsplit, const EpiStore& whole,
                                           const EpiPartial& part, float* smem) {
   constexpr int TS = 64 * W;
-  if constexpr (W == 2) {
-    auto store = [&](auto&& put) {
-      if (unsplit) put(whole);
-      else put(part);
-    };
-    if (bi == bj) split_tile_tri(op, bi * TS, kbeg, kend, smem, true, store);
-    else split_tile_full<W, W>(op, op, bi * TS, bj * TS, kbeg, kend, smem, store);
-  } else {
-    if (unsplit) gemm_tile_cfg<W, W, true>(op, op, bi * TS, bj * TS, kbeg, kend, bi == bj, whole, smem);
-    else gemm_tile_cfg<W, W, true>(op, op, bi * TS, bj * TS, kbeg, kend, bi == bj, part, smem);
-  }
+  auto store = [&](auto&& put) {
+    if (unsplit) put(whole);
+    else put(part);
+  };
+  if (bi == bj) split_tile_tri<W>(op, bi * TS, kbeg, kend, smem, true, store);
+  else split_tile_full<W>(op, op, bi * TS, bj * TS, kbeg, kend, smem, store);
 }
 template <int W>
 constexpr int syrk_lds_bytes() {
-  return W == 2 ? SplitCfg<2, 2>::SMEM_BYTES : Cfg<W, W>::SMEM_FLOATS * (int)sizeof(float);
+  return SplitCfg<W>::SMEM_BYTES;
 }
 
 // Sum the k-split partials of one tile in a fixed order and apply the epilogue
