@@ -834,6 +834,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void potrf_trail_kernel(const MatDesc*
 // 2177 -> 1922 us, and 2.5 times closer to float64 (6.7e-5 -> 2.7e-5 at 2900).
 // PMK / QMK: the operand has consecutive k next to each other (P(k, m) = p[m n + k]) instead of
 // consecutive m (p[k n + m]).
+// `fresh`: there are no old values (OLD false: known at compile time).
 // `upper`: only elements on and above the diagonal of C are stored, with `mirror` at their
 // mirror positions too (a tile on the diagonal is symmetric except for rounding).
 constexpr int STEP_THREADS = 512;
@@ -868,15 +869,16 @@ struct StepOperand {
         }
       }
     } else {
-      // (never the last block row: all 128 k are there)
       const int m = m0 + (t & 127);
       const int k = 64 * half + 8 * __builtin_amdgcn_readfirstlane(t >> 7);
       const unsigned off = m < n ? (unsigned)m * 4u : INV_M;
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-          v[8 * i + j] = buffer_load_at(rs, off, (unsigned)((k + 32 * i + j) * n) * 4u);
+        for (int j = 0; j < 8; ++j) {
+          const int at = k + 32 * i + j;
+          v[8 * i + j] = depth == DB || at < depth ? buffer_load_at(rs, off, (unsigned)(at * n) * 4u) : 0.f;
+        }
     }
   }
   __device__ __forceinline__ void commit(lds_c* at) const {
@@ -919,7 +921,7 @@ struct StepOperand {
   }
 };
 
-template <bool PMK, bool QMK>
+template <bool PMK, bool QMK, bool OLD = true>
 __device__ __forceinline__ void step_tile(const float* p, const float* q, float* C, int n, int m0,
                                           int n0, int depth, float sign, bool fresh, bool upper,
                                           bool mirror, lds_c* sm) {
@@ -977,7 +979,7 @@ __device__ __forceinline__ void step_tile(const float* p, const float* q, float*
     for (int e = 0; e < 16; ++e) {
       const int row = m0 + wm + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
       const bool in = !fresh && row < n && col < n && (!upper || row <= col);
-      old[i][e] = buffer_load(rc, in ? (unsigned)(row * n + col) * 4u : INV_M);
+      old[i][e] = OLD ? buffer_load(rc, in ? (unsigned)(row * n + col) * 4u : INV_M) : 0.f;
     }
   __syncthreads();
   products();
@@ -1079,13 +1081,14 @@ __global__ __launch_bounds__(DIAG_THREADS) void potrf_step_kernel(const MatDesc*
 constexpr int STEP_CUS = 256;
 static int step_workgroups(int nd, int tiles) { return std::min(tiles, std::max(STEP_CUS - nd, 64)); }
 
-// The row panel for launches of few tiles: the same 128x128x128 product, but by 16 waves
-// with one 32x32 block each instead of 4 waves with four.  A tile is a chain of
-// dependent-issue MFMAs, 256 per wave (7.8 us) in the tile engine and 64 here, and at the
-// end of a factorisation nothing else runs beside it.  Both operands are fetched whole (32
-// loads per thread in flight) into 128 KB of LDS.
-constexpr int FINE_THREADS = 1024;
-constexpr int FINE_SMEM_BYTES = 2 * DB * DB * (int)sizeof(float);
+// The row panel for launches of few tiles: the same 128x128x128 product as a tile beside a diagonal
+// block, one workgroup of 8 waves to a tile.  Alone it is a chain of latencies (93 tiles 12.7 us, 15.8
+// with 16 waves on the fp32 matrix instructions and both operands whole in LDS); beside the launches of
+// another stream what counts is that it fits into what one workgroup of the tile engine leaves: 98 KB
+// of LDS and 128 registers, where 128 KB had to wait for an empty compute unit, that is until the other
+// launch had handed out its last tile.
+constexpr int FINE_THREADS = STEP_THREADS;
+constexpr int FINE_SMEM_BYTES = 2 * STEP_OPERAND;
 constexpr int FINE_MAX_TILES = 256;      // one workgroup per CU
 
 // Tile `local` of row panel p.  U[p,j] = Y_pp^T A[p,j] in place for j > p, and in a sweep, after
@@ -1116,57 +1119,31 @@ __device__ __forceinline__ bool panel_tile(const MatDesc& m, int p, int local, P
   return true;
 }
 
-__global__ __launch_bounds__(FINE_THREADS) void potrf_fine_kernel(const MatDesc* table, int p,
-                                                                  const WorkList wl) {
+__global__ __launch_bounds__(FINE_THREADS, 4) void potrf_fine_kernel(const MatDesc* table, int p,
+                                                                     const WorkList wl) {
   extern __shared__ __attribute__((aligned(16))) float fsm[];
-  lds_f* const tp = (lds_f*)fsm;
-  lds_f* const tq = tp + DB * DB;
   int mat, local;
   work_find(wl, mat, local);
   const MatDesc m = table[mat];
-  const int n = m.n;
-  PanelTile pt;
-  if (!panel_tile(m, p, local, pt)) return;
-  // P(k, i) = Y_pp;  Q(k, j);  C[i][j], or C[j][i]
-  const float* P = m.Y + (size_t)p * DB * n + p * DB;
-  const int t = threadIdx.x;
-  const int wave = t >> 6, lane = t & 63;
-  const int r = lane & 31, h = lane >> 5;
-  const int wr = wave >> 2, wc = wave & 3;
-
-  const int mm = t & (DB - 1), kq = t >> 7;
-  const __amdgpu_buffer_rsrc_t rp = make_rsrc(P), rq = make_rsrc(pt.q);
-  float vp[16], vq[16];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const unsigned off = (unsigned)((kq + 8 * i) * n + mm) * 4u;
-    const bool in = kq + 8 * i < pt.rows;
-    vp[i] = buffer_load(rp, in && mm < pt.rows ? off : INV_M);
-    vq[i] = buffer_load(rq, in && mm < pt.cols ? off : INV_M);
-  }
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    tp[(kq + 8 * i) * DB + mm] = vp[i];
-    tq[(kq + 8 * i) * DB + mm] = vq[i];
-  }
-  __syncthreads();
-  // (the transposed result comes from the exchanged operands: rows j, and lanes along i)
-  const lds_f* const left = pt.z ? tq : tp;
-  const lds_f* const right = pt.z ? tp : tq;
-  const int nrow = pt.z ? pt.cols : pt.rows, ncol = pt.z ? pt.rows : pt.cols;
-  const v16f acc = lds_mma32(left + 32 * wr, DB, 1, right + 32 * wc, DB, 1, DB);
-#pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    const int row = 32 * wr + 8 * (e >> 2) + 4 * h + (e & 3), col = 32 * wc + r;
-    if (row < nrow && col < ncol) pt.c[(size_t)row * n + col] = acc[e];
+  const int n = m.n, row0 = p * DB, right = m.T - p - 1;
+  const float* const y = m.Y + (size_t)row0 * n;
+  if (local < right) {
+    step_tile<false, false, false>(y, m.U + (size_t)row0 * n, m.U, n, row0, (p + 1 + local) * BM, DB,
+                                   1.f, true, false, false, (lds_c*)fsm);
+  } else if (local - right < p) {
+    // (the transposed result comes from the exchanged operands)
+    step_tile<false, false, false>(y, y, m.Y, n, (local - right) * BM, row0, min(DB, n - row0), 1.f,
+                                   true, false, false, (lds_c*)fsm);
   }
 }
 
 // The same product for launches of very few tiles (at most SUB_MAX_TILES): every tile is
 // dealt to four workgroups, so that four CUs' matrix cores work on it.  The row panel
 // overwrites its own right-hand operand, so the pieces must not share columns: four
-// 128x32 column strips, four 32x32 blocks each.  8 waves: a wave does one block over half
-// of the 128-deep reduction and the halves are added through LDS.
+// 128x32 column strips, four 32x32 blocks each.  8 waves: the blocks' reductions, 32 to 128 deep
+// since Y_pp is triangular, are cut at 64 k, and the two parts of the longer ones are added through
+// LDS.  (All of them 128 deep, a half to a wave: 1153 us where this takes 1144, inverse and Cholesky
+// factor of 2305^2.)
 constexpr int SUB_THREADS = 512;
 constexpr int SUB_SMEM_BYTES = DB * (128 + 32) * (int)sizeof(float);
 constexpr int SUB_MAX_TILES = 64;        // 4 workgroups per tile, one workgroup per CU
@@ -1186,9 +1163,13 @@ __global__ __launch_bounds__(SUB_THREADS) void potrf_sub_kernel(const MatDesc* t
   if (!panel_tile(m, p, local, pt)) return;
   const float* P = m.Y + (size_t)p * DB * n + p * DB;
   const int t = threadIdx.x;
-  const int wave = t >> 6, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
   const int r = lane & 31, h = lane >> 5;
-  const int br = wave & 3, khalf = wave >> 2;
+  // block row br (k < 32 (br + 1): Y_pp is zero below its diagonal) and the wave's part of its
+  // reduction; waves w and w + 4 share a SIMD, so no SIMD has more than 96 k
+  // (a digit per wave: br = 3 3 2 1 0 2 - -, kbeg = 0 64 0 0 0 64 - -, kn = 64 64 64 64 32 32 0 0)
+  const int br = (0x00201233 >> (4 * wave)) & 15, kbeg = ((0x22 >> wave) & 1) * 64,
+            kn = ((0x00112222 >> (4 * wave)) & 15) * 32;
   const int row0 = 32 * br, col0 = WQ * sj;         // of this wave's block in the tile (U[p,j])
 
   const __amdgpu_buffer_rsrc_t rp = make_rsrc(P), rq = make_rsrc(pt.q);
@@ -1197,7 +1178,7 @@ __global__ __launch_bounds__(SUB_THREADS) void potrf_sub_kernel(const MatDesc* t
   for (int i = 0; i < WP / 4; ++i) {
     const int idx = t + SUB_THREADS * i;
     const int k = idx / WP, col = idx % WP;
-    vp[i] = buffer_load(rp, k < pt.rows && col < pt.rows ? (unsigned)(k * n + col) * 4u : INV_M);
+    vp[i] = buffer_load(rp, k <= (col | 31) && k < pt.rows && col < pt.rows ? (unsigned)(k * n + col) * 4u : INV_M);
   }
 #pragma unroll
   for (int i = 0; i < WQ / 4; ++i) {
@@ -1210,24 +1191,25 @@ __global__ __launch_bounds__(SUB_THREADS) void potrf_sub_kernel(const MatDesc* t
 #pragma unroll
   for (int i = 0; i < WQ / 4; ++i) tq[t + SUB_THREADS * i] = vq[i];
   __syncthreads();
-  const lds_f* const bp = tp + 64 * khalf * WP + 32 * br;
-  const lds_f* const bq = tq + 64 * khalf * WQ;
+  const lds_f* const bp = tp + kbeg * WP + row0;
+  const lds_f* const bq = tq + kbeg * WQ;
   // (the transposed result comes from the exchanged operands: rows j, and lanes along i)
-  const v16f acc = lds_mma32(pt.z ? bq : bp, pt.z ? WQ : WP, 1, pt.z ? bp : bq, pt.z ? WP : WQ, 1, 64);
+  v16f acc;
+  if (kn > 0) acc = lds_mma32(pt.z ? bq : bp, pt.z ? WQ : WP, 1, pt.z ? bp : bq, pt.z ? WP : WQ, 1, kn);
   __syncthreads();
-  // the second halves of the reduction travel through LDS (the operands are spent)
+  // the second parts of the reduction travel through LDS (the operands are spent)
   lds_f* const red = tp + br * 1024;
-  if (khalf == 1) {
+  if (kbeg > 0) {
 #pragma unroll
     for (int e = 0; e < 16; ++e) red[e * 64 + lane] = acc[e];
   }
   __syncthreads();
-  if (khalf == 0) {
+  if (kbeg == 0 && kn > 0) {
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
       const int at = 8 * (e >> 2) + 4 * h + (e & 3);
       const int row = (pt.z ? col0 : row0) + at, col = (pt.z ? row0 : col0) + r;
-      const float v = acc[e] + red[e * 64 + lane];
+      const float v = br >= 2 ? acc[e] + red[e * 64 + lane] : acc[e];
       if (row < (pt.z ? pt.cols : pt.rows) && col < (pt.z ? pt.rows : pt.cols))
         pt.c[(size_t)row * n + col] = v;
     }
