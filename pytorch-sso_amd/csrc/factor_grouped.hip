@@ -122,51 +122,84 @@ __global__ __launch_bounds__(256) void reduce_tile_grouped_kernel(const RdJob* _
 // One convolution input and its copy in planes (see ConvP).  Only the row phases that
 // some kernel tap reads are written (a 1x1 convolution of stride 2 reads one of two).
 constexpr int MAX_PLANES = 32;
-constexpr int PLANE_ITEM = 8192;      // elements of the copy per workgroup
+constexpr int PLANE_ITEM = 16384;     // elements of the copy per workgroup, at most
+constexpr int PLANE_LDS = 4096;       // elements of the input per workgroup, at most
 struct PlaneJob {
   const float* x;
   float* out;
-  int C, H, W, sh, sw, ph, pw, dw, KW, Hs, OW, nused, chunks, ones, image;
-  FastDiv by_ow, by_area, by_chunks, by_c;
+  int C, H, W, sh, sw, ph, pw, dw, KW, Hs, OW, nused, band, chunks, ones, image;
+  FastDiv by_ow, by_band, by_chunks, by_c;
   unsigned char used[MAX_PLANES];     // ry * KW + kw of the planes to write
 };
 
-// item = (channel image (n, c), chunk of its used planes): PLANE_ITEM elements, in order
+// item = (channel image (n, c), band of rows [ys0, ys0 + band) of all its used planes).  Row ys of the
+// planes with row phase ry is row ys * sh + ry - ph of the input, so a band reads one run of whole
+// rows: it comes into LDS once, in order, and every plane's part of the band is written from there in
+// order.  Bound by memory, and for small images by the workgroups' own latency; 32 images, copies of
+// element by element from global memory (each read once per kernel column, with a stride) / this:
+// the stem's 7x7 over 3x224x224 and 3x3 of stride 2 over 128x56x56 79.5 / 46.0 us (220 MB moved),
+// 3x3 of stride 2 over 256x28x28 28.4 / 22.8, over 512x14x14 27.4 / 25.7.
+// Where a row of every phase does not fit (sh * W > PLANE_LDS) the elements come from global memory.
 __global__ __launch_bounds__(256) void conv_planes_kernel(const PlaneJob* __restrict__ jobs,
                                                           const int* __restrict__ cum, int njobs) {
+  __shared__ float rows[PLANE_LDS];
+  __shared__ int4 planes_of[MAX_PLANES];       // output offset, first input row, first input column
   const int j = find_job(cum, njobs, blockIdx.x);
   const PlaneJob& jb = jobs[j];
   const int local = blockIdx.x - cum[j];
   const int img = jb.by_chunks.div(local);
   const int chunk = local - img * jb.chunks;
   const int n = jb.by_c.div(img), c = img - n * jb.C;
-  const int H = jb.H, W = jb.W, OW = jb.OW, area = jb.Hs * OW, planes = jb.sh * jb.KW;
+  const int H = jb.H, W = jb.W, OW = jb.OW, sh = jb.sh, sw = jb.sw;
+  const int area = jb.Hs * OW, planes = sh * jb.KW;
   const float* __restrict__ src = jb.x + (size_t)img * H * W;
   float* __restrict__ dst = jb.out + (size_t)n * jb.image + (size_t)c * planes * area;
-  const int total = jb.nused * area;
-  const int e1 = min(total, (chunk + 1) * PLANE_ITEM);
-  // four elements per thread and trip, so that four loads are in flight
-  for (int e0 = chunk * PLANE_ITEM + threadIdx.x; e0 < e1; e0 += 4 * 256) {
-    float v[4];
-    int at[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int e = e0 + 256 * q;
-      const int u = jb.by_area.div(e);
-      const int idx = e - u * area;
-      const int plane = jb.used[u & (MAX_PLANES - 1)];
-      const int ry = plane / jb.KW, kw = plane - ry * jb.KW;
-      const int ys = jb.by_ow.div(idx);
-      const int ow = idx - ys * OW;
-      const int y = ys * jb.sh + ry - jb.ph, x = ow * jb.sw + kw * jb.dw - jb.pw;
-      const bool in = e < e1 && (unsigned)y < (unsigned)H && (unsigned)x < (unsigned)W;
-      at[q] = e < e1 ? plane * area + idx : -1;
-      v[q] = in ? src[y * W + x] : 0.f;
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      if (at[q] >= 0) dst[at[q]] = v[q];
+  const int ys0 = chunk * jb.band, count = jb.band * OW;
+  const int left = area - ys0 * OW;              // elements of a plane from row ys0 on
+  const int y0 = max(ys0 * sh - jb.ph, 0), y1 = min((ys0 + jb.band) * sh - jb.ph, H);
+  const bool staged = jb.band * sh * W <= PLANE_LDS;
+  if (threadIdx.x < jb.nused) {
+    const int plane = jb.used[threadIdx.x];
+    const int ry = plane / jb.KW, kw = plane - ry * jb.KW;
+    planes_of[threadIdx.x] = int4{plane * area + ys0 * OW, ys0 * sh + ry - jb.ph, kw * jb.dw - jb.pw, 0};
   }
+  if (staged) {
+    const int size = (y1 - y0) * W;
+    const float* __restrict__ from = src + (size_t)y0 * W;
+    for (int e0 = threadIdx.x; e0 < size; e0 += 8 * 256) {
+      float v[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) v[q] = e0 + 256 * q < size ? from[e0 + 256 * q] : 0.f;
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        if (e0 + 256 * q < size) rows[e0 + 256 * q] = v[q];
+    }
+  }
+  __syncthreads();
+  const int total = jb.nused * count;
+  auto write = [&](auto&& element) {
+    for (int e0 = threadIdx.x; e0 < total; e0 += 4 * 256) {
+      float v[4];
+      int at[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int e = min(e0 + 256 * q, total - 1);
+        const int u = jb.by_band.div(e);
+        const int idx = e - u * count;
+        const int4 pl = planes_of[u];
+        const int ys = jb.by_ow.div(idx);
+        const int y = ys * sh + pl.y, x = (idx - ys * OW) * sw + pl.z;
+        at[q] = e0 + 256 * q < total && idx < left ? pl.x + idx : -1;
+        const bool in = at[q] >= 0 && (unsigned)y < (unsigned)H && (unsigned)x < (unsigned)W;
+        v[q] = in ? element(y, x) : 0.f;
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (at[q] >= 0) dst[at[q]] = v[q];
+    }
+  };
+  if (staged) write([&](int y, int x) { return rows[(y - y0) * W + x]; });
+  else write([&](int y, int x) { return src[(size_t)y * W + x]; });
   if (jb.ones && c == 0 && chunk == 0) {
     float* __restrict__ one = jb.out + (size_t)n * jb.image + (size_t)jb.C * planes * area;
     for (int idx = threadIdx.x; idx < jb.ones; idx += 256) one[idx] = 1.f;
@@ -622,11 +655,13 @@ static Launch fill_planes(TableWriter& tw, const GroupedPlan& gp, const kfac_fac
       for (int kw = 0; kw < j.kw && seen[ry]; ++kw)
         pj.used[pj.nused++] = (unsigned char)(ry * j.kw + kw);
     const int area = c.Hs * c.OW;
-    pj.chunks = cdiv(pj.nused * area, PLANE_ITEM);
+    pj.band = std::min(c.Hs, std::max(1, PLANE_ITEM / (pj.nused * c.OW)));
+    if (j.sh * j.W <= PLANE_LDS) pj.band = std::min(pj.band, PLANE_LDS / (j.sh * j.W));
+    pj.chunks = cdiv(c.Hs, pj.band);
     pj.ones = j.add_bias ? c.OH * c.OW : 0;
     pj.image = j.c * j.sh * j.kw * area + pj.ones;
     pj.by_ow = FastDiv((unsigned)c.OW);
-    pj.by_area = FastDiv((unsigned)area);
+    pj.by_band = FastDiv((unsigned)(pj.band * c.OW));
     pj.by_chunks = FastDiv((unsigned)pj.chunks);
     pj.by_c = FastDiv((unsigned)j.c);
     tab.push_back(pj);
