@@ -124,22 +124,26 @@ __global__ __launch_bounds__(256) void reduce_tile_grouped_kernel(const RdJob* _
 constexpr int MAX_PLANES = 32;
 constexpr int PLANE_ITEM = 16384;     // elements of the copy per workgroup, at most
 constexpr int PLANE_LDS = 4096;       // elements of the input per workgroup, at most
+constexpr int PLANE_GROUP = 4096;     // elements of the copies of several small images, at most
 struct PlaneJob {
   const float* x;
   float* out;
-  int C, H, W, sh, sw, ph, pw, dw, KW, Hs, OW, nused, band, chunks, ones, image;
-  FastDiv by_ow, by_band, by_chunks, by_c;
+  int C, H, W, sh, sw, ph, pw, dw, KW, Hs, OW, nused, band, staged, chunks, group, groups, ones, image;
+  FastDiv by_ow, by_band, by_image, by_chunks, by_groups;
   unsigned char used[MAX_PLANES];     // ry * KW + kw of the planes to write
 };
 
-// item = (channel image (n, c), band of rows [ys0, ys0 + band) of all its used planes).  Row ys of the
-// planes with row phase ry is row ys * sh + ry - ph of the input, so a band reads one run of whole
-// rows: it comes into LDS once, in order, and every plane's part of the band is written from there in
-// order.  Bound by memory, and for small images by the workgroups' own latency; 32 images, copies of
-// element by element from global memory (each read once per kernel column, with a stride) / this:
-// the stem's 7x7 over 3x224x224 and 3x3 of stride 2 over 128x56x56 79.5 / 46.0 us (220 MB moved),
-// 3x3 of stride 2 over 256x28x28 28.4 / 22.8, over 512x14x14 27.4 / 25.7.
-// Where a row of every phase does not fit (sh * W > PLANE_LDS) the elements come from global memory.
+// item = (channel image (n, c), band of rows [ys0, ys0 + band) of all its used planes), or several whole
+// images where they are small.  Row ys of the planes with row phase ry is row ys * sh + ry - ph of the
+// input, so a band reads one run of whole rows: it comes into LDS once, in order, and every plane's part
+// of the band is written from there in order.  Bound by memory, and for small images by the workgroups'
+// own latency; 32 images, copies of element by element from global memory (each read once per kernel
+// column, with a stride) / this with an image to an item / this:
+//   the stem's 7x7 over 3x224x224 and 3x3 of stride 2 over 128x56x56   79.5 / 46.0 us (220 MB moved)
+//   3x3 over 256x28x28 28.4 / 22.8 us, with the 1x1 over 512x28x28     38.6 / 31.1
+//   3x3 over 512x14x14 27.4 / 25.7 us, with the 1x1 over 1024x14x14    52.8 / 19.6
+// Where a row of every phase does not fit (sh * W > PLANE_LDS), or one plane is all there is, each element
+// being read once anyway (a pointwise convolution), the elements come from global memory.
 __global__ __launch_bounds__(256) void conv_planes_kernel(const PlaneJob* __restrict__ jobs,
                                                           const int* __restrict__ cum, int njobs) {
   __shared__ float rows[PLANE_LDS];
@@ -147,24 +151,25 @@ __global__ __launch_bounds__(256) void conv_planes_kernel(const PlaneJob* __rest
   const int j = find_job(cum, njobs, blockIdx.x);
   const PlaneJob& jb = jobs[j];
   const int local = blockIdx.x - cum[j];
-  const int img = jb.by_chunks.div(local);
-  const int chunk = local - img * jb.chunks;
-  const int n = jb.by_c.div(img), c = img - n * jb.C;
+  const int gi = jb.by_chunks.div(local);
+  const int chunk = local - gi * jb.chunks;
+  const int n = jb.by_groups.div(gi), c = (gi - n * jb.groups) * jb.group;
+  const int images = min(jb.group, jb.C - c);
   const int H = jb.H, W = jb.W, OW = jb.OW, sh = jb.sh, sw = jb.sw;
   const int area = jb.Hs * OW, planes = sh * jb.KW;
-  const float* __restrict__ src = jb.x + (size_t)img * H * W;
+  const float* __restrict__ src = jb.x + ((size_t)n * jb.C + c) * H * W;
   float* __restrict__ dst = jb.out + (size_t)n * jb.image + (size_t)c * planes * area;
   const int ys0 = chunk * jb.band, count = jb.band * OW;
   const int left = area - ys0 * OW;              // elements of a plane from row ys0 on
   const int y0 = max(ys0 * sh - jb.ph, 0), y1 = min((ys0 + jb.band) * sh - jb.ph, H);
-  const bool staged = jb.band * sh * W <= PLANE_LDS;
+  const bool staged = jb.staged;
   if (threadIdx.x < jb.nused) {
     const int plane = jb.used[threadIdx.x];
     const int ry = plane / jb.KW, kw = plane - ry * jb.KW;
     planes_of[threadIdx.x] = int4{plane * area + ys0 * OW, ys0 * sh + ry - jb.ph, kw * jb.dw - jb.pw, 0};
   }
   if (staged) {
-    const int size = (y1 - y0) * W;
+    const int size = jb.group > 1 ? images * H * W : (y1 - y0) * W;
     const float* __restrict__ from = src + (size_t)y0 * W;
     for (int e0 = threadIdx.x; e0 < size; e0 += 8 * 256) {
       float v[8];
@@ -176,7 +181,7 @@ __global__ __launch_bounds__(256) void conv_planes_kernel(const PlaneJob* __rest
     }
   }
   __syncthreads();
-  const int total = jb.nused * count;
+  const int per_image = jb.nused * count, total = images * per_image;
   auto write = [&](auto&& element) {
     for (int e0 = threadIdx.x; e0 < total; e0 += 4 * 256) {
       float v[4];
@@ -184,22 +189,23 @@ __global__ __launch_bounds__(256) void conv_planes_kernel(const PlaneJob* __rest
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int e = min(e0 + 256 * q, total - 1);
-        const int u = jb.by_band.div(e);
-        const int idx = e - u * count;
+        const int g = jb.by_image.div(e);
+        const int u = jb.by_band.div(e - g * per_image);
+        const int idx = e - g * per_image - u * count;
         const int4 pl = planes_of[u];
         const int ys = jb.by_ow.div(idx);
         const int y = ys * sh + pl.y, x = (idx - ys * OW) * sw + pl.z;
-        at[q] = e0 + 256 * q < total && idx < left ? pl.x + idx : -1;
+        at[q] = e0 + 256 * q < total && idx < left ? g * planes * area + pl.x + idx : -1;
         const bool in = at[q] >= 0 && (unsigned)y < (unsigned)H && (unsigned)x < (unsigned)W;
-        v[q] = in ? element(y, x) : 0.f;
+        v[q] = in ? element(g * H, y, x) : 0.f;
       }
 #pragma unroll
       for (int q = 0; q < 4; ++q)
         if (at[q] >= 0) dst[at[q]] = v[q];
     }
   };
-  if (staged) write([&](int y, int x) { return rows[(y - y0) * W + x]; });
-  else write([&](int y, int x) { return src[(size_t)y * W + x]; });
+  if (staged) write([&](int g, int y, int x) { return rows[(g + y - y0) * W + x]; });
+  else write([&](int g, int y, int x) { return src[(size_t)(g + y) * W + x]; });
   if (jb.ones && c == 0 && chunk == 0) {
     float* __restrict__ one = jb.out + (size_t)n * jb.image + (size_t)jb.C * planes * area;
     for (int idx = threadIdx.x; idx < jb.ones; idx += 256) one[idx] = 1.f;
@@ -307,9 +313,10 @@ static Classified classify_shape(const kfac_factor_job& j) {
     c.Hs = c.OH + (j.kh - 1) * j.dh / j.sh;
     const int64_t copy =
         j.rows * ((int64_t)j.c * j.sh * j.kw * c.Hs * c.OW + (bias ? c.OH * c.OW : 0)) * 4;
-    // (a pointwise convolution with a stride reads so little per product that the copy
-    // costs more than the bounds tests)
-    if (j.kh * j.kw > 1 && j.sh * j.kw <= MAX_PLANES && copy <= MAX_OPERAND_BYTES) {
+    // (pointwise: with a stride, too; three layers of a ResNet-50 139 us with bounds tests, 41 TFLOP/s,
+    // and 45 to 80 with the copy, which shares its launches with those of the k x k layers.  Without one,
+    // that is with padding or a bias, the copy would be of the whole input for the sake of its edge)
+    if ((j.kh * j.kw > 1 || j.sh * j.sw > 1) && j.sh * j.kw <= MAX_PLANES && copy <= MAX_OPERAND_BYTES) {
       c.path = P_CONVP;
       // (a k x 1 kernel, stride 1, no padding, no bias: one plane, Hs = H, OW = W)
       const bool as_is =
@@ -656,17 +663,26 @@ static Launch fill_planes(TableWriter& tw, const GroupedPlan& gp, const kfac_fac
         pj.used[pj.nused++] = (unsigned char)(ry * j.kw + kw);
     const int area = c.Hs * c.OW;
     pj.band = std::min(c.Hs, std::max(1, PLANE_ITEM / (pj.nused * c.OW)));
-    if (j.sh * j.W <= PLANE_LDS) pj.band = std::min(pj.band, PLANE_LDS / (j.sh * j.W));
+    pj.staged = pj.nused > 1 && j.sh * j.W <= PLANE_LDS;
+    if (pj.staged) pj.band = std::min(pj.band, PLANE_LDS / (j.sh * j.W));
     pj.chunks = cdiv(c.Hs, pj.band);
+    pj.group = 1;
+    if (pj.chunks == 1) {
+      int most = PLANE_GROUP / (pj.nused * area);
+      if (pj.staged) most = std::min(most, PLANE_LDS / (j.H * j.W));
+      pj.group = std::max(1, std::min(j.c, most));
+    }
+    pj.groups = cdiv(j.c, pj.group);
     pj.ones = j.add_bias ? c.OH * c.OW : 0;
     pj.image = j.c * j.sh * j.kw * area + pj.ones;
     pj.by_ow = FastDiv((unsigned)c.OW);
     pj.by_band = FastDiv((unsigned)(pj.band * c.OW));
     pj.by_chunks = FastDiv((unsigned)pj.chunks);
-    pj.by_c = FastDiv((unsigned)j.c);
+    pj.by_groups = FastDiv((unsigned)pj.groups);
+    pj.by_image = FastDiv((unsigned)(pj.nused * pj.band * c.OW));
     tab.push_back(pj);
     cum.push_back(items);
-    items += (int)j.rows * j.c * pj.chunks;
+    items += (int)j.rows * pj.groups * pj.chunks;
   }
   cum.push_back(items);
   Launch l;

@@ -1,5 +1,6 @@
 """Padded copies of a convolution's input in planes (factors of strided or padded k x k layers): bands
-of rows with a remainder, rows that do not fit into LDS, phases and columns outside of the image.
+of rows with a remainder, rows that do not fit into LDS, phases and columns outside of the image,
+several small images to a workgroup.
 Small whole numbers, so that every product and sum is exact and the factors have to be equal."""
 import pytest
 import torch
@@ -15,6 +16,10 @@ CASES = [   # input, kernel, stride, padding, dilation, bias
     ((1, 1, 70, 300), (3, 2), (14, 3), (2, 1), (1, 1), False),     # a row of all phases does not
     ((2, 2, 33, 21), (5, 3), (3, 2), (4, 2), (2, 3), True),        # dilated, wide padding
     ((1, 2, 3, 2), (5, 5), (2, 2), (4, 4), (1, 1), False),         # bands that lie in the padding
+    ((2, 37, 9, 9), (1, 1), (2, 2), (0, 0), (1, 1), False),        # pointwise with a stride, one row phase
+    ((3, 201, 6, 5), (1, 1), (2, 3), (0, 0), (1, 1), False),       # several images an item, with a remainder
+    ((2, 53, 11, 10), (3, 3), (2, 2), (1, 1), (1, 1), True),       # ... through LDS
+    ((2, 3, 70, 90), (1, 1), (3, 2), (1, 0), (1, 1), True),        # ... padded, with a bias
     ((1, 1, 400, 3), (2, 3), (2, 1), (0, 1), (1, 1), True),        # one pixel column of a stride, tall
 ]
 
