@@ -15,7 +15,8 @@
 //   XCD (own L2) walks a contiguous run of (split, tile) pairs, tile fastest, as in
 //   the single-product kernel.
 //
-// The input factor of a convolution that is not pointwise reads a copy of its input:
+// The input factor of a convolution that is not pointwise (and of one with a stride that is,
+// beside others in a call) reads a copy of its input:
 // zero-padded, one plane per row phase of the stride and per kernel column
 // (conv_planes_kernel, one launch for all such products of the call).  The operand then
 // needs no bounds test and reads consecutive addresses along the reduction.
@@ -267,7 +268,7 @@ struct Classified {
   int positions;         // P_CONVG, P_CONVP: index positions of an image (see padded_run)
 };
 
-static Classified classify_shape(const kfac_factor_job& j) {
+static Classified classify_shape(const kfac_factor_job& j, bool copy_pointwise) {
   Classified c{P_BAD, 0, 0, 0, 0, 0, 0, 0};
   if (j.rows <= 0 || j.c <= 0) return c;
   const int bias = j.add_bias ? 1 : 0;
@@ -313,10 +314,12 @@ static Classified classify_shape(const kfac_factor_job& j) {
     c.Hs = c.OH + (j.kh - 1) * j.dh / j.sh;
     const int64_t copy =
         j.rows * ((int64_t)j.c * j.sh * j.kw * c.Hs * c.OW + (bias ? c.OH * c.OW : 0)) * 4;
-    // (pointwise: with a stride, too; three layers of a ResNet-50 139 us with bounds tests, 41 TFLOP/s,
-    // and 45 to 80 with the copy, which shares its launches with those of the k x k layers.  Without one,
-    // that is with padding or a bias, the copy would be of the whole input for the sake of its edge)
-    if ((j.kh * j.kw > 1 || j.sh * j.sw > 1) && j.sh * j.kw <= MAX_PLANES && copy <= MAX_OPERAND_BYTES) {
+    // (pointwise: with a stride, in a call that copies other inputs anyway, whose launches it then
+    // shares.  Three layers of a ResNet-50 beside its 3x3 ones: 139 us with bounds tests, 41 TFLOP/s, 22 us of
+    // copies and 14 of products with it.  Without a stride, that is with padding or a bias, the copy
+    // would be of the whole input for the sake of its edge)
+    const bool wanted = j.kh * j.kw > 1 || (copy_pointwise && j.sh * j.sw > 1);
+    if (wanted && j.sh * j.kw <= MAX_PLANES && copy <= MAX_OPERAND_BYTES) {
       c.path = P_CONVP;
       // (a k x 1 kernel, stride 1, no padding, no bias: one plane, Hs = H, OW = W)
       const bool as_is =
@@ -328,8 +331,8 @@ static Classified classify_shape(const kfac_factor_job& j) {
 }
 
 // ... and the reduction index of products in runs, on 128-wide tiles with padded runs
-static Classified classify(const kfac_factor_job& j) {
-  Classified c = classify_shape(j);
+static Classified classify(const kfac_factor_job& j, bool copy_pointwise) {
+  Classified c = classify_shape(j, copy_pointwise);
   if (c.path != P_CONVG && c.path != P_CONVP) return c;
   const int run = c.path == P_CONVG ? j.H * j.W : c.OH * c.OW;
   c.positions = padded_run(run);
@@ -403,8 +406,11 @@ static GroupedPlan make_plan(int count, const kfac_factor_job* jobs) {
   gp.plans.resize(count);
   gp.partial_off.assign(count, 0);
   gp.copy_off.assign(count, 0);
+  bool copy_pointwise = false;
+  for (int i = 0; i < count && !copy_pointwise; ++i)
+    copy_pointwise = classify_shape(jobs[i], false).copy_bytes > 0;
   for (int i = 0; i < count; ++i) {
-    const Classified c = classify(jobs[i]);
+    const Classified c = classify(jobs[i], copy_pointwise);
     gp.cls[i] = c;
     if (c.path == P_BAD) {
       gp.ok = false;

@@ -40,5 +40,11 @@ def test_factor_equals_unfolded_product(shape, kernel, stride, padding, dilation
     xd = x.to(dev)
     job = _ops.factor_job('conv_a', xd, 1., out, add_bias=bias, kernel_size=kernel, stride=stride,
                           padding=padding, dilation=dilation)
+    # (a pointwise layer reads a copy in a call that makes others)
+    other = torch.full((9, 9), float('nan'), device=dev)
+    zeros = torch.zeros(1, 1, 5, 5, device=dev)
+    _ops.factor_grouped([job, _ops.factor_job('conv_a', zeros, 1., other, kernel_size=3, stride=2)], dev)
+    assert torch.equal(out.double().cpu(), ref) and not other.any().item()
+    out.fill_(float('nan'))
     _ops.factor_grouped([job], dev)
     assert torch.equal(out.double().cpu(), ref)
