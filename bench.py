@@ -37,9 +37,9 @@ sys.path.insert(0, os.path.join(ROOT, 'pytorch-sso_amd'))
 sys.path.insert(0, ROOT)
 
 METRIC = 'K-FAC step ms (factor+invert+precondition) & fp32 MFMA TFLOP/s, 1 MI355X'
-# Ceiling of float32 products: 128-wide tiles run as six bf16 matrix products each
-# (csrc/gemm_split.h), of 2500 dense bf16 TFLOP/s.  (The 64-wide tiles and the diagonal blocks use the
-# fp32 matrix instructions, 157.3 TFLOP/s; they are priced against the same ceiling.)
+# Ceiling of float32 products: tiles run as six bf16 matrix products each (csrc/gemm_split.h), of
+# 2500 dense bf16 TFLOP/s.  (The diagonal blocks use the fp32 matrix instructions, 157.3 TFLOP/s; they
+# are priced against the same ceiling.)
 PEAK_PRODUCT_TFLOPS = 2500. / 6.
 # rocprofv3 --pmc readings of the factor-build kernels of a resnet50 step, kept with the
 # profile summary they come from (counter runs cannot be made from inside this script):
