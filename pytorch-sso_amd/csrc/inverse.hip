@@ -30,6 +30,7 @@
 #include <vector>
 
 #include "common.h"
+#include "diag_schedule.h"
 #include "operands.h"
 
 namespace kfac {
@@ -134,10 +135,12 @@ __global__ __launch_bounds__(256) void inv_copy_damp_kernel(const MatDesc* table
 constexpr int DB = 128;          // diagonal block size
 constexpr int DLD = DB + 4;      // LDS leading dimension (rows of 16-byte pieces)
 // S and Z; what the steps of the strips leave; the A operands of one strip; marks by strip and block
-// column; write items taken
+// column, and of the waves that applied a pending panel; write items taken
 constexpr int DIAG_STEPS = 4 * 16 * 4;
 constexpr int DIAG_OPS = 16 * 64;
-constexpr int DIAG_MARKS = 4 * 8 * 8;
+constexpr int STRIP_MARKS = 4 * 8 * 8;
+constexpr int DIAG_MARKS = STRIP_MARKS + 16;
+static_assert(PENDING_WAVES <= 16, "a mark for each");
 constexpr int DIAG_SMEM_BYTES = (2 * DB * DLD + DIAG_STEPS + DIAG_OPS + DIAG_MARKS + 4) * (int)sizeof(float);
 
 __device__ __forceinline__ float lane_value(float v, int src_lane) {
@@ -375,49 +378,6 @@ __device__ __forceinline__ void collect(v16f& N, const Rows r0, v16f& M, const R
   }
 }
 
-// Which wave does what in strip q.  Block columns: 1-3 of S (the row panel), 4-7 = 0-3 of Z.
-//   LEAD: the leaf;  FOLLOW c: the block of column c;  COLLECT c: what strip q takes from the block
-//   of column c in strip q+1, which that wave then follows, or leads, with;  HELP: the rest.
-// A SIMD has the waves s, s+4, s+8 and issues one instruction at a time to its matrix core or its
-// vector unit; of a step, the leading wave takes it 160 cycles, a following one 90, a collecting
-// one 70, and a helper 1400 cycles for a block.  So the leading wave has no following one beside
-// it, and every SIMD has about the same to do:
-//   SIMD      0               1                     2                    3
-//   strip 0   lead, C4, H     F1, C1, H             F2, C2, H            F3, C3, F4
-//   strip 1   C4, F4, F5      lead, C5, H (1)       C2, F2, H (2)        C3, F3, H (2 blocks)
-//   strip 2   F4, C4, C5      F6, F5, C6            lead, H, H (2)       F3, C3, H (1)
-//   strip 3   F4, F5          F6, H                 F7, H, H             lead
-enum { ROLE_NONE = 0, ROLE_LEAD = 1, ROLE_FOLLOW = 2, ROLE_COLLECT = 3, ROLE_HELP = 4 };
-constexpr int STRIP_HELPERS = 3;
-struct StripRoles {
-  unsigned long long bits = 0;      // 5 bits a wave
-  static constexpr unsigned long long code(int kind, int c) {
-    return kind == ROLE_LEAD ? 1 : kind == ROLE_HELP ? 2 + c : kind == ROLE_FOLLOW ? 8 + c
-           : kind == ROLE_COLLECT ? 16 + c : 0;
-  }
-  constexpr StripRoles& set(int wave, int kind, int c = 0) {
-    bits |= code(kind, c) << (5 * wave);
-    return *this;
-  }
-};
-constexpr unsigned long long STRIP_ROLES[4] = {
-    StripRoles().set(0, ROLE_LEAD).set(4, ROLE_COLLECT, 4).set(8, ROLE_HELP, 0)
-        .set(1, ROLE_FOLLOW, 1).set(5, ROLE_COLLECT, 1).set(9, ROLE_HELP, 1)
-        .set(2, ROLE_FOLLOW, 2).set(10, ROLE_COLLECT, 2).set(6, ROLE_HELP, 2)
-        .set(3, ROLE_FOLLOW, 3).set(7, ROLE_COLLECT, 3).set(11, ROLE_FOLLOW, 4).bits,
-    StripRoles().set(0, ROLE_COLLECT, 4).set(4, ROLE_FOLLOW, 4).set(8, ROLE_FOLLOW, 5)
-        .set(5, ROLE_LEAD).set(9, ROLE_COLLECT, 5).set(1, ROLE_HELP, 0)
-        .set(2, ROLE_COLLECT, 2).set(10, ROLE_FOLLOW, 2).set(6, ROLE_HELP, 1)
-        .set(3, ROLE_COLLECT, 3).set(7, ROLE_FOLLOW, 3).set(11, ROLE_HELP, 2).bits,
-    StripRoles().set(0, ROLE_FOLLOW, 4).set(4, ROLE_COLLECT, 4).set(8, ROLE_COLLECT, 5)
-        .set(5, ROLE_FOLLOW, 6).set(9, ROLE_FOLLOW, 5).set(1, ROLE_COLLECT, 6)
-        .set(2, ROLE_LEAD).set(6, ROLE_HELP, 0).set(10, ROLE_HELP, 1)
-        .set(3, ROLE_FOLLOW, 3).set(7, ROLE_COLLECT, 3).set(11, ROLE_HELP, 2).bits,
-    StripRoles().set(4, ROLE_FOLLOW, 4).set(8, ROLE_FOLLOW, 5)
-        .set(1, ROLE_FOLLOW, 6).set(5, ROLE_HELP, 0)
-        .set(6, ROLE_FOLLOW, 7).set(2, ROLE_HELP, 1).set(10, ROLE_HELP, 2)
-        .set(7, ROLE_LEAD).bits};
-
 // Factors and inverts diagonal block p of matrix m: one workgroup of DIAG_THREADS threads
 // (12 waves) with DIAG_SMEM_BYTES of LDS at dsm: S, the block (upper triangle and the whole
 // diagonal 32-blocks; finished rows of U replace it strip by strip), and Z, the rows of
@@ -435,10 +395,10 @@ constexpr unsigned long long STRIP_ROLES[4] = {
 // SIMD.  One block alone 21.0 -> 17.1 us, with the pending panel 26.1 -> 21.2 (four waves that each
 // held the leaf and a second block, three barriers a strip, the pending panel on the fp32 instructions, 4-byte
 // accesses to memory); the inverse of a 2305^2 matrix and its Cholesky factor 1333 -> 1160 us.
-constexpr int DIAG_THREADS = 768;
+constexpr int DIAG_THREADS = 64 * DIAG_WAVES;
 typedef SplitChunk<DB> PendingGroup;                       // (HALF: 8 k of 128 columns)
 constexpr int PENDING_PLANE = 8 * PendingGroup::HALF;      // 64 k
-static_assert(3 * PENDING_PLANE <= (DB - 32) * DLD * (int)sizeof(float), "half of W lives in the LDS of Z");
+static_assert(3 * PENDING_PLANE <= (DB - PENDING_ROW0) * DLD * (int)sizeof(float), "half of W lives in the LDS of Z");
 
 // `pending`: the row panel above (block row p-1) has not been applied to this block yet
 // (the launch that holds this workgroup applies it to the rest of block row p meanwhile).
@@ -510,16 +470,16 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
     }
   }
   // S -= W^T W, split into bf16 parts as in gemm_split.h, half of the reduction after the other in
-  // the LDS of Z, a 32x32 block of S on each of ten waves; the waves 0-3 have the blocks that they
-  // start the first strip with, and do not wait for the others.
+  // the LDS of Z, a 32x32 block of S on each of ten waves; no barrier behind it: pending_row etc. say
+  // who may go ahead and who waits for whom.
+  lds_vf* const pending_marks = (lds_vf*)(marks + STRIP_MARKS);
   if (pending) {
     v16f acc, cor;
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[e] = cor[e] = 0.f;
-    // (behind the first 32 rows of Z, which the first strip writes)
-    lds_c* const planes = (lds_c*)(Z + 32 * DLD);
-    int bi = 0, bj = 0;
-    if (wave < 10) upper_tile(wave, 4, bi, bj);
+    // (behind the first rows of Z, which the first strip writes)
+    lds_c* const planes = (lds_c*)(Z + PENDING_ROW0 * DLD);
+    const int bi = pending_row(wave), bj = pending_col(wave);
     v4u ph[WGROUPS], pm[WGROUPS], pl[WGROUPS];
     // the pieces of one half of the reduction, split (the second half's under the first's products)
     auto split_half = [&](int half) {
@@ -550,7 +510,7 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
         *(lds_u4*)(at + 2 * PENDING_PLANE) = pl[g];
       }
       __syncthreads();
-      if (wave < 10) {
+      if (wave < PENDING_WAVES) {
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
           v8bf a[3], b[3];
@@ -570,11 +530,14 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
       }
       if (half == 0) split_half(1);
     }
-    if (wave < 10) {
+    if (wave < PENDING_WAVES) {
       add_corrections(acc, cor);
       lds_f* const at = S + (32 * bi + 4 * h) * DLD + 32 * bj + r;
 #pragma unroll
       for (int e = 0; e < 16; ++e) at[(8 * (e >> 2) + (e & 3)) * DLD] -= acc[e];
+      // (the compiler keeps the mark behind the accesses above, and LDS serves a wave's requests in order)
+      asm volatile("" ::: "memory");
+      pending_marks[wave] = 1.f;
     }
   } else {
     __syncthreads();
@@ -686,20 +649,26 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
       }
     } else if (code >= 2) {
       __builtin_amdgcn_s_setprio(0);
-      // what this strip takes from the rows further down:  block (i, i), (i, i+1), ... of S and
-      // (i, 0), ... (i, q) of Z for the block rows i > q + 1; at most five blocks, two to a wave
-      int found = 0, i0 = 0, k0 = 0, i1 = 0, k1 = 0, k = 0;
-      for (int i = q + 2; i < nq; ++i)
-        for (int b = 0; b < nq - i + q + 1; ++b, ++k)
-          if (k % STRIP_HELPERS == code - 2) {
-            i1 = i;
-            k1 = b < nq - i ? i + b : 4 + b - (nq - i);
-            i0 = found ? i0 : i1;
-            k0 = found ? k0 : k1;
-            ++found;
-          }
+      // what this strip takes from the rows further down
+      int found = 0, i0 = 0, k0 = 0, i1 = 0, k1 = 0;
+      helped_blocks(q, nq, code - 2, [&](int i, int col) {
+        i1 = i;
+        k1 = col;
+        i0 = found ? i0 : i1;
+        k0 = found ? k0 : k1;
+        ++found;
+      });
       auto rows_of = [&](int i, int col) {
         return Rows{rows_at(i), rows_at(col), marks_at(i), marks_at(col)};
+      };
+      // (the waves that applied the pending panel end, and wait for nobody behind its last barrier; a
+      // mark apiece, read by lane.  The blocks are read and written behind this.)
+      auto settle = [&]() {
+        if (!pending || !helper_awaits_pending(q)) return;
+        const lds_vf* const mark = pending_marks + min(lane, PENDING_WAVES - 1);
+        while (__builtin_amdgcn_ballot_w64(__builtin_bit_cast(int, (float)*mark) == 0) != 0) {
+        }
+        asm volatile("" ::: "memory");
       };
       auto apply = [&](int i, int col, const v16f& x) {
         lds_f* const at = block_at(col < 4, i, col & 3);
@@ -715,11 +684,13 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
       if (found == 2) {
         v16f x, y;
         collect<true>(x, rows_of(i0, k0), y, rows_of(i1, k1));
+        settle();
         apply(i0, k0, x);
         apply(i1, k1, y);
       } else if (found == 1) {
         v16f x;
         collect<false>(x, rows_of(i0, k0), x, rows_of(i0, k0));
+        settle();
         apply(i0, k0, x);
       }
     }
