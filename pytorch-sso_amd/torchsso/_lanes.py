@@ -197,13 +197,15 @@ def deferred_count():
         return sum(len(q.items) + len(q.bn) for q in _deferred.values())
 
 
-_events = []       # events of engine calls that are done with, for the next ones
+_events = {}       # device index -> events of engine calls that are done with, for the next ones there
+                   # (an event belongs to the device of its first record)
 
 
-def _drop(held):
-    """(under the lock) the calls in `held` keep nothing alive any more"""
-    if len(_events) < 64:
-        _events.extend(done for done, _, _ in held)
+def _drop(i, held):
+    """(under the lock) the calls in `held`, of device i, keep nothing alive any more"""
+    events = _events.setdefault(i, [])
+    if len(events) < 64:
+        events.extend(done for done, _, _ in held)
 
 
 def _run_deferred(only=None, bn_only=False, reader=False):
@@ -289,12 +291,13 @@ def _run_deferred(only=None, bn_only=False, reader=False):
             # the tensors stay referenced until the caller's stream has been made to wait
             # for the side stream (join), or until the side stream is seen to have passed
             with _lock:
-                done = _events.pop() if _events else torch.cuda.Event()
+                events = _events.get(i)
+                done = events.pop() if events else torch.cuda.Event()
                 done.record(side)
                 held, past = [], []
                 for h in _inflight.get(i, ()):
                     (past if h[0].query() else held).append(h)
-                _drop(past)
+                _drop(i, past)
                 held.append((done, items, set(job.C for job in jobs)))
                 _inflight[i] = held
                 _pending.setdefault(i, set()).add(lane)
@@ -382,7 +385,7 @@ def join(device=None):
                     waited.append(st)
                     st.wait_event(done)
         with _lock:
-            _drop(held)
+            _drop(i, held)
 
 
 def _at_exit():
