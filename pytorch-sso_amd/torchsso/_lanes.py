@@ -223,84 +223,94 @@ def _run_deferred(only=None, bn_only=False, reader=False):
                 todo.append((i, q.items, q.bn))
                 _deferred[i] = _Queue()
     for i, items, bn in todo:
-        device = torch.device('cuda', i)
-        cur = _current_stream(i)
-        if bn:
-            # the BatchNorm reductions stay on the caller's stream (one launch for all queued
-            # layers): they are bound by memory and run beside the factor products of the
-            # side streams; whoever reads their outputs does so on this stream, behind them
-            waited = []
-            for job, st in bn:
-                if st is not cur and st != cur:
-                    if st not in waited:
-                        waited.append(st)
-                        _hip.order_streams(i, cur, st)
-                    for t in (job[0], job[2]) + tuple(job[4:]):
-                        if t is not None:
-                            t.record_stream(cur)
-            _ops.bn_diag_cov_batched([job for job, _ in bn], device)
-        if not items:
-            continue
-        side = None
-        # the engine call goes to a side stream (the calls of a pass take turns), so that it runs
-        # beside whatever the caller's stream does next; a reader's stream does nothing before
-        # the call is done, unless it has BatchNorm reductions to run, and takes the call itself: no
-        # event forward and back (a fully connected network's step: 30 us of host time)
-        if _count > 0 and (bn or not reader):
-            _, lst = _lane_streams(device)
-            with _lock:
-                lane = _calls.get(i, 0) % _count
-                _calls[i] = _calls.get(i, 0) + 1
-            side = lst[lane][0]
-            if side == cur:
-                side = None
-        target = cur if side is None else side
-        # a product queued under another stream: its input is complete once that stream
-        # has run what it held at the time of the hook (all of it, to keep this simple)
-        others = []
-        for _, keep, st in items:
+        # (the handle of a null stream means that of the current device)
+        if i == torch.cuda.current_device():
+            _run_queue(i, items, bn, reader)
+        else:
+            with torch.cuda.device(i):
+                _run_queue(i, items, bn, reader)
+
+
+def _run_queue(i, items, bn, reader):
+    """What `_run_deferred` took from the queue of device i, which is current."""
+    device = torch.device('cuda', i)
+    cur = _current_stream(i)
+    if bn:
+        # the BatchNorm reductions stay on the caller's stream (one launch for all queued
+        # layers): they are bound by memory and run beside the factor products of the
+        # side streams; whoever reads their outputs does so on this stream, behind them
+        waited = []
+        for job, st in bn:
             if st is not cur and st != cur:
-                if st not in others and st != target:
-                    others.append(st)
-                for t in keep:
+                if st not in waited:
+                    waited.append(st)
+                    _hip.order_streams(i, cur, st)
+                for t in (job[0], job[2]) + tuple(job[4:]):
                     if t is not None:
-                        t.record_stream(target)
-        jobs = [job for job, _, _ in items]
-        if side is not None:
-            _hip.order_streams(i, side, cur)
+                        t.record_stream(cur)
+        _ops.bn_diag_cov_batched([job for job, _ in bn], device)
+    if not items:
+        return
+    side = None
+    # the engine call goes to a side stream (the calls of a pass take turns), so that it runs
+    # beside whatever the caller's stream does next; a reader's stream does nothing before
+    # the call is done, unless it has BatchNorm reductions to run, and takes the call itself: no
+    # event forward and back (a fully connected network's step: 30 us of host time)
+    if _count > 0 and (bn or not reader):
+        _, lst = _lane_streams(device)
         with _lock:
-            # a call still in flight on ANOTHER side stream that writes a buffer this
-            # call reads or adds to (factors accumulated over MC samples): wait for it
-            held = _inflight.get(i)
-            if held:
-                touched = set()
-                for job in jobs:
-                    touched.add(job.C)
-                    if job.C_prev:
-                        touched.add(job.C_prev)
-                for done, _, written in held:
-                    if not touched.isdisjoint(written):
-                        target.wait_event(done)
-        for st in others:
-            _hip.order_streams(i, target, st)
-        # (the call's workspace is the cached scratch of the stream it runs on; a pass under
-        # no_grad leaves its inputs referenced in the queue, or in `_inflight`, until the
-        # next flush or join)
-        _ops.factor_grouped(jobs, device, stream=side)
-        if side is not None:
-            # the tensors stay referenced until the caller's stream has been made to wait
-            # for the side stream (join), or until the side stream is seen to have passed
-            with _lock:
-                events = _events.get(i)
-                done = events.pop() if events else torch.cuda.Event()
-                done.record(side)
-                held, past = [], []
-                for h in _inflight.get(i, ()):
-                    (past if h[0].query() else held).append(h)
-                _drop(i, past)
-                held.append((done, items, set(job.C for job in jobs)))
-                _inflight[i] = held
-                _pending.setdefault(i, set()).add(lane)
+            lane = _calls.get(i, 0) % _count
+            _calls[i] = _calls.get(i, 0) + 1
+        side = lst[lane][0]
+        if side == cur:
+            side = None
+    target = cur if side is None else side
+    # a product queued under another stream: its input is complete once that stream
+    # has run what it held at the time of the hook (all of it, to keep this simple)
+    others = []
+    for _, keep, st in items:
+        if st is not cur and st != cur:
+            if st not in others and st != target:
+                others.append(st)
+            for t in keep:
+                if t is not None:
+                    t.record_stream(target)
+    jobs = [job for job, _, _ in items]
+    if side is not None:
+        _hip.order_streams(i, side, cur)
+    with _lock:
+        # a call still in flight on ANOTHER side stream that writes a buffer this
+        # call reads or adds to (factors accumulated over MC samples): wait for it
+        held = _inflight.get(i)
+        if held:
+            touched = set()
+            for job in jobs:
+                touched.add(job.C)
+                if job.C_prev:
+                    touched.add(job.C_prev)
+            for done, _, written in held:
+                if not touched.isdisjoint(written):
+                    target.wait_event(done)
+    for st in others:
+        _hip.order_streams(i, target, st)
+    # (the call's workspace is the cached scratch of the stream it runs on; a pass under
+    # no_grad leaves its inputs referenced in the queue, or in `_inflight`, until the
+    # next flush or join)
+    _ops.factor_grouped(jobs, device, stream=side)
+    if side is not None:
+        # the tensors stay referenced until the caller's stream has been made to wait
+        # for the side stream (join), or until the side stream is seen to have passed
+        with _lock:
+            events = _events.get(i)
+            done = events.pop() if events else torch.cuda.Event()
+            done.record(side)
+            held, past = [], []
+            for h in _inflight.get(i, ()):
+                (past if h[0].query() else held).append(h)
+            _drop(i, past)
+            held.append((done, items, set(job.C for job in jobs)))
+            _inflight[i] = held
+            _pending.setdefault(i, set()).add(lane)
 
 
 def _lane_streams(device):

@@ -107,3 +107,13 @@ def test_events_are_recorded_on_their_own_device(world):
             defer(i, ('G', i), 200 + i, backward=True)      # (runs the input factors on a side stream)
             _lanes.join(torch.device('cuda', i))
     assert [(st.device_index, c) for st, c in world.calls()] == 3 * [(0, [100]), (0, [200]), (1, [101]), (1, [201])]
+
+
+def test_products_of_two_devices_keep_to_their_devices(world):
+    for step in range(3):
+        for i in (0, 1):
+            defer(i, ('A', i), 100 + i)
+            defer(i, ('G', i), 200 + i, backward=True)      # (runs the input factors on a side stream)
+        _lanes.join()
+    assert [(st.device_index, c) for st, c in world.calls()] == 3 * [(0, [100]), (1, [101]), (0, [200]), (1, [201])]
+    assert world.device == 0
