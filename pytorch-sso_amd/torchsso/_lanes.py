@@ -255,8 +255,9 @@ def _run_queue(i, items, bn, reader):
     # the engine call goes to a side stream (the calls of a pass take turns), so that it runs
     # beside whatever the caller's stream does next; a reader's stream does nothing before
     # the call is done, unless it has BatchNorm reductions to run, and takes the call itself: no
-    # event forward and back (a fully connected network's step: 30 us of host time)
-    if _count > 0 and (bn or not reader):
+    # event forward and back (a fully connected network's step: 30 us of host time).  (Not the products
+    # of hooks that ran under another stream: that one has to wait for them too, see `join`.)
+    if _count > 0 and (bn or not reader or any(st is not cur and st != cur for _, _, st in items)):
         _, lst = _lane_streams(device)
         with _lock:
             lane = _calls.get(i, 0) % _count

@@ -117,3 +117,19 @@ def test_products_of_two_devices_keep_to_their_devices(world):
         _lanes.join()
     assert [(st.device_index, c) for st, c in world.calls()] == 3 * [(0, [100]), (1, [101]), (0, [200]), (1, [201])]
     assert world.device == 0
+
+
+def test_a_hooks_stream_waits_for_the_products_a_reader_runs(world):
+    """Its next pass may write the same factors, and the allocator hands what the products read out again there."""
+    reader, hook = world.streams[0], Stream(0)
+    world.streams[0] = hook
+    defer(0, ('A', 0), 100)
+    world.streams[0] = reader
+    _lanes.join()
+    (call, _), = world.calls()
+    at = [kind for kind, *_ in world.log].index('call')
+    behind = [(entry[1], entry[2]) for entry in world.log[at:] if entry[0] == 'order']
+    recorded = {id(event): st for kind, st, event in world.log[at:] if kind == 'record'}
+    behind += [(st, recorded[id(event)]) for kind, st, event in world.log[at:] if kind == 'wait']
+    assert (hook, call) in behind
+    assert call == reader or (reader, call) in behind
