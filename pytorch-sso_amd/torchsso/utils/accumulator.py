@@ -54,7 +54,9 @@ class TensorAccumulator(object):
             acc.check_type(data)
             as_list = data if isinstance(data, list) else [data]
             if not as_list[0].is_cuda:
-                acc.update(data, scale)
+                # (values only: a gradient may have a graph of its own)
+                plain = [d.detach() for d in as_list]
+                acc.update(plain if isinstance(data, list) else plain[0], scale)
                 continue
             src = [d if d.is_contiguous() else d.detach().contiguous() for d in as_list]
             have = acc._accumulation

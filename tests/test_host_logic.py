@@ -749,3 +749,18 @@ def test_layers_are_sorted_into_classes_by_the_length_of_their_factorisation():
     assert chain_classes([4608, 0, 0], 2048, 2) is None
     assert chain_classes([4608, 100], None, 2) is None
     assert chain_classes([4608, 100], 2048, 1) is None
+
+
+def test_gradients_are_accumulated_without_their_graph():
+    """Gradients of a backward pass with create_graph, which have one."""
+    p = nn.Parameter(torch.randn(3))
+    accs = [torchsso.utils.TensorAccumulator(), torchsso.utils.TensorAccumulator()]
+    for _ in range(2):
+        p.grad = None
+        (p ** 3).sum().backward(create_graph=True)
+        assert p.grad.requires_grad
+        torchsso.utils.TensorAccumulator.update_many(accs, [[p.grad], p.grad], scale=0.5)
+    a, b = accs[0].get(), accs[1].get()
+    assert not a[0].requires_grad and not b.requires_grad
+    assert torch.equal(a[0], 3 * p.detach() ** 2) and torch.equal(a[0], b)
+    p.grad = None
