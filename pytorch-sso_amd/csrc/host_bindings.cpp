@@ -21,7 +21,8 @@ void* address_of(PyObject* o) {
   const at::Tensor& t = THPVariable_Unpack(o);
   if (!t.is_cuda() || t.scalar_type() != at::kFloat || t.layout() != at::kStrided || !t.is_contiguous())
     return nullptr;
-  return const_cast<void*>(t.const_data_ptr());
+  // (as Tensor.data_ptr(): a lazily copied tensor gets memory of its own before it is written to)
+  return t.mutable_data_ptr();
 }
 
 // `fill(object, index, slot)` for every object of a list or tuple, into a bytes object of T; None where it

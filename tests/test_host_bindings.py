@@ -57,6 +57,22 @@ def test_addresses_and_jobs_of_device_tensors():
 
 
 @pytest.mark.gpu
+def test_a_lazily_copied_tensor_is_not_written_through():
+    dev = torch.device('cuda:0')
+    for through in ('call', 'job'):
+        a = torch.zeros(8, 8, device=dev)
+        b = torch._lazy_clone(a)
+        x = torch.ones(3, 8, device=dev)
+        if through == 'call':
+            _ops.axpby_batched([torch.full((8, 8), 3., device=dev)], [b], 1., 0.)
+        else:
+            job = _ops.factor_job('linear', x, 1., x.new_empty(8, 8))
+            _ops.factor_job_update(job, x, 1., b)
+            _ops.factor_grouped([job], dev)
+        assert not a.any().item() and bool((b == 3.).all())
+
+
+@pytest.mark.gpu
 def test_order_of_two_streams():
     dev = torch.device('cuda:0')
     x = torch.zeros(1 << 24, device=dev)
