@@ -79,9 +79,9 @@ struct SyrkPlan {
 static SyrkPlan plan_syrk(int d, long K) {
   SyrkPlan p;
   // 64-wide tiles up to 192 rows, and to 256 where the reduction is short: of 200 rows over 4096 / 16384 /
-  // 32768 / 60000 / 100000 terms 13.1 / 22.7 / 30.4 / 45.6 / 64.8 us, on 128-wide tiles 18.1 / 26.4 / 31.0 / 41.0 /
-  // 55.5; of 256 over the same 13.8 / 23.7 / 31.5 / 48.4 / 69.1 and 19.1 / 28.2 / 34.5 / 45.9 / 61.9.
-  p.w = d <= 192 || (d <= 256 && K <= 32768) ? 1 : 2;
+  // 32768 / 60000 / 100000 terms 13.8 / 24.7 / 34.1 / 51.1 / 74.1 us, on 128-wide tiles 18.4 / 26.9 / 31.2 / 40.7 /
+  // 55.6; of 256 over the same 14.2 / 25.8 / 34.9 / 55.2 / 80.4 and 19.0 / 28.8 / 35.0 / 46.2 / 62.4.
+  p.w = d <= 192 || (d <= 256 && K <= 24576) ? 1 : 2;
   p.ts = 64 * p.w;
   p.T = cdiv(d, p.ts);
   p.ntiles = p.T * (p.T + 1) / 2;

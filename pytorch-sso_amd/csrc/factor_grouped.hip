@@ -230,9 +230,11 @@ struct GroupPlan {
   }
 };
 
-// 64-wide tiles up to 192 rows; from there a 128-wide tile has at most a
-// quarter of padding, and it runs on the bf16 matrix cores (factors of a ResNet-50, 32 images: 4.57 ms,
-// and 5.1 ms with 64-wide tiles up to 256 rows; 128 rows make no difference there).
+// 64-wide tiles up to 192 rows; from there a 128-wide tile has at most a quarter of padding, and splits an
+// element once for twice the products.  64-wide up to 192 / up to 256 rows: output gradients of 32 images of
+// 256x56x56, one layer / three 72 / 77 and 182 / 224 us, six layers of 256x14x14 beside three of 1024x14x14
+// 169 / 192; but 4096 rows of 256 21.4 / 16.8, 128 rows of 256 20.9 / 11.1, six layers of 256x14x14 alone 55 / 47:
+// such calls, of little work, are not told apart.
 constexpr int GROUP_W1_MAX_DIM = 192;
 
 static GroupPlan plan_group(int d, long K, long target) {
@@ -330,7 +332,7 @@ static Classified classify_shape(const kfac_factor_job& j, bool copy_pointwise) 
   return c;
 }
 
-// ... and the reduction index of products in runs, on 128-wide tiles with padded runs
+// ... and the reduction index of products in runs, with padded runs
 static Classified classify(const kfac_factor_job& j, bool copy_pointwise) {
   Classified c = classify_shape(j, copy_pointwise);
   if (c.path != P_CONVG && c.path != P_CONVP) return c;

@@ -10,8 +10,9 @@
 // (An element below 2^-109, 1.5e-33, is that sum only down to 2^-133, the smallest bf16 number: it
 // enters rounded to a multiple of that, so that a product with a large factor keeps 2^-134 / |x|
 // instead of 2^-24.)
-// The bracket is at most 2^-23 and on average 2^-26 of x y, below the rounding of one float32
-// accumulation, and is left out; the other six run as v_mfma_f32_32x32x16_bf16.  The leading
+// The bracket is at most 2^-25 and on average 2^-26 of x y, below the rounding of one float32
+// accumulation, and is left out (on 64-wide tiles its last term only); the others run as
+// v_mfma_f32_32x32x16_bf16.  The leading
 // products and the five corrections have accumulators of their own: the leading ones are
 // rounded once per 16 reduction steps, the corrections are 2^-8 of them, and the two are
 // added at the end.  Measured against float64 on one 32x32 tile (relative 2-norm, this
@@ -59,10 +60,13 @@ struct SplitChunk {
 // The 32x32 blocks of a tile that one wave computes, and from which fragment rows (of 32) of the
 // operands.  TM x TN: the tile; NT: its threads; NB blocks a wave, block B = fragment row a(B) of P
 // against row b(B) of Q (SAME: of P: a diagonal tile of a symmetric product, of which only P is
-// staged); PF / QF fragment rows a wave.
+// staged); PF / QF fragment rows a wave.  PRODUCTS: how many of the nine partial products are taken;
+// SCALE: what elements are multiplied with before they are split (a power of two).
 // SplitTile: four waves, each a 64x64 quadrant of 128x128.
 struct SplitTile {
   static constexpr int TM = 128, TN = 128, NT = 256, NB = 4, PF = 2, QF = 2;
+  static constexpr int PRODUCTS = 6;
+  static constexpr float SCALE = 1.f;
   static constexpr bool SAME = false;
   static constexpr int a(int B) { return B >> 1; }
   static constexpr int b(int B) { return B & 1; }
@@ -77,6 +81,8 @@ struct SplitTile {
 // Every wave runs the same code, and the tile is done in three quarters of the time.
 struct SplitDiag {
   static constexpr int TM = 128, TN = 128, NT = 256, NB = 3, PF = 3, QF = 0;
+  static constexpr int PRODUCTS = 6;
+  static constexpr float SCALE = 1.f;
   static constexpr bool SAME = true;
   static constexpr int a(int B) { return B == 2 ? 1 : 0; }
   static constexpr int b(int B) { return B == 1 ? 2 : 1; }
@@ -85,17 +91,24 @@ struct SplitDiag {
 // stored).  A chunk is short work for a wave (6 matrix instructions), so what bounds these is the barrier and
 // the loads of each chunk, and workgroups in flight hide them: five to a CU at 100 registers.  (One wave
 // with the four blocks does with two thirds of the LDS reads, but needs 330 registers.)  On the fp32
-// matrix instructions, a wave to a tile, / here: output gradients of 32 images of 64x112x112 69 / 39 us,
-// 128x56x56 54 / 35, six layers of 64x56x56 82 / 45, of 160x13x13 23 / 18; 3x3 inputs of 64x56x56, three
-// layers, 480 / 319, the 3x224x224 of a 7x7 stem 261 / 162; 4096 rows of 100 28 / 15.
+// matrix instructions, a wave to a tile, / here with six partial products / here: output gradients of 32 images of
+// 64x112x112 68 / 41 / 44 us, 128x56x56 54 / 35 / 38, six layers of 64x56x56 82 / 44 / 50, of 160x13x13
+// 22 / 14.7 / 15.1; 3x3 inputs of 64x56x56, three layers, 485 / 326 / 357, the 3x224x224 of a 7x7 stem 262 / 160 /
+// 171; 4096 rows of 100 26 / 10.8 / 11.0.  (What the two more products cost is what makes every sum as good as
+// the fp32 instructions' own, see split_blocks; the scale costs nothing.)
+constexpr float SMALL_SCALE = 16777216.f;       // 2^24
 struct SmallTile {
   static constexpr int TM = 64, TN = 64, NT = 256, NB = 1, PF = 1, QF = 1;
+  static constexpr int PRODUCTS = 8;
+  static constexpr float SCALE = SMALL_SCALE;
   static constexpr bool SAME = false;
   static constexpr int a(int) { return 0; }
   static constexpr int b(int) { return 0; }
 };
 struct SmallDiag {
   static constexpr int TM = 64, TN = 64, NT = 256, NB = 1, PF = 2, QF = 0;
+  static constexpr int PRODUCTS = 8;
+  static constexpr float SCALE = SMALL_SCALE;
   static constexpr bool SAME = true;
   static constexpr int a(int) { return 0; }
   static constexpr int b(int) { return 1; }
@@ -247,6 +260,20 @@ struct SplitStager<OP, ROWS, NT, KM> {
     }
     ones[SET] = one;
   }
+  // the elements as they are (fp32_tile): rows of LDS_MK floats
+  __device__ __forceinline__ void commit_plain(lds_f* chunk) {
+    static_assert(KPT == 4, "one 16-byte store a column");
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      v4f v;
+#pragma unroll
+      for (int j = 0; j < KPT; ++j) {
+        v[j] = ((ones[0] >> (KPT * i + j)) & 1u) ? 1.f : regs[0][i][j];
+        if (squares_elements<OP>::value) v[j] *= v[j];
+      }
+      *(lds_f4*)(chunk + ((tid() + NT * i) & (ROWS - 1)) * LDS_MK + KPT * kgroup(i)) = v;
+    }
+  }
   template <int SET, int PIECE, int MODE, bool SCALED = false>
   __device__ __forceinline__ void commit(lds_c* chunk, float scale = 1.f) {
     typedef SplitChunk<ROWS> L;
@@ -362,6 +389,18 @@ struct SplitStager<OP, ROWS, NT, MK> {
     }
     kin[SET] = in;
   }
+  __device__ __forceinline__ void commit_plain(lds_f* chunk) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      v4f v = regs[0][i];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (OP::kruns == K_ANY) v[j] = ((ones >> i) & (kin[0] >> j) & 1u) ? 1.f : v[j];
+        if (squares_elements<OP>::value) v[j] *= v[j];
+      }
+      *(lds_f4*)(chunk + ((tid() >> 2) + STEP * i) * LDS_MK + 4 * (tid() & 3)) = v;
+    }
+  }
   template <int SET, int PIECE, int MODE, bool SCALED = false>
   __device__ __forceinline__ void commit(lds_c* chunk, float scale = 1.f) {
     typedef SplitChunk<ROWS> L;
@@ -421,11 +460,13 @@ struct SplitFrags {
   v8bf q[3][TILE::QF > 0 ? TILE::QF : 1];
 };
 
-// product PR of the six (in the order h h', h m', m h', m m', h l', l h'; then m l', l m') for block B
+// product PR for block B, in the order h h', h m', m h', m m', (m l', l m',) h l', l h': the last two leave
+// m's registers to the next chunk
 template <class TILE, int PR, int B>
 __device__ __forceinline__ void split_product(const SplitFrags<TILE>& fr, v16f& sum) {
-  constexpr int PA = PR == 2 || PR == 3 || PR == 6 ? 1 : PR == 5 || PR == 7 ? 2 : 0;
-  constexpr int PB = PR == 1 || PR == 3 || PR == 7 ? 1 : PR == 4 || PR == 6 ? 2 : 0;
+  constexpr int LAST = PR - (TILE::PRODUCTS - 2);
+  constexpr int PA = LAST == 0 ? 0 : LAST == 1 ? 2 : PR < 4 ? PR >> 1 : PR == 4 ? 1 : 2;
+  constexpr int PB = LAST == 0 ? 2 : LAST == 1 ? 0 : PR < 4 ? PR & 1 : PR == 4 ? 2 : 1;
   const v8bf a = fr.p[PA][TILE::a(B)];
   v8bf b;
   if constexpr (TILE::SAME) b = fr.p[PB][TILE::b(B)];
@@ -480,9 +521,9 @@ __device__ __forceinline__ void split_tile_loop(const OPP& P, const OPQ& Q, int 
   auto commit = [&](auto set_, auto piece_, lds_c* stage) {
     constexpr int SET = decltype(set_)::value, X = decltype(piece_)::value;
     if constexpr (X < SP::PIECES)
-      sp.template commit<SET, X, MODE>(stage);
+      sp.template commit<SET, X, MODE, C::SCALE != 1.f>(stage, C::SCALE);
     else
-      sq.template commit<SET, X - SP::PIECES, MODE>(stage + QOFF);
+      sq.template commit<SET, X - SP::PIECES, MODE, C::SCALE != 1.f>(stage + QOFF, C::SCALE);
   };
   SplitFrags<C> fr[2];
   auto load_frags = [&](auto set_, auto plane_) {
@@ -505,7 +546,7 @@ __device__ __forceinline__ void split_tile_loop(const OPP& P, const OPQ& Q, int 
   load_frags(S0, std::integral_constant<int, 0>{});
 
   // One chunk.  Its leading planes are in registers already; the loads of chunk c + 2 and the
-  // pieces of chunk c + 1 are dealt out between the matrix instructions of the first four
+  // pieces of chunk c + 1 are dealt out between the matrix instructions of all but two
   // products; then the workgroup meets (chunk c has been read and chunk c + 1 written by
   // every wave), and the leading planes of chunk c + 1 come in under the last two products.
   auto step = [&](auto set_, auto full_, int c) {
@@ -516,9 +557,9 @@ __device__ __forceinline__ void split_tile_loop(const OPP& P, const OPQ& Q, int 
     load_frags(set_, std::integral_constant<int, 2>{});
     if (!FULL) fetch(set_, c + 2);
     __builtin_amdgcn_sched_barrier(0);
-    static_for<6>([&](auto prod_) {
+    static_for<C::PRODUCTS>([&](auto prod_) {
       constexpr int PR = decltype(prod_)::value;
-      if constexpr (PR == 4) {
+      if constexpr (PR == C::PRODUCTS - 2) {
         __syncthreads();
         load_frags(std::integral_constant<int, SET ^ 1>{}, std::integral_constant<int, 0>{});
         __builtin_amdgcn_sched_barrier(0);
@@ -527,8 +568,8 @@ __device__ __forceinline__ void split_tile_loop(const OPP& P, const OPQ& Q, int 
         constexpr int B = decltype(blk_)::value;
         constexpr int IDX = PR * NB + B;
         split_product<C, PR, B>(fr[SET], PR == 0 ? acc[B] : cor[B]);
-        if constexpr (PR < 4) {
-          constexpr int LAST = 4 * NB;
+        if constexpr (PR < C::PRODUCTS - 2) {
+          constexpr int LAST = (C::PRODUCTS - 2) * NB;
           constexpr int l0 = IDX * LOADS / LAST, l1 = (IDX + 1) * LOADS / LAST;
           if constexpr (FULL)
             static_for<l1 - l0>([&](auto x) {
@@ -565,10 +606,6 @@ __device__ __forceinline__ void split_tile_loop(const OPP& P, const OPQ& Q, int 
 // loop has a third of the code and no chunk past the end.  Factor of 16 rows of 300 / 48 of 1000 /
 // 8 of 5000: 12.1 / 15.7 / 57.5 us by the loop above, 9.8 / 14.1 / 52.7 by this one (9.4 / 13.3 /
 // 51.8 on the fp32 tile engine); 64 rows of 512: 16.1 / 16.7.
-// The 64-wide tiles, which replaced fp32 instructions, take the two largest of the products left out as well:
-// in sums of one or two terms those are as large as a float32 sum's own roundings (relative 2-norm
-// of the factor of 1 / 2 rows of 17 ... 192: 2.51e-8 / 2.63e-8 without, 2.47e-8 / 2.59e-8
-// with them, 2.47e-8 / 3.10e-8 by the fp32 ones).
 constexpr int SHORT_K = 48;
 template <class C, class OPP, class OPQ>
 __device__ __forceinline__ void split_tile_rolled(const OPP& P, const OPQ& Q, int m0, int n0, int kbeg,
@@ -609,13 +646,47 @@ __device__ __forceinline__ void split_tile_rolled(const OPP& P, const OPQ& Q, in
 #pragma unroll
       for (int i = 0; i < C::QF; ++i) fr.q[pl][i] = load_frag<C::TN>(at + QOFF, rows.q[i], lane, pl);
     }
-    static_for<C::NB == 1 ? 8 : 6>([&](auto prod_) {
+    static_for<C::PRODUCTS>([&](auto prod_) {
       constexpr int PR = decltype(prod_)::value;
       static_for<C::NB>([&](auto blk_) {
         constexpr int B = decltype(blk_)::value;
         split_product<C, PR, B>(fr, PR == 0 ? acc[B] : cor[B]);
       });
     });
+  }
+}
+
+// The same on the fp32 instructions (64-wide tiles): what leaves the range of the split elements.
+template <class C, class OPP, class OPQ>
+__device__ __forceinline__ void fp32_tile(const OPP& P, const OPQ& Q, int m0, int n0, int kbeg, int kend,
+                                          lds_c* sm, const SplitRows& rows, v16f& acc) {
+  static_assert(C::NB == 1 && C::TM * LDS_MK * 4 <= SplitChunk<C::TM>::BYTES, "one block a wave, 64-wide chunks");
+  constexpr bool SAME = C::SAME;
+  constexpr int STAGE = SplitCfg<C::TM / 64>::STAGE;
+  constexpr int QOFF = SAME ? 0 : SplitChunk<C::TM>::BYTES;
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+  SplitStager<OPP, C::TM, C::NT> sp;
+  SplitStager<OPQ, C::TN, C::NT> sq;
+  sp.init(P, m0);
+  if (!SAME) sq.init(Q, n0);
+  int stage = 0;
+#pragma unroll 1
+  for (int k0 = kbeg; k0 < kend; k0 += KC) {
+    lds_c* const at = sm + stage;
+    stage ^= STAGE;
+    sp.template fetch<0>(P, k0, kend);
+    if (!SAME) sq.template fetch<0>(Q, k0, kend);
+    sp.commit_plain((lds_f*)at);
+    if (!SAME) sq.commit_plain((lds_f*)(at + QOFF));
+    __syncthreads();       // (every wave is done with the chunk before this one: its stage is free)
+    const lds_f* const pa = (const lds_f*)at + (rows.p[0] + r) * LDS_MK + 4 * h;
+    const lds_f* const pb = (const lds_f*)(at + QOFF) + ((SAME ? rows.p[1] : rows.q[0]) + r) * LDS_MK + 4 * h;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const v4f a = *(const lds_f4*)(pa + 8 * j), b = *(const lds_f4*)(pb + 8 * j);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s], b[s], acc, 0, 0, 0);
+    }
   }
 }
 
@@ -627,6 +698,14 @@ __device__ __forceinline__ void split_tile_rolled(const OPP& P, const OPQ& Q, in
 // from halves of the elements, and the sums taken four times: what is finite then, is what a
 // float32 sum gives, and what is not, is not there either.  (Half of an element is exact, but for
 // a last bit of 2^-149.)  The waves vote across the barrier that ends a tile anyway.
+// The 64-wide tiles are as good as fp32 instructions, which they replaced, at every element:
+//   they take the two largest of the partial products left out as well.  In sums of one or few terms
+//   those are as large as a float32 sum's own rounding (a single product is off by up to 1.7 half units in the
+//   last place without them, 1.0 with them);
+//   elements are multiplied by 2^24 before they are split, so that those below 2^-109 keep all their bits (to the
+//   last one of the smallest float32, 2^-149), and the sums by 2^-48;
+//   a tile with a sum that is then not finite, with an element from 2^104 or a sum from 2^80 on, that is,
+//   is computed once more by the fp32 instructions.
 template <class C, class OPP, class OPQ>
 __device__ __forceinline__ void split_blocks(const OPP& P, const OPQ& Q, int m0, int n0, int kbeg,
                                              int kend, float* smem, const SplitRows& rows,
@@ -649,7 +728,7 @@ __device__ __forceinline__ void split_blocks(const OPP& P, const OPQ& Q, int m0,
   clear();
   if (kend <= kbeg) return;
   if (kend - kbeg <= SHORT_K) {
-    split_tile_rolled<C>(P, Q, m0, n0, kbeg, kend, sm, rows, 1.f, acc, cor);
+    split_tile_rolled<C>(P, Q, m0, n0, kbeg, kend, sm, rows, C::SCALE, acc, cor);
   } else if (mode == FAST_K && qmode == FAST_K) {
     split_tile_loop<C, FAST_K>(P, Q, m0, n0, kbeg, kend, sm, rows, acc, cor);
   } else if (has_padded_runs<OPP>::value && mode == PADDED_K) {
@@ -673,7 +752,16 @@ __device__ __forceinline__ void split_blocks(const OPP& P, const OPQ& Q, int m0,
   unsigned any = 0;
 #pragma unroll
   for (int w = 0; w < C::NT / 64; ++w) any |= votes[w];
-  if (__builtin_expect(__builtin_amdgcn_readfirstlane((int)any) != 0, 0)) {
+  const bool again = __builtin_expect(__builtin_amdgcn_readfirstlane((int)any) != 0, 0);
+  if constexpr (NB == 1) {
+    if (again) {
+      clear();
+      fp32_tile<C>(P, Q, m0, n0, kbeg, kend, sm, rows, acc[0]);
+      __syncthreads();
+    } else {
+      acc[0] *= 1.f / (C::SCALE * C::SCALE);
+    }
+  } else if (again) {
     clear();
     split_tile_rolled<C>(P, Q, m0, n0, kbeg, kend, sm, rows, 0.5f, acc, cor);
 #pragma unroll

@@ -34,7 +34,7 @@ def test_dense(ops, dev, f, rows):  # noqa: F811
 
 # both sides of the change of tile
 @pytest.mark.parametrize('f', [193, 256])
-@pytest.mark.parametrize('rows', [32768, 32769])
+@pytest.mark.parametrize('rows', [24576, 24577, 32768, 32769])
 def test_long_reductions(ops, dev, f, rows):  # noqa: F811
     x = randn(dev, rows, f)
     out = ops.factor_linear(x, False, 1.)
@@ -82,3 +82,30 @@ def test_not_finite(ops, dev, rows):  # noqa: F811
         ok = want.isfinite()
         # (sums of positive terms: either side within rows roundings of the exact sum)
         assert ((out - want)[ok] / want[ok]).abs().max().item() < 2 * rows * 2. ** -24
+
+
+# one term apiece in sums of up to, and of more than, a rolled loop's length; magnitudes around 1, and from
+# below the range of split elements to sums beyond that of scaled ones
+@pytest.mark.parametrize('rows', [5, 48, 49, 300, 5000])
+@pytest.mark.parametrize('exponents', [(0, 0), (-36, 3), (-36, 18)])
+def test_single_terms_are_rounded_once(ops, dev, rows, exponents):  # noqa: F811
+    """Sums of which all terms but one are zero (inputs behind a ReLU, one-hot rows) are that product, rounded to
+    float32.  Allowed beyond that: the seven partial products added to the corrections, at most 2^-8 of the
+    product, each rounded by 2^-23 of those."""
+    f = 130
+    x = torch.zeros(rows, f, device=dev)
+    gen = torch.Generator(device=dev).manual_seed(rows)
+    lo, hi = exponents
+    x[rows // 2] = torch.randn(f, device=dev, generator=gen).sign() * 10. ** (
+        lo + (hi - lo) * torch.rand(f, device=dev, generator=gen, dtype=torch.float64)).float() * (
+        1 + torch.rand(f, device=dev, generator=gen))
+    want = x[rows // 2].double()[:, None] * x[rows // 2].double()
+    bound = want.abs() * 2. ** -24 * (1 + 7 * 2. ** -7) + 2. ** -149
+    grouped = torch.full((f, f), float('nan'), device=dev)
+    ops.factor_grouped([ops.factor_job('linear', x, 1., grouped)], dev)
+    positions = x.t().reshape(1, f, 1, rows).contiguous()
+    torch.cuda.synchronize()
+    for got in (ops.factor_linear(x, False, 1.), grouped, ops.factor_conv_g(positions, 1.)):
+        # (what a float32 cannot hold as a normal number is not looked at)
+        over = ((got.double() - want).abs() / bound)[want.abs() >= 2. ** -126]
+        assert over.max().item() <= 1., 'error %.2f times the bound' % over.max().item()
