@@ -472,6 +472,11 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
   // S -= W^T W, split into bf16 parts as in gemm_split.h, half of the reduction after the other in
   // the LDS of Z, a 32x32 block of S on each of ten waves; no barrier behind it: pending_row etc. say
   // who may go ahead and who waits for whom.
+  // (Eight of the nine partial products, as good as the fp32 instructions.  The ends of the range do
+  // not matter here: W is part of a Cholesky factor, so the sum of the squares of a column is at most the
+  // diagonal entry below it.  No element is above 2^64; and what one below 2^-109 loses, 2^-134 times the
+  // other column, is below the rounding 2^-24 sqrt(S_ii S_jj) of the entry it goes to wherever S_ii is a
+  // float32 that is not zero.)
   lds_vf* const pending_marks = (lds_vf*)(marks + STRIP_MARKS);
   if (pending) {
     v16f acc, cor;
@@ -526,6 +531,8 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
           cor = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[1], cor, 0, 0, 0);
           cor = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[2], cor, 0, 0, 0);
           cor = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2], b[0], cor, 0, 0, 0);
+          cor = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[2], cor, 0, 0, 0);
+          cor = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2], b[1], cor, 0, 0, 0);
         }
       }
       if (half == 0) split_half(1);
@@ -847,13 +854,18 @@ struct StepOperand {
       for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
+          // (no branch around the load: what is done with its value would move in there, and wait for it)
           const int at = k + 32 * i + j;
-          v[8 * i + j] = depth == DB || at < depth ? buffer_load_at(rs, off, (unsigned)(at * n) * 4u) : 0.f;
+          const bool in = depth == DB || at < depth;
+          v[8 * i + j] = buffer_load_at(rs, in ? off : INV_M, in ? (unsigned)(at * n) * 4u : 0u);
         }
     }
   }
-  __device__ __forceinline__ void commit(lds_c* at) const {
+  // (SCALED: multiplied by SMALL_SCALE)
+  template <bool SCALED>
+  __device__ __forceinline__ void commit(lds_c* at) {
     const int t = threadIdx.x;
+    const float f = SCALED ? SMALL_SCALE : 1.f;
     if constexpr (MKL) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -861,7 +873,7 @@ struct StepOperand {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
           unsigned a, b, c;
-          split_pair(v[4 * i + 2 * j], v[4 * i + 2 * j + 1], a, b, c);
+          split_pair(v[4 * i + 2 * j] * f, v[4 * i + 2 * j + 1] * f, a, b, c);
           h[j] = a;
           m[j] = b;
           l[j] = c;
@@ -878,7 +890,7 @@ struct StepOperand {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           unsigned a, b, c;
-          split_pair(v[8 * i + 2 * j], v[8 * i + 2 * j + 1], a, b, c);
+          split_pair(v[8 * i + 2 * j] * f, v[8 * i + 2 * j + 1] * f, a, b, c);
           h[j] = a;
           m[j] = b;
           l[j] = c;
@@ -887,10 +899,40 @@ struct StepOperand {
         *(lds_u4*)o = h;
         *(lds_u4*)(o + STEP_PLANE) = m;
         *(lds_u4*)(o + 2 * STEP_PLANE) = l;
+        if (SCALED) __builtin_amdgcn_sched_barrier(0);
       }
     }
   }
 };
+
+// Without old values (the row panels) a tile is as good as the fp32 instructions that it replaces, as a 64-wide one
+// of gemm_split.h is and in the same ways: eight of the nine partial products, elements multiplied by
+// 2^24 before they are split, and where a sum is then not finite, the tile on the fp32 instructions.
+constexpr int STEP_VOTES = 2 * STEP_OPERAND;        // a word per wave
+
+// C[m][n] of a wave's two 32x32 blocks at (m0, n0) and (m0 + 32, n0), k < depth, straight from memory
+// (consecutive m and n)
+__device__ __forceinline__ void step_fp32(const float* p, const float* q, int n, int m0, int n0, int depth,
+                                          v16f (&acc)[2]) {
+  const __amdgpu_buffer_rsrc_t rp = make_rsrc(p), rq = make_rsrc(q);
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[i][e] = 0.f;
+#pragma unroll 1
+  for (int k0 = 0; k0 < DB; k0 += 2) {
+    const int k = k0 + h;
+    const unsigned row = (unsigned)(k * n) * 4u;
+    const float b = buffer_load(rq, k < depth && n0 + r < n ? row + 4u * (n0 + r) : INV_M);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int m = m0 + 32 * i + r;
+      const float a = buffer_load(rp, k < depth && m < n ? row + 4u * m : INV_M);
+      acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc[i], 0, 0, 0);
+    }
+  }
+}
 
 template <bool PMK, bool QMK, bool OLD = true>
 __device__ __forceinline__ void step_tile(const float* p, const float* q, float* C, int n, int m0,
@@ -911,36 +953,49 @@ __device__ __forceinline__ void step_tile(const float* p, const float* q, float*
 #pragma unroll 1
     for (int ks = 0; ks < 4; ++ks) {
       v8bf a[3][2], b[3];
+      const lds_c* const at = sm + (2 * ks + h) * StepGroup::HALF + r * 16;
+      auto load_a = [&](int i) {
 #pragma unroll
-      for (int pl = 0; pl < 3; ++pl) {
-        const lds_c* const at = sm + pl * STEP_PLANE + (2 * ks + h) * StepGroup::HALF + r * 16;
+        for (int pl = 0; pl < 3; ++pl)
+          a[pl][i] = __builtin_bit_cast(v8bf, *(const lds_u4*)(at + pl * STEP_PLANE + (wm + 32 * i) * 16));
+      };
 #pragma unroll
-        for (int i = 0; i < 2; ++i) a[pl][i] = __builtin_bit_cast(v8bf, *(const lds_u4*)(at + (wm + 32 * i) * 16));
-        b[pl] = __builtin_bit_cast(v8bf, *(const lds_u4*)(at + STEP_OPERAND + wn * 16));
-      }
-      static_for<6>([&](auto prod_) {
+      for (int pl = 0; pl < 3; ++pl)
+        b[pl] = __builtin_bit_cast(v8bf, *(const lds_u4*)(at + pl * STEP_PLANE + STEP_OPERAND + wn * 16));
+      load_a(0);
+      if (OLD) load_a(1);
+      auto product = [&](auto prod_, int i) {
         constexpr int PR = decltype(prod_)::value;
-        constexpr int PA = PR == 2 || PR == 3 ? 1 : PR == 5 ? 2 : 0;
-        constexpr int PB = PR == 1 || PR == 3 ? 1 : PR == 4 ? 2 : 0;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          v16f& x = PR == 0 ? acc[i] : cor[i];
-          x = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[PA][i], b[PB], x, 0, 0, 0);
-        }
-      });
+        constexpr int PA = PR == 2 || PR == 3 || PR == 6 ? 1 : PR == 5 || PR == 7 ? 2 : 0;
+        constexpr int PB = PR == 1 || PR == 3 || PR == 7 ? 1 : PR == 4 || PR == 6 ? 2 : 0;
+        v16f& x = PR == 0 ? acc[i] : cor[i];
+        x = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[PA][i], b[PB], x, 0, 0, 0);
+      };
+      if constexpr (OLD) {
+        static_for<6>([&](auto prod_) {
+          product(prod_, 0);
+          product(prod_, 1);
+        });
+      } else {
+        // (one block after the other: the operands of both, eight products each, do not fit beside the half in flight)
+        static_for<8>([&](auto prod_) { product(prod_, 0); });
+        __builtin_amdgcn_sched_barrier(0);
+        load_a(1);
+        static_for<8>([&](auto prod_) { product(prod_, 1); });
+      }
     }
   };
   P.load(0);
   Q.load(0);
-  P.commit(sm);
-  Q.commit(sq);
+  P.template commit<!OLD>(sm);
+  Q.template commit<!OLD>(sq);
   P.load(1);
   Q.load(1);
   __syncthreads();
   products();
   __syncthreads();
-  P.commit(sm);
-  Q.commit(sq);
+  P.template commit<!OLD>(sm);
+  Q.template commit<!OLD>(sq);
   const __amdgpu_buffer_rsrc_t rc = make_rsrc(C);
   const int col = n0 + wn + r;
   float old[2][16];
@@ -954,9 +1009,33 @@ __device__ __forceinline__ void step_tile(const float* p, const float* q, float*
     }
   __syncthreads();
   products();
+  if constexpr (!OLD) {
+    static_assert(!PMK && !QMK, "step_fp32 reads consecutive m and n");
+    float probe = 0.f;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        acc[i][e] += cor[i][e];
+        probe = fmaf(acc[i][e], 0.f, probe);
+      }
+    lds_u* const votes = (lds_u*)(sm + STEP_VOTES);
+    votes[wave] = __builtin_amdgcn_ballot_w64(probe != 0.f) != 0;
+    __syncthreads();
+    unsigned any = 0;
+#pragma unroll
+    for (int w = 0; w < STEP_THREADS / 64; ++w) any |= votes[w];
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane((int)any) != 0, 0)) {
+      step_fp32(p, q, n, m0 + wm, n0 + wn, depth, acc);
+      __syncthreads();     // (a panel overwrites its own operand)
+    } else {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) acc[i] *= 1.f / (SMALL_SCALE * SMALL_SCALE);
+    }
+  }
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    add_corrections(acc[i], cor[i]);
+    if (OLD) add_corrections(acc[i], cor[i]);
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
       const int row = m0 + wm + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
@@ -1054,12 +1133,14 @@ static int step_workgroups(int nd, int tiles) { return std::min(tiles, std::max(
 
 // The row panel for launches of few tiles: the same 128x128x128 product as a tile beside a diagonal
 // block, one workgroup of 8 waves to a tile.  Alone it is a chain of latencies (93 tiles 12.7 us, 15.8
-// with 16 waves on the fp32 matrix instructions and both operands whole in LDS); beside the launches of
-// another stream what counts is that it fits into what one workgroup of the tile engine leaves: 98 KB
-// of LDS and 128 registers, where 128 KB had to wait for an empty compute unit, that is until the other
+// with 16 waves on the fp32 matrix instructions and both operands whole in LDS, and since then 66 tiles 10.6 ->
+// 11.8 for eight partial products instead of six and the vote); beside the launches of
+// another stream what counts is that it fits into what one workgroup of the tile engine leaves: 99 KiB
+// of LDS and 128 registers, where 128 KiB had to wait for an empty compute unit, that is until the other
 // launch had handed out its last tile.
 constexpr int FINE_THREADS = STEP_THREADS;
-constexpr int FINE_SMEM_BYTES = 2 * STEP_OPERAND;
+constexpr int FINE_SMEM_BYTES = STEP_VOTES + 4 * (FINE_THREADS / 64);
+static_assert(FINE_SMEM_BYTES + SplitCfg<2>::SMEM_BYTES <= 160 * 1024, "fits beside a workgroup of the tile engine");
 constexpr int FINE_MAX_TILES = 256;      // one workgroup per CU
 
 // Tile `local` of row panel p.  U[p,j] = Y_pp^T A[p,j] in place for j > p, and in a sweep, after

@@ -47,3 +47,28 @@ def test_inverse_and_factor_against_float64(ops, dev, count, sizes):
         rest = x @ m64 - torch.eye(n, dtype=torch.float64, device=dev)
         assert (rest.norm() / n ** 0.5).item() <= 2 * bound * (eig[-1] / eig[0]).item()
         assert torch.equal(xs[i], xs[i].t())
+
+
+# panels of 66 tiles in a sweep, of 240, 160 and 80 outside of one
+@pytest.mark.parametrize('count,sizes', [(33, (257, 300, 383, 384)), (80, (385, 416, 511, 512))])
+def test_matrices_of_any_magnitude(ops, dev, count, sizes):
+    """The same matrices times 2^-116 (many entries below 2^-118), 2^90 and 2^106 (beyond what the panels' elements
+    are multiplied with: computed in another way): errors as those of the matrices themselves, but for the few
+    entries that are rounded to multiples of 2^-149."""
+    distinct = [matrix(n, dev) for n in sizes]
+    eye = [torch.eye(n, dtype=torch.float64, device=dev) for n in sizes]
+
+    def errors(exponent):
+        mats = [distinct[i % len(sizes)] * 2. ** exponent for i in range(count)]
+        us, info = ops.cholesky_upper_batched(mats)
+        xs, info2 = ops.damped_inverse_batched(mats, [0.] * count)
+        assert not info.any().item() and not info2.any().item()
+        out = []
+        for i in range(count):
+            m, u, x = mats[i].double(), us[i].double(), xs[i].double()
+            out += [((u.t() @ u - m).norm() / m.norm()).item(), (x @ m - eye[i % len(sizes)]).norm().item()]
+        return torch.tensor(out)
+
+    base = errors(0)
+    for exponent in (-116, 90, 106):
+        assert (errors(exponent) / base).max().item() < 2.
