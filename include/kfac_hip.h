@@ -22,11 +22,10 @@
  *  - precision: products are float32 sums of exact products, infinities and NaN included.
  *    On 128-wide tiles (factors of more than 192 rows, k x k convolutions of stride 1 with more
  *    than 64 channels, element-wise factors of Linear layers, the updates of an inversion,
- *    preconditioning) terms
- *    below 2^-25 of a product are left out: a product that is alone in its sum is off by up to 1.7
- *    half units in the last place, where one rounding is 1.0.  There, too, an element below
- *    1.5e-33 (2^-109) enters rounded to a multiple of 2^-133: its products with large elements
- *    keep 2^-134 / |x| instead of 2^-24;
+ *    preconditioning) terms below 2^-25 of a product are left out: a product that is alone in its
+ *    sum is off by up to 1.7 half units in the last place, where one rounding is 1.0.  There, too,
+ *    an element below 1.5e-33 (2^-109) enters rounded to a multiple of 2^-133: its products with
+ *    large elements keep 2^-134 / |x| instead of 2^-24;
  *  - entry points are re-entrant: they may be called from any host thread
  *    (the backward hooks of the host code run on autograd's worker thread).
  */

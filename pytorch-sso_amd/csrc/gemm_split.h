@@ -822,6 +822,48 @@ __device__ __forceinline__ void store_blocks(const v16f (&acc)[NB], const int (&
       put(b, [&](int i, int row, int col) { epi.store(row, col, acc[b][i]); });
 }
 
+// A 64-wide tile with mirror images, a 32x32 block on each of four waves, through LDS (`smem`, free again when the sums
+// are done; the workgroup's last use of it): from the registers an image would be written by 4-byte pieces
+// of 64 rows at a time.  Results go there once (`old` values are read, and `epi` applied, for the blocks on and above
+// the diagonal only), and come back row by row.  TRI: a diagonal tile, whose upper triangle is the result.
+// Factor of 16 rows of 64 / 64 of 64 / 128 of 100: 7.2 / 8.4 / 9.5 us from the registers, 4.5 / 5.8 / 8.2 here
+// (on the fp32 instructions, whose diagonal blocks need no image, 5.4 / 7.8 / 24.1).
+constexpr int SMALL_LD = 65;
+static_assert(64 * SMALL_LD * 4 <= SplitCfg<1>::VOTES, "the result of a 64-wide tile lies where its chunks were");
+template <bool TRI, class EPI>
+__device__ __forceinline__ void store_small(const v16f& acc, int m0, int n0, int wm, int wn, float* smem,
+                                            const EPI& epi) {
+  lds_f* const t = (lds_f*)smem;
+  const int lane = threadIdx.x & 63;
+  const int row0 = wm + 4 * (lane >> 5), col = wn + (lane & 31);
+  if (!TRI || wm <= wn) {
+    float old[16];
+    bool reads = false;
+    if constexpr (reading_epilogue<EPI>::value) {
+      reads = epi.reads();
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        old[i] = reads ? epi.fetch(m0 + row0 + 8 * (i >> 2) + (i & 3), n0 + col) : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int row = row0 + 8 * (i >> 2) + (i & 3);
+      float o = epi.value(acc[i]);
+      if constexpr (reading_epilogue<EPI>::value) o = reads ? epi.value(acc[i], old[i]) : o;
+      t[row * SMALL_LD + col] = o;
+      if (!TRI) epi.put(m0 + row, n0 + col, o);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    // row r of the tile (TRI), or of its image
+    const int r = (int)(threadIdx.x >> 6) + 4 * i, c = lane;
+    if (TRI) epi.put(m0 + r, n0 + c, t[min(r, c) * SMALL_LD + max(r, c)]);
+    else epi.put(n0 + r, m0 + c, t[c * SMALL_LD + r]);
+  }
+}
+
 // a tile of a product of two operands, 64 W wide
 template <int W, class OPP, class OPQ, class STORE>
 __device__ __forceinline__ void split_tile_full(const OPP& P, const OPQ& Q, int m0, int n0, int kbeg,
@@ -832,7 +874,10 @@ __device__ __forceinline__ void split_tile_full(const OPP& P, const OPQ& Q, int 
     v16f acc[1];
     split_blocks<SmallTile>(P, Q, m0, n0, kbeg, kend, smem, SplitRows{{wm}, {wn}}, acc);
     const int row0[1] = {m0 + wm}, col0[1] = {n0 + wn}, what[1] = {BLK_PLAIN};
-    store([&](const auto& epi) { store_blocks<1>(acc, row0, col0, what, epi); });
+    store([&](const auto& epi) {
+      if (epi.mirror) store_small<false>(acc[0], m0, n0, wm, wn, smem, epi);
+      else store_blocks<1>(acc, row0, col0, what, epi);
+    });
   } else {
     v16f acc[4];
     split_blocks<SplitTile>(P, Q, m0, n0, kbeg, kend, smem, SplitRows{{wm, wm + 32}, {wn, wn + 32}}, acc);
@@ -849,15 +894,14 @@ template <int W, class OP, class STORE>
 __device__ __forceinline__ void split_tile_tri(const OP& P, int m0, int kbeg, int kend, float* smem,
                                                bool both, const STORE& store) {
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x & (SplitCfg<W>::NT - 1)) >> 6);
-  const int above = both ? BLK_BOTH : BLK_PLAIN, on = both ? BLK_UPPER_BOTH : BLK_UPPER;
   if constexpr (W == 1) {
     const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
     v16f acc[1];
     split_blocks<SmallDiag>(P, P, m0, m0, kbeg, kend, smem, SplitRows{{wm, wn}, {}}, acc);
-    const int row0[1] = {m0 + wm}, col0[1] = {m0 + wn};
-    const int what[1] = {wm == wn ? on : wm < wn ? above : (int)BLK_NONE};
-    store([&](const auto& epi) { store_blocks<1>(acc, row0, col0, what, epi); });
+    // (both triangles, always)
+    store([&](const auto& epi) { store_small<true>(acc[0], m0, m0, wm, wn, smem, epi); });
   } else {
+    const int above = both ? BLK_BOTH : BLK_PLAIN, on = both ? BLK_UPPER_BOTH : BLK_UPPER;
     const SplitTri t = split_tri(wave);
     const int r0 = 32 * t.r[0], r1 = 32 * t.r[1], r2 = 32 * t.r[2];
     v16f acc[3];

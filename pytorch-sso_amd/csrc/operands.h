@@ -285,6 +285,12 @@ struct EpiStore {
       if (mirror && row != col) C[(size_t)col * ld + row] = o;
     }
   }
+  // the two halves of a store, for epilogues that rearrange results in between
+  __device__ __forceinline__ float value(float v, float old) const { return fmaf(alpha, v, beta * old); }
+  __device__ __forceinline__ float value(float v) const { return alpha * v; }
+  __device__ __forceinline__ void put(int row, int col, float o) const {
+    if (row < M && col < N) C[(size_t)row * ld + col] = o;
+  }
   __device__ __forceinline__ void store(int row, int col, float v) const {
     if (row < M && col < N) {
       const size_t idx = (size_t)row * ld + col;
@@ -298,8 +304,11 @@ struct EpiStore {
 
 // raw partial sums of one k-split into a tile-packed workspace
 struct EpiPartial {
+  static constexpr bool mirror = false;
   float* ws;      // already offset to this (split, tile)
   int m0, n0, M, N, tn;   // tn = tile width
+  __device__ __forceinline__ float value(float v) const { return v; }
+  __device__ __forceinline__ void put(int row, int col, float o) const { store(row, col, o); }
   __device__ __forceinline__ void store(int row, int col, float v) const {
     if (row < M && col < N) ws[(row - m0) * tn + (col - n0)] = v;
   }
