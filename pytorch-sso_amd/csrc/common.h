@@ -13,7 +13,7 @@ namespace kfac {
 inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 
 // Dynamic LDS sizes are registered once per kernel (required above 64 KiB, as
-// for the 148 KiB of the diagonal-block kernel; harmless below).
+// for the 138 KiB of the diagonal-block kernel; harmless below).
 bool enable_large_lds(const void* kernel, int bytes);
 
 #define KFAC_LAUNCH_TILE2(kernel, grid, stream, ...)                                         \

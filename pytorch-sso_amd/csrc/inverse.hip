@@ -770,8 +770,8 @@ __device__ __forceinline__ bool trail_tile(int T, int row_lo, int row_hi, int lo
 // the whole group at once (nk = GROUP_BLOCKS), which cuts the read-modify-write passes over
 // the trailing matrix by that factor (a rank-128 update of a large trailing matrix is
 // bound by memory traffic, not by the matrix cores).  Taller groups cost the factors of a ResNet-50
-// more than they bring to larger matrices (height 4 / 6 / 8: 3.71 / 3.81 / 3.92 ms; 9217 / 4097 / 4097
-// and smaller 7.44 / 7.32 / 7.39), and accuracy: on the fp32 tile engine the error of the
+// more than they bring to larger matrices (height 4 / 6 / 8: 4.67 / 4.83 / 4.88 ms; 9217 / 4097 / 4097
+// and smaller 9.35 / 9.21 / 9.45), and accuracy: on the fp32 tile engine the error of the
 // inverse of a 9217^2 factor with condition number 9e2 grew from 2.2e-5 (height 1) over
 // 5.2e-5 (4; scipy's float32 LU inverse: 4.7e-5) to 1.0e-4 (16), because a deeper product
 // accumulates more terms before it meets the entry it nearly cancels.
@@ -779,8 +779,9 @@ constexpr int GROUP_BLOCKS = 4;
 // The last TAIL_BLOCKS diagonal blocks of the largest matrices form one group: the deeper
 // update of the rows beyond a group is a launch that lasts as long as one 512-deep tile
 // however few tiles it has, while the rank-128 updates of a short trailing matrix
-// fit beside the next diagonal block.  16 / 24 / 32 / 40: the factors of a ResNet-50 3.76 / 3.71 /
-// 4.00 / 4.40 ms, matrices of 9217 / 4097 / 4097 and smaller 7.48 / 7.44 / 7.35 / 7.36.
+// fit beside the next diagonal block.  16 / 24 / 32 / 40: the factors of a ResNet-50 4.60 / 4.67 /
+// 4.96 / 5.42 ms, matrices of 9217 / 4097 / 4097 and smaller 9.38 / 9.35 / 9.25 / 9.28, the Cholesky factor of
+// 3500^2 0.94 / 0.89 / 0.87 / 0.87.
 constexpr int TAIL_BLOCKS = 24;
 
 __global__ __launch_bounds__(NTHREADS, 2) void potrf_trail_kernel(const MatDesc* table, int kb0,
@@ -1198,6 +1199,7 @@ __global__ __launch_bounds__(FINE_THREADS, 4) void potrf_fine_kernel(const MatDe
 // factor of 2305^2.)
 constexpr int SUB_THREADS = 512;
 constexpr int SUB_SMEM_BYTES = DB * (128 + 32) * (int)sizeof(float);
+// (32 instead of 64: inverse of 4600^2 1856 / 1976 us, three of 2305^2 1012 / 1064)
 constexpr int SUB_MAX_TILES = 64;        // 4 workgroups per tile, one workgroup per CU
 
 __global__ __launch_bounds__(SUB_THREADS) void potrf_sub_kernel(const MatDesc* table, int p,
@@ -1565,9 +1567,11 @@ enum { MODE_INVERSE = 0, MODE_CHOLESKY = 1 };
 // 2 log2(T) + 1 launches, each as long as its longest tile, of deep products.  So the line
 // lies where the tiles of a step, about T^2 / 2 per matrix, no longer fit beside a diagonal block:
 // three per compute unit.  Recursive / sweep, one matrix of n rows, us (same step tiles):
-//     300: 191 / 164   1000: 472 / 346   2305: 1049 / 753   3500 (406 tiles): 1575 / 1367
-//     4600 (666): 2230 / 2177;   five matrices of 728 tiles in all: 2418 / 2264
-//     the layers of a ResNet-50 (several thousand): 10.8 / 12.3 ms
+//     300: 140 / 102   1000: 401 / 263   2305: 940 / 611   3500 (406 tiles): 1408 / 1075
+//     4600 (666): 2001 / 1856;   three of 2305 (570): 1042 / 1012;   five of 2200 (855): 1189 / 1265
+//     the layers of a ResNet-50 (several thousand): 4.67 / 7.32 ms
+// (between 600 and 765 tiles several matrices are better off without: four of 2305 (760) 1191 / 1276,
+// twenty of 1000 (720) 569 / 609; one of 4600 is not.)
 // (a matrix of one block has no panels: Y Y^T by its own kernel, 70 us instead of 75.)
 constexpr long SWEEP_MAX_TILES = 3 * 255;
 static bool use_sweep(const std::vector<int>& Ts) {

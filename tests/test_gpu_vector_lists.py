@@ -63,3 +63,38 @@ def test_lists_against_float64(ops, dev, count):
     out = [torch.empty_like(t) for t in v]
     ops.sqrt_batched(v, out)
     same(out, [t.double().sqrt() for t in v])
+
+
+# 130: with tensors of more blocks than a tensor's share of a launch, accessed by 4 and by 16 bytes
+@pytest.mark.parametrize('count', [8, 9, 64, 65, 130])
+def test_other_operations_against_float64(ops, dev, count):
+    def lists(seed, positive=False):
+        out = tensors(count, seed, dev, positive)
+        if count == 130:
+            big = torch.randn(300000, generator=torch.Generator().manual_seed(seed)).clamp_(-4, 4)
+            big = (big.abs() + 0.1 if positive else big).to(dev)
+            out[1], out[count - 2] = big, big[1:70002]
+            assert out[1].data_ptr() % 16 == 0 and out[count - 2].data_ptr() % 16 == 4
+        return [t.clone() if i % 5 == 1 else t for i, t in enumerate(out)]      # (aligned next to others that are not)
+
+    inv, grad = lists(11, True), lists(12)
+    want = [a.double() * b.double() for a, b in zip(inv, grad)]
+    ops.diag_precondition_batched(inv, grad)
+    same(grad, want)
+
+    x, y = lists(13), lists(14)
+    want = [torch.maximum(a.double(), b.double()) for a, b in zip(x, y)]
+    ops.max_batched(x, y)
+    same(y, want)
+
+    ema = lists(15, True)
+    for use_sqrt in (False, True):
+        out = [torch.full_like(t, float('nan')) for t in ema]
+        ops.diag_inverse_batched(ema, out, [1. + i % 3 for i in range(count)], use_sqrt)
+        same(out, [1 / ((t.double().sqrt() if use_sqrt else t.double()) + 1. + i % 3) for i, t in enumerate(ema)])
+
+    mean, std, noise = lists(16), lists(17, True), lists(18)
+    scales = [0.25 * (i % 4) for i in range(count)]
+    want = [m.double() + s * n.double() * d.double() for m, d, n, s in zip(mean, std, noise, scales)]
+    ops.diag_sample_batched(mean, std, noise, scales)
+    same(noise, want)
