@@ -474,9 +474,10 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
   // who may go ahead and who waits for whom.
   // (Eight of the nine partial products, as good as the fp32 instructions.  The ends of the range do
   // not matter here: W is part of a Cholesky factor, so the sum of the squares of a column is at most the
-  // diagonal entry below it.  No element is above 2^64; and what one below 2^-109 loses, 2^-134 times the
+  // diagonal entry below it.  No element is above 2^64; what one below 2^-108 loses, 2^-133 times the
   // other column, is below the rounding 2^-24 sqrt(S_ii S_jj) of the entry it goes to wherever S_ii is a
-  // float32 that is not zero.)
+  // float32 that is not zero; and halves of the elements keep leading sums finite that are rounded up from
+  // near the largest float32.)
   lds_vf* const pending_marks = (lds_vf*)(marks + STRIP_MARKS);
   if (pending) {
     v16f acc, cor;
@@ -494,7 +495,7 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
           unsigned x, y, z;
-          split_pair(w[g][2 * k], w[g][2 * k + 1], x, y, z);
+          split_pair(0.5f * w[g][2 * k], 0.5f * w[g][2 * k + 1], x, y, z);
           ph[g][k] = x;
           pm[g][k] = y;
           pl[g][k] = z;
@@ -541,7 +542,10 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
       add_corrections(acc, cor);
       lds_f* const at = S + (32 * bi + 4 * h) * DLD + 32 * bj + r;
 #pragma unroll
-      for (int e = 0; e < 16; ++e) at[(8 * (e >> 2) + (e & 3)) * DLD] -= acc[e];
+      for (int e = 0; e < 16; ++e) {
+        lds_f* const s = at + (8 * (e >> 2) + (e & 3)) * DLD;
+        *s = fmaf(-4.f, acc[e], *s);
+      }
       // (the compiler keeps the mark behind the accesses above, and LDS serves a wave's requests in order)
       asm volatile("" ::: "memory");
       pending_marks[wave] = 1.f;

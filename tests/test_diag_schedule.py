@@ -101,5 +101,5 @@ def test_the_kernel_takes_its_schedule_from_the_header():
                  'helper_awaits_pending'):
         assert name in block
     # marked behind the last access, awaited in front of the first one of either way through a helper's blocks
-    assert block.index('pending_marks[wave] = 1.f') > block.index('-= acc[e]')
+    assert block.index('pending_marks[wave] = 1.f') > block.index('*s = fmaf(-4.f, acc[e], *s)')
     assert block.count('settle();\n        apply(') == 2

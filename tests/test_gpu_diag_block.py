@@ -71,3 +71,17 @@ def test_values_that_are_not_finite_end_and_are_reported(ops, dev):
         assert info[6].item() == 0 and bool(torch.isfinite(outs[6]).all())
         if value != float('inf'):
             assert (info[:6] > 0).all()
+
+
+def test_entries_close_to_the_largest_float(ops, dev):
+    """A second block that the first one explains but for 1e-3: the sums of squares that the pending panel takes
+    from it lie above 0.995 of the largest float32."""
+    g = torch.Generator().manual_seed(5)
+    x = torch.randn(600, 128, generator=g, dtype=torch.float64)
+    x = torch.cat([x, x + 0.03 * torch.randn(600, 128, generator=g, dtype=torch.float64)], 1)
+    x = x / x.norm(dim=0)
+    m = (x.t() @ x * (0.9995 * torch.finfo(torch.float32).max)).float().to(dev)
+    (u,), info = ops.cholesky_upper_batched([m])
+    assert info.item() == 0 and bool(u.isfinite().all())
+    m64, u64 = m.double(), u.double()
+    assert ((u64.t() @ u64 - m64).norm() / m64.norm()).item() <= 257 * U * 16
