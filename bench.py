@@ -38,13 +38,14 @@ sys.path.insert(0, ROOT)
 
 METRIC = 'K-FAC step ms (factor+invert+precondition) & fp32 MFMA TFLOP/s, 1 MI355X'
 # Ceiling of float32 products: tiles run as six bf16 matrix products each (csrc/gemm_split.h), of
-# 2500 dense bf16 TFLOP/s.  (The diagonal blocks use the fp32 matrix instructions, 157.3 TFLOP/s; they
-# are priced against the same ceiling.)
+# 2500 dense bf16 TFLOP/s.  (The diagonal blocks use the fp32 matrix instructions, 157.3 TFLOP/s, and
+# the 64-wide tiles eight bf16 products; they are priced against the same ceiling.)
 PEAK_PRODUCT_TFLOPS = 2500. / 6.
 # rocprofv3 --pmc readings of the factor-build kernels of a resnet50 step, kept with the
 # profile summary they come from (counter runs cannot be made from inside this script):
 #   traffic_bytes_per_launch   HBM bytes per launch (FETCH_SIZE, WRITE_SIZE, calibrated)
-#   executed_flop_per_step_pmc 512 x (SQ_INSTS_VALU_MFMA_MOPS_F32 + SQ_INSTS_VALU_MFMA_MOPS_BF16 / 6)
+#   executed_flop_per_step_pmc 512 x (SQ_INSTS_VALU_MFMA_MOPS_F32 + SQ_INSTS_VALU_MFMA_MOPS_BF16 / 6,
+#                              on 64-wide tiles / 8)
 # The second one is the check on the plan arithmetic below: if the flops this script
 # derives from the library's tile / split plan differ from it by more than 3 %, the plan
 # has changed since the counters were read, and the line says so instead of quoting them.
