@@ -275,8 +275,12 @@ def inverse_precondition_executed_flops(specs, batch):
         dims += [a, g]
         dA.append(a)
         dG.append(g)
-    inv = lib.kfac_inverse_executed_flops(len(dims), _hip.int_array(dims),
-                                          _hip.int_array([fact(d) for d in dims]))
+    halved = [d for d in dA if fact(d) and d >= (KronCurvature.halved_inverse_min_dim or 1 << 30)]
+    if sum(float(d) ** 3 for d in halved) < KronCurvature.halved_inverse_min_work:
+        halved = []
+    forms = [fact(d) for d in dims]
+    forms[::2] = [2 if d in halved else f for d, f in zip(dA, forms[::2])]
+    inv = lib.kfac_inverse_executed_flops(len(dims), _hip.int_array(dims), _hip.int_array(forms))
     pre = lib.kfac_precondition_executed_flops(len(dG), _hip.int_array(dG), _hip.int_array(dA),
                                                _hip.int_array([fact(d) for d in dG]),
                                                _hip.int_array([fact(d) for d in dA]))

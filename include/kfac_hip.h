@@ -167,7 +167,8 @@ size_t kfac_inverse_workspace_bytes(int count, const int* dims);
 /* Plan query: the flops of float32 products that the batched inversion executes on the matrix
  * cores for matrices of these sizes (HOST arrays): blocked Cholesky (diagonal blocks, row panels, trailing updates
  * with whole diagonal tiles), the triangular inverse, and Y Y^T for the matrices whose
- * explicit inverse is formed (factored[i] == 0, or factored == NULL). */
+ * explicit inverse is formed (factored[i] == 0, or factored == NULL); without the last merge of the
+ * triangular inverse for those left in two halves (factored[i] == 2). */
 double kfac_inverse_executed_flops(int count, const int* dims, const int* factored);
 
 /* For every layer l:  pi = sqrt((tr A/dA) / (tr G/dG)), r = sqrt(damping[l]),
@@ -225,6 +226,29 @@ int kfac_pi_damped_inverse_factored_batched(int layers, const int* dA, const int
                                             float* const* Ainv, float* const* Ginv,
                                             float* const* Afac, float* const* Gfac, int* info,
                                             void* workspace, size_t workspace_bytes, void* stream);
+
+/* kfac_pi_damped_inverse_factored_batched, with factors of A that may be left in two halves: A_halves is
+ * a HOST array of `layers` ints, != 0 where Afac[l] may be; on return it is 1 where it is and 0
+ * elsewhere (small batches are inverted in a way that has whole factors at no extra cost; a matrix of
+ * one 128-block has no halves).  With h = 128 * floor(ceil(d / 128) / 2), such a factor
+ * holds the diagonal blocks [0, h) and [h, d) of the triangular factor Y and, at [0, h) x [h, d), that
+ * block U12 of the Cholesky factor (U^T U the damped matrix, Y = U^-1), where Y has -Y11 U12 Y22, three
+ * quarters of the work of the triangular inverse.  kfac_precondition_halves_batched applies it with the
+ * multiply-adds of a whole one; kfac_factor_complete_batched makes a whole one of it.  Replaces the same
+ * call site, torchsso/curv/curvature.py:302-312. */
+int kfac_pi_damped_inverse_halves_batched(int layers, const int* dA, const int* dG,
+                                          const float* const* A, const float* const* G,
+                                          const float* damping,
+                                          float* const* Ainv, float* const* Ginv,
+                                          float* const* Afac, float* const* Gfac,
+                                          int* A_halves, int* info,
+                                          void* workspace, size_t workspace_bytes, void* stream);
+
+/* Factors of sizes dims[i] in two halves -> whole ones, in place (what is left of
+ * KronCurvature.update_inv, torchsso/curv/curvature.py:302-312, when the inverse itself is read). */
+size_t kfac_factor_complete_workspace_bytes(int count);
+int kfac_factor_complete_batched(int count, const int* dims, float* const* factors,
+                                 void* workspace, size_t workspace_bytes, void* stream);
 
 /* dst[i] = (src[i] + damp[i]*I)^-1 for `count` symmetric positive definite
  * matrices of sizes dims[i]; damp may be NULL (no shift).  Host arrays as
@@ -303,6 +327,18 @@ int kfac_precondition_factored_batched(int layers, const int* dG, const int* dA,
                                        const int* g_factored, const int* a_factored,
                                        float* const* gradW, float* const* gradb,
                                        void* workspace, size_t workspace_bytes, void* stream);
+
+/* kfac_precondition_factored_batched where Aop[l] is a factor in two halves (see
+ * kfac_pi_damped_inverse_halves_batched) if a_halves[l] != 0 and a_factored[l] != 0.  Replaces the same
+ * call sites, torchsso/curv/cov/linear.py:69-84 and cov/conv.py:76-92. */
+size_t kfac_precondition_halves_workspace_bytes(int layers, const int* dG, const int* dA,
+                                                const int* a_halves);
+int kfac_precondition_halves_batched(int layers, const int* dG, const int* dA,
+                                     const float* const* Gop, const float* const* Aop,
+                                     const int* g_factored, const int* a_factored,
+                                     const int* a_halves,
+                                     float* const* gradW, float* const* gradb,
+                                     void* workspace, size_t workspace_bytes, void* stream);
 
 /* For every layer:  [paramW | paramb] = [meanW | meanb] + std_scale * U_G * E * U_A
  * with U_G, U_A the upper Cholesky factors of the inverses and E = noise[l], a

@@ -15,7 +15,8 @@
 //      two launches per panel), the rows beyond the group receive the whole group
 //      in one deeper product;
 //   3. Y = U^-1 by recursive doubling over the 128-blocks:
-//      Y12 = -Y11 * U12 * Y22, two MFMA products per level, log2(n/128) levels;
+//      Y12 = -Y11 * U12 * Y22, two MFMA products per level, log2(n/128) levels
+//      (without the last one for a factor that may stay in two halves, see half_cut);
 //   4. dst = Y Y^T on the MFMA tile engine (upper tiles, mirrored).
 //   Batches whose tiles fit beside a diagonal block have steps 3 and 4 done by the launches of
 //   step 2 (the sweep, potrf_step_kernel).
@@ -50,7 +51,7 @@ struct MatDesc {
   int rev;       // 1: the work matrix is src with rows and columns reversed (see run_batched)
   float* W;      // rev only: receives the upper Cholesky factor of the inverse, else nullptr
   int noinv;     // 1: the explicit inverse is not wanted, Y is the result (Y Y^T = inverse)
-  int pad;
+  int cut;       // > 0 (with noinv): Y is left in two halves, cut in front of this block
 };
 
 constexpr int SETUP_CHUNK = 48;
@@ -1517,8 +1518,15 @@ __global__ __launch_bounds__(256) void std_from_inverse_factor_kernel(const MatD
   }
 }
 
+// Two halves.  The last merge of the triangular inverse, Y12 = -Y11 U12 Y22 at depth 0, is n^3/4
+// of its n^3/3 multiply-adds; whoever applies Y to a matrix can do without it and use U12 as it is,
+//   V Y = [V1 Y11, (V2 - (V1 Y11) U12) Y22],
+// at the cost of applying Y.  Such a factor holds Y11, Y22 and, in the place of Y12, U12.
+static int half_cut(int T) { return T >> 1; }       // (segment(0, 0, T).mid)
+
 // zero the strictly lower triangle of a triangular result: of U for every matrix
-// (Cholesky-factor output), or, with `of_y`, of Y for the matrices whose result Y is
+// (Cholesky-factor output), or, with `of_y`, of Y for the matrices whose result Y is (whose
+// U12 comes to Y here where it is left in two halves)
 __global__ __launch_bounds__(256) void zero_lower_kernel(const MatDesc* table, int of_y,
                                                          const WorkList wl) {
   int mat, local;
@@ -1529,7 +1537,25 @@ __global__ __launch_bounds__(256) void zero_lower_kernel(const MatDesc* table, i
   const int n = m.n;
   const int T = m.T;
   const int bi = local / T, bj = local - bi * T;
-  if (bj > bi) return;
+  if (bj > bi) {
+    if (!of_y || bi >= m.cut || bj < m.cut) return;
+    // 16 loads in flight, then 16 stores
+    const float* const from = m.U;
+    for (int e0 = threadIdx.x; e0 < BM * BN; e0 += 256 * 16) {
+      float v[16];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        const int e = e0 + 256 * k, row = bi * BM + (e >> 7), col = bj * BN + (e & 127);
+        v[k] = col < n ? from[(size_t)row * n + col] : 0.f;
+      }
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        const int e = e0 + 256 * k, row = bi * BM + (e >> 7), col = bj * BN + (e & 127);
+        if (col < n) X[(size_t)row * n + col] = v[k];
+      }
+    }
+    return;
+  }
   for (int e = threadIdx.x; e < BM * BN; e += 256) {
     const int row = bi * BM + (e >> 7);
     const int col = bj * BN + (e & 127);
@@ -1555,6 +1581,7 @@ struct HostMat {
                           // std of Noisy K-FAC)
   float* fac = nullptr;   // non-null (then dst and std are null): deliver the inverse as its
                           // triangular factor only, Y upper with Y Y^T = inverse
+  bool halves = false;    // with fac: it may be left in two halves
 };
 
 static size_t inverse_workspace_bytes(const std::vector<int>& dims) {
@@ -1616,8 +1643,10 @@ static int run_batched(std::vector<HostMat>& mats, int mode, int* info, void* wo
   MatDesc* table = (MatDesc*)workspace;
   char* ybase = (char*)workspace + align256(nmat * sizeof(MatDesc));
   size_t yoff = 0;
-  int Tmax = 0;
-  std::vector<int> Ts(nmat);
+  std::vector<int> Ts(nmat), cuts(nmat);
+  for (int s = 0; s < nmat; ++s) Ts[s] = cdiv(mats[order[s]].n, DB);
+  const int Tmax = Ts[0];
+  const bool sweep = mode == MODE_INVERSE && use_sweep(Ts);
   bool any_pi = false;
   for (auto& h : mats) any_pi |= h.partner >= 0;
   for (int s0 = 0; s0 < nmat; s0 += SETUP_CHUNK) {
@@ -1630,7 +1659,7 @@ static int run_batched(std::vector<HostMat>& mats, int mode, int* info, void* wo
       // the slot of the workspace holds Y, or, when Y goes straight to the caller, the
       // Cholesky factor that nobody asked for
       d.noinv = h.fac != nullptr;
-      d.pad = 0;
+      d.cut = d.noinv && h.halves && !sweep ? half_cut(cdiv(h.n, DB)) : 0;
       d.U = d.noinv ? (float*)(ybase + yoff) : h.dst;
       d.Y = d.noinv ? h.fac : (float*)(ybase + yoff);
       yoff += align256((size_t)h.n * h.n * sizeof(float));
@@ -1643,8 +1672,7 @@ static int run_batched(std::vector<HostMat>& mats, int mode, int* info, void* wo
       d.trace = 0.f;
       d.rev = h.std != nullptr;
       d.W = h.std;
-      Ts[s0 + k] = d.T;
-      Tmax = std::max(Tmax, d.T);
+      cuts[s0 + k] = d.cut;
     }
     if (any_pi)
       hipLaunchKernelGGL(inv_trace_kernel, dim3(cnt), dim3(256), 0, stream, chunk, table, s0);
@@ -1682,7 +1710,6 @@ static int run_batched(std::vector<HostMat>& mats, int mode, int* info, void* wo
     hipLaunchKernelGGL(inv_copy_damp_kernel, dim3(grid), dim3(256), 0, stream, table, info, wl);
   });
 
-  const bool sweep = mode == MODE_INVERSE && use_sweep(Ts);
   // (a matrix factored back to front is written back through a reversal: its Y Y^T comes after)
   auto sweep_x = [&](int s) {
     const HostMat& h = mats[order[s]];
@@ -1786,12 +1813,15 @@ static int run_batched(std::vector<HostMat>& mats, int mode, int* info, void* wo
     while ((1 << D) < Tmax) ++D;
     const int na = active(2);
     for (int depth = D - 1; depth >= 0 && na > 0; --depth) {
-      // matrices with fewer than 2^depth blocks have no merge this deep
-      auto pairs = [&](int T) { return (1 << depth) < T ? merge_tiles(T, depth) : 0; };
-      for_worklists(na, pairs, [&](const WorkList& wl, int grid) {
+      // matrices with fewer than 2^depth blocks have no merge this deep, those left in two halves
+      // not the last one
+      auto pairs = [&](int s) {
+        return (1 << depth) < Ts[s] && (depth > 0 || cuts[s] == 0) ? merge_tiles(Ts[s], depth) : 0;
+      };
+      for_matrices(na, pairs, [&](const WorkList& wl, int grid) {
         KFAC_LAUNCH_TILE2(trtri_w_kernel, dim3(grid), stream, table, depth, wl);
       });
-      for_worklists(na, pairs, [&](const WorkList& wl, int grid) {
+      for_matrices(na, pairs, [&](const WorkList& wl, int grid) {
         KFAC_LAUNCH_TILE2(trtri_y_kernel, dim3(grid), stream, table, depth, wl);
       });
     }
@@ -1934,7 +1964,7 @@ double kfac_inverse_executed_flops(int count, const int* dims, const int* factor
     const int Ti = (int)T;
     int D = 0;
     while ((1 << D) < Ti) ++D;
-    for (int depth = 0; depth < D; ++depth)
+    for (int depth = factored && factored[i] == 2 ? 1 : 0; depth < D; ++depth)
       for (int P = 0; P < (1 << depth); ++P) {
         const Segment sg = segment(P, depth, Ti);
         const double r = sg.mid - sg.p0, c = sg.p1 - sg.mid;
@@ -2010,16 +2040,16 @@ int kfac_pi_damped_inverse_std_batched(int layers, const int* dA, const int* dG,
   return run_batched(mats, MODE_INVERSE, info, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
-int kfac_pi_damped_inverse_factored_batched(int layers, const int* dA, const int* dG,
-                                            const float* const* A, const float* const* G,
-                                            const float* damping, float* const* Ainv,
-                                            float* const* Ginv, float* const* Afac,
-                                            float* const* Gfac, int* info, void* workspace,
-                                            size_t workspace_bytes, void* stream) {
+// A_halves: NULL, or which factors of A may be left in two halves; on return, which are
+static int factored_batched(int layers, const int* dA, const int* dG, const float* const* A,
+                            const float* const* G, const float* damping, float* const* Ainv,
+                            float* const* Ginv, float* const* Afac, float* const* Gfac, int* A_halves,
+                            int* info, void* workspace, size_t workspace_bytes, hipStream_t stream) {
   if (layers < 0 || (layers > 0 && (!dA || !dG || !A || !G || !damping || !Ainv || !Ginv ||
                                     !Afac || !Gfac || !info)))
     return KFAC_ERR_ARG;
   std::vector<HostMat> mats(2 * layers);
+  std::vector<int> Ts(2 * layers);
   for (int l = 0; l < layers; ++l) {
     if (dA[l] <= 0 || dG[l] <= 0 || dA[l] > 16384 || dG[l] > 16384 || !A[l] || !G[l] ||
         !(damping[l] >= 0.f))
@@ -2030,10 +2060,86 @@ int kfac_pi_damped_inverse_factored_batched(int layers, const int* dA, const int
     if (Ainv[l] == A[l] || Afac[l] == A[l] || Ginv[l] == G[l] || Gfac[l] == G[l])
       return KFAC_ERR_ARG;
     const float r = sqrtf(damping[l]);
-    mats[2 * l] = HostMat{A[l], Ainv[l], dA[l], r, 2 * l + 1, 1, 2 * l, nullptr, Afac[l]};
+    mats[2 * l] = HostMat{A[l], Ainv[l], dA[l], r, 2 * l + 1, 1, 2 * l, nullptr, Afac[l],
+                          A_halves && A_halves[l]};
     mats[2 * l + 1] = HostMat{G[l], Ginv[l], dG[l], r, 2 * l, 0, 2 * l + 1, nullptr, Gfac[l]};
+    Ts[2 * l] = cdiv(dA[l], DB);
+    Ts[2 * l + 1] = cdiv(dG[l], DB);
   }
-  return run_batched(mats, MODE_INVERSE, info, workspace, workspace_bytes, (hipStream_t)stream);
+  // (the sweep has whole factors at no extra cost)
+  const bool whole = use_sweep(Ts);
+  for (int l = 0; A_halves && l < layers; ++l)
+    A_halves[l] = A_halves[l] && Afac[l] && !whole && half_cut(Ts[2 * l]) > 0;
+  return run_batched(mats, MODE_INVERSE, info, workspace, workspace_bytes, stream);
+}
+
+int kfac_pi_damped_inverse_factored_batched(int layers, const int* dA, const int* dG,
+                                            const float* const* A, const float* const* G,
+                                            const float* damping, float* const* Ainv,
+                                            float* const* Ginv, float* const* Afac,
+                                            float* const* Gfac, int* info, void* workspace,
+                                            size_t workspace_bytes, void* stream) {
+  return factored_batched(layers, dA, dG, A, G, damping, Ainv, Ginv, Afac, Gfac, nullptr, info,
+                          workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+int kfac_pi_damped_inverse_halves_batched(int layers, const int* dA, const int* dG,
+                                          const float* const* A, const float* const* G,
+                                          const float* damping, float* const* Ainv,
+                                          float* const* Ginv, float* const* Afac,
+                                          float* const* Gfac, int* A_halves, int* info,
+                                          void* workspace, size_t workspace_bytes, void* stream) {
+  if (layers > 0 && !A_halves) return KFAC_ERR_ARG;
+  return factored_batched(layers, dA, dG, A, G, damping, Ainv, Ginv, Afac, Gfac, A_halves, info,
+                          workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+size_t kfac_factor_complete_workspace_bytes(int count) {
+  return count > 0 ? align256((size_t)count * sizeof(MatDesc)) : 0;
+}
+
+int kfac_factor_complete_batched(int count, const int* dims, float* const* factors,
+                                 void* workspace, size_t workspace_bytes, void* stream_) {
+  if (count < 0 || (count > 0 && (!dims || !factors))) return KFAC_ERR_ARG;
+  if (count == 0) return KFAC_OK;
+  if (!workspace || workspace_bytes < kfac_factor_complete_workspace_bytes(count))
+    return KFAC_ERR_WORKSPACE;
+  for (int i = 0; i < count; ++i)
+    if (dims[i] <= 0 || dims[i] > 16384 || !factors[i]) return KFAC_ERR_ARG;
+  hipStream_t stream = (hipStream_t)stream_;
+  MatDesc* const table = (MatDesc*)workspace;
+  for (int s0 = 0; s0 < count; s0 += SETUP_CHUNK) {
+    DescChunk chunk{};
+    const int cnt = std::min(SETUP_CHUNK, count - s0);
+    for (int k = 0; k < cnt; ++k) {
+      MatDesc& d = chunk.d[k];
+      d.U = d.Y = factors[s0 + k];         // (the merge leaves W below the diagonal, and U12 is read before Y12 is written)
+      d.n = dims[s0 + k];
+      d.T = cdiv(d.n, DB);
+      d.partner = -1;
+      d.noinv = 1;
+    }
+    hipLaunchKernelGGL(inv_setup_kernel, dim3(1), dim3(SETUP_CHUNK), 0, stream, chunk, table, s0, cnt);
+  }
+  for (int s0 = 0; s0 < count; s0 += WL_MAX) {
+    auto list = [&](auto&& items) {
+      WorkList wl;
+      wl.first = s0;
+      wl.n = std::min(WL_MAX, count - s0);
+      wl.cum[0] = 0;
+      for (int i = 0; i < wl.n; ++i) wl.cum[i + 1] = wl.cum[i] + items(cdiv(dims[s0 + i], DB));
+      for (int i = wl.n + 1; i <= WL_MAX; ++i) wl.cum[i] = wl.cum[wl.n];
+      return wl;
+    };
+    const WorkList merges = list([](int T) { return T > 1 ? merge_tiles(T, 0) : 0; });
+    const WorkList tiles = list([](int T) { return T * T; });
+    if (merges.cum[merges.n] == 0) continue;
+    KFAC_LAUNCH_TILE2(trtri_w_kernel, dim3(merges.cum[merges.n]), stream, table, 0, merges);
+    KFAC_LAUNCH_TILE2(trtri_y_kernel, dim3(merges.cum[merges.n]), stream, table, 0, merges);
+    hipLaunchKernelGGL(zero_lower_kernel, dim3(tiles.cum[tiles.n]), dim3(256), 0, stream, table, 1,
+                       tiles);
+  }
+  return launch_status();
 }
 
 int kfac_cholesky_upper_batched(int count, const int* dims, const float* const* src,

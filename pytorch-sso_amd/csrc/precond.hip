@@ -27,9 +27,12 @@ struct LayerDesc {
   float* Tt;             // dA x dG scratch
   int dG, dA, dAw;       // dAw = dA - (has bias)
   float scale;
-  int flags;         // factored preconditioning: bit 0 L is Wg, bit 1 R is Wa (else the inverses)
+  int flags;         // factored preconditioning: L_FACTOR, ... (none: the inverses)
   float* parts;      // pieces of the tiles whose reduction is cut (see tile_item)
 };
+
+// what the operands of a layer are: triangular factors (else explicit inverses), R's in two halves
+enum { L_FACTOR = 1, R_FACTOR = 2, R_HALVES = 4 };
 
 constexpr int LAYER_CHUNK = 32;
 struct LayerChunk {
@@ -49,6 +52,7 @@ struct EpiSplit {
   const float* mb;
   int dG, dA, dAw;
   float scale;
+  float* copy = nullptr;     // dG x dA: the result once more, as one matrix (without means only)
   static constexpr bool reads_output = true;     // the means, when sampling
   __device__ __forceinline__ bool reads() const { return mW != nullptr; }
   __device__ __forceinline__ float fetch(int row, int col) const {
@@ -74,6 +78,7 @@ struct EpiSplit {
       } else {
         b[row] = (mb ? mb[row] : 0.f) + scale * v;
       }
+      if (copy) copy[(size_t)row * dA + col] = scale * v;
     }
   }
 };
@@ -97,6 +102,18 @@ struct EpiSplit {
 // results in between live in the two halves of the layer's scratch (T^T in the first; the
 // result of the second and third product in whichever half that product does not read).
 //
+// A factor Ya in two halves (R_HALVES) holds Y11 and Y22, the diagonal halves of Y, and in the place of
+// Y12 the block U12 of the Cholesky factor (Y12 = -Y11 U12 Y22, the last and largest product of
+// the triangular inversion, was not formed).  Its products are done in three steps, the tiles
+// of one half (PART_A), the coupling of the other half's input to their result, and the tiles of
+// the other half (PART_B):
+//   second   j in 1    T^T[a][i]  -= sum_{a' in 1} U12[a'][a] X[i][a']   a in 2    j in 2
+//   third    j in 2    X[i][a]    -= sum_{j in 2} X'[i][j] U12[a][j]     a in 1    j in 1
+// as many multiply-adds as with the whole factor.  The steps are launches of their own, shared by
+// all layers of the call; the others have all their tiles in the first.  (For Yg, whose products
+// are shorter, the launches cost more than the inversion saves: a ResNet-50 8688 instead of 8733 us a
+// step, AlexNet's layers 13876 / 13967, 4000-1500-3000-100 3147 / 2998, 4900-4900-100 6277 / 6202.)
+//
 // The reduction of a tile against a triangular operand runs from or to the tile's own
 // position along one tile index (`fast` below), so its length varies from one block to all
 // of them.  Such a layer's tiles are dispatched longest first: all tiles of the longest
@@ -117,6 +134,20 @@ struct EpiSplit {
 // applies the epilogue (precond_finish_kernel).  Piece j exists for the tiles whose
 // reduction is longer than j * pb blocks: tfast - j * pb values of `fast`.  pb == 0: no
 // reduction is cut.
+enum { PART_A = 0, COUPLING = 1, PART_B = 2, STEPS = 3 };
+__host__ __device__ inline int half_of(int T) { return T >> 1; }     // blocks of the first half
+
+// which of the T tiles along the reduction a part holds (`grows`: the reduction gets longer with the
+// tile index, so that the first half comes first); their reductions start or end where the part does
+struct TileRange {
+  int first, count;
+};
+__host__ __device__ inline TileRange part_tiles(int T, bool halves, bool grows, int part) {
+  if (!halves) return part == PART_A ? TileRange{0, T} : TileRange{0, 0};
+  const int h = half_of(T);
+  return (part == PART_A) == grows ? TileRange{0, h} : TileRange{h, T - h};
+}
+
 // work items of a layer in one product: tiles x pieces
 __host__ __device__ inline int piece_items(int tslow, int tfast, bool tri, int pb) {
   if (pb <= 0) return tslow * tfast;
@@ -195,9 +226,12 @@ __device__ __forceinline__ EpiSplit second_epilogue(const LayerDesc& m) {
 __device__ __forceinline__ EpiSplit sample_epilogue(const LayerDesc& m) {
   return EpiSplit{m.outW, m.outb, m.meanW, m.meanb, m.dG, m.dA, m.dAw, m.scale};
 }
-__device__ __forceinline__ EpiSplit third_epilogue(const LayerDesc& m) {
-  return (m.flags & 1) ? EpiSplit{m.Tt, nullptr, nullptr, nullptr, m.dG, m.dA, m.dA, 1.f}
-                       : EpiSplit{m.outW, m.outb, nullptr, nullptr, m.dG, m.dA, m.dAw, 1.f};
+// (the coupling of the third product reads its first part as one matrix)
+__device__ __forceinline__ EpiSplit third_epilogue(const LayerDesc& m, int part) {
+  return (m.flags & L_FACTOR)
+             ? EpiSplit{m.Tt, nullptr, nullptr, nullptr, m.dG, m.dA, m.dA, 1.f}
+             : EpiSplit{m.outW, m.outb, nullptr, nullptr, m.dG, m.dA, m.dAw, 1.f,
+                        (m.flags & R_HALVES) && part == PART_A ? m.Tt : nullptr};
 }
 __device__ __forceinline__ EpiSplit fourth_epilogue(const LayerDesc& m) {
   return EpiSplit{m.outW, m.outb, nullptr, nullptr, m.dG, m.dA, m.dAw, 1.f};
@@ -221,7 +255,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void precond_first_kernel(const LayerD
     tile_or_piece(m, it, bi + ta * bj, piece_count(tg, pb), pb, P, Q, bi * BM, bj * BN, m.dA, m.dG,
                   bj * BN, m.dG, epi, smem);
   } else {
-    const bool tri = m.flags & 1;
+    const bool tri = m.flags & L_FACTOR;
     const TileItem it = tile_item(local, ta, tg, tri, true, pb);
     const int bi = it.slow, bj = it.fast;            // bi over dA, bj over dG
     DenseKM P{m.V, m.vb, m.dAw, m.dA, m.vb ? 2 : 0};
@@ -233,7 +267,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void precond_first_kernel(const LayerD
 
 template <bool SAMPLE>
 __global__ __launch_bounds__(NTHREADS, 2) void precond_second_kernel(const LayerDesc* table,
-                                                                 const WorkList wl, int pb) {
+                                                                 const WorkList wl, int pb, int part) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
   int layer, local;
   work_find(wl, layer, local);
@@ -248,28 +282,30 @@ __global__ __launch_bounds__(NTHREADS, 2) void precond_second_kernel(const Layer
     tile_or_piece(m, it, bi + tg * bj, piece_count(ta, pb), pb, P, Q, bi * BM, bj * BN, m.dG, m.dA,
                   0, min(m.dA, (bj + 1) * BN), sample_epilogue(m), smem);
   } else {
-    const bool tri = m.flags & 2;
-    const TileItem it = tile_item(local, tg, ta, tri, true, pb);
-    const int bi = it.slow, bj = it.fast;            // bi over dG, bj over dA
-    tile_or_piece(m, it, bi + tg * bj, piece_count(ta, pb), pb, P, Q, bi * BM, bj * BN, m.dG, m.dA,
-                  0, tri ? min(m.dA, (bj + 1) * BN) : m.dA, second_epilogue(m), smem);
+    const bool tri = m.flags & R_FACTOR;
+    const TileRange rg = part_tiles(ta, m.flags & R_HALVES, true, part);
+    const TileItem it = tile_item(local, tg, rg.count, tri, true, pb);
+    const int bi = it.slow, bj = rg.first + it.fast; // bi over dG, bj over dA
+    tile_or_piece(m, it, bi + tg * it.fast, piece_count(rg.count, pb), pb, P, Q, bi * BM, bj * BN, m.dG,
+                  m.dA, rg.first * BM, tri ? min(m.dA, (bj + 1) * BN) : m.dA, second_epilogue(m), smem);
   }
 }
 
 // third product, layers whose R is the factor Ya:  X' = X Ya^T, reduction a >= j
 __global__ __launch_bounds__(NTHREADS, 2) void precond_third_kernel(const LayerDesc* table,
-                                                                const WorkList wl, int pb) {
+                                                                const WorkList wl, int pb, int part) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
   int layer, local;
   work_find(wl, layer, local);
   const LayerDesc m = table[layer];
   const int ta = tiles128(m.dA), tg = tiles128(m.dG);
-  const TileItem it = tile_item(local, tg, ta, true, false, pb);
-  const int bi = it.slow, bj = it.fast;              // bi over dG, bj over dA
+  const TileRange rg = part_tiles(ta, m.flags & R_HALVES, false, part);
+  const TileItem it = tile_item(local, tg, rg.count, true, false, pb);
+  const int bi = it.slow, bj = rg.first + it.fast;   // bi over dG, bj over dA
   DenseMK P{second_half(m), m.dA, m.dG};
   DenseMK Q{m.R, m.dA, m.dA};
-  tile_or_piece(m, it, bi + tg * bj, piece_count(ta, pb), pb, P, Q, bi * BM, bj * BN, m.dG, m.dA,
-                bj * BN, m.dA, third_epilogue(m), smem);
+  tile_or_piece(m, it, bi + tg * it.fast, piece_count(rg.count, pb), pb, P, Q, bi * BM, bj * BN, m.dG,
+                m.dA, bj * BN, min(m.dA, (rg.first + rg.count) * BN), third_epilogue(m, part), smem);
 }
 
 // fourth product, layers whose L is the factor Yg:  U = Yg X', reduction k >= i
@@ -283,41 +319,95 @@ __global__ __launch_bounds__(NTHREADS, 2) void precond_fourth_kernel(const Layer
   const TileItem it = tile_item(local, ta, tg, true, false, pb);
   const int bi = it.fast, bj = it.slow;              // bi over dG, bj over dA
   DenseMK P{m.L, m.dG, m.dG};
-  DenseKM Q{(m.flags & 2) ? m.Tt : second_half(m), nullptr, m.dA, m.dA, 0};
+  DenseKM Q{(m.flags & R_FACTOR) ? m.Tt : second_half(m), nullptr, m.dA, m.dA, 0};
   tile_or_piece(m, it, bj + ta * bi, piece_count(tg, pb), pb, P, Q, bi * BM, bj * BN, m.dG, m.dA,
                 bi * BM, m.dG, fourth_epilogue(m), smem);
 }
 
-// The tiles of product `product` (0..3) whose reduction was cut: pieces added up in order,
-// result through the product's epilogue.  One work item per tile of the layers that take
+// The couplings of the second (`product` 1) and third (2) product: the tiles of PART_B's input, `slow`
+// over dG and `fast` over its blocks of dA; reductions over all of PART_A, `depth` blocks.
+struct CouplingShape {
+  int first, count;              // blocks of PART_B
+  int kfirst, depth;             // of PART_A
+};
+__host__ __device__ inline CouplingShape coupling_shape(int product, int ta, int flags) {
+  const bool grows = product == 1;
+  const TileRange a = part_tiles(ta, true, grows, PART_A), b = part_tiles(ta, true, grows, PART_B);
+  return CouplingShape{b.first, flags & R_HALVES ? b.count : 0, a.first, a.count};
+}
+__device__ __forceinline__ EpiStore coupling_epilogue(const LayerDesc& m, int product) {
+  return product == 1 ? EpiStore{m.Tt, m.dG, m.dA, m.dG, -1.f, 1.f, false}
+                      : EpiStore{second_half(m), m.dA, m.dG, m.dA, -1.f, 1.f, false};
+}
+
+template <int PRODUCT>
+__global__ __launch_bounds__(NTHREADS, 2) void precond_coupling_kernel(const LayerDesc* table,
+                                                                   const WorkList wl, int pb) {
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  int layer, local;
+  work_find(wl, layer, local);
+  const LayerDesc m = table[layer];
+  const int tg = tiles128(m.dG);
+  const CouplingShape cs = coupling_shape(PRODUCT, tiles128(m.dA), m.flags);
+  const int tiles = tg * cs.count;
+  TileItem it;
+  it.pieces = piece_count(cs.depth, pb);
+  it.piece = local / tiles;
+  const int id = xcd_remap(local - it.piece * tiles, tiles);
+  it.fast = id / tg;
+  it.slow = id - it.fast * tg;
+  const int i0 = it.slow * BM, a0 = (cs.first + it.fast) * BM;
+  const int k0 = cs.kfirst * BM, k1 = min(m.dA, k0 + cs.depth * BM);
+  if constexpr (PRODUCT == 1) {
+    DenseKM P{m.R, nullptr, m.dA, m.dA, 0};
+    DenseMK Q{second_half(m), m.dA, m.dG};
+    tile_or_piece(m, it, id, it.pieces, pb, P, Q, a0, i0, m.dA, m.dG, k0, k1, coupling_epilogue(m, 1), smem);
+  } else {
+    DenseMK P{m.Tt, m.dA, m.dG};
+    DenseMK Q{m.R, m.dA, m.dA};
+    tile_or_piece(m, it, id, it.pieces, pb, P, Q, i0, a0, m.dG, m.dA, k0, k1, coupling_epilogue(m, 2), smem);
+  }
+}
+
+// The tiles of step `step` of product `product` (0..3) whose reduction was cut: pieces added up in
+// order, result through the product's epilogue.  One work item per tile of the layers that take
 // part with a triangular operand; a tile of one piece was finished by its product.
 __global__ __launch_bounds__(NTHREADS) void precond_finish_kernel(const LayerDesc* table,
                                                                   const WorkList wl, int product,
-                                                                  int pb, int sample) {
+                                                                  int step, int pb, int sample) {
   int layer, local;
   work_find(wl, layer, local);
   const LayerDesc m = table[layer];
   const int ta = tiles128(m.dA), tg = tiles128(m.dG);
+  if (step == COUPLING) {
+    const CouplingShape cs = coupling_shape(product, ta, m.flags);
+    const int pieces = piece_count(cs.depth, pb);
+    if (pieces == 1) return;
+    const int fast = local / tg, i0 = (local - fast * tg) * BM, a0 = (cs.first + fast) * BM;
+    const float* parts = m.parts + (size_t)local * pieces * (BM * BN);
+    splitk_sum(parts, pieces, product == 1 ? a0 : i0, product == 1 ? i0 : a0, coupling_epilogue(m, product));
+    return;
+  }
   // (slow, fast) as the product numbers them; `local` = slow + tslow * fast = the tile id
   const bool over_g = product == 0 || product == 3;      // the reduction runs over dG
-  const int tslow = over_g ? ta : tg, tfast = over_g ? tg : ta;
-  const int fast = local / tslow, slow = local - fast * tslow;
   const bool grows = sample ? product == 1 : product < 2;
-  const bool tri = sample || (m.flags & (over_g ? 1 : 2));
+  const TileRange rg = part_tiles(over_g ? tg : ta, !over_g && (m.flags & R_HALVES), grows, step);
+  const int tslow = over_g ? ta : tg, tfast = rg.count;
+  const int fast = local / tslow, slow = local - fast * tslow;
+  const bool tri = sample || (m.flags & (over_g ? L_FACTOR : R_FACTOR));
   const int pieces = piece_count(!tri ? tfast : (grows ? fast + 1 : tfast - fast), pb);
   if (pieces == 1) return;
   const float* parts = m.parts + (size_t)local * piece_count(tfast, pb) * (BM * BN);
   // rows of the result: dA for the first product (T^T), dG for the others
   int bi, bj;
-  if (product == 0) { bi = slow; bj = fast; }          // bi over dA, bj over dG
-  else if (product == 3) { bi = fast; bj = slow; }     // bi over dG, bj over dA
-  else { bi = slow; bj = fast; }                       // bi over dG, bj over dA
+  if (product == 3) { bi = rg.first + fast; bj = slow; }       // bi over dG, bj over dA
+  else { bi = slow; bj = rg.first + fast; }
   if (product == 0)
     splitk_sum(parts, pieces, bi * BM, bj * BN, EpiStore{m.Tt, m.dG, m.dA, m.dG, 1.f, 0.f, false});
   else if (product == 1)
     splitk_sum(parts, pieces, bi * BM, bj * BN, sample ? sample_epilogue(m) : second_epilogue(m));
   else if (product == 2)
-    splitk_sum(parts, pieces, bi * BM, bj * BN, third_epilogue(m));
+    splitk_sum(parts, pieces, bi * BM, bj * BN, third_epilogue(m, step));
   else
     splitk_sum(parts, pieces, bi * BM, bj * BN, fourth_epilogue(m));
 }
@@ -326,117 +416,128 @@ static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 constexpr int PRODUCTS = 4;
 
-// Piece size of each product from the shape of its launch.  flags == nullptr: every side of
-// every layer is a triangular factor (what the scratch is sized for).
-static void plan_pieces(int layers, const int* dG, const int* dA, const int* flags, bool any_tri,
-                        int (&pbs)[4], bool sample = false) {
-  for (int product = 0; product < 4; ++product) {
-    long work = 0;
-    int longest = 0;
-    const bool over_g = product == 0 || product == 3;
-    for (int l = 0; any_tri && !(sample && product >= 2) && l < layers; ++l) {
-      const int ta = cdiv(dA[l], BN), tg = cdiv(dG[l], BM);
-      const int f = flags ? flags[l] : 3;
-      const int tslow = over_g ? ta : tg, tfast = over_g ? tg : ta;
-      const bool tri = over_g ? (f & 1) : (f & 2);
-      if (product >= 2 && !tri) continue;
-      work += tri ? (long)tslow * tfast * (tfast + 1) / 2 : (long)tslow * tfast * tfast;
-      longest = std::max(longest, tfast);
-    }
-    pbs[product] = any_tri ? piece_blocks(work, longest) : 0;
+// what a layer does in one step of a product: `tiles` tiles with reductions of up to `longest` blocks
+// (tri: of 1 to `longest`, with `tslow` of each length), `work` blocks in all
+struct StepShape {
+  int tiles, longest, tslow;
+  bool tri;
+  long work;
+};
+static StepShape step_shape(int product, int step, int dG, int dA, int flags, bool sample) {
+  const int ta = cdiv(dA, BN), tg = cdiv(dG, BM);
+  const bool over_g = product == 0 || product == 3;
+  const bool tri = sample || (flags & (over_g ? L_FACTOR : R_FACTOR));
+  if ((product >= 2 && (!tri || sample)) || (sample && step != PART_A)) return StepShape{0, 0, 1, false, 0};
+  const bool halves = !over_g && (flags & R_HALVES);
+  if (step == COUPLING) {
+    const CouplingShape cs = coupling_shape(product, ta, flags);
+    return halves ? StepShape{tg * cs.count, cs.depth, tg, false, (long)tg * cs.count * cs.depth}
+                  : StepShape{0, 0, 1, false, 0};
   }
+  const int count = part_tiles(over_g ? tg : ta, halves, product < 2, step).count;
+  const int tslow = over_g ? ta : tg;
+  return StepShape{tslow * count, count, tslow, tri,
+                   tri ? (long)tslow * count * (count + 1) / 2 : (long)tslow * count * count};
+}
+
+// Piece size of each step of each product from the shape of its launch.  flags == nullptr: every side
+// of every layer is a triangular factor (what the scratch is sized for, but for halves).
+typedef int PieceSizes[PRODUCTS][STEPS];
+static void plan_pieces(int layers, const int* dG, const int* dA, const int* flags, PieceSizes& pbs,
+                        bool sample = false) {
+  for (int product = 0; product < PRODUCTS; ++product)
+    for (int step = 0; step < STEPS; ++step) {
+      long work = 0;
+      int longest = 0;
+      for (int l = 0; l < layers; ++l) {
+        const StepShape sh = step_shape(product, step, dG[l], dA[l], flags ? flags[l] : L_FACTOR | R_FACTOR,
+                                        sample);
+        work += sh.work;
+        longest = std::max(longest, sh.longest);
+      }
+      pbs[product][step] = piece_blocks(work, longest);
+    }
 }
 
 // floats of the piece area of a layer under the piece sizes `pbs`: room for the pieces of
 // the longest reduction, for every tile
-static size_t piece_floats(int dG, int dA, const int (&pbs)[4]) {
-  const int ta = cdiv(dA, BN), tg = cdiv(dG, BM);
-  int most = 1;
-  for (int product = 0; product < 4; ++product) {
-    const bool over_g = product == 0 || product == 3;
-    most = std::max(most, piece_count(over_g ? tg : ta, pbs[product]));
-  }
-  return most > 1 ? (size_t)ta * tg * most * (BM * BN) : 0;
+static size_t piece_floats(int dG, int dA, int flags, const PieceSizes& pbs) {
+  size_t most = 0;
+  for (int product = 0; product < PRODUCTS; ++product)
+    for (int step = 0; step < STEPS; ++step) {
+      const StepShape sh = step_shape(product, step, dG, dA, flags, false);
+      const int pieces = piece_count(sh.longest, pbs[product][step]);
+      if (pieces > 1) most = std::max(most, (size_t)sh.tiles * pieces);
+    }
+  return most * (BM * BN);
 }
 
 // scratch: the descriptor tables, then per layer dG*dA floats (twice that when
 // `factored`: a layer with a factored side keeps two results in flight) and its piece area
-static size_t precond_workspace(int layers, const int* dG, const int* dA, bool factored) {
-  size_t bytes = PRODUCTS * align256((size_t)layers * sizeof(LayerDesc));
-  // (the piece area is there for both queries: posterior sampling, which shares the query of
+// (`flags` as in plan_pieces)
+static size_t precond_workspace(int layers, const int* dG, const int* dA, bool factored, const int* flags) {
+  size_t bytes = align256((size_t)2 * layers * sizeof(LayerDesc));
+  // (the piece area is there for all queries: posterior sampling, which shares the query of
   // the explicit preconditioning, multiplies by triangular factors as well)
-  int pbs[4];
-  plan_pieces(layers, dG, dA, nullptr, true, pbs);
+  PieceSizes pbs;
+  plan_pieces(layers, dG, dA, flags, pbs);
   for (int l = 0; l < layers; ++l) {
     bytes += align256((size_t)(factored ? 2 : 1) * dG[l] * dA[l] * sizeof(float));
-    bytes += align256(piece_floats(dG[l], dA[l], pbs) * sizeof(float));
+    bytes += align256(piece_floats(dG[l], dA[l], flags ? flags[l] : L_FACTOR | R_FACTOR, pbs) * sizeof(float));
   }
   return bytes;
 }
 
-// flags: per layer, bit 0 L is the factor Yg, bit 1 R is the factor Ya (nullptr: none)
+// flags: per layer, L_FACTOR etc. (nullptr: explicit inverses); room_flags: those that the workspace
+// was sized for (see plan_pieces)
 static int run_layers(int layers, const int* dG, const int* dA, const float* const* L,
                       const float* const* R, const float* const* V, const float* const* vb,
                       const float* const* meanW, const float* const* meanb, float* const* outW,
                       float* const* outb, const int* has_bias, float scale, bool sample,
-                      const int* flags, void* workspace, size_t workspace_bytes,
-                      hipStream_t stream) {
+                      const int* flags, const int* room_flags, void* workspace,
+                      size_t workspace_bytes, hipStream_t stream) {
   if (layers == 0) return KFAC_OK;
-  if (!workspace || workspace_bytes < precond_workspace(layers, dG, dA, flags != nullptr))
+  if (!workspace || workspace_bytes < precond_workspace(layers, dG, dA, flags != nullptr, room_flags))
     return KFAC_ERR_WORKSPACE;
-  bool any[PRODUCTS] = {true, true, false, false};
-  for (int l = 0; flags && l < layers; ++l) {
-    any[2] |= (flags[l] & 2) != 0;
-    any[3] |= (flags[l] & 1) != 0;
-  }
   // Longest tiles first, so that the tail of a launch is made of short tiles: each
   // product walks the layers in the order of ITS reduction length (dG for the first and
   // fourth, dA for the second and third), through a descriptor table in that order.
   // (two orders, so two tables, one behind the other; uploaded together, which for a few
   // layers is one launch)
-  char* tbase = (char*)workspace + PRODUCTS * align256((size_t)layers * sizeof(LayerDesc));
+  char* tbase = (char*)workspace + align256((size_t)2 * layers * sizeof(LayerDesc));
   // pieces as large as the scratch was sized for, at least (the query assumed that every
   // side is a triangular factor), and none where it left no room
   const std::vector<int> no_flags(layers, 0);     // explicit inverses on both sides
-  int pbs_room[4], pbs[PRODUCTS];
-  const int* const real_flags = flags ? flags : (sample ? nullptr : no_flags.data());
-  plan_pieces(layers, dG, dA, nullptr, true, pbs_room);
-  plan_pieces(layers, dG, dA, real_flags, true, pbs, sample);
+  const int* const real_flags = flags ? flags : no_flags.data();
+  PieceSizes pbs_room, pbs;
+  plan_pieces(layers, dG, dA, room_flags, pbs_room);
+  plan_pieces(layers, dG, dA, real_flags, pbs, sample);
   for (int product = 0; product < PRODUCTS; ++product)
-    pbs[product] = pbs[product] > 0 && pbs_room[product] > 0
-                       ? std::max(pbs[product], pbs_room[product]) : 0;
+    for (int step = 0; step < STEPS; ++step) {
+      int& pb = pbs[product][step];
+      const int room = pbs_room[product][step];
+      pb = pb > 0 && room > 0 ? std::max(pb, room) : 0;
+    }
   std::vector<size_t> toff(layers), poff(layers);
   size_t off = 0;
   for (int l = 0; l < layers; ++l) {
     toff[l] = off;
     off += align256((size_t)(flags ? 2 : 1) * dG[l] * dA[l] * sizeof(float));
     poff[l] = off;
-    off += align256(piece_floats(dG[l], dA[l], pbs_room) * sizeof(float));
+    off += align256(piece_floats(dG[l], dA[l], room_flags ? room_flags[l] : L_FACTOR | R_FACTOR, pbs_room) *
+                    sizeof(float));
   }
-  // per product: is the reduction of layer l against a triangular operand, over how many
-  // blocks (tfast), with how many tiles across (tslow)
-  auto shape = [&](int product, int l, bool& takes_part, bool& tri, int& tslow, int& tfast) {
-    const int ta = cdiv(dA[l], BN), tg = cdiv(dG[l], BM);
-    const bool gfac = sample || (flags && (flags[l] & 1)), afac = sample || (flags && (flags[l] & 2));
-    const bool over_g = product == 0 || product == 3;
-    tslow = over_g ? ta : tg;
-    tfast = over_g ? tg : ta;
-    tri = over_g ? gfac : afac;
-    takes_part = product < 2 || (tri && !sample);
+  // work items of layer l in a step: its tiles x pieces
+  auto items = [&](int product, int step, int l) {
+    const StepShape sh = step_shape(product, step, dG[l], dA[l], real_flags[l], sample);
+    const int pb = pbs[product][step];
+    if (sh.tiles == 0) return 0;
+    return sh.tri ? piece_items(sh.tslow, sh.longest, true, pb) : sh.tiles * piece_count(sh.longest, pb);
   };
-  // work items of layer l in a product: its tiles x pieces, or none where it takes no part
-  auto items = [&](int product, int l) {
-    bool part, tri;
-    int tslow, tfast;
-    shape(product, l, part, tri, tslow, tfast);
-    return part ? piece_items(tslow, tfast, tri, pbs[product]) : 0;
-  };
-  // ... and in the launch that finishes the cut tiles of the product
-  auto finish_items = [&](int product, int l) {
-    bool part, tri;
-    int tslow, tfast;
-    shape(product, l, part, tri, tslow, tfast);
-    return part && piece_count(tfast, pbs[product]) > 1 ? tslow * tfast : 0;
+  // ... and in the launch that finishes the cut tiles of the step
+  auto finish_items = [&](int product, int step, int l) {
+    const StepShape sh = step_shape(product, step, dG[l], dA[l], real_flags[l], sample);
+    return piece_count(sh.longest, pbs[product][step]) > 1 ? sh.tiles : 0;
   };
   std::vector<int> by_g(layers), by_a(layers);
   for (int l = 0; l < layers; ++l) by_g[l] = by_a[l] = l;
@@ -462,54 +563,54 @@ static int run_layers(int layers, const int* dG, const int* dA, const float* con
       d.dA = dA[l];
       d.dAw = dA[l] - (has_bias[l] ? 1 : 0);
       d.scale = scale;
-      d.flags = flags ? flags[l] : 0;
+      d.flags = real_flags[l];
       d.parts = (float*)(tbase + poff[l]);
     }
     hipLaunchKernelGGL(layer_setup_kernel, dim3(1), dim3(LAYER_CHUNK), 0, stream, chunk,
                        (LayerDesc*)workspace, s0, cnt);
   }
   for (int product = 0; product < PRODUCTS; ++product) {
-    if (!any[product]) continue;
     const bool g_order = product == 0 || product == 3;
     const std::vector<int>& order = g_order ? by_g : by_a;
     LayerDesc* const table = (LayerDesc*)workspace + (g_order ? 0 : layers);
-    // every launch of a product is enqueued before any of the next one (stream order is
-    // the dependency)
-    const int pb = pbs[product];
-    for (int s0 = 0; s0 < layers; s0 += WL_MAX) {
-      WorkList wl;
-      wl.first = s0;
-      wl.n = std::min(WL_MAX, layers - s0);
-      wl.cum[0] = 0;
-      for (int i = 0; i < wl.n; ++i) wl.cum[i + 1] = wl.cum[i] + items(product, order[s0 + i]);
-      for (int i = wl.n + 1; i <= WL_MAX; ++i) wl.cum[i] = wl.cum[wl.n];
-      if (wl.cum[wl.n] == 0) continue;
-      const dim3 grid(wl.cum[wl.n]);
-      if (product == 0) {
-        if (sample) KFAC_LAUNCH_TILE2(precond_first_kernel<true>, grid, stream, table, wl, pb);
-        else KFAC_LAUNCH_TILE2(precond_first_kernel<false>, grid, stream, table, wl, pb);
-      } else if (product == 1) {
-        if (sample) KFAC_LAUNCH_TILE2(precond_second_kernel<true>, grid, stream, table, wl, pb);
-        else KFAC_LAUNCH_TILE2(precond_second_kernel<false>, grid, stream, table, wl, pb);
-      } else if (product == 2) {
-        KFAC_LAUNCH_TILE2(precond_third_kernel, grid, stream, table, wl, pb);
-      } else {
-        KFAC_LAUNCH_TILE2(precond_fourth_kernel, grid, stream, table, wl, pb);
-      }
-    }
-    if (pb > 0)
+    // `launch(worklist, grid)` for all layers, WL_MAX at a time, with count(layer) work items each
+    auto for_layers = [&](auto&& count, auto&& launch) {
       for (int s0 = 0; s0 < layers; s0 += WL_MAX) {
         WorkList wl;
         wl.first = s0;
         wl.n = std::min(WL_MAX, layers - s0);
         wl.cum[0] = 0;
-        for (int i = 0; i < wl.n; ++i)
-          wl.cum[i + 1] = wl.cum[i] + finish_items(product, order[s0 + i]);
+        for (int i = 0; i < wl.n; ++i) wl.cum[i + 1] = wl.cum[i] + count(order[s0 + i]);
         for (int i = wl.n + 1; i <= WL_MAX; ++i) wl.cum[i] = wl.cum[wl.n];
-        if (wl.cum[wl.n] == 0) continue;
-        hipLaunchKernelGGL(precond_finish_kernel, dim3(wl.cum[wl.n]), dim3(NTHREADS), 0, stream,
-                           table, wl, product, pb, sample ? 1 : 0);
+        if (wl.cum[wl.n] > 0) launch(wl, dim3(wl.cum[wl.n]));
       }
+    };
+    // every launch of a step is enqueued before any of the next one (stream order is
+    // the dependency)
+    for (int step = 0; step < STEPS; ++step) {
+      const int pb = pbs[product][step];
+      for_layers([&](int l) { return items(product, step, l); }, [&](const WorkList& wl, dim3 grid) {
+        if (step == COUPLING) {
+          if (product == 1) KFAC_LAUNCH_TILE2(precond_coupling_kernel<1>, grid, stream, table, wl, pb);
+          else KFAC_LAUNCH_TILE2(precond_coupling_kernel<2>, grid, stream, table, wl, pb);
+        } else if (product == 0) {
+          if (sample) KFAC_LAUNCH_TILE2(precond_first_kernel<true>, grid, stream, table, wl, pb);
+          else KFAC_LAUNCH_TILE2(precond_first_kernel<false>, grid, stream, table, wl, pb);
+        } else if (product == 1) {
+          if (sample) KFAC_LAUNCH_TILE2(precond_second_kernel<true>, grid, stream, table, wl, pb, step);
+          else KFAC_LAUNCH_TILE2(precond_second_kernel<false>, grid, stream, table, wl, pb, step);
+        } else if (product == 2) {
+          KFAC_LAUNCH_TILE2(precond_third_kernel, grid, stream, table, wl, pb, step);
+        } else {
+          KFAC_LAUNCH_TILE2(precond_fourth_kernel, grid, stream, table, wl, pb);
+        }
+      });
+      if (pb > 0)
+        for_layers([&](int l) { return finish_items(product, step, l); }, [&](const WorkList& wl, dim3 grid) {
+          hipLaunchKernelGGL(precond_finish_kernel, grid, dim3(NTHREADS), 0, stream, table, wl, product,
+                             step, pb, sample ? 1 : 0);
+        });
+    }
   }
   return launch_status();
 }
@@ -537,7 +638,7 @@ double kfac_precondition_executed_flops(int layers, const int* dG, const int* dA
 
 size_t kfac_precondition_workspace_bytes(int layers, const int* dG, const int* dA) {
   if (layers <= 0 || !dG || !dA) return 0;
-  return precond_workspace(layers, dG, dA, false);
+  return precond_workspace(layers, dG, dA, false, nullptr);
 }
 
 static int check_layers(int layers, const int* dG, const int* dA, const float* const* Gop,
@@ -566,12 +667,45 @@ int kfac_precondition_batched(int layers, const int* dG, const int* dA,
   if (st != KFAC_OK) return st;
   return run_layers(layers, dG, dA, Ginv, Ainv, (const float* const*)gradW,
                     (const float* const*)gradb, nullptr, nullptr, gradW, gradb, hb.data(), 1.f,
-                    false, nullptr, workspace, workspace_bytes, (hipStream_t)stream);
+                    false, nullptr, nullptr, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 size_t kfac_precondition_factored_workspace_bytes(int layers, const int* dG, const int* dA) {
   if (layers <= 0 || !dG || !dA) return 0;
-  return precond_workspace(layers, dG, dA, true);
+  return precond_workspace(layers, dG, dA, true, nullptr);
+}
+
+// what is in halves, as plan_pieces wants it (a matrix of one block has none)
+static std::vector<int> halves_room(int layers, const int* dA, const int* a_halves) {
+  std::vector<int> flags(layers, L_FACTOR | R_FACTOR);
+  for (int l = 0; l < layers; ++l)
+    if (a_halves[l] && half_of(cdiv(dA[l], BM)) > 0) flags[l] |= R_HALVES;
+  return flags;
+}
+
+size_t kfac_precondition_halves_workspace_bytes(int layers, const int* dG, const int* dA,
+                                                const int* a_halves) {
+  if (layers <= 0 || !dG || !dA || !a_halves) return 0;
+  return precond_workspace(layers, dG, dA, true, halves_room(layers, dA, a_halves).data());
+}
+
+static int precondition_factored(int layers, const int* dG, const int* dA, const float* const* Gop,
+                                 const float* const* Aop, const int* g_factored,
+                                 const int* a_factored, const int* room_flags, float* const* gradW,
+                                 float* const* gradb, void* workspace, size_t workspace_bytes,
+                                 void* stream) {
+  std::vector<int> hb;
+  const int st = check_layers(layers, dG, dA, Gop, Aop, gradW, gradb, hb);
+  if (st != KFAC_OK) return st;
+  std::vector<int> flags(layers);
+  for (int l = 0; l < layers; ++l) {
+    const bool a = !a_factored || a_factored[l];
+    flags[l] = ((!g_factored || g_factored[l]) ? L_FACTOR : 0) | (a ? R_FACTOR : 0) |
+               (a && room_flags ? room_flags[l] & R_HALVES : 0);
+  }
+  return run_layers(layers, dG, dA, Gop, Aop, (const float* const*)gradW,
+                    (const float* const*)gradb, nullptr, nullptr, gradW, gradb, hb.data(), 1.f,
+                    false, flags.data(), room_flags, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 int kfac_precondition_factored_batched(int layers, const int* dG, const int* dA,
@@ -579,15 +713,19 @@ int kfac_precondition_factored_batched(int layers, const int* dG, const int* dA,
                                        const int* g_factored, const int* a_factored,
                                        float* const* gradW, float* const* gradb, void* workspace,
                                        size_t workspace_bytes, void* stream) {
-  std::vector<int> hb;
-  const int st = check_layers(layers, dG, dA, Gop, Aop, gradW, gradb, hb);
-  if (st != KFAC_OK) return st;
-  std::vector<int> flags(layers);
-  for (int l = 0; l < layers; ++l)
-    flags[l] = ((!g_factored || g_factored[l]) ? 1 : 0) | ((!a_factored || a_factored[l]) ? 2 : 0);
-  return run_layers(layers, dG, dA, Gop, Aop, (const float* const*)gradW,
-                    (const float* const*)gradb, nullptr, nullptr, gradW, gradb, hb.data(), 1.f,
-                    false, flags.data(), workspace, workspace_bytes, (hipStream_t)stream);
+  return precondition_factored(layers, dG, dA, Gop, Aop, g_factored, a_factored, nullptr, gradW,
+                               gradb, workspace, workspace_bytes, stream);
+}
+
+int kfac_precondition_halves_batched(int layers, const int* dG, const int* dA,
+                                     const float* const* Gop, const float* const* Aop,
+                                     const int* g_factored, const int* a_factored,
+                                     const int* a_halves, float* const* gradW, float* const* gradb,
+                                     void* workspace, size_t workspace_bytes, void* stream) {
+  if (layers < 0 || (layers > 0 && (!dA || !a_halves))) return KFAC_ERR_ARG;
+  return precondition_factored(layers, dG, dA, Gop, Aop, g_factored, a_factored,
+                               halves_room(layers, dA, a_halves).data(), gradW, gradb, workspace,
+                               workspace_bytes, stream);
 }
 
 int kfac_sample_batched(int layers, const int* dG, const int* dA, const float* const* U_G,
@@ -609,7 +747,7 @@ int kfac_sample_batched(int layers, const int* dG, const int* dA, const float* c
     if (hb[l] && (!meanb[l] || dA[l] < 2)) return KFAC_ERR_ARG;
   }
   return run_layers(layers, dG, dA, U_G, U_A, noise, nullptr, meanW, meanb, paramW, paramb,
-                    hb.data(), std_scale, true, nullptr, workspace, workspace_bytes,
+                    hb.data(), std_scale, true, nullptr, nullptr, workspace, workspace_bytes,
                     (hipStream_t)stream);
 }
 

@@ -77,6 +77,11 @@ _SIGNATURES = {
     'kfac_pi_damped_inverse_factored_batched': (c_int, [c_int, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr,
                                                         c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr,
                                                         c_size, c_ptr]),
+    'kfac_pi_damped_inverse_halves_batched': (c_int, [c_int] + [c_ptr] * 11 + [c_ptr, c_size, c_ptr]),
+    'kfac_factor_complete_workspace_bytes': (c_size, [c_int]),
+    'kfac_factor_complete_batched': (c_int, [c_int, c_ptr, c_ptr, c_ptr, c_size, c_ptr]),
+    'kfac_precondition_halves_workspace_bytes': (c_size, [c_int] + [c_ptr] * 3),
+    'kfac_precondition_halves_batched': (c_int, [c_int] + [c_ptr] * 10 + [c_size, c_ptr]),
     'kfac_precondition_factored_workspace_bytes': (c_size, [c_int, c_ptr, c_ptr]),
     'kfac_precondition_factored_batched': (c_int, [c_int, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr,
                                                    c_ptr, c_ptr, c_ptr, c_size, c_ptr]),

@@ -239,8 +239,9 @@ def pi_damped_inverse_batched(As, Gs, dampings, A_invs=None, G_invs=None, info=N
 
 
 def _pi_inverse_two_outputs(entry, As, Gs, dampings, A_invs, G_invs, A_others, G_others, info,
-                            check):
-    """Common part of the pi-damped inversions that write up to two results per matrix."""
+                            check, *more):
+    """Common part of the pi-damped inversions that write up to two results per matrix (`more`:
+    arguments of the entry point between those and `info`)."""
     lib = _hip.load()
     layers = len(As)
     if layers == 0:
@@ -263,7 +264,7 @@ def _pi_inverse_two_outputs(entry, As, Gs, dampings, A_invs, G_invs, A_others, G
         layers, _hip.ints(dA), _hip.ints(dG), _hip.ptr_array(As, 'A'),
         _hip.ptr_array(Gs, 'G'), _hip.floats(dampings), _hip.ptr_array(A_invs, 'A_inv', True),
         _hip.ptr_array(G_invs, 'G_inv', True), _hip.ptr_array(A_others, 'A output', True),
-        _hip.ptr_array(G_others, 'G output', True), info.data_ptr(), _ws_ptr(ws), ws_bytes,
+        _hip.ptr_array(G_others, 'G output', True), *more, info.data_ptr(), _ws_ptr(ws), ws_bytes,
         _hip.stream_ptr(dev))
     _hip.check(st, entry)
     return info
@@ -280,22 +281,46 @@ def pi_damped_inverse_std_batched(As, Gs, dampings, A_invs, G_invs, A_stds, G_st
                                    A_invs, G_invs, A_stds, G_stds, info, check)
 
 
-def pi_damped_inverse_factored_batched(As, Gs, dampings, A_invs, G_invs, A_facs, G_facs, info=None):
+def pi_damped_inverse_factored_batched(As, Gs, dampings, A_invs, G_invs, A_facs, G_facs, info=None,
+                                       a_halves=None):
     """The pi-damped inverses, each in exactly one of two forms: the matrix itself (a tensor in
     A_invs / G_invs, None in A_facs / G_facs) or only its upper-triangular factor Y with
-    Y Y^T = inverse (the other way round), for which the explicit inverse is never formed."""
+    Y Y^T = inverse (the other way round), for which the explicit inverse is never formed.
+    `a_halves`: a list, which factors of A may be left in two halves (see
+    kfac_pi_damped_inverse_halves_batched); on return, which are."""
     def check(l, what, inv, fac):
         if (inv is None) == (fac is None):
             raise _hip.KfacHipError('layer %d: exactly one of inverse and factor must be asked for %s'
                                     % (l, what))
-    return _pi_inverse_two_outputs('kfac_pi_damped_inverse_factored_batched', As, Gs, dampings,
-                                   A_invs, G_invs, A_facs, G_facs, info, check)
+    if a_halves is None:
+        return _pi_inverse_two_outputs('kfac_pi_damped_inverse_factored_batched', As, Gs, dampings,
+                                       A_invs, G_invs, A_facs, G_facs, info, check)
+    flags = _hip.int_array([int(bool(v)) for v in a_halves])
+    info = _pi_inverse_two_outputs('kfac_pi_damped_inverse_halves_batched', As, Gs, dampings,
+                                   A_invs, G_invs, A_facs, G_facs, info, check, flags)
+    a_halves[:] = [bool(v) for v in flags]
+    return info
 
 
-def precondition_factored_batched(G_ops, A_ops, grad_ws, grad_bs, g_factored=None, a_factored=None):
+def factor_complete_batched(factors):
+    """Triangular factors in two halves -> whole ones, in place."""
+    lib = _hip.load()
+    if len(factors) == 0:
+        return
+    dev = factors[0].device
+    dims = _square_dims(factors, 'factor')
+    ws, ws_bytes = _hip.workspace(dev, lib.kfac_factor_complete_workspace_bytes(len(factors)))
+    st = lib.kfac_factor_complete_batched(len(factors), _hip.ints(dims), _hip.ptr_array(factors, 'factor'),
+                                          _ws_ptr(ws), ws_bytes, _hip.stream_ptr(dev))
+    _hip.check(st, 'kfac_factor_complete_batched')
+
+
+def precondition_factored_batched(G_ops, A_ops, grad_ws, grad_bs, g_factored=None, a_factored=None,
+                                  a_halves=None):
     """[gW | gb] <- G^-1 [gW | gb] A^-1 in place for every layer (gb may be None), with the
     inverses given by their upper-triangular factors (Y Y^T = inverse) where the flag of that
-    side is true (no flag list: all of them), and as the explicit matrices elsewhere."""
+    side is true (no flag list: all of them), and as the explicit matrices elsewhere.
+    `a_halves`: which of the factors of A are in two halves (None: none)."""
     lib = _hip.load()
     layers = len(G_ops)
     if layers == 0:
@@ -307,12 +332,17 @@ def precondition_factored_batched(G_ops, A_ops, grad_ws, grad_bs, g_factored=Non
     dGa, dAa = _hip.ints(dG), _hip.ints(dA)
     flags = [None if f is None else _hip.ints([int(bool(v)) for v in f])
              for f in (g_factored, a_factored)]
-    ws, ws_bytes = _hip.workspace(dev, lib.kfac_precondition_factored_workspace_bytes(layers, dGa, dAa))
-    st = lib.kfac_precondition_factored_batched(
+    entry, query = 'kfac_precondition_factored_batched', 'kfac_precondition_factored_workspace_bytes'
+    halves = ()
+    if a_halves is not None:
+        halves = (_hip.ints([int(bool(v)) for v in a_halves]),)
+        entry, query = 'kfac_precondition_halves_batched', 'kfac_precondition_halves_workspace_bytes'
+    ws, ws_bytes = _hip.workspace(dev, getattr(lib, query)(layers, dGa, dAa, *halves))
+    st = getattr(lib, entry)(
         layers, dGa, dAa, _hip.ptr_array(G_ops, 'G operand'), _hip.ptr_array(A_ops, 'A operand'),
-        flags[0], flags[1], _hip.ptr_array(grad_ws, 'weight grad'),
+        flags[0], flags[1], *halves, _hip.ptr_array(grad_ws, 'weight grad'),
         _hip.ptr_array(grad_bs, 'bias grad', True), _ws_ptr(ws), ws_bytes, _hip.stream_ptr(dev))
-    _hip.check(st, 'kfac_precondition_factored_batched')
+    _hip.check(st, entry)
 
 
 def damped_inverse_batched(mats, damps=None, outs=None, info=None):

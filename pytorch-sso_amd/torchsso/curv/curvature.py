@@ -270,9 +270,25 @@ class KronCurvature(Curvature):
     # a missing inverse on first access.  None: update_inv forms every inverse explicitly.
     factored_inverse_min_dim = 256
 
+    # ... and the factor of A of a layer whose inverses are renewed after every use is left in
+    # two halves, Y11 and Y22 with the Cholesky factor's block between them, where an inversion
+    # holds factors of at least this many rows of enough work in all (the sum of their rows^3): the
+    # last product of the triangular inversion, three quarters of it, is not formed, and
+    # preconditioning takes four launches more for the same multiply-adds.  In us a step, halves / whole:
+    #   layers of a ResNet-50, 64 and 48 planes (3 x 4608^3 = 2.9e11, 3 x 3456^3 = 1.2e11)  8733 / 9035, 4005 / 4087
+    #   9216-4096-4096-1000 (7.8e11) 13967 / 14868    4800-700-4900-10 (2.3e11) 3839 / 4005
+    #   3800-3800-3800-100 (1.6e11) 5487 / 5609       4900-4900-100 (2.4e11) 6202 / 6370
+    #   600-4900-600 (1.2e11) 3312 / 3321             4000-1500-3000-100 (9e10) 2998 / 2903
+    # A step with inverses it already has is slower with halves (a ResNet-50's 5983 / 5786 us), hence
+    # the rule on their use.  None: always whole.
+    halved_inverse_min_dim = 2048
+    halved_inverse_min_work = 1e11
+
     def __init__(self, *args, **kwargs):
         self._inv = None
         self._inv_factors = [None, None]
+        self._a_in_halves = False        # the factor of A's inverse is in two halves
+        self._inv_uses = 0               # preconditionings with the inverses there are
         super(KronCurvature, self).__init__(*args, **kwargs)
         self._A = None
         self._G = None
@@ -294,6 +310,9 @@ class KronCurvature(Curvature):
         if self._inv is not None:
             for k, y in enumerate(self._inv_factors):
                 if self._inv[k] is None and y is not None:
+                    if k == 0 and self._a_in_halves:
+                        _ops.factor_complete_batched([y])
+                        self._a_in_halves = False
                     self._inv[k] = _ops.factor_linear(y.t().contiguous(), False, 1.)
         return self._inv
 
@@ -301,6 +320,8 @@ class KronCurvature(Curvature):
     def inv(self, value):
         self._inv = None if value is None else list(value)
         self._inv_factors = [None, None]      # inverses given from outside have no factors
+        self._a_in_halves = False
+        self._inv_uses = 0
 
     def _inverse_outputs(self, with_std):
         """Output buffers for one update_inv of this layer, None where that output is not
@@ -564,6 +585,21 @@ def update_ema_all(curvs):
     _ops.max_batched(xs, ys)
 
 
+def _left_in_halves(kron):
+    """Which factors of A an inversion of these curvatures may leave in two halves, or None (see
+    `halved_inverse_min_dim`): those whose last inverses were used once, as these will be then."""
+    work = 0.
+    flags = []
+    for c in kron:
+        fac, low = c._inv_factors[0], c.halved_inverse_min_dim
+        half = (fac is not None and low is not None and fac.shape[0] >= low and c._inv_uses == 1
+                and fac.is_cuda)
+        flags.append(half)
+        if half:
+            work += float(fac.shape[0]) ** 3
+    return flags if work >= KronCurvature.halved_inverse_min_work and work > 0 else None
+
+
 def update_inv_all(curvs, with_std=()):
     """update_inv for every curvature: one batched pi-damped inversion for all
     Kronecker layers (reference: curvature.py:302-312), one element-wise launch
@@ -580,13 +616,22 @@ def update_inv_all(curvs, with_std=()):
     wanted = {id(c) for c in with_std}
     if kron:
         outs = [c._inverse_outputs(id(c) in wanted) for c in kron]
+        for c in kron:
+            c._a_in_halves = False
         column = lambda which, k: [o[which][k] for o in outs]
         args = ([c.ema[0] for c in kron], [c.ema[1] for c in kron], [c.damping for c in kron])
         if any(f is not None for _, facs, _ in outs for f in facs):
             # (a layer with a std to deliver has no factored side, but others may: its std
             # then takes a launch of its own below)
+            more = {}
+            halves = _left_in_halves(kron)
+            if halves is not None:
+                more['a_halves'] = halves
             info = _ops.pi_damped_inverse_factored_batched(*args, column(0, 0), column(0, 1),
-                                                           column(1, 0), column(1, 1))
+                                                           column(1, 0), column(1, 1), **more)
+            if halves is not None:
+                for c, h in zip(kron, halves):
+                    c._a_in_halves = h
             for c in kron:
                 c._info_reversed = False
                 if id(c) in wanted:
@@ -606,6 +651,7 @@ def update_inv_all(curvs, with_std=()):
                 c._info_reversed = False
         for c, status in zip(kron, info.view(-1, 2).unbind()):
             c.info = status
+            c._inv_uses = 0
     if diag:
         by_sqrt = {False: ([], [], []), True: ([], [], [])}
         for c in diag:
@@ -811,6 +857,7 @@ def precondition_all(pairs):
     in place by G^-1 [dW|db] A^-1 (reference: cov/linear.py:69-84,
     cov/conv.py:76-92) or inv * grad (curvature.py:234-238)."""
     kron = ([], [], [], [], [], [])     # G operand, A operand, gW, gb, G is a factor, A is a factor
+    a_halves = []                       # A's factor is in two halves
     dinv, dgrad = [], []
     for c, params in pairs:
         if c.kind == 'kron':
@@ -828,6 +875,8 @@ def precondition_all(pairs):
                                      fa if fa is not None else c._inv[0],
                                      w.grad, gb, fg is not None, fa is not None)):
                 lst.append(v)
+            a_halves.append(c._a_in_halves)
+            c._inv_uses += 1
         elif c.kind == 'diag':
             for p, inv in zip(params, c.inv):
                 if not p.grad.is_contiguous():
@@ -835,7 +884,9 @@ def precondition_all(pairs):
                 dinv.append(inv)
                 dgrad.append(p.grad)
         # 'full' curvatures do not precondition (reference: cov/linear.py:24-25)
-    if any(kron[4]) or any(kron[5]):
+    if any(a_halves):
+        _ops.precondition_factored_batched(*kron, a_halves=a_halves)
+    elif any(kron[4]) or any(kron[5]):
         # one call for all layers, explicit ones included: every product is then one launch
         _ops.precondition_factored_batched(*kron)
     elif kron[0]:
