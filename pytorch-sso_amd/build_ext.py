@@ -40,7 +40,7 @@ def host_command(hipcc):
              '-I' + sysconfig.get_paths()['include'], '-I' + os.path.join(root, 'include'),
              '-I' + os.path.join(root, 'include', 'torch', 'csrc', 'api', 'include'),
              '-I' + os.path.join(rocm, 'include'), '-L' + os.path.join(root, 'lib'), '-L' + os.path.join(rocm, 'lib'),
-             '-ltorch_python', '-ltorch_cpu', '-lc10', '-lamdhip64'])
+             '-ltorch_python', '-ltorch_cpu', '-lc10', '-lc10_hip', '-lamdhip64'])
 
 
 def build(verbose=True):

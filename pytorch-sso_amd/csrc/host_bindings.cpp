@@ -5,11 +5,15 @@
 //
 // A tensor is taken if it is a contiguous float32 tensor on a HIP device.  Where one is not, the
 // functions return None (or False) and the caller finds out which and raises; nothing is launched here.
+#include <ATen/ops/empty.h>
+#include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <climits>
 #include <map>
 #include <mutex>
+#include <vector>
 
 #include "../../include/kfac_hip.h"
 
@@ -114,6 +118,170 @@ PyObject* floats(PyObject*, PyObject* list) {
   });
 }
 
+// The elements of some lists of equal lengths, side by side
+struct Columns {
+  std::vector<PyObject*> lists;          // (as PySequence_Fast gives them)
+  Py_ssize_t n = 0;
+  bool ok = true;
+  Columns(PyObject* const* args, int count) {
+    for (int i = 0; i < count && ok; ++i) {
+      PyObject* const seq = PySequence_Fast(args[i], "expected a list or tuple");
+      if (!seq) {
+        ok = false;
+        return;
+      }
+      lists.push_back(seq);
+      if (i == 0) n = PySequence_Fast_GET_SIZE(seq);
+      else if (PySequence_Fast_GET_SIZE(seq) != n) ok = false;
+    }
+  }
+  ~Columns() {
+    for (PyObject* l : lists) Py_DECREF(l);
+  }
+  PyObject* at(int list, Py_ssize_t i) const { return PySequence_Fast_GET_ITEM(lists[list], i); }
+};
+const at::Tensor* tensor_of(PyObject* o) { return THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }
+PyObject* int_list(const std::vector<int64_t>& v) {
+  PyObject* const l = PyList_New((Py_ssize_t)v.size());
+  if (!l) return nullptr;
+  for (size_t i = 0; i < v.size(); ++i) {
+    PyObject* const x = PyLong_FromLongLong(v[i]);
+    if (!x) {
+      Py_DECREF(l);
+      return nullptr;
+    }
+    PyList_SET_ITEM(l, (Py_ssize_t)i, x);
+  }
+  return l;
+}
+
+// square_dims(tensors) -> their sizes, or None where one is no square matrix
+PyObject* square_dims(PyObject*, PyObject* list) {
+  return guarded([&]() -> PyObject* {
+    const Columns c(&list, 1);
+    if (!c.ok) return nullptr;
+    std::vector<int64_t> dims;
+    for (Py_ssize_t i = 0; i < c.n; ++i) {
+      const at::Tensor* const t = tensor_of(c.at(0, i));
+      if (!t || t->dim() != 2 || t->size(0) != t->size(1)) Py_RETURN_NONE;
+      dims.push_back(t->size(0));
+    }
+    return int_list(dims);
+  });
+}
+
+// outputs_fit(xs, firsts, seconds, exactly one) -> is there, for every x, a first output (with `exactly
+// one`: either of the two and not both), and are the outputs of x's shape
+PyObject* outputs_fit(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 4) {
+    PyErr_SetString(PyExc_TypeError, "outputs_fit(xs, firsts, seconds, exactly_one)");
+    return nullptr;
+  }
+  const int exactly_one = PyObject_IsTrue(args[3]);
+  if (exactly_one < 0) return nullptr;
+  return guarded([&]() -> PyObject* {
+    const Columns c(args, 3);
+    if (PyErr_Occurred()) return nullptr;
+    if (!c.ok) Py_RETURN_FALSE;
+    for (Py_ssize_t i = 0; i < c.n; ++i) {
+      const at::Tensor* const x = tensor_of(c.at(0, i));
+      if (!x) Py_RETURN_FALSE;
+      bool have[2];
+      for (int k = 0; k < 2; ++k) {
+        PyObject* const o = c.at(1 + k, i);
+        have[k] = o != Py_None;
+        const at::Tensor* const t = have[k] ? tensor_of(o) : nullptr;
+        if (have[k] && (!t || t->sizes() != x->sizes())) Py_RETURN_FALSE;
+      }
+      if (exactly_one ? have[0] == have[1] : !have[0]) Py_RETURN_FALSE;
+    }
+    Py_RETURN_TRUE;
+  });
+}
+
+// kron_dims(Ls, Rs, Ws, bs) -> (dG, dA) of layers whose weight- and bias-shaped tensors fit their factors, or None
+PyObject* kron_dims(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 4) {
+    PyErr_SetString(PyExc_TypeError, "kron_dims(Ls, Rs, Ws, bs)");
+    return nullptr;
+  }
+  return guarded([&]() -> PyObject* {
+    const Columns c(args, 4);
+    if (PyErr_Occurred()) return nullptr;
+    if (!c.ok) Py_RETURN_NONE;
+    std::vector<int64_t> dG, dA;
+    for (Py_ssize_t i = 0; i < c.n; ++i) {
+      const at::Tensor *const L = tensor_of(c.at(0, i)), *const R = tensor_of(c.at(1, i)),
+                       *const W = tensor_of(c.at(2, i));
+      const bool bias = c.at(3, i) != Py_None;
+      const at::Tensor* const b = bias ? tensor_of(c.at(3, i)) : nullptr;
+      if (!L || !R || !W || (bias && !b) || L->dim() < 1 || R->dim() < 1 || W->dim() < 1) Py_RETURN_NONE;
+      const int64_t g = L->size(0), a = R->size(0);
+      if (W->numel() != g * (a - (bias ? 1 : 0)) || W->size(0) != g || (b && b->numel() != g)) Py_RETURN_NONE;
+      dG.push_back(g);
+      dA.push_back(a);
+    }
+    PyObject* const l = int_list(dG);
+    PyObject* const r = l ? int_list(dA) : nullptr;
+    PyObject* const both = r ? PyTuple_Pack(2, l, r) : nullptr;
+    Py_XDECREF(l);
+    Py_XDECREF(r);
+    return both;
+  });
+}
+
+// rowsq_sum(address of kfac_rowsq_sum, x, channels, scale or None, shift or None) -> the sums, or None
+// where x is not what the engine takes as it is
+PyObject* rowsq_sum(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 5) {
+    PyErr_SetString(PyExc_TypeError, "rowsq_sum(function, x, channels, scale, shift)");
+    return nullptr;
+  }
+  const auto run = (decltype(&kfac_rowsq_sum))PyLong_AsVoidPtr(args[0]);
+  const long long channels = PyLong_AsLongLong(args[2]);
+  if (PyErr_Occurred()) return nullptr;
+  return guarded([&]() -> PyObject* {
+    const float* const x = (const float*)address_of(args[1]);
+    const float* const scale = args[3] == Py_None ? nullptr : (const float*)address_of(args[3]);
+    const float* const shift = args[4] == Py_None ? nullptr : (const float*)address_of(args[4]);
+    if (!run || !x || (args[3] != Py_None && !scale) || (args[4] != Py_None && !shift)) Py_RETURN_NONE;
+    const at::Tensor& t = THPVariable_Unpack(args[1]);
+    if (t.dim() < 2 || channels <= 0 || channels > INT_MAX || t.size(1) != channels || t.size(0) <= 0) Py_RETURN_NONE;
+    const int64_t rows = t.size(0) * channels, len = t.numel() / rows;
+    if (len <= 0 || len > INT_MAX) Py_RETURN_NONE;
+    const at::Tensor out = at::empty({t.size(0), (int64_t)channels}, t.options().requires_grad(false));
+    if (run(x, rows, (int)channels, (int)len, scale, shift, out.mutable_data_ptr<float>(),
+            c10::hip::getCurrentHIPStream(t.device().index()).stream()) != KFAC_OK)
+      Py_RETURN_NONE;
+    return THPVariable_Wrap(out);
+  });
+}
+
+// vectors(tensor, size, count) -> `count` new float32 vectors on the tensor's device
+PyObject* vectors(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 3 || !THPVariable_Check(args[0])) {
+    PyErr_SetString(PyExc_TypeError, "vectors(tensor, size, count)");
+    return nullptr;
+  }
+  const long long size = PyLong_AsLongLong(args[1]);
+  const long count = PyLong_AsLong(args[2]);
+  if (PyErr_Occurred()) return nullptr;
+  return guarded([&]() -> PyObject* {
+    const auto options = at::TensorOptions().dtype(at::kFloat).device(THPVariable_Unpack(args[0]).device());
+    PyObject* const l = PyList_New(count);
+    if (!l) return nullptr;
+    for (long i = 0; i < count; ++i) {
+      PyObject* const t = THPVariable_Wrap(at::empty({(int64_t)size}, options));
+      if (!t) {
+        Py_DECREF(l);
+        return nullptr;
+      }
+      PyList_SET_ITEM(l, i, t);
+    }
+    return l;
+  });
+}
+
 // update_job(address of a kfac_factor_job, x, out, prev or None, alpha, beta) -> done
 PyObject* update_job(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (nargs != 6) {
@@ -196,6 +364,11 @@ PyMethodDef methods[] = {
     {"floats", floats, METH_O, "float32 values"},
     {"update_job", KFAC_FAST(update_job), "update_job(job, x, out, prev, alpha, beta)"},
     {"jobs", jobs, METH_O, "factor jobs by address, one behind the other"},
+    {"square_dims", square_dims, METH_O, "sizes of square matrices, or None"},
+    {"outputs_fit", KFAC_FAST(outputs_fit), "outputs_fit(xs, firsts, seconds, exactly_one)"},
+    {"kron_dims", KFAC_FAST(kron_dims), "kron_dims(Ls, Rs, Ws, bs): (dG, dA), or None"},
+    {"rowsq_sum", KFAC_FAST(rowsq_sum), "rowsq_sum(function, x, channels, scale, shift): the sums, or None"},
+    {"vectors", KFAC_FAST(vectors), "vectors(tensor, size, count): new vectors on its device"},
     {"order", KFAC_FAST(order), "order(device, waiting stream, stream waited for)"},
     {nullptr, nullptr, 0, nullptr}};
 

@@ -198,8 +198,12 @@ def load():
             fn = getattr(lib, name)
             fn.restype = res
             fn.argtypes = args
+        _addresses['kfac_rowsq_sum'] = ctypes.cast(lib.kfac_rowsq_sum, ctypes.c_void_p).value
         _lib = lib
     return _lib
+
+
+_addresses = {}      # entry points that the native helpers call themselves
 
 
 def check(status, what):

@@ -136,15 +136,13 @@ def defer(device, key, job, keep, work=0., backward=False):
     queued, so that the input factors are computed beside the backward pass."""
     idx = device.index if device.index is not None else torch.cuda.current_device()
     stream = _current_stream(idx)
+    q = _deferred.get(idx)
+    if q is not None and (key in q.keys or (backward and q.forward)):
+        _run_deferred(idx)
     with _lock:
         q = _deferred.get(idx)
         if q is None:
             q = _deferred[idx] = _Queue()
-        run_first = key in q.keys or (backward and q.forward)
-    if run_first:
-        _run_deferred(idx)
-    with _lock:
-        q = _deferred[idx]
         q.keys.add(key)
         q.forward = q.forward or not backward
         q.items.append((job, keep, stream))
@@ -162,15 +160,13 @@ def defer_bn(device, key, job):
     one of a pass runs what the forward hooks have queued."""
     idx = device.index if device.index is not None else torch.cuda.current_device()
     stream = _current_stream(idx)
+    q = _deferred.get(idx)
+    if q is not None and (key in q.keys or q.forward):
+        _run_deferred(idx)
     with _lock:
         q = _deferred.get(idx)
         if q is None:
             q = _deferred[idx] = _Queue()
-        run_first = key in q.keys or q.forward
-    if run_first:
-        _run_deferred(idx)
-    with _lock:
-        q = _deferred[idx]
         q.keys.add(key)
         q.bn.append((job, stream))
         q.bn_bytes += job[0].numel() * 4
@@ -184,10 +180,8 @@ def flush_if_queued(device, key):
     """Runs the queue of `device` if it holds a product for `key` (the caller is about to
     reuse that product's job object or output buffer)."""
     idx = device.index if device.index is not None else torch.cuda.current_device()
-    with _lock:
-        q = _deferred.get(idx)
-        dup = q is not None and key in q.keys
-    if dup:
+    q = _deferred.get(idx)
+    if q is not None and key in q.keys:
         _run_deferred(idx)
 
 

@@ -199,6 +199,9 @@ def _ws_ptr(ws):
 
 
 def _square_dims(mats, what):
+    dims = None if _hip._host is None else _hip._host.square_dims(mats)
+    if dims is not None:
+        return dims
     dims = []
     for i, m in enumerate(mats):
         if m.dim() != 2 or m.shape[0] != m.shape[1]:
@@ -239,9 +242,10 @@ def pi_damped_inverse_batched(As, Gs, dampings, A_invs=None, G_invs=None, info=N
 
 
 def _pi_inverse_two_outputs(entry, As, Gs, dampings, A_invs, G_invs, A_others, G_others, info,
-                            check, *more):
-    """Common part of the pi-damped inversions that write up to two results per matrix (`more`:
-    arguments of the entry point between those and `info`)."""
+                            exactly_one, *more):
+    """Common part of the pi-damped inversions that write up to two results per matrix: the inverse
+    and possibly another one, or `exactly_one` of the two (`more`: arguments of the entry point
+    between those and `info`)."""
     lib = _hip.load()
     layers = len(As)
     if layers == 0:
@@ -250,8 +254,14 @@ def _pi_inverse_two_outputs(entry, As, Gs, dampings, A_invs, G_invs, A_others, G
     dA = _square_dims(As, 'A')
     dG = _square_dims(Gs, 'G')
     for what, srcs, invs, others in (('A', As, A_invs, A_others), ('G', Gs, G_invs, G_others)):
+        if _hip._host.outputs_fit(srcs, invs, others, exactly_one):
+            continue
         for l, (x, i, o) in enumerate(zip(srcs, invs, others)):
-            check(l, what, i, o)
+            if exactly_one and (i is None) == (o is None):
+                raise _hip.KfacHipError('layer %d: exactly one of inverse and factor must be asked '
+                                        'for %s' % (l, what))
+            if not exactly_one and i is None:
+                raise _hip.KfacHipError('layer %d: no buffer for the inverse of %s' % (l, what))
             if any(t is not None and t.shape != x.shape for t in (i, o)):
                 raise _hip.KfacHipError('layer %d: output buffers of %s have the wrong shape' % (l, what))
     if info is None:
@@ -274,11 +284,8 @@ def pi_damped_inverse_std_batched(As, Gs, dampings, A_invs, G_invs, A_stds, G_st
     """pi_damped_inverse_batched that also writes, for the matrices whose A_stds / G_stds entry
     is a tensor (None: no std for it), the upper Cholesky factor of the inverse
     (std^T std = inverse), read off the triangular inverse instead of a second factorisation."""
-    def check(l, what, inv, std):
-        if inv is None:
-            raise _hip.KfacHipError('layer %d: no buffer for the inverse of %s' % (l, what))
     return _pi_inverse_two_outputs('kfac_pi_damped_inverse_std_batched', As, Gs, dampings,
-                                   A_invs, G_invs, A_stds, G_stds, info, check)
+                                   A_invs, G_invs, A_stds, G_stds, info, False)
 
 
 def pi_damped_inverse_factored_batched(As, Gs, dampings, A_invs, G_invs, A_facs, G_facs, info=None,
@@ -288,16 +295,12 @@ def pi_damped_inverse_factored_batched(As, Gs, dampings, A_invs, G_invs, A_facs,
     Y Y^T = inverse (the other way round), for which the explicit inverse is never formed.
     `a_halves`: a list, which factors of A may be left in two halves (see
     kfac_pi_damped_inverse_halves_batched); on return, which are."""
-    def check(l, what, inv, fac):
-        if (inv is None) == (fac is None):
-            raise _hip.KfacHipError('layer %d: exactly one of inverse and factor must be asked for %s'
-                                    % (l, what))
     if a_halves is None:
         return _pi_inverse_two_outputs('kfac_pi_damped_inverse_factored_batched', As, Gs, dampings,
-                                       A_invs, G_invs, A_facs, G_facs, info, check)
+                                       A_invs, G_invs, A_facs, G_facs, info, True)
     flags = _hip.int_array([int(bool(v)) for v in a_halves])
     info = _pi_inverse_two_outputs('kfac_pi_damped_inverse_halves_batched', As, Gs, dampings,
-                                   A_invs, G_invs, A_facs, G_facs, info, check, flags)
+                                   A_invs, G_invs, A_facs, G_facs, info, True, flags)
     a_halves[:] = [bool(v) for v in flags]
     return info
 
@@ -387,6 +390,9 @@ def cholesky_upper_batched(mats, outs=None, info=None):
 
 
 def _kron_dims(Ls, Rs, Ws, bs, what):
+    dims = None if _hip._host is None else _hip._host.kron_dims(Ls, Rs, Ws, bs)
+    if dims is not None:
+        return dims
     dG, dA = [], []
     for l, (L, R, W, b) in enumerate(zip(Ls, Rs, Ws, bs)):
         g, a = L.shape[0], R.shape[0]
@@ -606,6 +612,9 @@ def sgd_update_batched(params, grads, bufs, lrs, momenta, weight_decays):
 def rowsq_sum(x, channels, scale=None, shift=None):
     """[n, c] tensor of sum over the trailing dims of ((x - shift[c]) / scale[c])^2."""
     lib = _hip.load()
+    out = _hip._host.rowsq_sum(_hip._addresses['kfac_rowsq_sum'], x, channels, scale, shift)
+    if out is not None:
+        return out
     x = x.contiguous()
     n = x.shape[0]
     if x.shape[1] != channels:
@@ -618,6 +627,14 @@ def rowsq_sum(x, channels, scale=None, shift=None):
                             out.data_ptr(), _hip.stream_ptr(x.device))
     _hip.check(st, 'kfac_rowsq_sum')
     return out
+
+
+def vectors(like, size, count):
+    """`count` new float32 vectors of `size` elements on the device of the tensor `like`."""
+    made = None if _hip._host is None else _hip._host.vectors(like, size, count)
+    if made is not None:
+        return made
+    return [torch.empty(size, dtype=torch.float32, device=like.device) for _ in range(count)]
 
 
 def bn_diag_combine(sx, sg, alpha, bias):

@@ -11,7 +11,7 @@ import torch
 import torch.nn as nn
 
 from torchsso import _lanes, _ops
-from torchsso.curv.curvature import Curvature, DiagCurvature, _attach
+from torchsso.curv.curvature import Curvature, DiagCurvature, _attach, _parameter
 
 
 class CovBatchNorm1d(Curvature):
@@ -39,13 +39,14 @@ class _DiagCovBatchNorm(DiagCurvature):
             raise TypeError('expected a BatchNorm module, got %s' % type(bn).__name__)
         out = output.detach()
         # [n, c] sums over the spatial positions of ((out - bias) / weight)^2
-        self._sx = _ops.rowsq_sum(out, bn.num_features, bn.weight.detach(), bn.bias.detach())
+        weight, bias = _parameter(bn, 'weight').detach(), _parameter(bn, 'bias').detach()
+        self._sx = _ops.rowsq_sum(out, bn.num_features, weight, bias)
         # module.data_input: x_hat, as the reference keeps it (curvature.py:123-136), only
         # on request: it costs a pass over the activation and a tensor of its size that
         # nothing here reads
         if self.expose_normalized_input:
             shape = (1, -1) + (1,) * (out.dim() - 2)
-            x_hat = (out - bn.bias.detach().view(shape)) / bn.weight.detach().view(shape)
+            x_hat = (out - bias.view(shape)) / weight.view(shape)
         else:
             x_hat = None
         _attach(module, 'data_input', x_hat)
@@ -83,10 +84,10 @@ class _DiagCovBatchNorm(DiagCurvature):
         if (_lanes.mode() == 'grouped' and device.type == 'cuda'
                 and n <= _ops.BN_BATCH_MAX_ROWS):
             g = grad_output.contiguous()
-            w = torch.empty(channels, dtype=torch.float32, device=device)
-            b = torch.empty(channels, dtype=torch.float32, device=device) if self.bias else None
-            _lanes.defer_bn(device, (id(self), 'bn'), (g, channels, self._sx, float(n), w, b))
-            self._data = [w] if b is None else [w, b]
+            data = _ops.vectors(g, channels, 2 if self.bias else 1)
+            _lanes.defer_bn(device, (id(self), 'bn'),
+                            (g, channels, self._sx, float(n), data[0], data[1] if len(data) > 1 else None))
+            self._data = data
             self._queued = True
             return
         w, b = _ops.bn_diag_cov(grad_output, channels, self._sx, float(n), self.bias)   # n^2 / n

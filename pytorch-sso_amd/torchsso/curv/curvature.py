@@ -36,11 +36,20 @@ def _attach(module, name, value):
     ResNet-50 pass)."""
     if ((value is None or type(value) is torch.Tensor)
             and type(module).__setattr__ is nn.Module.__setattr__
-            and name not in module._parameters and name not in module._buffers
-            and name not in module._modules and not hasattr(type(module), name)):
+            and (name in module.__dict__
+                 or (name not in module._parameters and name not in module._buffers
+                     and name not in module._modules))
+            and not hasattr(type(module), name)):
         module.__dict__[name] = value
     else:
         setattr(module, name, value)
+
+
+def _parameter(module, name, *default):
+    """getattr(module, name, *default) for what is a parameter as a rule, looked up where a module
+    keeps those first (getattr comes to them last)."""
+    kept = module._parameters
+    return kept[name] if name in kept else getattr(module, name, *default)
 
 
 class Curvature(object):
@@ -113,7 +122,7 @@ class Curvature(object):
 
     @property
     def bias(self):
-        return getattr(self._module, 'bias', None) is not None
+        return _parameter(self._module, 'bias', None) is not None
 
     @property
     def damping(self):
@@ -389,7 +398,7 @@ class KronCurvature(Curvature):
             # (the job object of this factor is reused from pass to pass: the engine copies
             # it when the queue runs, and a second product of a queued factor runs the queue)
             _lanes.flush_if_queued(device, (id(self), idx))
-            sig = (kind, tuple(source.shape), add_bias, tuple(sorted(geometry.items())))
+            sig = (kind, source.shape, add_bias, geometry)
             cached = self._jobs[idx]
             if cached is None or cached[0] != sig:
                 d = self._factor_dim(idx, source, kind, add_bias, geometry)
