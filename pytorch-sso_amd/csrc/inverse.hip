@@ -389,11 +389,14 @@ __device__ __forceinline__ void collect(v16f& N, const Rows r0, v16f& M, const R
 // when the last strip is: no back substitution, no doubling.  What a strip takes from the rows
 // below it goes
 //   to strip q+1 while strip q is eliminated, by the waves that then have those blocks (COLLECT);
-//   to the rows further down, in LDS, by the helping waves.
-// The finished rows of strip q are written to memory during strip q+1, by the waves that are done.
+//   to the rows further down, in LDS, by the helping waves, in the strip before those rows' own.
+// The finished rows of strip q are written to memory during strip q+1, by the collecting waves before they
+// collect, in the last strip by those without a block.
 // Bound by latency and, in the strips, by the issue of a SIMD's matrix core and vector unit, which take
 // turns: the steps of a strip take the leading wave 200 cycles each where nothing else is on its
-// SIMD.  One block alone 21.0 -> 17.1 us, with the pending panel 26.1 -> 21.2 (four waves that each
+// SIMD.  One block alone 17.5 -> 15.8 us, with the pending panel 22.1 -> 19.5, the inverse of a 2305^2 matrix
+// and its Cholesky factor 1166 -> 1075 (with the helping waves and the writes at the end of the strip that they
+// belong to); before that 21.0 -> 17.1 and 26.1 -> 21.2 (four waves that each
 // held the leaf and a second block, three barriers a strip, the pending panel on the fp32 instructions, 4-byte
 // accesses to memory); the inverse of a 2305^2 matrix and its Cholesky factor 1333 -> 1160 us.
 constexpr int DIAG_THREADS = 64 * DIAG_WAVES;
@@ -421,7 +424,7 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
   const int r = lane & 31, h = lane >> 5;
   if (t < DIAG_STEPS) steps[t] = 0.f;
   if (t < DIAG_MARKS) marks[t] = 0.f;
-  if (t < 4) taken[t] = 0;
+  if (t == 0) *taken = 0;
 
   // pending: W, tile (p-1, p) of U, all of its 128 rows, in the same round trip as the block; 8
   // consecutive k of one column a piece, wave by wave
@@ -601,11 +604,13 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
     const int c = code & 7;
     const bool in_s = c < 4;
     const bool there = in_s ? c < nq : c - 4 <= q;        // (a matrix may end in this block)
-    // first row of this strip in block column k, with the lane's row and column
-    auto rows_at = [&](int k) {
-      return (lds_vf*)((k < 4 ? S : Z) + (c0 + h) * DLD + 32 * (k & 3) + r);
+    // first row of a strip (of this one) in block column k, with the lane's row and column
+    auto rows_in = [&](int strip, int k) {
+      return (lds_vf*)((k < 4 ? S : Z) + (32 * strip + h) * DLD + 32 * (k & 3) + r);
     };
-    auto marks_at = [&](int k) { return (lds_vf*)(marks + (8 * q + k) * 8); };
+    auto marks_in = [&](int strip, int k) { return (lds_vf*)(marks + (8 * strip + k) * 8); };
+    auto rows_at = [&](int k) { return rows_in(q, k); };
+    auto marks_at = [&](int k) { return marks_in(q, k); };
     lds_vf2* const step = (lds_vf2*)(steps + 64 * q);
     lds_vf* const op = (lds_vf*)(ops + lane);
     if (code == 1) {
@@ -636,6 +641,11 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
       }
     } else if (code >= 16) {
       __builtin_amdgcn_s_setprio(1);
+      // the rows of the strip above to memory first, a quarter each: what is to be collected comes later
+      if (q > 0) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) write_item(q - 1, 4 * (c - q - 1) + k);
+      }
       const Rows from{rows_at(q + 1), rows_at(c), marks_at(q + 1), marks_at(c)};
       if (there && q + 1 < nq) collect<false>(N, from, N, from);
     } else if (code >= 8) {
@@ -661,57 +671,54 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
       }
     } else if (code >= 2) {
       __builtin_amdgcn_s_setprio(0);
-      // what this strip takes from the rows further down
-      int found = 0, i0 = 0, k0 = 0, i1 = 0, k1 = 0;
-      helped_blocks(q, nq, code - 2, [&](int i, int col) {
-        i1 = i;
-        k1 = col;
-        i0 = found ? i0 : i1;
-        k0 = found ? k0 : k1;
-        ++found;
-      });
-      auto rows_of = [&](int i, int col) {
-        return Rows{rows_at(i), rows_at(col), marks_at(i), marks_at(col)};
+      // what the strips above this one take from a block of the next one (their rows are all there)
+      int i = 0, col = 0;
+      if (q > 0)
+        helped_blocks(q - 1, nq, code - 2, [&](int row, int c) {
+          i = row == q + 1 ? row : i;
+          col = row == q + 1 ? c : col;
+        });
+      auto rows_of = [&](int strip) {
+        return Rows{rows_in(strip, i), rows_in(strip, col), marks_in(strip, i), marks_in(strip, col)};
       };
       // (the waves that applied the pending panel end, and wait for nobody behind its last barrier; a
-      // mark apiece, read by lane.  The blocks are read and written behind this.)
+      // mark apiece, read by lane.  The block is read and written behind this.)
       auto settle = [&]() {
-        if (!pending || !helper_awaits_pending(q)) return;
+        if (!pending || !helper_awaits_pending(q - 1)) return;
         const lds_vf* const mark = pending_marks + min(lane, PENDING_WAVES - 1);
         while (__builtin_amdgcn_ballot_w64(__builtin_bit_cast(int, (float)*mark) == 0) != 0) {
         }
         asm volatile("" ::: "memory");
       };
-      auto apply = [&](int i, int col, const v16f& x) {
+      auto apply = [&](const v16f& x) {
         lds_f* const at = block_at(col < 4, i, col & 3);
-        // (a block of Z below the diagonal starts at zero: the strip of its column is the
-        // first to update it, and finds it uninitialised)
-        const bool fresh = col == 4 + q;
+        // (a block of Z below the diagonal starts at zero, and finds it uninitialised)
         float old[16];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) old[e] = fresh ? 0.f : at[(8 * (e >> 2) + (e & 3)) * DLD];
+        for (int e = 0; e < 16; ++e) old[e] = col < 4 ? at[(8 * (e >> 2) + (e & 3)) * DLD] : 0.f;
 #pragma unroll
         for (int e = 0; e < 16; ++e) at[(8 * (e >> 2) + (e & 3)) * DLD] = old[e] - x[e];
       };
-      if (found == 2) {
+      // (block column 4 + c of Z has rows from strip c on)
+      if (i > 0 && q > 1 && col <= 4) {
         v16f x, y;
-        collect<true>(x, rows_of(i0, k0), y, rows_of(i1, k1));
+        collect<true>(x, rows_of(q - 1), y, rows_of(q - 2));
+        x += y;
         settle();
-        apply(i0, k0, x);
-        apply(i1, k1, y);
-      } else if (found == 1) {
+        apply(x);
+      } else if (i > 0) {
         v16f x;
-        collect<false>(x, rows_of(i0, k0), x, rows_of(i0, k0));
+        collect<false>(x, rows_of(q - 1), x, rows_of(q - 1));
         settle();
-        apply(i0, k0, x);
+        apply(x);
       }
     }
-    // the rows of the strip above to memory, by whoever is done
-    if (q > 0) {
+    // (in the last strip of a whole block, which nobody collects from, by the waves without a block)
+    if (q == 3 && code < 8 && code != 1) {
       for (;;) {
         int item = 0;
         if (lane == 0)
-          item = __hip_atomic_fetch_add(taken + q, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          item = __hip_atomic_fetch_add(taken, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         item = __builtin_amdgcn_readfirstlane(item);
         if (item >= WRITE_ITEMS) break;
         write_item(q - 1, item);
