@@ -228,9 +228,9 @@ int kfac_pi_damped_inverse_factored_batched(int layers, const int* dA, const int
                                             void* workspace, size_t workspace_bytes, void* stream);
 
 /* kfac_pi_damped_inverse_factored_batched, with factors of A that may be left in two halves: A_halves is
- * a HOST array of `layers` ints, != 0 where Afac[l] may be; on return it is 1 where it is and 0
- * elsewhere (small batches are inverted in a way that has whole factors at no extra cost; a matrix of
- * one 128-block has no halves).  With h = 128 * floor(ceil(d / 128) / 2), such a factor
+ * a HOST array of `layers` ints, 1 where Afac[l] may be and 2 where it has to be; on return it is 1 where
+ * it is and 0 elsewhere (small batches are inverted in a way that has whole factors at no extra cost,
+ * unless one has to be in halves; a matrix of one 128-block has no halves).  With h = 128 * floor(ceil(d / 128) / 2), such a factor
  * holds the diagonal blocks [0, h) and [h, d) of the triangular factor Y and, at [0, h) x [h, d), that
  * block U12 of the Cholesky factor (U^T U the damped matrix, Y = U^-1), where Y has -Y11 U12 Y22, three
  * quarters of the work of the triangular inverse.  kfac_precondition_halves_batched applies it with the

@@ -1588,7 +1588,7 @@ struct HostMat {
                           // std of Noisy K-FAC)
   float* fac = nullptr;   // non-null (then dst and std are null): deliver the inverse as its
                           // triangular factor only, Y upper with Y Y^T = inverse
-  bool halves = false;    // with fac: it may be left in two halves
+  int halves = 0;         // with fac: 1 it may be left in two halves, 2 it has to be
 };
 
 static size_t inverse_workspace_bytes(const std::vector<int>& dims) {
@@ -1653,7 +1653,9 @@ static int run_batched(std::vector<HostMat>& mats, int mode, int* info, void* wo
   std::vector<int> Ts(nmat), cuts(nmat);
   for (int s = 0; s < nmat; ++s) Ts[s] = cdiv(mats[order[s]].n, DB);
   const int Tmax = Ts[0];
-  const bool sweep = mode == MODE_INVERSE && use_sweep(Ts);
+  bool any_cut = false;
+  for (int s = 0; s < nmat; ++s) any_cut |= mats[order[s]].halves == 2;
+  const bool sweep = mode == MODE_INVERSE && !any_cut && use_sweep(Ts);
   bool any_pi = false;
   for (auto& h : mats) any_pi |= h.partner >= 0;
   for (int s0 = 0; s0 < nmat; s0 += SETUP_CHUNK) {
@@ -2047,7 +2049,7 @@ int kfac_pi_damped_inverse_std_batched(int layers, const int* dA, const int* dG,
   return run_batched(mats, MODE_INVERSE, info, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
-// A_halves: NULL, or which factors of A may be left in two halves; on return, which are
+// A_halves: NULL, or which factors of A may (1) or have to (2) be left in two halves; on return, which are
 static int factored_batched(int layers, const int* dA, const int* dG, const float* const* A,
                             const float* const* G, const float* damping, float* const* Ainv,
                             float* const* Ginv, float* const* Afac, float* const* Gfac, int* A_halves,
@@ -2057,6 +2059,7 @@ static int factored_batched(int layers, const int* dA, const int* dG, const floa
     return KFAC_ERR_ARG;
   std::vector<HostMat> mats(2 * layers);
   std::vector<int> Ts(2 * layers);
+  bool any_cut = false;
   for (int l = 0; l < layers; ++l) {
     if (dA[l] <= 0 || dG[l] <= 0 || dA[l] > 16384 || dG[l] > 16384 || !A[l] || !G[l] ||
         !(damping[l] >= 0.f))
@@ -2068,15 +2071,15 @@ static int factored_batched(int layers, const int* dA, const int* dG, const floa
       return KFAC_ERR_ARG;
     const float r = sqrtf(damping[l]);
     mats[2 * l] = HostMat{A[l], Ainv[l], dA[l], r, 2 * l + 1, 1, 2 * l, nullptr, Afac[l],
-                          A_halves && A_halves[l]};
+                          A_halves && Afac[l] && half_cut(cdiv(dA[l], DB)) > 0 ? A_halves[l] : 0};
+    any_cut |= mats[2 * l].halves == 2;
     mats[2 * l + 1] = HostMat{G[l], Ginv[l], dG[l], r, 2 * l, 0, 2 * l + 1, nullptr, Gfac[l]};
     Ts[2 * l] = cdiv(dA[l], DB);
     Ts[2 * l + 1] = cdiv(dG[l], DB);
   }
   // (the sweep has whole factors at no extra cost)
-  const bool whole = use_sweep(Ts);
-  for (int l = 0; A_halves && l < layers; ++l)
-    A_halves[l] = A_halves[l] && Afac[l] && !whole && half_cut(Ts[2 * l]) > 0;
+  const bool whole = !any_cut && use_sweep(Ts);
+  for (int l = 0; A_halves && l < layers; ++l) A_halves[l] = mats[2 * l].halves && !whole;
   return run_batched(mats, MODE_INVERSE, info, workspace, workspace_bytes, stream);
 }
 

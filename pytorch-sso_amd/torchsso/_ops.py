@@ -293,12 +293,12 @@ def pi_damped_inverse_factored_batched(As, Gs, dampings, A_invs, G_invs, A_facs,
     """The pi-damped inverses, each in exactly one of two forms: the matrix itself (a tensor in
     A_invs / G_invs, None in A_facs / G_facs) or only its upper-triangular factor Y with
     Y Y^T = inverse (the other way round), for which the explicit inverse is never formed.
-    `a_halves`: a list, which factors of A may be left in two halves (see
+    `a_halves`: a list, which factors of A may (1) or have to (2) be left in two halves (see
     kfac_pi_damped_inverse_halves_batched); on return, which are."""
     if a_halves is None:
         return _pi_inverse_two_outputs('kfac_pi_damped_inverse_factored_batched', As, Gs, dampings,
                                        A_invs, G_invs, A_facs, G_facs, info, True)
-    flags = _hip.int_array([int(bool(v)) for v in a_halves])
+    flags = _hip.int_array([int(v) for v in a_halves])
     info = _pi_inverse_two_outputs('kfac_pi_damped_inverse_halves_batched', As, Gs, dampings,
                                    A_invs, G_invs, A_facs, G_facs, info, True, flags)
     a_halves[:] = [bool(v) for v in flags]

@@ -293,11 +293,16 @@ class KronCurvature(Curvature):
     halved_inverse_min_dim = 2048
     halved_inverse_min_work = 1e11
 
+    # (on the class, for objects that were pickled before they had these)
+    _a_in_halves = False        # the factor of A's inverse is in two halves
+    _inv_uses = 0               # preconditionings with the inverses there are
+    # ... the form that a recorded graph has to find and leave it in: a graph that inverts or preconditions
+    # does at every replay what it did when it was captured, so that neither may change from then on
+    _form_captured = None
+
     def __init__(self, *args, **kwargs):
         self._inv = None
         self._inv_factors = [None, None]
-        self._a_in_halves = False        # the factor of A's inverse is in two halves
-        self._inv_uses = 0               # preconditionings with the inverses there are
         super(KronCurvature, self).__init__(*args, **kwargs)
         self._A = None
         self._G = None
@@ -320,8 +325,10 @@ class KronCurvature(Curvature):
             for k, y in enumerate(self._inv_factors):
                 if self._inv[k] is None and y is not None:
                     if k == 0 and self._a_in_halves:
+                        # (a copy: to read the inverse under another stream, or from another thread, writes
+                        # nothing that preconditioning reads)
+                        y = y.clone()
                         _ops.factor_complete_batched([y])
-                        self._a_in_halves = False
                     self._inv[k] = _ops.factor_linear(y.t().contiguous(), False, 1.)
         return self._inv
 
@@ -594,19 +601,33 @@ def update_ema_all(curvs):
     _ops.max_batched(xs, ys)
 
 
+def _keep_captured_forms(kron):
+    """Where the current stream is being captured: the factors stay in the form that they have (see
+    `KronCurvature._form_captured`)."""
+    if torch.cuda.is_initialized() and torch.cuda.is_current_stream_capturing():
+        for c in kron:
+            if c._form_captured is None:
+                c._form_captured = c._a_in_halves
+
+
 def _left_in_halves(kron):
-    """Which factors of A an inversion of these curvatures may leave in two halves, or None (see
-    `halved_inverse_min_dim`): those whose last inverses were used once, as these will be then."""
+    """Which factors of A an inversion of these curvatures may (1) or has to (2) leave in two halves, or
+    None (see `halved_inverse_min_dim`): those whose last inverses were used once, as these will be then."""
     work = 0.
     flags = []
     for c in kron:
         fac, low = c._inv_factors[0], c.halved_inverse_min_dim
-        half = (fac is not None and low is not None and fac.shape[0] >= low and c._inv_uses == 1
-                and fac.is_cuda)
-        flags.append(half)
-        if half:
+        half = 0
+        if fac is not None and c._form_captured is not None:
+            half = 2 if c._form_captured else 0
+        elif (fac is not None and low is not None and fac.shape[0] >= low and c._inv_uses == 1
+                and fac.is_cuda):
+            half = 1
             work += float(fac.shape[0]) ** 3
-    return flags if work >= KronCurvature.halved_inverse_min_work and work > 0 else None
+        flags.append(half)
+    if work < KronCurvature.halved_inverse_min_work:
+        flags = [half if half == 2 else 0 for half in flags]
+    return flags if any(flags) else None
 
 
 def update_inv_all(curvs, with_std=()):
@@ -624,9 +645,9 @@ def update_inv_all(curvs, with_std=()):
     full = [c for c in curvs if c.kind == 'full']
     wanted = {id(c) for c in with_std}
     if kron:
+        _keep_captured_forms(kron)
         outs = [c._inverse_outputs(id(c) in wanted) for c in kron]
-        for c in kron:
-            c._a_in_halves = False
+        halves = None
         column = lambda which, k: [o[which][k] for o in outs]
         args = ([c.ema[0] for c in kron], [c.ema[1] for c in kron], [c.damping for c in kron])
         if any(f is not None for _, facs, _ in outs for f in facs):
@@ -638,9 +659,6 @@ def update_inv_all(curvs, with_std=()):
                 more['a_halves'] = halves
             info = _ops.pi_damped_inverse_factored_batched(*args, column(0, 0), column(0, 1),
                                                            column(1, 0), column(1, 1), **more)
-            if halves is not None:
-                for c, h in zip(kron, halves):
-                    c._a_in_halves = h
             for c in kron:
                 c._info_reversed = False
                 if id(c) in wanted:
@@ -658,8 +676,9 @@ def update_inv_all(curvs, with_std=()):
             _, _, info = _ops.pi_damped_inverse_batched(*args, column(0, 0), column(0, 1))
             for c in kron:
                 c._info_reversed = False
-        for c, status in zip(kron, info.view(-1, 2).unbind()):
+        for c, status, half in zip(kron, info.view(-1, 2).unbind(), halves or [False] * len(kron)):
             c.info = status
+            c._a_in_halves = half
             c._inv_uses = 0
     if diag:
         by_sqrt = {False: ([], [], []), True: ([], [], [])}
@@ -893,6 +912,8 @@ def precondition_all(pairs):
                 dinv.append(inv)
                 dgrad.append(p.grad)
         # 'full' curvatures do not precondition (reference: cov/linear.py:24-25)
+    if a_halves:
+        _keep_captured_forms([c for c, _ in pairs if c.kind == 'kron'])
     if any(a_halves):
         _ops.precondition_factored_batched(*kron, a_halves=a_halves)
     elif any(kron[4]) or any(kron[5]):

@@ -168,9 +168,93 @@ def test_optimizer_keeps_halves_where_inverses_are_used_once(monkeypatch):
     got = [p.grad.clone() for p in model[3].parameters()]
     for a, b in zip(curv.inv, invs):
         assert rel(a, b) < TOL
-    assert not curv._a_in_halves
+    assert curv._a_in_halves           # (reading the inverse changes nothing)
     for p, r in zip(model[3].parameters(), closure.raw):
         p.grad = r.clone()
     curv.precondition_grad(list(model[3].parameters()))
     for p, g in zip(model[3].parameters(), got):
         assert rel(p.grad, g.double().cpu()) < TOL
+
+
+def test_one_factor_that_has_to_be_in_halves_takes_the_batch_with_it():
+    """(alone it would be inverted whole; matrices of one block have no halves)"""
+    dev = torch.device('cuda', 0)
+    A64, G64 = spd(300, 1), spd(100, 2)
+    pi = ((A64.trace() / 300) / (G64.trace() / 100)).sqrt()
+    want = operand(A64 + 0.1 * pi * torch.eye(300, dtype=A64.dtype), 'H')[0]
+    a, g = A64.float().to(dev), G64.float().to(dev)
+    af, gf, af1, gf1 = torch.empty_like(a), torch.empty_like(g), torch.empty_like(g), torch.empty_like(g)
+    halves = [2, 2]
+    ops.pi_damped_inverse_factored_batched([a, g], [g, g], [1e-2] * 2, [None] * 2, [None] * 2, [af, af1], [gf, gf1],
+                                           a_halves=halves)
+    assert halves == [True, False]
+    assert rel(af, want) < TOL
+
+
+@pytest.mark.parametrize('form', ['whole', 'halves'])
+def test_captured_graphs_find_the_form_they_were_captured_with(form, monkeypatch):
+    """Graphs of a preconditioning and of an inversion, replayed between calls that choose a form anew."""
+    import torch.nn as nn
+    import torchsso
+    from torchsso.curv import curvature
+    monkeypatch.setattr(curvature.KronCurvature, 'halved_inverse_min_dim', 256)
+    monkeypatch.setattr(curvature.KronCurvature, 'halved_inverse_min_work', 1.)
+    dev = torch.device('cuda', 0)
+    torch.manual_seed(0)
+    model = nn.Sequential(*[nn.Linear(1000, 1000, device=dev) for _ in range(13)])
+    opt = torchsso.optim.SecondOrderOptimizer(model, 'Cov', {'Linear': 'Kron'}, {'damping': 1e-1}, lr=0.)
+    x = torch.randn(256, 1000, device=dev)
+
+    def closure():
+        opt.zero_grad(set_to_none=False)
+        out = model(x)
+        loss = out.pow(2).mean()
+        loss.backward()
+        return loss, out
+    opt.step(closure=closure)
+    curvs = [g['curv'] for g in opt.param_groups]
+    pairs = [(g['curv'], g['params']) for g in opt.param_groups]
+    for k, d in enumerate((1001, 1000)):     # (of a scale at which neither form passes for the other)
+        factor = spd(d, d).float().to(dev)
+        for c in curvs:
+            c.ema[k].copy_(factor)
+    if form == 'whole':
+        curvature.precondition_all(pairs)    # (used twice)
+    curvature.update_inv_all(curvs)
+    assert [c._a_in_halves for c in curvs] == [form == 'halves'] * 13
+
+    def restored():
+        for i, (_, params) in enumerate(pairs):
+            gen = torch.Generator(device=dev).manual_seed(i)
+            for p in params:
+                p.grad.copy_(torch.randn(p.shape, device=dev, generator=gen))
+
+    def graph_of(run):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            run()
+        return graph
+    restored()
+    A, G = (e.double().cpu() for e in curvs[3].ema)
+    pi = ((A.trace() / A.shape[0]) / (G.trace() / G.shape[0])).sqrt()
+    r = curvs[3].damping ** 0.5
+    v = torch.cat([pairs[3][1][0].grad, pairs[3][1][1].grad[:, None]], 1).double().cpu()
+    want = (torch.linalg.inv(G + r / pi * torch.eye(G.shape[0], dtype=G.dtype)) @ v
+            @ torch.linalg.inv(A + r * pi * torch.eye(A.shape[0], dtype=A.dtype)))
+
+    def check():
+        w, b = (p.grad for p in pairs[3][1])
+        assert rel(torch.cat([w, b[:, None]], 1), want) < TOL
+    precondition = graph_of(lambda: curvature.precondition_all(pairs))
+    invert = graph_of(lambda: curvature.update_inv_all(curvs))
+    eager_inversions = [lambda: curvature.update_inv_all(curvs), lambda: curvature.update_inv_all([curvs[3]]),
+                        lambda: None]
+    for again in eager_inversions * 2:
+        for inversion in (invert.replay, again):
+            inversion()
+            for run in (lambda: curvature.precondition_all(pairs), precondition.replay):
+                restored()
+                run()
+                check()
+    for c in curvs:
+        c.inv = None             # (nothing of the graphs' memory is used behind them)
