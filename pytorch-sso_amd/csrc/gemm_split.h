@@ -774,11 +774,10 @@ __device__ __forceinline__ void split_blocks(const OPP& P, const OPQ& Q, int m0,
 }
 
 // The 32x32 blocks of a wave, rows from `row0`, columns from `col0`, through the epilogue.
-// `what`: nothing (the block is another wave's), the block, the block and its mirror image, or,
-// for a block on the diagonal, its upper triangle with or without the mirror image.  (The two
-// orders in which the corrections h m' and m h' are added round differently, so that only
-// one triangle of such a block is used: the result is symmetric to the bit.)
-enum { BLK_NONE = 0, BLK_PLAIN = 1, BLK_BOTH = 2, BLK_UPPER = 3, BLK_UPPER_BOTH = 4 };
+// `what`: nothing (the block is another wave's), the block or, for a block on the diagonal, its upper
+// triangle.  (The two orders in which the corrections h m' and m h' are added round differently, so that
+// only one triangle of such a block is used: the result is symmetric to the bit.)
+enum { BLK_NONE = 0, BLK_PLAIN = 1, BLK_UPPER = 2 };
 template <int NB, class EPI>
 __device__ __forceinline__ void store_blocks(const v16f (&acc)[NB], const int (&row0)[NB],
                                              const int (&col0)[NB], const int (&what)[NB],
@@ -790,8 +789,7 @@ __device__ __forceinline__ void store_blocks(const v16f (&acc)[NB], const int (&
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int row = row_of(b, i), col = col0[b] + r;
-      if (what[b] < BLK_UPPER || row <= col) element(i, row, col);
-      if (what[b] == BLK_BOTH || (what[b] == BLK_UPPER_BOTH && row < col)) element(i, col, row);
+      if (what[b] != BLK_UPPER || row <= col) element(i, row, col);
     }
   };
   if constexpr (reading_epilogue<EPI>::value) {
@@ -807,7 +805,6 @@ __device__ __forceinline__ void store_blocks(const v16f (&acc)[NB], const int (&
 #pragma unroll
           for (int i = 0; i < 16; ++i)
             old[b - b0][i] = what[b] != BLK_NONE ? epi.fetch(row_of(b, i), col0[b] + r) : 0.f;
-        // (the old values are symmetric like the new ones)
 #pragma unroll
         for (int b = b0; b < b0 + 2 && b < NB; ++b)
           if (what[b] != BLK_NONE)
@@ -820,6 +817,61 @@ __device__ __forceinline__ void store_blocks(const v16f (&acc)[NB], const int (&
   for (int b = 0; b < NB; ++b)
     if (what[b] != BLK_NONE)
       put(b, [&](int i, int row, int col) { epi.store(row, col, acc[b][i]); });
+}
+
+// An epilogue with value() and put() can have the images of a tile's blocks across the diagonal stored as well.
+template <class T, class = void>
+struct imaging_epilogue : std::false_type {};
+template <class T>
+struct imaging_epilogue<T, std::void_t<decltype(std::declval<const T&>().put(0, 0, 0.f))>> : std::true_type {};
+
+// store_blocks, with the image of every block.  It goes through the wave's own piece of LDS (`smem`, free again when
+// the sums are done; the workgroup's last use of it), a block at a time, and to memory by its rows: from the
+// registers it is written by 4-byte pieces of 64 rows at a time.  The old values of all blocks are in flight
+// together (they are symmetric like the new ones).  Bound by memory, 16 bytes an element of the triangle.  Running
+// average of a factor, us with the images from the registers / here: 256 rows of 9216 285 / 244 (2.8 TB/s), of 4096
+// 83 / 68, 64 rows of 4096 59 / 44 (3.0 TB/s), 32 of 2048 23.7 / 19.7, 16 of 1000 18.9 / 16.9; 256 of 2048 38.4 / 38.8.
+constexpr int IMAGE_LD = 33;
+static_assert(NTHREADS / 64 * 32 * IMAGE_LD * 4 <= SplitCfg<2>::VOTES, "the images lie where the tile's chunks were");
+template <int NB, class EPI>
+__device__ __forceinline__ void store_images(const v16f (&acc)[NB], const int (&row0)[NB],
+                                             const int (&col0)[NB], const int (&what)[NB], float* smem,
+                                             const EPI& epi) {
+  const int lane = threadIdx.x & 63;
+  const int r = lane & 31, h = lane >> 5;
+  lds_f* const t = (lds_f*)smem + ((int)(threadIdx.x & (NTHREADS - 1)) >> 6) * 32 * IMAGE_LD;
+  float old[NB][16];
+  bool reads = false;
+  if constexpr (reading_epilogue<EPI>::value) {
+    reads = epi.reads();
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        old[b][i] = reads && what[b] != BLK_NONE
+                        ? epi.fetch(row0[b] + 8 * (i >> 2) + 4 * h + (i & 3), col0[b] + r) : 0.f;
+  }
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    if (what[b] == BLK_NONE) continue;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int row = 8 * (i >> 2) + 4 * h + (i & 3);
+      float o = epi.value(acc[b][i]);
+      if constexpr (reading_epilogue<EPI>::value) o = reads ? epi.value(acc[b][i], old[b][i]) : o;
+      if (what[b] != BLK_UPPER || row <= r) epi.put(row0[b] + row, col0[b] + r, o);
+      t[r * IMAGE_LD + row] = o;
+    }
+    // (other lanes' values: a wave's accesses to LDS are done in order)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int row = 2 * i + h;         // of the image
+      const float o = t[row * IMAGE_LD + r];
+      if (what[b] != BLK_UPPER || r < row) epi.put(col0[b] + row, row0[b] + r, o);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
 }
 
 // A 64-wide tile with mirror images, a 32x32 block on each of four waves, through LDS (`smem`, free again when the sums
@@ -884,7 +936,15 @@ __device__ __forceinline__ void split_tile_full(const OPP& P, const OPQ& Q, int 
     const int row0[4] = {m0 + wm, m0 + wm, m0 + wm + 32, m0 + wm + 32};
     const int col0[4] = {n0 + wn, n0 + wn + 32, n0 + wn, n0 + wn + 32};
     const int what[4] = {BLK_PLAIN, BLK_PLAIN, BLK_PLAIN, BLK_PLAIN};
-    store([&](const auto& epi) { store_blocks<4>(acc, row0, col0, what, epi); });
+    store([&](const auto& epi) {
+      if constexpr (imaging_epilogue<std::decay_t<decltype(epi)>>::value) {
+        if (epi.mirror) {
+          store_images<4>(acc, row0, col0, what, smem, epi);
+          return;
+        }
+      }
+      store_blocks<4>(acc, row0, col0, what, epi);
+    });
   }
 }
 
@@ -901,15 +961,22 @@ __device__ __forceinline__ void split_tile_tri(const OP& P, int m0, int kbeg, in
     // (both triangles, always)
     store([&](const auto& epi) { store_small<true>(acc[0], m0, m0, wm, wn, smem, epi); });
   } else {
-    const int above = both ? BLK_BOTH : BLK_PLAIN, on = both ? BLK_UPPER_BOTH : BLK_UPPER;
     const SplitTri t = split_tri(wave);
     const int r0 = 32 * t.r[0], r1 = 32 * t.r[1], r2 = 32 * t.r[2];
     v16f acc[3];
     split_blocks<SplitDiag>(P, P, m0, m0, kbeg, kend, smem, SplitRows{{r0, r1, r2}, {}}, acc);
     const int row0[3] = {m0 + r0, m0 + r0, m0 + r1};
     const int col0[3] = {m0 + r1, m0 + r2, m0 + r1};
-    const int what[3] = {above, t.r[0] == t.r[2] ? on : above, t.last ? on : (int)BLK_NONE};
-    store([&](const auto& epi) { store_blocks<3>(acc, row0, col0, what, epi); });
+    const int what[3] = {BLK_PLAIN, t.r[0] == t.r[2] ? BLK_UPPER : BLK_PLAIN, t.last ? BLK_UPPER : BLK_NONE};
+    store([&](const auto& epi) {
+      if constexpr (imaging_epilogue<std::decay_t<decltype(epi)>>::value) {
+        if (both) {
+          store_images<3>(acc, row0, col0, what, smem, epi);
+          return;
+        }
+      }
+      store_blocks<3>(acc, row0, col0, what, epi);
+    });
   }
 }
 

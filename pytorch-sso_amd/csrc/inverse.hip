@@ -1464,19 +1464,17 @@ __device__ __forceinline__ void lauum_tile(int T, int local, int& bi, int& bj) {
   bi = bj = 0;       // not reached: the classes hold exactly ntiles tiles
 }
 
-// C[f(row)][f(col)] = v and its mirror image, f(i) = base + sign * i: the identity, or the
+// C[f(row)][f(col)] = v (and, by put(), its mirror image), f(i) = base + sign * i: the identity, or the
 // reversal i -> n - 1 - i that undoes the reversed read of a matrix factored back to front
 struct EpiSymFlip {
   float* C;
   int n, base, sign;
   bool mirror;
-  __device__ __forceinline__ void store(int row, int col, float v) const {
-    if (row < n && col < n) {
-      const int r = base + sign * row, c = base + sign * col;
-      C[(size_t)r * n + c] = v;
-      if (mirror && row != col) C[(size_t)c * n + r] = v;
-    }
+  __device__ __forceinline__ float value(float v) const { return v; }
+  __device__ __forceinline__ void put(int row, int col, float o) const {
+    if (row < n && col < n) C[(size_t)(base + sign * row) * n + base + sign * col] = o;
   }
+  __device__ __forceinline__ void store(int row, int col, float v) const { put(row, col, v); }
 };
 
 // dst = Y Y^T over the upper tiles (k >= the later block), mirrored

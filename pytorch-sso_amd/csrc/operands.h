@@ -265,8 +265,8 @@ struct ConvP {
 // Epilogues
 // ---------------------------------------------------------------------------
 
-// C[row][col] = alpha*acc + beta*Cin[row][col] ; optionally also the mirrored
-// element.  Cin == nullptr: the old values of C itself.
+// C[row][col] = alpha*acc + beta*Cin[row][col].  Cin == nullptr: the old values of C itself.
+// `mirror`: of a symmetric C, whose other triangle gets the images of what is stored (put()).
 struct EpiStore {
   static constexpr bool reads_output = true;
   float* C;
@@ -280,9 +280,7 @@ struct EpiStore {
   }
   __device__ __forceinline__ void store_with(int row, int col, float v, float old) const {
     if (row < M && col < N) {
-      const float o = alpha * v + beta * old;
-      C[(size_t)row * ld + col] = o;
-      if (mirror && row != col) C[(size_t)col * ld + row] = o;
+      C[(size_t)row * ld + col] = alpha * v + beta * old;
     }
   }
   // the two halves of a store, for epilogues that rearrange results in between
@@ -297,7 +295,6 @@ struct EpiStore {
       float o = alpha * v;
       if (beta != 0.f) o += beta * (Cin ? Cin : C)[idx];
       C[idx] = o;
-      if (mirror && row != col) C[(size_t)col * ld + row] = o;
     }
   }
 };
