@@ -260,11 +260,6 @@ __device__ __forceinline__ void gemm_tile(const OPP& P, const OPQ& Q, int m0, in
 // the device-wide fences it needs write back and invalidate the whole L2 of an XCD each
 // time, and the operand panels that the other workgroups share through that L2 with them.)
 // ---------------------------------------------------------------------------
-// pieces of a reduction of `blocks` 128-blocks cut at `pb` blocks (pb <= 0: not cut)
-__host__ __device__ inline int piece_count(int blocks, int pb) {
-  return pb > 0 ? (blocks + pb - 1) / pb : 1;
-}
-
 // (`stride`: floats from one piece of the tile to the next)
 template <class EPI>
 __device__ __forceinline__ void splitk_sum(const float* parts, int nparts, int m0, int n0,

@@ -12,8 +12,11 @@
 
 #include "common.h"
 #include "operands.h"
+#include "precond_plan.h"
 
 namespace kfac {
+
+static_assert(BM == PLAN_TILE && BN == PLAN_TILE, "the plan counts 128-wide tiles");
 
 struct LayerDesc {
   const float* L;        // dG x dG : G^-1 (symmetric) or U_G (upper, sampling)
@@ -30,9 +33,6 @@ struct LayerDesc {
   int flags;         // factored preconditioning: L_FACTOR, ... (none: the inverses)
   float* parts;      // pieces of the tiles whose reduction is cut (see tile_item)
 };
-
-// what the operands of a layer are: triangular factors (else explicit inverses), R's in two halves
-enum { L_FACTOR = 1, R_FACTOR = 2, R_HALVES = 4 };
 
 constexpr int LAYER_CHUNK = 32;
 struct LayerChunk {
@@ -124,38 +124,6 @@ struct EpiSplit {
 // mapping.  Posterior sampling (U_G E U_A, both upper triangular) uses the first two
 // products with its own operand layouts.
 // ---------------------------------------------------------------------------
-
-// A reduction against a triangular operand of T blocks is up to T blocks long, and a launch
-// lasts at least as long as its longest tile: a 4608-deep tile is 150 MFLOP on ONE compute
-// unit.  Where that is longer than the launch would take if its work were spread evenly
-// (few layers, or few tiles: the driver decides per product), the reductions are cut into
-// pieces of at most `pb` blocks, each a work item of the same launch that stores a raw
-// partial tile; a second, short launch adds the pieces of every cut tile up in order and
-// applies the epilogue (precond_finish_kernel).  Piece j exists for the tiles whose
-// reduction is longer than j * pb blocks: tfast - j * pb values of `fast`.  pb == 0: no
-// reduction is cut.
-enum { PART_A = 0, COUPLING = 1, PART_B = 2, STEPS = 3 };
-__host__ __device__ inline int half_of(int T) { return T >> 1; }     // blocks of the first half
-
-// which of the T tiles along the reduction a part holds (`grows`: the reduction gets longer with the
-// tile index, so that the first half comes first); their reductions start or end where the part does
-struct TileRange {
-  int first, count;
-};
-__host__ __device__ inline TileRange part_tiles(int T, bool halves, bool grows, int part) {
-  if (!halves) return part == PART_A ? TileRange{0, T} : TileRange{0, 0};
-  const int h = half_of(T);
-  return (part == PART_A) == grows ? TileRange{0, h} : TileRange{h, T - h};
-}
-
-// work items of a layer in one product: tiles x pieces
-__host__ __device__ inline int piece_items(int tslow, int tfast, bool tri, int pb) {
-  if (pb <= 0) return tslow * tfast;
-  if (!tri) return tslow * tfast * piece_count(tfast, pb);    // dense: all reductions tfast blocks
-  int n = 0;
-  for (int j = 0; j * pb < tfast; ++j) n += tslow * (tfast - j * pb);
-  return n;
-}
 
 // (slow, fast) tile indices of work item `local` of a layer with tslow x tfast tiles.
 // `tri`: the reduction length depends on `fast`; it grows with it if `grows`.
@@ -324,17 +292,6 @@ __global__ __launch_bounds__(NTHREADS, 2) void precond_fourth_kernel(const Layer
                 bi * BM, m.dG, fourth_epilogue(m), smem);
 }
 
-// The couplings of the second (`product` 1) and third (2) product: the tiles of PART_B's input, `slow`
-// over dG and `fast` over its blocks of dA; reductions over all of PART_A, `depth` blocks.
-struct CouplingShape {
-  int first, count;              // blocks of PART_B
-  int kfirst, depth;             // of PART_A
-};
-__host__ __device__ inline CouplingShape coupling_shape(int product, int ta, int flags) {
-  const bool grows = product == 1;
-  const TileRange a = part_tiles(ta, true, grows, PART_A), b = part_tiles(ta, true, grows, PART_B);
-  return CouplingShape{b.first, flags & R_HALVES ? b.count : 0, a.first, a.count};
-}
 __device__ __forceinline__ EpiStore coupling_epilogue(const LayerDesc& m, int product) {
   return product == 1 ? EpiStore{m.Tt, m.dG, m.dA, m.dG, -1.f, 1.f, false}
                       : EpiStore{second_half(m), m.dA, m.dG, m.dA, -1.f, 1.f, false};
@@ -414,64 +371,6 @@ __global__ __launch_bounds__(NTHREADS) void precond_finish_kernel(const LayerDes
 
 static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
-constexpr int PRODUCTS = 4;
-
-// what a layer does in one step of a product: `tiles` tiles with reductions of up to `longest` blocks
-// (tri: of 1 to `longest`, with `tslow` of each length), `work` blocks in all
-struct StepShape {
-  int tiles, longest, tslow;
-  bool tri;
-  long work;
-};
-static StepShape step_shape(int product, int step, int dG, int dA, int flags, bool sample) {
-  const int ta = cdiv(dA, BN), tg = cdiv(dG, BM);
-  const bool over_g = product == 0 || product == 3;
-  const bool tri = sample || (flags & (over_g ? L_FACTOR : R_FACTOR));
-  if ((product >= 2 && (!tri || sample)) || (sample && step != PART_A)) return StepShape{0, 0, 1, false, 0};
-  const bool halves = !over_g && (flags & R_HALVES);
-  if (step == COUPLING) {
-    const CouplingShape cs = coupling_shape(product, ta, flags);
-    return halves ? StepShape{tg * cs.count, cs.depth, tg, false, (long)tg * cs.count * cs.depth}
-                  : StepShape{0, 0, 1, false, 0};
-  }
-  const int count = part_tiles(over_g ? tg : ta, halves, product < 2, step).count;
-  const int tslow = over_g ? ta : tg;
-  return StepShape{tslow * count, count, tslow, tri,
-                   tri ? (long)tslow * count * (count + 1) / 2 : (long)tslow * count * count};
-}
-
-// Piece size of each step of each product from the shape of its launch.  flags == nullptr: every side
-// of every layer is a triangular factor (what the scratch is sized for, but for halves).
-typedef int PieceSizes[PRODUCTS][STEPS];
-static void plan_pieces(int layers, const int* dG, const int* dA, const int* flags, PieceSizes& pbs,
-                        bool sample = false) {
-  for (int product = 0; product < PRODUCTS; ++product)
-    for (int step = 0; step < STEPS; ++step) {
-      long work = 0;
-      int longest = 0;
-      for (int l = 0; l < layers; ++l) {
-        const StepShape sh = step_shape(product, step, dG[l], dA[l], flags ? flags[l] : L_FACTOR | R_FACTOR,
-                                        sample);
-        work += sh.work;
-        longest = std::max(longest, sh.longest);
-      }
-      pbs[product][step] = piece_blocks(work, longest);
-    }
-}
-
-// floats of the piece area of a layer under the piece sizes `pbs`: room for the pieces of
-// the longest reduction, for every tile
-static size_t piece_floats(int dG, int dA, int flags, const PieceSizes& pbs) {
-  size_t most = 0;
-  for (int product = 0; product < PRODUCTS; ++product)
-    for (int step = 0; step < STEPS; ++step) {
-      const StepShape sh = step_shape(product, step, dG, dA, flags, false);
-      const int pieces = piece_count(sh.longest, pbs[product][step]);
-      if (pieces > 1) most = std::max(most, (size_t)sh.tiles * pieces);
-    }
-  return most * (BM * BN);
-}
-
 // scratch: the descriptor tables, then per layer dG*dA floats (twice that when
 // `factored`: a layer with a factored side keeps two results in flight) and its piece area
 // (`flags` as in plan_pieces)
@@ -505,19 +404,11 @@ static int run_layers(int layers, const int* dG, const int* dA, const float* con
   // (two orders, so two tables, one behind the other; uploaded together, which for a few
   // layers is one launch)
   char* tbase = (char*)workspace + align256((size_t)2 * layers * sizeof(LayerDesc));
-  // pieces as large as the scratch was sized for, at least (the query assumed that every
-  // side is a triangular factor), and none where it left no room
   const std::vector<int> no_flags(layers, 0);     // explicit inverses on both sides
   const int* const real_flags = flags ? flags : no_flags.data();
   PieceSizes pbs_room, pbs;
   plan_pieces(layers, dG, dA, room_flags, pbs_room);
-  plan_pieces(layers, dG, dA, real_flags, pbs, sample);
-  for (int product = 0; product < PRODUCTS; ++product)
-    for (int step = 0; step < STEPS; ++step) {
-      int& pb = pbs[product][step];
-      const int room = pbs_room[product][step];
-      pb = pb > 0 && room > 0 ? std::max(pb, room) : 0;
-    }
+  call_pieces(layers, dG, dA, real_flags, pbs_room, pbs, sample);
   std::vector<size_t> toff(layers), poff(layers);
   size_t off = 0;
   for (int l = 0; l < layers; ++l) {
@@ -675,14 +566,6 @@ size_t kfac_precondition_factored_workspace_bytes(int layers, const int* dG, con
   return precond_workspace(layers, dG, dA, true, nullptr);
 }
 
-// what is in halves, as plan_pieces wants it (a matrix of one block has none)
-static std::vector<int> halves_room(int layers, const int* dA, const int* a_halves) {
-  std::vector<int> flags(layers, L_FACTOR | R_FACTOR);
-  for (int l = 0; l < layers; ++l)
-    if (a_halves[l] && half_of(cdiv(dA[l], BM)) > 0) flags[l] |= R_HALVES;
-  return flags;
-}
-
 size_t kfac_precondition_halves_workspace_bytes(int layers, const int* dG, const int* dA,
                                                 const int* a_halves) {
   if (layers <= 0 || !dG || !dA || !a_halves) return 0;
@@ -697,12 +580,7 @@ static int precondition_factored(int layers, const int* dG, const int* dA, const
   std::vector<int> hb;
   const int st = check_layers(layers, dG, dA, Gop, Aop, gradW, gradb, hb);
   if (st != KFAC_OK) return st;
-  std::vector<int> flags(layers);
-  for (int l = 0; l < layers; ++l) {
-    const bool a = !a_factored || a_factored[l];
-    flags[l] = ((!g_factored || g_factored[l]) ? L_FACTOR : 0) | (a ? R_FACTOR : 0) |
-               (a && room_flags ? room_flags[l] & R_HALVES : 0);
-  }
+  const std::vector<int> flags = operand_flags(layers, g_factored, a_factored, room_flags);
   return run_layers(layers, dG, dA, Gop, Aop, (const float* const*)gradW,
                     (const float* const*)gradb, nullptr, nullptr, gradW, gradb, hb.data(), 1.f,
                     false, flags.data(), room_flags, workspace, workspace_bytes, (hipStream_t)stream);

@@ -79,6 +79,25 @@ def test_precondition(case):
     assert all(torch.equal(a, b) for a, b in zip(before, Go + Ao))
 
 
+def test_an_explicit_inverse_is_not_in_halves_whatever_the_list_says():
+    """(reductions of this call are cut into pieces, and those over an explicit inverse are twice as long)"""
+    dev = torch.device('cuda', 0)
+    gen = torch.Generator().manual_seed(9)
+    layers = [(300, 1025, 'I'), (129, 640, 'H'), (64, 385, 'I')]
+    Go, Ao, gw, gb, want = [], [], [], [], []
+    for dG, dA, form in layers:
+        v = torch.randn(dG, dA, generator=gen, dtype=torch.float64)
+        (go, gi), (ao, ai) = operand(spd(dG, dG), 'F'), operand(spd(dA, dA), form)
+        want.append(gi @ v @ ai)
+        Go.append(go.float().contiguous().to(dev))
+        Ao.append(ao.float().contiguous().to(dev))
+        gw.append(v[:, :-1].float().contiguous().to(dev))
+        gb.append(v[:, -1].float().contiguous().to(dev))
+    ops.precondition_factored_batched(Go, Ao, gw, gb, None, [f != 'I' for _, _, f in layers], a_halves=[True] * 3)
+    for w, b, ref in zip(gw, gb, want):
+        assert rel(torch.cat([w, b[:, None]], 1), ref) < TOL
+
+
 # (22 matrices of 8 blocks are more than the sweep takes)
 DIMS = [(1000, 1024), (1025, 897)] * 6
 
