@@ -296,8 +296,8 @@ class KronCurvature(Curvature):
     # (on the class, for objects that were pickled before they had these)
     _a_in_halves = False        # the factor of A's inverse is in two halves
     _inv_uses = 0               # preconditionings with the inverses there are
-    # ... the form that a recorded graph has to find and leave it in: a graph that inverts or preconditions
-    # does at every replay what it did when it was captured, so that neither may change from then on
+    # ... the form that a recorded graph has to find and leave it in: a graph that inverts, preconditions or
+    # forms `inv` does at every replay what it did when it was captured, so that none may change from then on
     _form_captured = None
 
     def __init__(self, *args, **kwargs):
@@ -324,6 +324,8 @@ class KronCurvature(Curvature):
         if self._inv is not None:
             for k, y in enumerate(self._inv_factors):
                 if self._inv[k] is None and y is not None:
+                    if k == 0:
+                        _keep_captured_forms([self])
                     if k == 0 and self._a_in_halves:
                         # (a copy: to read the inverse under another stream, or from another thread, writes
                         # nothing that preconditioning reads)

@@ -277,3 +277,55 @@ def test_captured_graphs_find_the_form_they_were_captured_with(form, monkeypatch
                 check()
     for c in curvs:
         c.inv = None             # (nothing of the graphs' memory is used behind them)
+
+
+@pytest.mark.parametrize('form', ['whole', 'halves'])
+def test_captured_reads_of_an_inverse_find_the_form_they_were_captured_with(form, monkeypatch):
+    """A graph of `inv` alone (which multiplies the factor by its transpose, and completes a copy of one in halves
+    first), replayed behind inversions that choose a form anew."""
+    import torch.nn as nn
+    import torchsso
+    from torchsso.curv import curvature
+    monkeypatch.setattr(curvature.KronCurvature, 'halved_inverse_min_dim', 256)
+    monkeypatch.setattr(curvature.KronCurvature, 'halved_inverse_min_work', 1.)
+    dev = torch.device('cuda', 0)
+    torch.manual_seed(0)
+    model = nn.Sequential(*[nn.Linear(1000, 1000, device=dev) for _ in range(13)])
+    opt = torchsso.optim.SecondOrderOptimizer(model, 'Cov', {'Linear': 'Kron'}, {'damping': 1e-1}, lr=0.)
+    x = torch.randn(256, 1000, device=dev)
+
+    def closure():
+        opt.zero_grad(set_to_none=False)
+        out = model(x)
+        loss = out.pow(2).mean()
+        loss.backward()
+        return loss, out
+    opt.step(closure=closure)
+    curvs = [g['curv'] for g in opt.param_groups]
+    pairs = [(g['curv'], g['params']) for g in opt.param_groups]
+    for k, d in enumerate((1001, 1000)):
+        factor = spd(d, d).float().to(dev)
+        for c in curvs:
+            c.ema[k].copy_(factor)
+    if form == 'whole':
+        curvature.precondition_all(pairs)    # (used twice)
+    curvature.update_inv_all(curvs)
+    assert [c._a_in_halves for c in curvs] == [form == 'halves'] * 13
+    A, G = (e.double().cpu() for e in curvs[3].ema)
+    pi = ((A.trace() / A.shape[0]) / (G.trace() / G.shape[0])).sqrt()
+    r = curvs[3].damping ** 0.5
+    want = [torch.linalg.inv(m + s * torch.eye(m.shape[0], dtype=m.dtype)) for m, s in ((A, r * pi), (G, r / pi))]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        read = list(curvs[3].inv)
+    for uses in (0, 1, 2, 1, 0):
+        for _ in range(uses):
+            curvature.precondition_all(pairs)
+        curvature.update_inv_all(curvs)
+        for t in read:
+            t.fill_(float('nan'))
+        graph.replay()
+        for t, w in zip(read, want):
+            assert rel(t, w) < TOL
+    for c in curvs:
+        c.inv = None             # (nothing of the graph's memory is used behind it)
