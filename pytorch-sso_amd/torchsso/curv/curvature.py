@@ -297,7 +297,8 @@ class KronCurvature(Curvature):
     _a_in_halves = False        # the factor of A's inverse is in two halves
     _inv_uses = 0               # preconditionings with the inverses there are
     # ... the form that a recorded graph has to find and leave it in: a graph that inverts, preconditions or
-    # forms `inv` does at every replay what it did when it was captured, so that none may change from then on
+    # forms `inv` does at every replay what it did when it was captured, so that none may change for as long
+    # as the factor lies where it lay then (also when the graph is gone)
     _form_captured = None
 
     def __init__(self, *args, **kwargs):
@@ -339,7 +340,12 @@ class KronCurvature(Curvature):
         self._inv = None if value is None else list(value)
         self._inv_factors = [None, None]      # inverses given from outside have no factors
         self._a_in_halves = False
+        self._form_captured = None
         self._inv_uses = 0
+
+    def __setstate__(self, state):
+        self.__dict__.update(state)
+        self._form_captured = None            # (graphs know the buffers of the object that this one is a copy of)
 
     def _inverse_outputs(self, with_std):
         """Output buffers for one update_inv of this layer, None where that output is not
@@ -360,6 +366,9 @@ class KronCurvature(Curvature):
                 invs[k] = reuse(old_inv[k], e)
                 if with_std:
                     stds[k] = reuse(old_std[k], e)
+        if facs[0] is not self._inv_factors[0]:
+            self._a_in_halves = False
+            self._form_captured = None
         self._inv = list(invs)
         self._inv_factors = list(facs)
         if with_std:
@@ -647,8 +656,8 @@ def update_inv_all(curvs, with_std=()):
     full = [c for c in curvs if c.kind == 'full']
     wanted = {id(c) for c in with_std}
     if kron:
-        _keep_captured_forms(kron)
         outs = [c._inverse_outputs(id(c) in wanted) for c in kron]
+        _keep_captured_forms(kron)
         halves = None
         column = lambda which, k: [o[which][k] for o in outs]
         args = ([c.ema[0] for c in kron], [c.ema[1] for c in kron], [c.damping for c in kron])
