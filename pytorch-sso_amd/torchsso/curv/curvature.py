@@ -289,13 +289,17 @@ class KronCurvature(Curvature):
     #   3800-3800-3800-100 (1.6e11) 5487 / 5609       4900-4900-100 (2.4e11) 6202 / 6370
     #   600-4900-600 (1.2e11) 3312 / 3321             4000-1500-3000-100 (9e10) 2998 / 2903
     # A step with inverses it already has is slower with halves (a ResNet-50's 5983 / 5786 us), hence
-    # the rule on their use.  None: always whole.
+    # the rule on their use.  None: always whole.  To read `inv` of a factor in halves takes a copy of it and the
+    # merge that was left out, once behind an inversion (9217 rows: 340 MB, 1.2 ms); a factor that a recorded graph
+    # finds in halves stays in halves, and inversions that it takes part in are not done by the sweep.
     halved_inverse_min_dim = 2048
     halved_inverse_min_work = 1e11
 
     # (on the class, for objects that were pickled before they had these)
     _a_in_halves = False        # the factor of A's inverse is in two halves
-    _inv_uses = 0               # preconditionings with the inverses there are
+    # preconditionings with the inverses there are; one whose factor `inv` has read counts as used more than
+    # once (to complete the factor costs what the inversion was spared: read at every step, it stays whole)
+    _inv_uses = 0
     # ... the form that a recorded graph has to find and leave it in: a graph that inverts, preconditions or
     # forms `inv` does at every replay what it did when it was captured, so that none may change for as long
     # as the factor lies where it lay then (also when the graph is gone)
@@ -327,6 +331,7 @@ class KronCurvature(Curvature):
                 if self._inv[k] is None and y is not None:
                     if k == 0:
                         _keep_captured_forms([self])
+                        self._inv_uses += 2
                     if k == 0 and self._a_in_halves:
                         # (a copy: to read the inverse under another stream, or from another thread, writes
                         # nothing that preconditioning reads)

@@ -329,3 +329,33 @@ def test_captured_reads_of_an_inverse_find_the_form_they_were_captured_with(form
             assert rel(t, w) < TOL
     for c in curvs:
         c.inv = None             # (nothing of the graph's memory is used behind it)
+
+
+def test_inverses_that_are_read_every_time_stay_whole(monkeypatch):
+    """(to complete a factor in halves costs a read what the inversion was spared)"""
+    import torch.nn as nn
+    import torchsso
+    from torchsso.curv.curvature import KronCurvature
+    monkeypatch.setattr(KronCurvature, 'halved_inverse_min_dim', 256)
+    monkeypatch.setattr(KronCurvature, 'halved_inverse_min_work', 1.)
+    dev = torch.device('cuda', 0)
+    torch.manual_seed(0)
+    model = nn.Sequential(*[nn.Linear(1000, 1000, device=dev) for _ in range(13)])
+    opt = torchsso.optim.SecondOrderOptimizer(model, 'Cov', {'Linear': 'Kron'}, {'damping': 1e-1}, lr=0.)
+    x = torch.randn(256, 1000, device=dev)
+
+    def closure():
+        opt.zero_grad()
+        out = model(x)
+        loss = out.pow(2).mean()
+        loss.backward()
+        return loss, out
+    forms = []
+    for read in (True, True, True, False, False, True, True):
+        opt.step(closure=closure)
+        forms.append([g['curv']._a_in_halves for g in opt.param_groups[2:4]])
+        if read:
+            opt.param_groups[2]['curv'].inv
+    # (the inverses of the third layer are in halves only behind a step without a read)
+    assert forms == [[False, False], [False, True], [False, True], [False, True], [True, True], [True, True],
+                     [False, True]]
