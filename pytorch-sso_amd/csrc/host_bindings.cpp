@@ -250,9 +250,14 @@ PyObject* rowsq_sum(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const int64_t rows = t.size(0) * channels, len = t.numel() / rows;
     if (len <= 0 || len > INT_MAX) Py_RETURN_NONE;
     const at::Tensor out = at::empty({t.size(0), (int64_t)channels}, t.options().requires_grad(false));
-    if (run(x, rows, (int)channels, (int)len, scale, shift, out.mutable_data_ptr<float>(),
-            c10::hip::getCurrentHIPStream(t.device().index()).stream()) != KFAC_OK)
-      Py_RETURN_NONE;
+    float* const sums = out.mutable_data_ptr<float>();
+    const hipStream_t stream = c10::hip::getCurrentHIPStream(t.device().index()).stream();
+    int status;
+    // (a launch may wait for room in the stream's queue: other threads go on meanwhile)
+    Py_BEGIN_ALLOW_THREADS
+    status = run(x, rows, (int)channels, (int)len, scale, shift, sums, stream);
+    Py_END_ALLOW_THREADS
+    if (status != KFAC_OK) Py_RETURN_NONE;
     return THPVariable_Wrap(out);
   });
 }
