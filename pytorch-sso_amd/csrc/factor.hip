@@ -66,10 +66,11 @@ static void upload_chunk(const char* host, size_t bytes, unsigned* dst, hipStrea
   hipLaunchKernelGGL(upload_kernel<WORDS>, dim3(1), dim3(WORDS / 4), 0, stream, c, dst, (int)words);
 }
 
-// 15 KiB a launch, as few launches as that takes, and 3 KiB where that is enough: a launch is 5 us whatever it
-// carries, and the tables of a ResNet-50 are 26 of 3.75 KiB or 12 (a step with old inverses, from an idle
-// device, 6026 -> 5937 us).
-constexpr int UPLOAD_SMALL = 768, UPLOAD_WORDS = 3840;
+// 15 KiB a launch, as few launches as that takes, and 3.75 KiB where that is enough.  One behind the other the
+// launches take what the host needs for them: with 1 / 3 / 3.75 / 7.5 / 15 KiB of arguments 2.8 / 2.9 / 3.0 / 3.2 / 3.6 us
+// (the kernel itself 1.3 to 1.8).  The tables of a ResNet-50 are 26 launches of 3.75 KiB or 13 (a step with old inverses,
+// from an idle device, 6026 -> 5937 us).
+constexpr int UPLOAD_SMALL = 960, UPLOAD_WORDS = 3840;
 void upload_table(const void* host, size_t bytes, void* dev, hipStream_t stream) {
   for (size_t at = 0; at < bytes; at += UPLOAD_WORDS * 4) {
     const size_t n = std::min(bytes - at, (size_t)UPLOAD_WORDS * 4);
