@@ -63,15 +63,17 @@ constexpr void helped_blocks(int q, int nq, int helper, F&& take) {
       if (k % STRIP_HELPERS == helper) take(i, b < nq - i ? i + b : 4 + b - (nq - i));
 }
 
+// The first strip that gives something to a block of block column `col` further down: the rows of S begin with
+// strip 0, those of block column 4 + c of Z with strip c.  A helper of strip q takes the strips from there to q - 1.
+constexpr int helped_from(int col) { return col < 4 ? 0 : col - 4; }
+
 // A pending panel is applied by ten waves, a 32x32 block of S each, from parts that lie in the rows of Z from
 // PENDING_ROW0 on.  The waves 0-3 have the blocks that they begin strip 0 with, and go on without waiting for
-// anybody.  Nothing of the others' is read or written in strip 0: its collecting waves read its own rows, and the
-// blocks of the rows below, also those of Z that lie over the parts, belong to the strips behind the next barrier.
-// Each wave leaves a mark when it is done with the panel, behind its last access to S and to the parts, and who
-// applies something of strip 0 to a block waits for all of them before it touches that.
+// anybody.  Nothing of the others' is read or written in strip 0: its collecting waves read its own rows, its helpers
+// have no block yet, and the blocks of the rows below, also those of Z that lie over the parts, belong to the
+// strips behind the barrier that ends strip 0.
 constexpr int PENDING_WAVES = 10, PENDING_ROW0 = 32;
 constexpr int pending_row(int wave) { return (int)(0x3221110000ull >> (4 * wave)) & 3; }
 constexpr int pending_col(int wave) { return (int)(0x3321233012ull >> (4 * wave)) & 3; }
-constexpr bool helper_awaits_pending(int q) { return q == 0; }
 
 }  // namespace kfac

@@ -139,8 +139,7 @@ constexpr int DLD = DB + 4;      // LDS leading dimension (rows of 16-byte piece
 // column, and of the waves that applied a pending panel; write items taken
 constexpr int DIAG_STEPS = 4 * 16 * 4;
 constexpr int DIAG_OPS = 16 * 64;
-constexpr int STRIP_MARKS = 4 * 8 * 8;
-constexpr int DIAG_MARKS = STRIP_MARKS + 16;
+constexpr int DIAG_MARKS = 4 * 8 * 8;
 static_assert(PENDING_WAVES <= 16, "a mark for each");
 constexpr int DIAG_SMEM_BYTES = (2 * DB * DLD + DIAG_STEPS + DIAG_OPS + DIAG_MARKS + 4) * (int)sizeof(float);
 
@@ -474,15 +473,14 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
     }
   }
   // S -= W^T W, split into bf16 parts as in gemm_split.h, half of the reduction after the other in
-  // the LDS of Z, a 32x32 block of S on each of ten waves; no barrier behind it: pending_row etc. say
-  // who may go ahead and who waits for whom.
+  // the LDS of Z, a 32x32 block of S on each of ten waves; no barrier behind it but the one that ends the
+  // first strip: pending_row etc. say why.
   // (Eight of the nine partial products, as good as the fp32 instructions.  The ends of the range do
   // not matter here: W is part of a Cholesky factor, so the sum of the squares of a column is at most the
   // diagonal entry below it.  No element is above 2^64; what one below 2^-108 loses, 2^-133 times the
   // other column, is below the rounding 2^-24 sqrt(S_ii S_jj) of the entry it goes to wherever S_ii is a
   // float32 that is not zero; and halves of the elements keep leading sums finite that are rounded up from
   // near the largest float32.)
-  lds_vf* const pending_marks = (lds_vf*)(marks + STRIP_MARKS);
   if (pending) {
     v16f acc, cor;
 #pragma unroll
@@ -550,9 +548,6 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
         lds_f* const s = at + (8 * (e >> 2) + (e & 3)) * DLD;
         *s = fmaf(-4.f, acc[e], *s);
       }
-      // (the compiler keeps the mark behind the accesses above, and LDS serves a wave's requests in order)
-      asm volatile("" ::: "memory");
-      pending_marks[wave] = 1.f;
     }
   } else {
     __syncthreads();
@@ -681,15 +676,6 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
       auto rows_of = [&](int strip) {
         return Rows{rows_in(strip, i), rows_in(strip, col), marks_in(strip, i), marks_in(strip, col)};
       };
-      // (the waves that applied the pending panel end, and wait for nobody behind its last barrier; a
-      // mark apiece, read by lane.  The block is read and written behind this.)
-      auto settle = [&]() {
-        if (!pending || !helper_awaits_pending(q - 1)) return;
-        const lds_vf* const mark = pending_marks + min(lane, PENDING_WAVES - 1);
-        while (__builtin_amdgcn_ballot_w64(__builtin_bit_cast(int, (float)*mark) == 0) != 0) {
-        }
-        asm volatile("" ::: "memory");
-      };
       auto apply = [&](const v16f& x) {
         lds_f* const at = block_at(col < 4, i, col & 3);
         // (a block of Z below the diagonal starts at zero, and finds it uninitialised)
@@ -699,17 +685,14 @@ __device__ __forceinline__ void diag_block(const MatDesc& m, int p, int* info, f
 #pragma unroll
         for (int e = 0; e < 16; ++e) at[(8 * (e >> 2) + (e & 3)) * DLD] = old[e] - x[e];
       };
-      // (block column 4 + c of Z has rows from strip c on)
-      if (i > 0 && q > 1 && col <= 4) {
+      if (i > 0 && helped_from(col) < q - 1) {
         v16f x, y;
         collect<true>(x, rows_of(q - 1), y, rows_of(q - 2));
         x += y;
-        settle();
         apply(x);
       } else if (i > 0) {
         v16f x;
         collect<false>(x, rows_of(q - 1), x, rows_of(q - 1));
-        settle();
         apply(x);
       }
     }

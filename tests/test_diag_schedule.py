@@ -1,6 +1,7 @@
 """The order of LDS accesses in a diagonal block with a panel pending (csrc/diag_schedule.h, which the kernel
-takes its schedule from): whatever a wave touches in the first strip, the waves that may still be applying
-the panel to it, or reading the panel's parts from under it, are waited for."""
+takes its schedule from): whatever a wave touches in the first strip, no other wave may still be applying
+the panel to it, or reading the panel's parts from under it; and in every strip each block has one wave, which
+finds the rows that it needs there."""
 import os
 import subprocess
 
@@ -20,8 +21,8 @@ int main() {
     for (int nq = q + 1; nq <= 4; ++nq)
       for (int h = 0; h < STRIP_HELPERS; ++h)
         helped_blocks(q, nq, h, [&](int i, int col) { printf("helped %d %d %d %d %d\n", q, nq, h, i, col); });
-    printf("awaits %d %d\n", q, (int)helper_awaits_pending(q));
   }
+  for (int col = 0; col < 8; ++col) printf("from %d %d\n", col, helped_from(col));
   printf("row0 %d\n", PENDING_ROW0);
 }
 '''
@@ -71,35 +72,66 @@ def test_helped_blocks_are_the_rows_further_down(schedule):
             assert got == sorted(want)
 
 
+def touched(schedule, q, nq):
+    """(wave, role, block) of every block of S or Z that a wave reads or writes in strip q of a block of nq strips.
+    Collecting waves read finished rows of the strip only, behind their marks."""
+    for s, w, code in schedule['role']:
+        kind, c = role(code)
+        if s != q:
+            continue
+        if kind == 'lead':
+            yield w, kind, (q, q)
+        elif kind == 'follow' and (c < nq if c < 4 else c - 4 <= q):
+            yield w, kind, (q, c)
+        elif kind == 'help' and q > 0:
+            for r in schedule.get('helped', []):
+                if r[:3] == (q - 1, nq, c) and r[3] == q + 1:
+                    yield w, kind, r[3:]
+
+
 @pytest.mark.parametrize('nq', [1, 2, 3, 4])
 def test_no_access_of_the_first_strip_overtakes_the_pending_panel(schedule, nq):
     owner = {(i, j): w for w, i, j in schedule['pending']}
     row0 = schedule['row0'][0][0]
-    roles = {w: role(code) for s, w, code in schedule['role'] if s == 0}
-    awaits = dict(schedule['awaits'])[0]
-    for w, (kind, c) in roles.items():
-        if kind == 'lead' or (kind == 'follow' and 0 < c < min(nq, 4)):
-            touched = [(0, c)]
-        elif kind == 'follow' and c == 4:
-            touched = [(0, 4)]
-        elif kind == 'help':
-            touched = [r[3:] for r in schedule.get('helped', []) if r[:3] == (0, nq, c)]
-        else:
-            touched = []         # (collecting: finished rows of the strip, behind their marks)
-        for i, col in touched:
-            # whose accesses have to be over: the block's owner's, or, where the panel's parts lie, everybody's
-            before = {owner[i, col]} if col < 4 else set(owner.values()) if 32 * i + 31 >= row0 else set()
-            assert before <= ({w} if not (kind == 'help' and awaits) else set(owner.values()) | {w}), \
-                'wave %d in block (%d, %d)' % (w, i, col)
+    blocks = list(touched(schedule, 0, nq))
+    assert len(blocks) == nq + 1 and all(kind != 'help' for _, kind, _ in blocks)
+    for w, _, (i, col) in blocks:
+        # whose accesses have to be over: the block's owner's, or, where the panel's parts lie, everybody's
+        before = {owner[i, col]} if col < 4 else set(owner.values()) if 32 * i + 31 >= row0 else set()
+        assert before <= {w}, 'wave %d in block (%d, %d)' % (w, i, col)
+
+
+@pytest.mark.parametrize('nq', [1, 2, 3, 4])
+def test_helpers_take_what_the_strips_above_give_to_the_next_one(schedule, nq):
+    """A helper of strip q: one block at most, of block row q + 1, which nobody else touches then; the strips that
+    it takes from are above q, at most two, and all that give something to the block but strip q, which the
+    block's own wave collects."""
+    first = dict(schedule['from'])
+    for q in range(nq):
+        blocks = list(touched(schedule, q, nq))
+        assert len(set(b for _, _, b in blocks)) == len(blocks) == len(set(w for w, _, _ in blocks))
+        helped = sorted(b for _, kind, b in blocks if kind == 'help')
+        want = [(q + 1, j) for j in list(range(q + 1, nq)) + [4 + c for c in range(q)]] if 0 < q < nq - 1 else []
+        assert helped == want
+        for i, col in helped:
+            gives = [s for s in range(i) if col < 4 or s >= col - 4]
+            assert gives == list(range(first[col], q + 1)) and 1 <= q - first[col] <= 2
+
+
+def test_every_row_is_written_once(schedule):
+    """Rows of strip q - 1, in sixteen pieces: in strip q the collecting waves have the pieces 4 (c - q - 1) + (0 ... 3);
+    strip 3 has no such waves, but some without a block."""
+    for q in (1, 2):
+        columns = [role(code)[1] for s, _, code in schedule['role'] if s == q and role(code)[0] == 'collect']
+        assert sorted(4 * (c - q - 1) + k for c in columns for k in range(4)) == list(range(16))
+    last = [role(code)[0] for s, _, code in schedule['role'] if s == 3]
+    assert 'collect' not in last and any(kind in ('help', 'none') for kind in last)
 
 
 def test_the_kernel_takes_its_schedule_from_the_header():
     with open(os.path.join(CSRC, 'inverse.hip')) as f:
         text = f.read()
     block = text[text.index('void diag_block('):text.index('void potrf_diag_kernel')]
-    for name in ('STRIP_ROLES', 'helped_blocks', 'pending_row', 'pending_col', 'PENDING_WAVES', 'PENDING_ROW0',
-                 'helper_awaits_pending'):
+    for name in ('STRIP_ROLES', 'helped_blocks', 'helped_from', 'pending_row', 'pending_col', 'PENDING_WAVES',
+                 'PENDING_ROW0'):
         assert name in block
-    # marked behind the last access, awaited in front of the first one of either way through a helper's blocks
-    assert block.index('pending_marks[wave] = 1.f') > block.index('*s = fmaf(-4.f, acc[e], *s)')
-    assert block.count('settle();\n        apply(') == 2
